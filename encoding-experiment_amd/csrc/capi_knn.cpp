@@ -51,15 +51,9 @@ void run_scores(larql_hip_ctx* c, const KnnPlan& p, size_t n_layers, const float
     if (nq > 0x7FFFFFFF / static_cast<size_t>(p.K)) fail(LARQL_HIP_ERR_INVALID, "gate KNN: too many queries");
     const int Q = static_cast<int>(nq);
     if (p.format == LARQL_F32) {
-        // rows of the device gate are f32_row_stride(K) apart; queries are padded to match
-        const size_t Kp = larql::f32_row_stride(static_cast<size_t>(p.K));
-        const float* X = queries;
-        if (Kp != static_cast<size_t>(p.K)) {
-            float* xp = static_cast<float*>(larql::ensure(c, c->knn_xpad, nq * Kp * sizeof(float)));
-            larql::launch_pad_rows_f32(queries, xp, nq, static_cast<size_t>(p.K), Kp, 0.0f, s);
-            X = xp;
-        }
-        larql::launch_gate_scores_f32(p.a, static_cast<int>(n_layers), X, scores, p.F, static_cast<int>(Kp), Q, s);
+        const size_t nws = larql::gate_scores_f32_ws_floats(p.K, Q);
+        float* ws = nws ? static_cast<float*>(larql::ensure(c, c->knn_xpad, nws * sizeof(float))) : nullptr;
+        larql::launch_gate_scores_f32(p.a, static_cast<int>(n_layers), queries, ws, scores, p.F, p.K, Q, s);
     } else {
         int8_t* q8 = static_cast<int8_t*>(larql::ensure(c, c->knn_q8, nq * p.K));
         float* q8s = static_cast<float*>(larql::ensure(c, c->knn_q8s, nq * (p.K / 32) * sizeof(float)));

@@ -14,8 +14,12 @@ struct KnnLayers {
 };
 
 // S[l][q][f] = G_l[f, :] . X[q, :], one fma chain over k from +0 per element.
-void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* S, int F, int K, int Q,
+// Gate rows lie f32_row_stride(K) floats apart, padded with -0 (a padded term leaves a
+// chain as it is); X [Q][K] is dense.  ws: gate_scores_f32_ws_floats(K, Q) floats (the
+// queries k-major; none for one query whose rows need no padding).
+void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, float* S, int F, int K, int Q,
                             hipStream_t s);
+size_t gate_scores_f32_ws_floats(int K, int Q);
 // S[l][q][f] = sum_b (float)isum * (f16(scale) * XS[q][b]) in block order (Q4_0 x Q8).
 // XA / XSP: work buffers of q4_xa_bytes / q4_xsp_bytes (the queries as MFMA operands).
 void launch_gate_scores_q4(const KnnLayers& nibbles, const KnnLayers& scales, int n_layers, const int8_t* X8,

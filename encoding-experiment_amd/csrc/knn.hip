@@ -26,43 +26,184 @@ namespace {
 
 constexpr int kThreads = 256;
 
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+
 // ── f32 scores ─────────────────────────────────────────────────────────────
-// Workgroup tile: 64 features x 256 queries; thread tile 8 queries x 8 features
-// (64 accumulators).  K advances in LDS stages of 16, double-buffered, with the
-// next stage's global loads in registers while the current stage is consumed.
+// A lane owns NF features and walks k in order, so a score is one fma chain held in one
+// register; a wave serves QW queries, whose values at one k come as scalar operands
+// (XT[block][k][query], read through the scalar cache: one v_fmac_f32 v, s, v per term and no LDS
+// traffic for the queries).  The gate rows are staged by global_load_lds: 64 NF rows x 32 k
+// per stage, a ring of ND stages, whole 128-byte lines per row, no registers in flight.
+// Chunk j (4 k) of row r sits in slot j ^ (r & 7) of the row's eight, so eight consecutive
+// lanes reading the same chunk of their rows touch eight different bank groups.  The NW
+// waves of a workgroup share the staged rows and serve QW queries each.
+// Bound: HBM for few queries (34 x [10240 x 2560], 3.57 GB: 587 us for one query, 6.1 TB/s,
+// against 4.8 ms in a 64 x 256 tile that computes 256 queries whatever their number), the
+// scalar loads' latency and fp32 VALU issue for more: 636 us for 2, 838 for 8, 1.22 ms for 32,
+// 1.86 for 64, 3.46 for 128.
+constexpr int kF32Stage = 32;
+
+// A query block of a k: QW consecutive floats at a wave-uniform address, read with scalar loads.
+typedef const float __attribute__((address_space(4))) * scalar_f32_ptr;
+
+// XT[b][k][QW] = the QW queries of block b at k: X[QW b + i][k] for existing queries and
+// k < K, else +0 (b < Qp / QW, k < Kp).
+__global__ void queries_t_kernel(const float* __restrict__ X, float* __restrict__ XT, int Q, int K, int Kp, int Qp,
+                                 int qw) {
+    __shared__ float t[32][33];
+    const int nk = (Kp + 31) / 32, k0 = 32 * static_cast<int>(blockIdx.x % nk), q0 = 32 * static_cast<int>(blockIdx.x / nk);
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int q = q0 + ty + 8 * i, k = k0 + tx;
+        t[ty + 8 * i][tx] = (q < Q && k < K) ? X[static_cast<size_t>(q) * K + k] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int k = k0 + ty + 8 * i, q = q0 + tx;
+        if (k < Kp && q < Qp) XT[(static_cast<size_t>(q / qw) * Kp + k) * qw + q % qw] = t[tx][ty + 8 * i];
+    }
+}
+
+// Four float4 of a lane's staged row (chunks 4 HALF .. 4 HALF + 3), read and waited for in
+// one block: the compiler does not see the loads that fill the ring, so its own LDS reads
+// would wait for every one of them.
+template <int HALF>
+__device__ __forceinline__ void ring_read4(uint32_t a, floatx4_t (&v)[4]) {
+    const uint32_t a0 = a ^ (16u * (4 * HALF)), a1 = a ^ (16u * (4 * HALF + 1)), a2 = a ^ (16u * (4 * HALF + 2)),
+                   a3 = a ^ (16u * (4 * HALF + 3));
+    asm volatile(
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+        : "v"(a0), "v"(a1), "v"(a2), "v"(a3)
+        : "memory");
+}
+
+// At most N vector memory operations of the wave still in flight.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int QW, int NF, int NW, int ND>
+__global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, const float* __restrict__ XT,
+                                                                  float* __restrict__ S, int F, int K, int Q) {
+    constexpr int kRows = 64 * NF, kPer = 8 * NF / NW;  // rows per stage; load instructions per wave and stage
+    static_assert(kPer * NW == 8 * NF, "the waves split a stage's loads evenly");
+    __shared__ __align__(128) float4 ring[ND][kRows * 8];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int f0 = blockIdx.x * kRows, q0 = (blockIdx.y * NW + wave) * QW, l = blockIdx.z;
+    const float* __restrict__ G = static_cast<const float*>(g.p[l]);
+    // load instruction i of the wave: rows 8 (kPer wave + i) .. + 7, eight lanes a row
+    const float* gp[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; i++) {
+        const int r = 8 * (kPer * wave + i) + (lane >> 3);
+        gp[i] = G + static_cast<size_t>(min(f0 + r, F - 1)) * K;
+    }
+    const int chunk = 4 * ((lane & 7) ^ (lane >> 3));
+    auto gload = [&](int st, int slot) __attribute__((always_inline)) {
+        // (a chunk past the row re-reads its last one: staged, never used)
+        const int k = min(kF32Stage * st + chunk, K - 4);
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)(gp[i] + k),
+                (__attribute__((address_space(3))) void*)&ring[slot][64 * (kPer * wave + i)], 16, 0, 0);
+    };
+    const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) void*)&ring[0][0]));
+    const uint32_t mine = ring0 + 128u * lane + 16u * (lane & 7);
+    float acc[NF][QW];
+#pragma unroll
+    for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int q = 0; q < QW; q++) acc[f][q] = 0.f;
+
+    const int ns = (K + kF32Stage - 1) / kF32Stage, last = ns - 1;
+#pragma unroll
+    for (int d = 0; d < ND - 1; d++) gload(min(d, last), d);
+    int slot = 0;
+    const scalar_f32_ptr xt = (scalar_f32_ptr)(reinterpret_cast<uintptr_t>(XT) + sizeof(float) * (static_cast<size_t>(q0) * K));
+    // 16 k of the stage in slot `slot`
+    auto half = [&](int k0, auto hc) __attribute__((always_inline)) {
+        constexpr int H = decltype(hc)::value;
+        floatx4_t v[NF][4];
+#pragma unroll
+        for (int f = 0; f < NF; f++)
+            ring_read4<H>(mine + static_cast<uint32_t>(slot) * (kRows * 128u) + 8192u * f, v[f]);
+        scalar_f32_ptr x = xt + static_cast<size_t>(k0 + 16 * H) * QW;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+#pragma unroll
+                for (int q = 0; q < QW; q++) {
+                    const float xv = x[(4 * j + e) * QW + q];
+#pragma unroll
+                    for (int f = 0; f < NF; f++) acc[f][q] = fmaf(v[f][j][e], xv, acc[f][q]);
+                }
+            }
+    };
+    for (int st = 0; st < ns; st++) {
+        // stage st has landed (this wave's loads, then everyone's), and every wave is past
+        // stage st - 1, whose slot the next loads overwrite
+        wait_vmcnt<kPer * (ND - 2)>();
+        if constexpr (NW > 1) asm volatile("s_barrier" ::: "memory");
+        gload(min(st + ND - 1, last), slot == 0 ? ND - 1 : slot - 1);
+        half(kF32Stage * st, std::integral_constant<int, 0>{});
+        if (kF32Stage * st + 16 < K) half(kF32Stage * st, std::integral_constant<int, 1>{});
+        slot = slot + 1 == ND ? 0 : slot + 1;
+    }
+    wait_vmcnt<0>();  // nothing may land in LDS after the workgroup has ended
+    float* Sl = S + static_cast<size_t>(l) * Q * F;
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const int fo = f0 + 64 * f + lane;
+        if (fo >= F) continue;
+#pragma unroll
+        for (int q = 0; q < QW; q++)
+            if (q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + fo] = acc[f][q];
+    }
+}
+
+// More than 128 queries: the chains are bound by fp32 VALU issue and the scalar operands of the
+// kernel above do not arrive fast enough (7.4 ms for 256), so the queries go through LDS as
+// well: 5.33 ms for 256 at 34 x [10240 x 2560], 85 TFLOP/s (5.51 with a thread's eight queries
+// adjacent and the queries transposed on their way into LDS).  A thread tile of 8 features x 16
+// queries took 5.82 ms (two waves per SIMD).
+// Workgroup tile: 64 features x 256 queries, thread tile 8 x 8 (64 accumulators); K in
+// double-buffered LDS stages of 16, the next stage's global loads in registers meanwhile.  A
+// thread's queries are two groups of four, 128 apart, so that a wave's query reads are
+// contiguous.
 constexpr int kF32TileF = 64, kF32TileQ = 256, kF32Ks = 16;
 
-__global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_kernel(KnnLayers g, const float* __restrict__ X,
-                                                                   float* __restrict__ S, int F, int K, int Q) {
+__global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLayers g, const float* __restrict__ XT,
+                                                                        float* __restrict__ S, int F, int K, int Q) {
     __shared__ float Gs[2][kF32Ks][kF32TileF];
     __shared__ float Xs[2][kF32Ks][kF32TileQ];
     const int l = blockIdx.z;
     const float* __restrict__ G = static_cast<const float*>(g.p[l]);
     const int f0 = blockIdx.x * kF32TileF, q0 = blockIdx.y * kF32TileQ;
     const int tid = threadIdx.x;
-    const int tq = tid & 31, tf = tid >> 5;  // queries q0 + 8 tq .., features f0 + 8 tf ..
-    // global -> LDS: G row f0 + (tid & 63), k-quarter tid >> 6; X row q0 + tid, all 16 k
-    const int lf = tid & 63, lk = 4 * (tid >> 6);
+    const int tq = tid & 31, tf = tid >> 5;  // queries q0 + 128 i + 4 tq .., features f0 + 8 tf ..
+    // global -> LDS: G row f0 + (tid & 63), k-quarter tid >> 6; XT rows (tid >> 6) + 4 i
+    const int lf = tid & 63, lk = 4 * (tid >> 6), xq = 4 * (tid & 63), xk = tid >> 6;
     const float* gp = G + static_cast<size_t>(min(f0 + lf, F - 1)) * K + lk;
-    const float* xp = X + static_cast<size_t>(min(q0 + tid, Q - 1)) * K;
-    float4 gr, xr[4];
+    const float* xp = XT + static_cast<size_t>(q0) * K + static_cast<size_t>(xk) * kF32TileQ + xq;
+    floatx4_t gr, xr[4];
     auto gload = [&](int k0) __attribute__((always_inline)) {
-        gr = *reinterpret_cast<const float4*>(gp + k0);
+        gr = *reinterpret_cast<const floatx4_t*>(gp + k0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) xr[i] = *reinterpret_cast<const float4*>(xp + k0 + 4 * i);
+        for (int i = 0; i < 4; i++) xr[i] = *reinterpret_cast<const floatx4_t*>(xp + static_cast<size_t>(k0 + 4 * i) * kF32TileQ);
     };
     auto lstore = [&](int b) __attribute__((always_inline)) {
-        Gs[b][lk + 0][lf] = gr.x;
-        Gs[b][lk + 1][lf] = gr.y;
-        Gs[b][lk + 2][lf] = gr.z;
-        Gs[b][lk + 3][lf] = gr.w;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            Xs[b][4 * i + 0][tid] = xr[i].x;
-            Xs[b][4 * i + 1][tid] = xr[i].y;
-            Xs[b][4 * i + 2][tid] = xr[i].z;
-            Xs[b][4 * i + 3][tid] = xr[i].w;
-        }
+        for (int i = 0; i < 4; i++) Gs[b][lk + i][lf] = gr[i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) *reinterpret_cast<floatx4_t*>(&Xs[b][xk + 4 * i][xq]) = xr[i];
     };
     float acc[8][8];
 #pragma unroll
@@ -76,19 +217,18 @@ __global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_kernel(KnnLayers 
     __syncthreads();
     for (int s = 0; s < nk; s++) {
         const int b = s & 1;
-        if (s + 1 < nk) gload((s + 1) * kF32Ks);
+        gload(min(s + 1, nk - 1) * kF32Ks);
 #pragma unroll 2
         for (int k = 0; k < kF32Ks; k++) {
-            const float4 xa = *reinterpret_cast<const float4*>(&Xs[b][k][tq * 8]);
-            const float4 xb = *reinterpret_cast<const float4*>(&Xs[b][k][tq * 8 + 4]);
-            const float4 ga = *reinterpret_cast<const float4*>(&Gs[b][k][tf * 8]);
-            const float4 gb = *reinterpret_cast<const float4*>(&Gs[b][k][tf * 8 + 4]);
-            const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-            const float gv[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+            floatx4_t xv[2], gv[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) xv[i] = *reinterpret_cast<const floatx4_t*>(&Xs[b][k][128 * i + 4 * tq]);
+#pragma unroll
+            for (int i = 0; i < 2; i++) gv[i] = *reinterpret_cast<const floatx4_t*>(&Gs[b][k][8 * tf + 4 * i]);
 #pragma unroll
             for (int i = 0; i < 8; i++)
 #pragma unroll
-                for (int j = 0; j < 8; j++) acc[i][j] = fmaf(gv[j], xv[i], acc[i][j]);
+                for (int j = 0; j < 8; j++) acc[i][j] = fmaf(gv[j >> 2][j & 3], xv[i >> 2][i & 3], acc[i][j]);
         }
         // buffer b ^ 1 was last read in stage s - 1, before that stage's barrier
         if (s + 1 < nk) lstore(b ^ 1);
@@ -97,11 +237,11 @@ __global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_kernel(KnnLayers 
     float* Sl = S + static_cast<size_t>(l) * Q * F;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int q = q0 + tq * 8 + i;
+        const int q = q0 + 128 * (i >> 2) + 4 * tq + (i & 3);
         if (q >= Q) continue;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const int f = f0 + tf * 8 + j;
+            const int f = f0 + 8 * tf + j;
             if (f < F) Sl[static_cast<size_t>(q) * F + f] = acc[i][j];
         }
     }
@@ -845,11 +985,74 @@ __global__ __launch_bounds__(64 * kWWaves) void topk_wave_kernel(const float* __
 
 }  // namespace
 
-void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* S, int F, int K, int Q,
+// Queries per wave (qw) and waves per workgroup (nw) of a walk of Q queries.  Few queries per
+// wave and more waves: a wave waits for its scalar loads every 16 k, and only other waves can
+// issue meanwhile (8 queries of one wave 1.78 ms, of four waves 0.84; 32 of four waves 1.87,
+// of eight 1.22; 64 of four waves 3.1, of eight 1.86).  Above 128 the tile kernel: 128 queries
+// cost 3.46 ms here and 4.9 there, 256 7.4 ms here and 5.3 there.
+namespace {
+struct F32Plan {
+    int qw, nw;
+};
+F32Plan f32_plan(int Q) {
+    if (Q <= 2) return {Q, 1};
+    if (Q <= 8) return {2, Q <= 4 ? 2 : 4};
+    if (Q <= 32) return {4, Q <= 16 ? 4 : 8};
+    if (Q <= 128) return {Q <= 64 ? 8 : 16, 8};
+    return {kF32TileQ, 1};  // the tile kernel
+}
+int f32_qp(int Q) {
+    const F32Plan p = f32_plan(Q);
+    const int b = p.qw * p.nw;
+    return (Q + b - 1) / b * b;
+}
+}  // namespace
+
+size_t gate_scores_f32_ws_floats(int K, int Q) {
+    const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
+    return Q == 1 && Kp == K ? 0 : static_cast<size_t>(Kp) * f32_qp(Q);
+}
+
+void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, float* S, int F, int K, int Q,
                             hipStream_t s) {
-    if (K % kF32Ks) fail(LARQL_HIP_ERR_INVALID, "gate scores: hidden must be a multiple of 16");
-    const dim3 grid((F + kF32TileF - 1) / kF32TileF, (Q + kF32TileQ - 1) / kF32TileQ, n_layers);
-    gate_scores_f32_kernel<<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, K, Q);
+    const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
+    const F32Plan p = f32_plan(Q);
+    const int Qp = f32_qp(Q);
+    const float* XT = X;  // one query of a whole row: as it lies
+    if (gate_scores_f32_ws_floats(K, Q)) {
+        if (!ws) fail(LARQL_HIP_ERR_INVALID, "gate scores: no workspace for the queries");
+        queries_t_kernel<<<dim3(((Kp + 31) / 32) * ((Qp + 31) / 32)), dim3(256), 0, s>>>(X, ws, Q, K, Kp, Qp, p.qw);
+        LARQL_HIP_CHECK(hipGetLastError());
+        XT = ws;
+    }
+    auto go = [&](auto qw, auto nf, auto nw, auto nd) {
+        constexpr int QW = decltype(qw)::value, NF = decltype(nf)::value, NW = decltype(nw)::value,
+                      ND = decltype(nd)::value;
+        const dim3 grid((F + 64 * NF - 1) / (64 * NF), Qp / (QW * NW), n_layers);
+        gate_scores_f32_kernel<QW, NF, NW, ND><<<grid, dim3(64 * NW), 0, s>>>(g, XT, S, F, Kp, Q);
+    };
+    using std::integral_constant;
+    const integral_constant<int, 1> c1;
+    const integral_constant<int, 2> c2;
+    const integral_constant<int, 4> c4;
+    const integral_constant<int, 8> c8;
+    const integral_constant<int, 16> c16;
+    if (p.qw == kF32TileQ) {
+        const dim3 grid((F + kF32TileF - 1) / kF32TileF, Qp / kF32TileQ, n_layers);
+        gate_scores_f32_tile_kernel<<<grid, dim3(kThreads), 0, s>>>(g, XT, S, F, Kp, Q);
+    } else if (p.nw == 1) {
+        if (p.qw == 1) go(c1, c1, c1, c4);
+        else go(c2, c1, c1, c4);
+    } else if (p.qw == 2) {
+        if (p.nw == 2) go(c2, c1, c2, c4);
+        else go(c2, c1, c4, c4);
+    } else if (p.qw == 4) {
+        if (p.nw == 4) go(c4, c1, c4, c4);
+        else go(c4, c1, c8, c4);
+    } else {
+        if (p.qw == 8) go(c8, c1, c8, c4);
+        else go(c16, c1, c8, c4);
+    }
     LARQL_HIP_CHECK(hipGetLastError());
 }
 

@@ -70,6 +70,30 @@ def test_gate_scores_f32_bit_exact(hip):
         hip.release_weight(h)
 
 
+@pytest.mark.parametrize("nq", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("features,hidden", [(1, 16), (65, 48), (130, 30), (64, 100)])
+def test_gate_scores_f32_query_counts_bit_exact(hip, nq, features, hidden):
+    """Every split of the queries over waves and workgroups (their edges), rows whose last stage
+    of 32 holds 16 or fewer real k, padded rows, partial feature blocks: the oracle's chain bit
+    for bit, over two layers."""
+    torch = pytest.importorskip("torch")
+    print(f"[scores f32] F={features} K={hidden} nq={nq}", flush=True)
+    gates = [oracle.gauss(60 + l, features * hidden, 0.0, 0.02).reshape(features, hidden) for l in range(2)]
+    queries = oracle.gauss(62, nq * hidden).reshape(nq, hidden)
+    hs = [hip.register_weight(larql_hip.F32, g, features, hidden) for g in gates]
+    try:
+        dq = torch.from_numpy(queries).cuda()
+        ds = torch.empty(2 * nq * features, device="cuda", dtype=torch.float32)
+        hip.gate_scores_dev(hs, dq, nq, ds)
+        hip.synchronize()
+        got = ds.cpu().numpy().reshape(2, nq, features)
+        ref = np.stack([[oracle.gate_scores_f32(g, q, features, hidden) for q in queries] for g in gates])
+        np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
+    finally:
+        for h in hs:
+            hip.release_weight(h)
+
+
 @pytest.mark.parametrize("features,hidden,nq,k", [(10240, 2560, 6, 32), (1000, 2560, 130, 17), (64, 64, 2, 64)])
 def test_gate_knn_q4_bit_exact(hip, features, hidden, nq, k):
     print(f"[knn q4] F={features} K={hidden} nq={nq} k={k}", flush=True)
