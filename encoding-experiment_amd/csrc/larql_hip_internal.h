@@ -287,6 +287,12 @@ struct GemmSplits {
 void launch_q4k_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
                          hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr,
                          GemmSplits* defer = nullptr);
+// Q4_0 or Q8_0 weights (cols a multiple of 128) x any number of Q8 rows, block order as the
+// matvecs (gemm_int.hip); w2 / out2: a second weight of the same format and shape in the same
+// launch.  Output rows ldo floats apart (0: w.rows).
+bool int_gemm_takes(const DevWeight& w);
+void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
+                     float* out2, size_t m, size_t ldo, hipStream_t s);
 void launch_q4_0_matvec(const DevWeight& w, const int8_t* q8x, const float* q8s, float* out,
                         size_t m, hipStream_t s);
 // Two Q4_0 matrices of one shape times the same Q8 rows, in one launch per pass.

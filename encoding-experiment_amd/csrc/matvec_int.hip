@@ -874,10 +874,20 @@ void launch_int_mv_batched(const DevWeight& w, const int8_t* q8x, const float* q
     }
 }
 
+// One launch of the int GEMM instead of passes of up to 8 rows (a pass streams the weights
+// again).  Weights of fewer than 8192 rows are worth it above 16 activation rows: their few
+// workgroups leave one wave per SIMD, and a wave's chain of blocks then takes as long as two
+// passes (Q8_0 [4096 x 4096]: 16 rows 15.8 us in two passes, 20.1 in the GEMM; 64 rows 63.5
+// against 20.0; Q4_0 [14336 x 4096]: 9 rows 20.8 against 20.2, 128 rows 204 against 65 us).
+bool int_gemm_pays(const DevWeight& w, size_t m) {
+    return m > (w.rows >= 8192 ? 8u : 16u) && int_gemm_takes(w) && m <= 0x7FFFFFFF / w.cols;
+}
+
 }  // namespace
 
 void launch_q4_0_matvec(const DevWeight& w, const int8_t* q8x, const float* q8s, float* out, size_t m,
                         hipStream_t s) {
+    if (int_gemm_pays(w, m)) return launch_int_gemm(w, nullptr, q8x, q8s, out, nullptr, m, 0, s);
     launch_int_mv_batched<LARQL_Q4_0>(w, q8x, q8s, out, m, s);
 }
 
@@ -885,6 +895,7 @@ void launch_q4_0_matvec_pair(const DevWeight& w1, const DevWeight& w2, const int
                              float* out1, float* out2, size_t m, hipStream_t s) {
     if (w1.format != LARQL_Q4_0 || w2.format != LARQL_Q4_0 || w1.rows != w2.rows || w1.cols != w2.cols)
         fail(LARQL_HIP_ERR_INVALID, "q4_0 matvec pair: two Q4_0 matrices of one shape");
+    if (int_gemm_pays(w1, m)) return launch_int_gemm(w1, &w2, q8x, q8s, out1, out2, m, 0, s);
     launch_int_mv_batched<LARQL_Q4_0>(w1, q8x, q8s, out1, m, s, &w2, out2);
 }
 
@@ -987,6 +998,7 @@ void launch_q4_0_f32_matvec(const DevWeight& w, const float* x, float* out, hipS
 void launch_q8_matvec(const DevWeight& w, const int8_t* q8x, const float* q8s, float* out, size_t m,
                       hipStream_t s) {
     const int nb = static_cast<int>(w.cols / 32);
+    if (int_gemm_pays(w, m)) return launch_int_gemm(w, nullptr, q8x, q8s, out, nullptr, m, 0, s);
     const bool mfma_ok = nb % 2 == 0 && mfma_lds_bytes(nb) <= kLdsLimit && w.rows * w.cols < (size_t{1} << 31);
     if (m <= 4 || !mfma_ok) {
         launch_int_mv_batched<LARQL_Q8_0>(w, q8x, q8s, out, m, s);

@@ -210,6 +210,39 @@ def test_q4_0_matvec_batched_dev_bit_exact(hip, m, rows, cols):
         assert np.array_equal(got[i].view(np.uint32), ref.view(np.uint32)), i
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,rows,cols", [(17, 64, 128), (18, 70, 256), (32, 1, 384), (33, 130, 640), (48, 200, 1152),
+                                         (65, 129, 512), (130, 300, 2560), (9, 8200, 128), (16, 8250, 256)])
+def test_int_gemm_bit_exact(hip, fmt, m, rows, cols):
+    """Many activation rows through the device entry point: every row equals the single-row
+    block order bit for bit.  Token counts at the edges of 16-token tiles and of one to four
+    tiles per workgroup, row counts at the edges of the 16-row tiles and of one or two tiles per
+    wave (rows from 8192 on: from 9 tokens), 1 .. 20 stages of four blocks (odd counts)."""
+    torch = pytest.importorskip("torch")
+    print(f"[int gemm] {fmt} m={m} rows={rows} cols={cols}", flush=True)
+    w = oracle.gauss(530 + rows, rows * cols, 0.0, 0.02)
+    xs = [oracle.quantize_to_q8(oracle.gauss(630 + i, cols)) for i in range(m)]
+    if fmt == "q4_0":
+        q = oracle.quantize_q4_0(w)
+        h = hip.register_weight(larql_hip.Q4_0, q, rows, cols)
+        ref = lambda a, b: oracle.q4_0_matvec_blockint(q, a, b, rows, cols)  # noqa: E731
+    else:
+        q, sc = oracle.quantize_weights_q8(w, rows, cols)
+        h = hip.register_weight(larql_hip.Q8_0, q, rows, cols, sc)
+        ref = lambda a, b: oracle.q8_matvec(q, sc, a, b, rows, cols)  # noqa: E731
+    try:
+        dq = torch.from_numpy(np.concatenate([a for a, _ in xs])).cuda()
+        ds = torch.from_numpy(np.concatenate([b for _, b in xs])).cuda()
+        dy = torch.full((m * rows,), 7.0, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dq, dy, m=m, x_scales=ds)
+        hip.synchronize()
+        got = dy.cpu().numpy().reshape(m, rows)
+        for i, (a, b) in enumerate(xs):
+            assert np.array_equal(got[i].view(np.uint32), ref(a, b).view(np.uint32)), i
+    finally:
+        hip.release_weight(h)
+
+
 def test_quantize_to_q8_bit_exact(hip):
     x = oracle.gauss(901, 32 * 1000)
     x[:32] = 0.0                                     # zero block -> scale 0, q 0
