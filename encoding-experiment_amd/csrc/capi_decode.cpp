@@ -781,72 +781,169 @@ extern "C" int larql_hip_decode_token(larql_hip_ctx* c, const larql_pipeline_lay
     });
 }
 
-// The batched prompt pass takes layers with gate/up fused in Q4_K and every other
-// projection Q4_K or Q6_K (Q4_K and Q4_K_M files); others run position by position.
-static bool prompt_batchable(const larql_hip_model* m) {
-    auto ok = [](const larql::DevWeight& w) { return w.format == LARQL_Q4_K || w.format == LARQL_Q6_K; };
-    for (const LayerDev& L : m->layers) {
-        if (L.split_gu || L.gateup.format != LARQL_Q4_K || !ok(L.wo) || !ok(L.down)) return false;
-        if (L.split_qkv ? !(ok(L.wq) && ok(L.wk) && ok(L.wv)) : !ok(L.qkv)) return false;
-    }
-    return true;
+// A projection the batched prompt pass runs over all positions: the Q8-input formats on the
+// ordered int GEMM, the others (and Q4_0 as the down projection) on the f32-accuracy GEMM.
+static bool batched_proj(const DevWeight& w, bool is_down) {
+    return takes_q8(w, is_down) ? larql::int_gemm_takes(w) : larql::gemm_f32_takes(w);
 }
 
-// One projection of all M positions (X rows ldx = w.cols apart) -> Y rows ldy apart: the
-// f32-accuracy GEMM, Q4_K or Q6_K.
-static void prompt_proj(const larql::DevWeight& w, const float* X, size_t ldx, float* Y, size_t ldy, size_t M,
-                        float* spl, size_t split_n, hipStream_t s, const larql::GemmRowStats* pre = nullptr,
-                        larql::GemmSplits* defer = nullptr) {
-    if (ldx != w.cols) fail(LARQL_HIP_ERR_INVALID, "prompt pass: input rows do not match the weight");
-    larql::launch_q4k_gemm_f32(w, X, Y, M, spl, split_n, s, ldy, pre, defer);
+// Floats of the batched prompt pass's work buffer, in the order of its regions.
+namespace {
+size_t a4(size_t n) { return (n + 3) & ~size_t{3}; }
+
+struct PromptLayout {
+    size_t wide, gw, rows, split, st_h, st_q, st_a, xp, q8, q8s;
+    size_t total() const { return rows + a4(split) + st_h + st_q + st_a + xp + q8 + q8s; }
+};
+
+PromptLayout prompt_layout(const larql_hip_model* m, size_t M) {
+    PromptLayout p{};
+    const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim;
+    p.wide = std::max({hidden, qmax, inter});
+    p.gw = std::max(hidden, 2 * inter);
+    size_t part_n = 0;  // partials of attention shapes without the one-pass prompt kernel
+    bool any_int = false;
+    // GEMM workspace: K-split partial products (and operands it packs itself)
+    auto need = [&](const DevWeight& w, bool is_down) {
+        if (takes_q8(w, is_down)) any_int = true;
+        else p.split = std::max(p.split, larql::gemm_f32_part_floats(w, M));
+    };
+    for (const LayerDev& L : m->layers) {
+        if (!larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd))
+            part_n = m->part_per_split * larql::attn_prompt_splits(1, static_cast<int>(M), 0) * M;
+        if (L.split_qkv) need(L.wq, false), need(L.wk, false), need(L.wv, false);
+        else need(L.qkv, false);
+        need(L.wo, false), need(L.down, true);
+        if (L.split_gu) need(L.gate, false), need(L.up, false);
+        else need(L.gateup, false);
+    }
+    p.rows = a4(2 * M * hidden + M * p.wide + M * m->qkv_dim + M * qmax + M * p.gw + M * inter + part_n);
+    // row statistics of the normed hidden rows, of the attention rows and of the activation
+    // rows (separate regions: a producer may still read the previous GEMM's partial products),
+    // the packed operands and the Q8 codes of one input
+    p.st_h = a4(larql::gemm_row_stats_floats(M, hidden));
+    p.st_q = a4(larql::gemm_row_stats_floats(M, qmax));
+    p.st_a = a4(larql::gemm_row_stats_floats(M, inter));
+    p.xp = larql::gemm_x_pack_floats(M, p.wide);
+    if (any_int) {
+        p.q8 = a4((M * p.wide + 3) / 4);
+        p.q8s = a4(M * (p.wide / 32));
+    }
+    return p;
 }
+}  // namespace
+
+// The batched prompt pass takes layers whose projections are Q4_K, Q6_K, Q8_0 or Q4_0, with
+// gate/up fused in Q4_K or both Q8-input (Q4_K, Q4_K_M and Q8_0 / Q4_0 files); others run
+// position by position.  So do Q8_0 / Q4_0 prompts that position by position need no more
+// than a step's buffers and batched would not fit: past 31-bit row blocks, attention shapes that
+// hold every query's partials at more than 4096 positions, or a work buffer beyond the free memory.
+static bool prompt_batchable(const larql_hip_model* m, size_t M) {
+    bool any_int = false;
+    auto ok = [&](const DevWeight& w, bool is_down) {
+        any_int |= w.format == LARQL_Q4_0 || w.format == LARQL_Q8_0;
+        return batched_proj(w, is_down);
+    };
+    bool one_pass = true;
+    for (const LayerDev& L : m->layers) {
+        if (!ok(L.wo, false) || !ok(L.down, true)) return false;
+        if (L.split_gu ? !(takes_q8(L.gate, false) && takes_q8(L.up, false) && ok(L.gate, false) && ok(L.up, false))
+                       : L.gateup.format != LARQL_Q4_K)
+            return false;
+        if (L.split_qkv ? !(ok(L.wq, false) && ok(L.wk, false) && ok(L.wv, false)) : !ok(L.qkv, false)) return false;
+        one_pass &= larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd);
+    }
+    if (!any_int) return true;
+    if (M > 0x7FFFFFFF / std::max({m->hidden, 2 * m->inter, m->qkv_dim}) || (!one_pass && M > 4096)) return false;
+    const size_t bytes = prompt_layout(m, M).total() * sizeof(float);
+    if (bytes <= m->prompt.n || bytes <= (size_t{1} << 30)) return true;
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return bytes + (size_t{1} << 30) <= free_b;
+}
+
+namespace {
+
+// The prompt pass's projections of M positions: the GEMM workspaces, and which form of the
+// current input rows they hold (packed operands and row statistics, or Q8 codes).
+struct PromptProj {
+    size_t M;
+    float* spl;
+    size_t split_n;
+    float* xp;     // packed operands of the current input
+    int8_t* q8;    // its quantize_to_q8 codes and scales
+    float* q8s;
+    hipStream_t s;
+    const float* packed = nullptr;
+    const float* quantized = nullptr;
+
+    // A new input row block at X (the same buffer with other contents included).
+    void input() { packed = quantized = nullptr; }
+    void pack(const float* X, size_t K, larql::GemmRowStats& st, bool have_stats) {
+        st.xp = xp;
+        if (packed == X) return;
+        if (!have_stats) larql::launch_gemm_row_stats(X, M, K, st, s);
+        larql::launch_gemm_x_pack(X, M, K, st, s);
+        packed = X;
+    }
+    void quantize(const float* X, size_t K) {
+        if (quantized == X) return;
+        larql::launch_quantize_q8(X, K, M, q8, q8s, s);
+        quantized = X;
+    }
+    // One projection (input rows w.cols apart) -> Y rows ldy apart.  st: the rows' statistics,
+    // computed if have_stats.  defer: K-split partial products left to the caller.
+    void run(const DevWeight& w, bool is_down, const float* X, float* Y, size_t ldy, larql::GemmRowStats st,
+             bool have_stats, larql::GemmSplits* defer = nullptr) {
+        if (takes_q8(w, is_down)) {
+            quantize(X, w.cols);
+            if (ldy != w.rows) larql::launch_int_gemm(w, nullptr, q8, q8s, Y, nullptr, M, ldy, s);
+            else if (w.format == LARQL_Q8_0) larql::launch_q8_matvec(w, q8, q8s, Y, M, s);
+            else larql::launch_q4_0_matvec(w, q8, q8s, Y, M, s);
+            if (defer) *defer = {nullptr, 1};
+            return;
+        }
+        pack(X, w.cols, st, have_stats);
+        larql::launch_gemm_f32(w, X, Y, M, spl, split_n, s, ldy, &st, defer);
+    }
+};
+
+}  // namespace
 
 static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, size_t M, float* dout, hipStream_t s,
                        const PromptAttn& pa = {}) {
     auto& kv = c->kv;
     kv_ensure_model(c, m, M);
     const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim, ldmax = m->qkv_dim;
-    const size_t wide = std::max({hidden, qmax, inter}), gw = std::max(hidden, 2 * inter);
-    const int S = larql::attn_prompt_splits(1, static_cast<int>(M), 0);
-    const size_t part_n = m->part_per_split * S * M;
-    size_t split_n = 0;  // GEMM workspace: row exponents and K-split partial products
-    auto need = [&](const larql::DevWeight& w) {
-        split_n = std::max(split_n, larql::q4k_gemm_f32_part_floats(w, M));
-    };
-    for (const LayerDev& L : m->layers) {
-        if (L.split_qkv) need(L.wq), need(L.wk), need(L.wv);
-        else need(L.qkv);
-        need(L.wo), need(L.gateup), need(L.down);
-    }
-    // row statistics of the normed hidden rows and of the activation rows, computed by the
-    // kernels that produce those rows (two separate regions: a producer may still read
-    // the previous GEMM's partial products in SPL)
-    const size_t st_h = larql::gemm_row_stats_floats(M, hidden), st_a = larql::gemm_row_stats_floats(M, inter);
-    const size_t n_f = 2 * M * hidden + M * wide + M * ldmax + M * qmax + M * gw + M * inter + part_n + split_n +
-                       st_h + st_a + 8;
-    float* base = static_cast<float*>(larql::ensure(c, m->prompt, n_f * sizeof(float)));
-    float *H0 = base, *H1 = H0 + M * hidden, *XN = H1 + M * hidden, *QKV = XN + M * wide, *ATT = QKV + M * ldmax;
-    float *G = ATT + M * qmax, *ACT = G + M * gw, *PART = ACT + M * inter, *SPL = PART + part_n;
-    const larql::GemmRowStats xn_st = larql::gemm_row_stats_at(SPL + split_n, M, hidden);
-    const larql::GemmRowStats act_st = larql::gemm_row_stats_at(SPL + split_n + st_h + 4, M, inter);
+    const PromptLayout lay = prompt_layout(m, M);
+    float* base = static_cast<float*>(larql::ensure(c, m->prompt, lay.total() * sizeof(float)));
+    float *H0 = base, *H1 = H0 + M * hidden, *XN = H1 + M * hidden, *QKV = XN + M * lay.wide, *ATT = QKV + M * ldmax;
+    float *G = ATT + M * qmax, *ACT = G + M * lay.gw, *PART = ACT + M * inter, *SPL = base + lay.rows;
+    float* ST = SPL + a4(lay.split);
+    float *XP = ST + lay.st_h + lay.st_q + lay.st_a, *Q8 = XP + lay.xp, *Q8S = Q8 + lay.q8;
+    const larql::GemmRowStats xn_st = larql::gemm_row_stats_at(ST, M, hidden);
+    const larql::GemmRowStats att_st = larql::gemm_row_stats_at(ST + lay.st_h, M, qmax);
+    const larql::GemmRowStats act_st = larql::gemm_row_stats_at(ST + lay.st_h + lay.st_q, M, inter);
+    PromptProj pj{M, SPL, lay.split, XP, reinterpret_cast<int8_t*>(Q8), Q8S, s};
     larql::launch_copy_f32(dx, H0, M * hidden, s);
     bool xn_ready = false;  // XN holds this layer's normed input and xn_st its statistics
     for (size_t l = 0; l < m->layers.size(); l++) {
         const LayerDev& L = m->layers[l];
         // this layer's [q | k | v] rows, ld floats apart, and attention rows qd apart
         const size_t qd = static_cast<size_t>(L.nq) * L.hd, kvd = static_cast<size_t>(L.nkv) * L.hd, ld = qd + 2 * kvd;
-        if (!xn_ready) {
-            larql::launch_rmsnorm_rows(H0, L.input_norm, L.norm_offset, XN, M, hidden, L.eps, s);
-            larql::launch_gemm_row_stats(XN, M, hidden, xn_st, s);
+        if (!xn_ready) larql::launch_rmsnorm_rows(H0, L.input_norm, L.norm_offset, XN, M, hidden, L.eps, s);
+        pj.input();
+        if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
+            pj.run(L.wq, false, XN, QKV, ld, xn_st, xn_ready);
+            pj.run(L.wk, false, XN, QKV + qd, ld, xn_st, xn_ready);
+            pj.run(L.wv, false, XN, QKV + qd + kvd, ld, xn_st, xn_ready);
+        } else {
+            pj.run(L.qkv, false, XN, QKV, ld, xn_st, xn_ready);
         }
         xn_ready = false;
-        if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
-            prompt_proj(L.wq, XN, hidden, QKV, ld, M, SPL, split_n, s, &xn_st);
-            prompt_proj(L.wk, XN, hidden, QKV + qd, ld, M, SPL, split_n, s, &xn_st);
-            prompt_proj(L.wv, XN, hidden, QKV + qd + kvd, ld, M, SPL, split_n, s, &xn_st);
-        } else {
-            prompt_proj(L.qkv, XN, hidden, QKV, ld, M, SPL, split_n, s, &xn_st);
-        }
         if (L.v_norm) larql::launch_vnorm_rows(QKV + qd + kvd, M, ld, L.nkv, L.hd, L.eps, s);
         const float2* rope = rope_table(c, L.rope_base, L.rdim, s);
         larql::launch_rope_kv_rows(QKV, M, 0, qd, kvd, L.hd, L.rdim, rope, kv.k[l], kv.v[l], L.nkv, s);
@@ -870,30 +967,55 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
         at.softcap = pa.softcap;
         larql::launch_attention(at, s);
         const float scale = L.layer_scalar != 0.0f ? L.layer_scalar : 1.0f;
-        if (L.post_norms || hidden > larql::kFusedRowMax || inter > larql::kFusedRowMax) {
-            prompt_proj(L.wo, ATT, qd, G, hidden, M, SPL, split_n, s);
-            larql::launch_resid_norm_rows(H0, G, L.post_attn_norm, L.norm_offset, 1.0f, H1, M, hidden, L.eps, s);
-            larql::launch_rmsnorm_rows(H1, L.pre_ffn_norm, L.norm_offset, XN, M, hidden, L.eps, s);
-            prompt_proj(L.gateup, XN, hidden, G, 2 * inter, M, SPL, split_n, s);
-            larql::launch_gated_pair_rows(G, ACT, M * inter, L.act, s);
-            prompt_proj(L.down, ACT, inter, G, hidden, M, SPL, split_n, s);
-            larql::launch_resid_norm_rows(H1, G, L.post_ffn_norm, L.norm_offset, scale, H0, M, hidden, L.eps, s);
-            continue;
-        }
         // the split sums of wo and down, the residual adds, the next norm and the row
-        // statistics of the next GEMM's input: one row kernel after each projection
+        // statistics of the next GEMM's input: one row kernel after each projection, unless
+        // the projection's output is normed before its residual add
+        const bool fused = !L.post_norms && hidden <= larql::kFusedRowMax && inter <= larql::kFusedRowMax;
         larql::GemmSplits sp{};
-        prompt_proj(L.wo, ATT, qd, G, hidden, M, SPL, split_n, s, nullptr, &sp);
-        larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H0, 1.0f, H1,
-                                            L.post_attn_norm, L.norm_offset, XN, M, hidden, L.eps, xn_st, s);
-        prompt_proj(L.gateup, XN, hidden, G, 2 * inter, M, SPL, split_n, s, &xn_st);
-        larql::launch_gated_pair_stats_rows(G, ACT, M, inter, L.act, act_st, s);
-        prompt_proj(L.down, ACT, inter, G, hidden, M, SPL, split_n, s, &act_st, &sp);
+        pj.input();
+        pj.run(L.wo, false, ATT, G, hidden, att_st, false, fused ? &sp : nullptr);
+        if (fused) {
+            larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H0, 1.0f, H1,
+                                                L.post_attn_norm, L.norm_offset, XN, M, hidden, L.eps, xn_st, s);
+        } else if (L.post_norms) {
+            larql::launch_resid_norm_rows(H0, G, L.post_attn_norm, L.norm_offset, 1.0f, H1, M, hidden, L.eps, s);
+            larql::launch_rmsnorm_rows(H1, L.pre_ffn_norm, L.pre_ffn_norm ? L.norm_offset : 0.0f, XN, M, hidden, L.eps, s);
+        } else {
+            larql::launch_add_rows(H0, G, H1, M * hidden, s);
+            larql::launch_rmsnorm_rows(H1, L.post_attn_norm, L.norm_offset, XN, M, hidden, L.eps, s);
+        }
+        pj.input();
+        bool act_ready = false;  // act_st holds ACT's statistics
+        if (L.split_gu) {
+            float* U = G + M * inter;
+            pj.quantize(XN, hidden);
+            if (L.gate.format == LARQL_Q4_0 && L.up.format == LARQL_Q4_0) {
+                larql::launch_q4_0_matvec_pair(L.gate, L.up, pj.q8, pj.q8s, G, U, M, s);
+            } else {
+                pj.run(L.gate, false, XN, G, inter, xn_st, fused);
+                pj.run(L.up, false, XN, U, inter, xn_st, fused);
+            }
+            larql::launch_gated_mul(G, U, ACT, M * inter, L.act, s);
+        } else {
+            pj.run(L.gateup, false, XN, G, 2 * inter, xn_st, fused);
+            if (fused) larql::launch_gated_pair_stats_rows(G, ACT, M, inter, L.act, act_st, s);
+            else larql::launch_gated_pair_rows(G, ACT, M * inter, L.act, s);
+            act_ready = fused;
+        }
+        pj.input();
+        pj.run(L.down, true, ACT, G, hidden, act_st, act_ready, fused ? &sp : nullptr);
         const LayerDev* nx = l + 1 < m->layers.size() ? &m->layers[l + 1] : nullptr;
-        larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H1, scale, H0,
-                                            nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f,
-                                            nx ? XN : nullptr, M, hidden, nx ? nx->eps : 0.0, xn_st, s);
-        xn_ready = nx != nullptr;
+        if (fused) {
+            larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H1, scale, H0,
+                                                nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f,
+                                                nx ? XN : nullptr, M, hidden, nx ? nx->eps : 0.0, xn_st, s);
+            xn_ready = nx != nullptr;
+        } else if (L.post_norms) {
+            larql::launch_resid_norm_rows(H1, G, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, scale, H0, M,
+                                          hidden, L.eps, s);
+        } else {
+            larql::launch_add_rows(H1, G, H0, M * hidden, s, scale);
+        }
     }
     larql::launch_copy_f32(H0, dout, M * hidden, s);
     kv.current_len = M;
@@ -916,7 +1038,7 @@ extern "C" int larql_hip_prefill_q4(larql_hip_ctx* c, const larql_pipeline_layer
         const float* dx = stage_upload(c, c->stage_in, x, seq_len * hidden);
         float* dout = static_cast<float*>(larql::ensure(c, c->stage_out, seq_len * hidden * sizeof(float)));
         const PromptAttn pa{use_qk_norm != 0, softcap};
-        if (seq_len > 1 && prompt_batchable(m))
+        if (seq_len > 1 && prompt_batchable(m, seq_len))
             run_prompt(c, m, dx, seq_len, dout, c->stream, pa);
         else
             for (size_t p = 0; p < seq_len; p++)
@@ -949,7 +1071,7 @@ extern "C" int larql_hip_full_pipeline_q4(larql_hip_ctx* c, const larql_pipeline
         const float* dx = stage_upload(c, c->stage_in, x, seq_len * hidden);
         float* dout = static_cast<float*>(larql::ensure(c, c->stage_out, seq_len * hidden * sizeof(float)));
         const PromptAttn pa{use_qk_norm != 0, softcap};
-        if (seq_len > 1 && prompt_batchable(m))
+        if (seq_len > 1 && prompt_batchable(m, seq_len))
             run_prompt(c, m, dx, seq_len, dout, c->stream, pa);
         else
             for (size_t p = 0; p < seq_len; p++)
@@ -1082,7 +1204,7 @@ extern "C" int larql_hip_model_prefill_dev(larql_hip_ctx* c, larql_hip_model* m,
         hipStream_t s = pick_stream(c, stream);
         kv_ensure_model(c, m, seq_len);
         c->kv.current_len = 0;
-        if (seq_len > 1 && prompt_batchable(m))
+        if (seq_len > 1 && prompt_batchable(m, seq_len))
             run_prompt(c, m, x_dev, seq_len, out_dev, s);
         else
             for (size_t p = 0; p < seq_len; p++)

@@ -34,6 +34,8 @@ void launch_attention(const AttnArgs& a, hipStream_t s);
 // queries T0 .. T0 + batch - 1 (its partials stride).
 int attn_splits(int T, int t_begin);
 int attn_prompt_splits(int T0, int batch, int window);
+// Prompt mode in one pass per block of queries, without partials.
+bool attn_prompt_one_pass(int reps, int hd);
 // Floats per partial entry (o[hd], max, sum).  A partial buffer holds batch x num_q x S
 // entries.
 int attn_partial_stride(int hd);

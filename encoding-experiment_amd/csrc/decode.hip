@@ -771,6 +771,8 @@ int attn_prompt_splits(int T0, int batch, int window) {
     return S;
 }
 
+bool attn_prompt_one_pass(int reps, int hd) { return hd <= 256 && 16 % reps == 0; }
+
 // f(std::integral_constant<int, hd>) for the instantiated head dims, the multiples of 32
 // from HD up to 512; false for any other hd.
 template <int HD, typename F>
@@ -787,7 +789,7 @@ void launch_attention(const AttnArgs& a0, hipStream_t s) {
     AttnArgs a = a0;
     const int reps = a.num_q / a.num_kv;
     if (!attn_supported(reps, a.hd)) fail(LARQL_HIP_ERR_UNSUPPORTED, "attention: head geometry");
-    if (a.batch && a.hd <= 256 && 16 % reps == 0) {  // prompt mode: one pass per block of queries
+    if (a.batch && attn_prompt_one_pass(reps, a.hd)) {  // prompt mode: one pass per block of queries
         const int qpb = 4 * (16 / reps);
         const dim3 gp(static_cast<unsigned>((a.batch + qpb - 1) / qpb), a.num_kv), bp(kAttnThreads);
         if (!dispatch_head_dim<32>(a.hd, [&](auto h) {

@@ -258,35 +258,38 @@ void launch_f32_matmul(const float* A, const float* B, float* C, size_t m, size_
 // MFMA operands.
 size_t q4k_gemm_ws_bytes(size_t m, size_t cols);
 void launch_q4k_gemm(const DevWeight& w, const float* X, float* Y, size_t m, void* ws, hipStream_t s);
-// The same product from f32 X at f32 accuracy (fp16 operand pairs, three products each,
-// X rows scaled into range by per-token powers of two): ~1e-6 instead of ~1e-4, for
-// chains of projections (the batched prompt pass).  `part` is the workspace (floats:
-// q4k_gemm_f32_part_floats): the m row exponents, and the partial products when small
-// grids split K over up to four workgroups per tile (summed in split order).
-size_t q4k_gemm_f32_part_floats(const DevWeight& w, size_t m);
-// Row statistics of an f32-accuracy GEMM input (row exponents; the scaled sub-block sums
-// that Q4_K weights use, m x cols / 32 floats from a 16-byte boundary), computed by a
-// caller that fuses them into the kernel producing the input: the floats of workspace
-// for m rows of `cols`, their place in it, and the standalone computation.
+// The same product at f32 accuracy for Q4_K, Q6_K and Q4_0 weights (gemm_hp.hip: X as fp16
+// operand pairs scaled into range by per-token powers of two): ~1e-6 instead of ~1e-4, for
+// chains of projections (the batched prompt pass) and small batches.
+bool gemm_f32_takes(const DevWeight& w);
+// Row statistics of an input (row exponents xe; the scaled sub-block sums xs that Q4_K weights
+// use, m x cols / 32 floats from a 16-byte boundary), which a caller may fuse into the kernel
+// that produces the input, and its packed operands xp (gemm_x_pack_floats, 16-byte aligned;
+// null: the GEMM packs X in its workspace).  The floats of workspace for m rows of `cols`, their
+// place in it, and the standalone computations.
 struct GemmRowStats {
-    int* xe;
-    float* xs;
+    int* xe = nullptr;
+    float* xs = nullptr;
+    float* xp = nullptr;
 };
 size_t gemm_row_stats_floats(size_t m, size_t cols);
 GemmRowStats gemm_row_stats_at(float* ws, size_t m, size_t cols);
 void launch_gemm_row_stats(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s);
+size_t gemm_x_pack_floats(size_t m, size_t cols);
+void launch_gemm_x_pack(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s);
 // K-split partial products left to the caller to sum in split order (splits 1: part null,
 // Y was written): split z of row r at part + (z m + r) rows.
 struct GemmSplits {
     const float* part;
     int splits;
 };
-// Q4_K or Q6_K weights.  Y rows are ldy floats apart (0: w.rows), so a projection can
-// fill a column slice.  pre: X's row statistics, already computed (for Q4_K weights with
-// the sub-block sums).  defer: leave the split partial products unsummed (ldy = w.rows).
-void launch_q4k_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
-                         hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr,
-                         GemmSplits* defer = nullptr);
+// Y rows are ldy floats apart (0: w.rows), so a projection can fill a column slice.  part:
+// workspace of gemm_f32_part_floats.  pre: X's row statistics, already computed, and its packed
+// operands if xp is set (for Q4_K weights with the sub-block sums).  defer: leave the split
+// partial products unsummed (ldy = w.rows).
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m);
+void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
+                     hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr, GemmSplits* defer = nullptr);
 // Q4_0 or Q8_0 weights (cols a multiple of 128) x any number of Q8 rows, block order as the
 // matvecs (gemm_int.hip); w2 / out2: a second weight of the same format and shape in the same
 // launch.  Output rows ldo floats apart (0: w.rows).

@@ -304,6 +304,66 @@ def test_decode_q8_attention_q4_0_ffn(hip, formats, variant):
     run_sequence(hip, T0=21, n_tokens=2, n_layers=2, formats=formats, variant=variant)
 
 
+# Formats of Q8_0 / Q4_0 layers: all projections, separate Q / K / V beside Q4_K, gate and up in
+# different formats with a Q8_0 down.
+Q8_ATTN_Q4_FFN = {n: "q8_0" for n in ("wq", "wk", "wv", "wo")} | {n: "q4_0" for n in ("gate", "up", "down")}
+Q8_PROMPTS = [(2, Q8_ATTN_Q4_FFN, None), (17, Q8_ATTN_Q4_FFN, None), (49, Q8_ATTN_Q4_FFN, None),
+              (18, {"wq": "q8_0", "wv": "q8_0", "wk": "q6_k", "down": "q4_0"}, None),
+              (33, {"wq": "q8_0", "wo": "q4_0", "gate": "q8_0", "up": "q4_0", "down": "q8_0"}, None),
+              (16, {"gate": "q8_0", "up": "q8_0", "down": "q6_k"}, None),
+              (20, Q8_ATTN_Q4_FFN, dict(has_post_norms=True, norm_offset=1.0, activation="gelu_tanh", layer_scalar=0.5))]
+
+
+@pytest.mark.parametrize("seq,formats,variant", Q8_PROMPTS)
+def test_prefill_q8_q4_0_layers(hip, seq, formats, variant):
+    """prefill_q4 of Q8_0 / Q4_0 layers, every position at once: against the oracle layers and
+    against decoding the prompt token by token, then the next decode_token.  The attention sums in
+    another order than the decode kernel's, so an activation next to a rounding tie may take the
+    neighbouring Q8 code: a step of max|x| / 127 in one of 512 elements, ~3 sigma / 127 of sqrt(512)
+    sigma = 1e-3 of that input, and half a dozen quantized inputs over the two layers add in
+    quadrature: 3e-3 of the output's scale."""
+    tol = 3e-3
+    n_layers, hidden, inter, nq, nkv, hd = 2, 512, 1024, 8, 2, 64
+    print(f"[prefill q8] seq={seq} formats={formats} variant={variant}", flush=True)
+    m = SmallModel(n_layers, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=78, formats=formats, variant=variant)
+    layers = m.hip_layers(10000.0)
+    x = np.stack([oracle.gauss(8100 + p, hidden) for p in range(seq)])
+    args = (hidden, inter, nq * hd, nkv * hd)
+    hip.reset_kv_cache()
+    got = hip.prefill_q4(layers, x, *args, seq, nq, nkv, hd, 10000.0)
+    assert got is not None and hip.kv_cache_len() == seq
+    nxt = oracle.gauss(9001, hidden)
+    after = hip.decode_token(layers, nxt, *args, nq, nkv, hd, 10000.0)
+    hip.reset_kv_cache()
+    step = np.stack([hip.decode_token(layers, x[p], *args, nq, nkv, hd, 10000.0) for p in range(seq)])
+    after_step = hip.decode_token(layers, nxt, *args, nq, nkv, hd, 10000.0)
+    ref = []
+    for p in range(seq):
+        h = x[p].copy()
+        for L in m.layers:
+            h = oracle.decode_layer(L, h, p, hidden, inter, nq, nkv, hd, 10000.0)
+        ref.append(h)
+    e_ref = max(rel_err(got[p], ref[p]) for p in range(seq))
+    e_step = max(rel_err(got[p], step[p].astype(np.float64)) for p in range(seq))
+    e_next = rel_err(after, after_step.astype(np.float64))
+    print(f"  oracle {e_ref:.2e}, step by step {e_step:.2e}, next token {e_next:.2e}", flush=True)
+    assert e_ref <= tol and e_step <= tol and e_next <= tol
+
+
+def test_prefill_wide_ffn_residual(hip):
+    """An FFN wider than the row kernels hold (inter > 16384): the residual adds of a layer without
+    post-norms, position by position against the oracle."""
+    hidden, inter, nq, nkv, hd, seq = 256, 16640, 4, 2, 64, 3
+    print(f"[prefill wide] inter={inter}", flush=True)
+    m = SmallModel(1, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=79)
+    x = np.stack([oracle.gauss(8200 + p, hidden) for p in range(seq)])
+    hip.reset_kv_cache()
+    got = hip.prefill_q4(m.hip_layers(10000.0), x, hidden, inter, nq * hd, nkv * hd, seq, nq, nkv, hd, 10000.0)
+    for p in range(seq):
+        ref = oracle.decode_layer(m.layers[0], x[p].copy(), p, hidden, inter, nq, nkv, hd, 10000.0)
+        assert rel_err(got[p], ref) <= REL_TOL, p
+
+
 def _oracle_positions(m, x, hidden, inter, nq, nkv, hd, rope):
     out = []
     for p in range(x.shape[0]):

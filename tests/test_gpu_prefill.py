@@ -94,7 +94,12 @@ def test_q4k_matmul_m1_equals_matvec(hip):
 # (4096, 14336, 64): the Llama-3-8B down projection; (300, 512, 37): a ragged tile; (70, 1024,
 # 9, scaled): token rows scaled by 1e6 .. 1e-30, far outside fp16 (the GEMM's operand pairs
 # are fp16: each row must be brought into range by its own power of two), and a zero row
-@pytest.mark.parametrize("rows,cols,m,scaled", [(4096, 14336, 64, False), (300, 512, 37, False), (70, 1024, 9, True)])
+# the others: the edges of 16-token tiles and of one to three tiles per workgroup, of 16-row
+# tiles and 256-row workgroups, and K split over 1 .. 16 workgroups
+@pytest.mark.parametrize("rows,cols,m,scaled", [(4096, 14336, 64, False), (300, 512, 37, False), (70, 1024, 9, True),
+                                                (300, 256, 16, False), (70, 512, 17, False), (257, 1024, 48, False),
+                                                (64, 256, 49, False), (1, 4096, 33, False), (272, 2304, 97, False),
+                                                (520, 4352, 2, False)])
 def test_q6k_gemm_rows_match_matvec_oracle(hip, rows, cols, m, scaled):
     """The Q6_K f32-accuracy GEMM of the prompt pass (matvec_dev with m > 1 on a Q6_K handle)
     at the Llama-3-8B down-projection shape: every token row against the oracle's Q6_K
