@@ -13,6 +13,7 @@ struct AttnArgs {
     float* part;       // [num_q][S][pst]: unnormalised o[hd], chunk max, chunk sum (attn_part_floats)
     int num_q, num_kv, hd, rdim;
     int T, t_begin, S;  // S is set by launch_attention
+    int chunks = 1;     // 64-position chunks per split, set by launch_attention
     int pst = 0;        // partial entry stride in floats (attn_partial_stride), set by launch_attention
     float scale;
     const float2* rope;  // [cap][rdim / 2] cos, sin (launch_rope_table)

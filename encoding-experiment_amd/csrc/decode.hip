@@ -131,102 +131,97 @@ __device__ __forceinline__ void attn_select_query(AttnArgs& a) {
     a.out += static_cast<size_t>(p) * a.num_q * a.hd;
 }
 
-// o = sum_s e_s o_s / sum_s e_s l_s with e_s = exp(m_s - max_s m_s), in split order, for
-// HD dims of nh consecutive query heads: partial entry (head h, split s) at
-// base + (h sst + s) pst = {o[HD], ...}, its (m, l) pair mlo floats further, outputs at
-// out + h HD.  One workgroup; ml holds 2 nh S floats of LDS.
-// The loads of every (m, l) pair and of the first PF splits of each thread's first output
-// pair are issued together, so for S <= PF (T <= 2176) the merge waits on memory once.
+// o = sum_s e_s o_s / sum_s e_s l_s with e_s = exp(m_s - max_s m_s) for the HD dims of a query
+// head: its partial entry of split s at base + s pst = {o[HD], m, l}.  One workgroup; ml holds 2 S
+// floats of LDS.  The threads are G groups of HD / 2 (two dims each), group k taking the k-th of
+// G runs of splits, in order, the runs' sums added in order.
+// The loads of every (m, l) pair and of the first PF splits of each group's run are issued
+// together, so for S <= G PF (the splits of a decode step: 68 of head_dim 128) the merge waits
+// on memory once.
 template <int HD>
-__device__ __forceinline__ void attn_merge_heads(const float* __restrict__ base, int mlo, int pst, int sst, int S,
-                                                 int nh, float* __restrict__ out, float* ml, float* inv_l) {
-    constexpr int H2 = HD / 2, PF = 34;
+__device__ __forceinline__ void attn_merge_head(const float* __restrict__ base, int pst, int S,
+                                                float* __restrict__ out, float* ml, float* inv_l) {
+    constexpr int H2 = HD / 2, G = kAttnThreads / H2, PF = G == 1 ? 34 : 17;
+    __shared__ float2 sums[G][H2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nout = nh * H2;  // float2 outputs
+    const int grp = min(tid / H2, G - 1), d = 2 * (tid % H2);  // (threads past G H2 repeat others' work)
+    const int per = (S + G - 1) / G, s0 = min(grp * per, S), s1 = min(s0 + per, S);
     // the first (m, l) pair of each thread first: loads complete in order, so storing it
     // to LDS then waits for it alone, not for the prefetch behind it
-    const int nk = nh * S, k0 = min(tid, nk - 1);
-    const float2 ml0 = [&] {
-        const int h = k0 / S, s = k0 - h * S;
-        return *reinterpret_cast<const float2*>(base + (static_cast<size_t>(h) * sst + s) * pst + mlo);
-    }();
+    const int k0 = min(tid, S - 1);
+    const float2 ml0 = *reinterpret_cast<const float2*>(base + static_cast<size_t>(k0) * pst + HD);
     __builtin_amdgcn_sched_barrier(0);
     float2 ov[PF];
-    {
-        // unconditional loads (thread and split clamped into range; a load under a
-        // condition becomes a branch, and the loads would then wait one by one): threads
-        // past nout and splits past S load data they do not use
-        const int t = min(tid, nout - 1), h = t / H2, d = 2 * (t - h * H2);
-        const float* src = base + static_cast<size_t>(h) * sst * pst + d;
+    const float* src = base + d;
+    // unconditional loads (split clamped into range; a load under a condition becomes a branch,
+    // and the loads would then wait one by one): splits past the run load data it does not use
 #pragma unroll
-        for (int u = 0; u < PF; u++) ov[u] = *reinterpret_cast<const float2*>(src + static_cast<size_t>(min(u, S - 1)) * pst);
-    }
-    ml[2 * k0] = ml0.x;  // (threads past nk write pair nk - 1's value again)
+    for (int u = 0; u < PF; u++)
+        ov[u] = *reinterpret_cast<const float2*>(src + static_cast<size_t>(min(s0 + u, S - 1)) * pst);
+    ml[2 * k0] = ml0.x;  // (threads past S write pair S - 1's value again)
     ml[2 * k0 + 1] = ml0.y;
-    for (int k = tid + kAttnThreads; k < nk; k += kAttnThreads) {
-        const int h = k / S, s = k - h * S;
-        const float2 v = *reinterpret_cast<const float2*>(base + (static_cast<size_t>(h) * sst + s) * pst + mlo);
+    for (int k = tid + kAttnThreads; k < S; k += kAttnThreads) {
+        const float2 v = *reinterpret_cast<const float2*>(base + static_cast<size_t>(k) * pst + HD);
         ml[2 * k] = v.x;
         ml[2 * k + 1] = v.y;
     }
     lds_barrier();
-    for (int h = wave; h < nh; h += kAttnThreads / 64) {  // one wave per head
+    if (wave == 0) {
         float mx = -INFINITY;
-        for (int s = lane; s < S; s += 64) mx = fmaxf(mx, ml[2 * (h * S + s)]);
+        for (int s = lane; s < S; s += 64) mx = fmaxf(mx, ml[2 * s]);
         mx = wave_max_dpp(mx);
         float L = 0.f;
         for (int s = lane; s < S; s += 64) {
-            const float e = expf(ml[2 * (h * S + s)] - mx);
-            ml[2 * (h * S + s)] = e;
-            L = fmaf(ml[2 * (h * S + s) + 1], e, L);
+            const float e = expf(ml[2 * s] - mx);
+            ml[2 * s] = e;
+            L = fmaf(ml[2 * s + 1], e, L);
         }
         L = wave_sum_dpp(L);
-        if (lane == 0) inv_l[h] = 1.0f / L;
+        if (lane == 0) *inv_l = 1.0f / L;
     }
     lds_barrier();
-    for (int i = tid; i < nout; i += kAttnThreads) {
-        const int h = i / H2, d = 2 * (i - h * H2);
-        const float* e = ml + 2 * h * S;
-        const float* src = base + static_cast<size_t>(h) * sst * pst + d;
-        float2 o = make_float2(0.f, 0.f);
-        int s = 0;
-        if (i == tid) {
-            // every weight read from LDS before the first is used; splits past S keep o
-            float ev[PF];
+    float2 o = make_float2(0.f, 0.f);
+    {
+        // every weight read from LDS before the first is used; splits past the run keep o
+        float ev[PF];
 #pragma unroll
-            for (int u = 0; u < PF; u++) ev[u] = e[2 * min(u, S - 1)];
+        for (int u = 0; u < PF; u++) ev[u] = ml[2 * min(s0 + u, S - 1)];
 #pragma unroll
-            for (int u = 0; u < PF; u++) {
-                const float x = fmaf(ov[u].x, ev[u], o.x), y = fmaf(ov[u].y, ev[u], o.y);
-                o.x = u < S ? x : o.x;
-                o.y = u < S ? y : o.y;
-            }
-            s = PF;
+        for (int u = 0; u < PF; u++) {
+            const float x = fmaf(ov[u].x, ev[u], o.x), y = fmaf(ov[u].y, ev[u], o.y);
+            o.x = s0 + u < s1 ? x : o.x;
+            o.y = s0 + u < s1 ? y : o.y;
         }
-        for (; s < S; s += 16) {  // splits past PF: sixteen loads in flight per round
-            float2 v[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                v[u] = s + u < S ? *reinterpret_cast<const float2*>(src + static_cast<size_t>(s + u) * pst)
-                                 : make_float2(0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (s + u < S) {
-                    o.x = fmaf(v[u].x, e[2 * (s + u)], o.x);
-                    o.y = fmaf(v[u].y, e[2 * (s + u)], o.y);
-                }
-        }
-        const float il = inv_l[h];
-        *reinterpret_cast<float2*>(out + static_cast<size_t>(h) * HD + d) = make_float2(o.x * il, o.y * il);
     }
+    for (int s = s0 + PF; s < s1; s += 16) {  // splits past PF: sixteen loads in flight per round
+        float2 v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            v[u] = *reinterpret_cast<const float2*>(src + static_cast<size_t>(min(s + u, s1 - 1)) * pst);
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            if (s + u < s1) {
+                o.x = fmaf(v[u].x, ml[2 * (s + u)], o.x);
+                o.y = fmaf(v[u].y, ml[2 * (s + u)], o.y);
+            }
+    }
+    if constexpr (G > 1) {
+        sums[grp][tid % H2] = o;
+        lds_barrier();
+        if (tid >= H2) return;
+        o = sums[0][tid];
+#pragma unroll
+        for (int k = 1; k < G; k++) o.x += sums[k][tid].x, o.y += sums[k][tid].y;
+    }
+    const float il = *inv_l;
+    *reinterpret_cast<float2*>(out + d) = make_float2(o.x * il, o.y * il);
 }
 
 // LDS of one head's merge: S (m, l) pairs and its reciprocal sum.
 constexpr int kMergeLdsMax = 48 * 1024;
-constexpr int kMergeParts = 1;  // workgroups per query head, each merging HD / kMergeParts dims
 inline size_t merge_lds_bytes(int S) { return sizeof(float) * (2 * static_cast<size_t>(S) + 8); }
 
-template <int HD>
+template <int HD, bool MULTI>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     attn_select_query(a);
     constexpr int KS = HD / 32;                 // score k-steps
@@ -239,6 +234,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     __shared__ v4u qop[KS * 64];                // score B operands
     __shared__ float p_s[8][kAttnChunk];
     __shared__ float ml_s[16];
+    __shared__ float alpha_s[8];                // MULTI: a head's factor on its sums so far
     __shared__ v4u pop[2 * 64];                 // P.V B operands
     __shared__ __attribute__((aligned(16))) uint16_t knew[HD];
     __shared__ uint16_t vnew[HD];
@@ -247,12 +243,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     const int s = blockIdx.x, kvh = blockIdx.y;
     const int reps = a.num_q / a.num_kv, half = a.rdim / 2;
     const int q_dim = a.num_q * HD, kv_dim = a.num_kv * HD;
-    const int t0 = (a.t_begin & ~7) + s * kAttnChunk;
+    const int nc = MULTI ? a.chunks : 1;  // chunks of this workgroup, from t0 on
+    int t0 = (a.t_begin & ~7) + s * nc * kAttnChunk;
     const int pos = a.T - 1;
     if (t0 > pos) return;  // prompt mode: a chunk past this query's position
     // the last chunk holds pos; outside prompt mode its row comes from the projections
-    const bool owner = pos < t0 + kAttnChunk;
-    const bool fresh = owner && a.batch == 0;
+    bool owner = pos < t0 + kAttnChunk;
+    const bool fresh = pos < t0 + nc * kAttnChunk && a.batch == 0;
     const int klim = a.batch ? pos + 1 : pos;  // K rows read from the cache: t < klim
 
     // 1. Global loads, all issued up front: first the query heads, the RoPE row and the
@@ -276,28 +273,34 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
         krv[u] = fresh && d < HD ? a.qkv[q_dim + static_cast<size_t>(kvh) * HD + d] : 0.f;
         vnv[u] = fresh && d < HD ? a.qkv[q_dim + kv_dim + static_cast<size_t>(kvh) * HD + d] : 0.f;
     }
-    const int tk = t0 + 16 * wave + c;
-    v4u kA[KS];
+    struct Kv {
+        v4u k[KS];
+        v4u v[DTW][2];
+    };
+    auto load_kv = [&](int at, Kv& o) __attribute__((always_inline)) {
+        const int tk = at + 16 * wave + c;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++)
-    {   // (unconditional loads from a row inside the cache, then a select: no branch around
-        // the loads, so each later wait counts only the loads issued after the one it needs)
-        const v4u kv = *reinterpret_cast<const v4u*>(
-            a.kc + (static_cast<size_t>(max(min(tk, klim - 1), 0)) * a.num_kv + kvh) * HD + 32 * ks + 8 * g);
-        kA[ks] = tk < klim ? kv : v4u{0u, 0u, 0u, 0u};
-    }
-    v4u vA[DTW][2];
-#pragma unroll
-    for (int i = 0; i < DTW; i++) {
-        const int dt = wave + 4 * i;
-#pragma unroll
-        for (int ts = 0; ts < 2; ts++) {
-            const int tv = t0 + 32 * ts + 8 * g;
-            const v4u vv = *reinterpret_cast<const v4u*>(
-                a.vc + ((static_cast<size_t>(min(tv, pos) >> 3) * a.num_kv + kvh) * HD + 16 * min(dt, NDT - 1) + c) * 8);
-            vA[i][ts] = (dt < NDT && tv <= pos) ? vv : v4u{0u, 0u, 0u, 0u};
+        for (int ks = 0; ks < KS; ks++) {
+            // (unconditional loads from a row inside the cache, then a select: no branch around
+            // the loads, so each later wait counts only the loads issued after the one it needs)
+            const v4u kv = *reinterpret_cast<const v4u*>(
+                a.kc + (static_cast<size_t>(max(min(tk, klim - 1), 0)) * a.num_kv + kvh) * HD + 32 * ks + 8 * g);
+            o.k[ks] = tk < klim ? kv : v4u{0u, 0u, 0u, 0u};
         }
-    }
+#pragma unroll
+        for (int i = 0; i < DTW; i++) {
+            const int dt = wave + 4 * i;
+#pragma unroll
+            for (int ts = 0; ts < 2; ts++) {
+                const int tv = at + 32 * ts + 8 * g;
+                const v4u vv = *reinterpret_cast<const v4u*>(
+                    a.vc + ((static_cast<size_t>(min(tv, pos) >> 3) * a.num_kv + kvh) * HD + 16 * min(dt, NDT - 1) + c) * 8);
+                o.v[i][ts] = (dt < NDT && tv <= pos) ? vv : v4u{0u, 0u, 0u, 0u};
+            }
+        }
+    };
+    Kv cur;
+    load_kv(t0, cur);
 #pragma unroll
     for (int u = 0; u < QPT; u++) {
         const int i = tid + u * kAttnThreads;
@@ -345,10 +348,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
         }
         qop[i] = op;
     }
+    auto new_row = [&]() __attribute__((always_inline)) {
     if (owner) {
-        if (fresh && tk == pos) {
+        if (fresh && t0 + 16 * wave + c == pos) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) kA[ks] = *reinterpret_cast<const v4u*>(&knew[32 * ks + 8 * g]);
+            for (int ks = 0; ks < KS; ks++) cur.k[ks] = *reinterpret_cast<const v4u*>(&knew[32 * ks + 8 * g]);
         }
         // the block holding pos: the new value at pos (prompt mode: the cached one), zeros
         // above it (beyond this query)
@@ -364,23 +368,34 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
                     const uint32_t vn = sub ? vnew[16 * dt + c] : 0u;
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const uint32_t w = vA[i][ts][k];
+                        const uint32_t w = cur.v[i][ts][k];
                         const uint32_t lo = 2 * k < e ? (w & 0xFFFFu)
                                                       : (2 * k == e ? (sub ? vn : (w & 0xFFFFu)) : 0u);
                         const uint32_t hi = 2 * k + 1 < e ? (w >> 16) : (2 * k + 1 == e ? (sub ? vn : (w >> 16)) : 0u);
-                        vA[i][ts][k] = lo | (hi << 16);
+                        cur.v[i][ts][k] = lo | (hi << 16);
                     }
                 }
             }
         }
     }
+    };
+    floatx4 oacc[DTW];  // MULTI: the chunks' sums so far
+#pragma unroll
+    for (int i = 0; i < DTW; i++) oacc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (MULTI && tid < 8) ml_s[2 * tid] = -INFINITY, ml_s[2 * tid + 1] = 0.f;
+    new_row();
     lds_barrier();
+    Kv nxt;
+    for (int ci = 0;; ci++) {
+    if constexpr (MULTI) {  // the next chunk's rows (past the last: rows it has, unused) meanwhile
+        load_kv(t0 + kAttnChunk, nxt);
+    }
 
     // 2. Scores of positions t0 + 16 w + 4 g + r for lanes (g, col < reps).
     floatx4 sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
-        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, kA[ks]),
+        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.k[ks]),
                                                       __builtin_bit_cast(half8, qop[ks * 64 + lane]), sacc, 0, 0, 0);
     sacc = add_lane_plus(sacc, reps);
     if (c < reps) {
@@ -393,16 +408,24 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
         }
     }
     lds_barrier();
-    // 3. Softmax partials of the chunk: one wave per head.
+    // 3. Softmax partials of the chunk: one wave per head.  MULTI: relative to the largest score so
+    // far, with the factor that takes the sums so far there.
     for (int h = wave; h < reps; h += kAttnThreads / 64) {
         const float sc = p_s[h][lane];
-        const float m = wave_max_dpp(sc);
+        float m = wave_max_dpp(sc), al = 0.f;
+        if constexpr (MULTI) {
+            const float m0 = ml_s[2 * h];
+            m = fmaxf(m, m0);
+            al = m0 == -INFINITY ? 0.f : expf(m0 - m);
+        }
         const float p = sc == -INFINITY ? 0.f : expf(sc - m);
-        const float l = wave_sum_dpp(p);
+        float l = wave_sum_dpp(p);
+        if constexpr (MULTI) l = fmaf(ml_s[2 * h + 1], al, l);
         p_s[h][lane] = p;
         if (lane == 0) {
             ml_s[2 * h] = m;
             ml_s[2 * h + 1] = l;
+            if constexpr (MULTI) alpha_s[h] = al;
         }
     }
     lds_barrier();
@@ -425,13 +448,29 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
         floatx4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ts = 0; ts < 2; ts++)
-            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, vA[i][ts]),
+            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.v[i][ts]),
                                                        __builtin_bit_cast(half8, pop[ts * 64 + lane]), o, 0, 0, 0);
         o = add_lane_plus(o, reps);
-        if (c < reps) {
+        if constexpr (MULTI) {
+            const float al = alpha_s[min(c, reps - 1)];
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = fmaf(oacc[i][r], al, o[r]);
+        }
+        oacc[i] = o;
+    }
+    if (!MULTI || ci + 1 == nc || t0 + kAttnChunk > pos) break;
+    t0 += kAttnChunk;
+    owner = pos < t0 + kAttnChunk;
+    cur = nxt;
+    new_row();
+    }
+#pragma unroll
+    for (int i = 0; i < DTW; i++) {
+        const int dt = wave + 4 * i;
+        if (dt < NDT && c < reps) {
             float* dst = a.part + (static_cast<size_t>(kvh * reps + c) * a.S + s) * a.pst;
 #pragma unroll
-            for (int r = 0; r < 4; r++) dst[16 * dt + 4 * g + r] = o[r];
+            for (int r = 0; r < 4; r++) dst[16 * dt + 4 * g + r] = oacc[i][r];
         }
     }
     if (tid < reps) {
@@ -454,13 +493,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(AttnArgs a) 
     extern __shared__ float lds[];
     const int sst = a.S;  // partial stride per head
     attn_select_query(a);
-    const int S = (a.T - (a.t_begin & ~7) + kAttnChunk - 1) / kAttnChunk;  // this query's splits
-    // query head h, dims [p DH, (p + 1) DH)
-    constexpr int DH = HD / kMergeParts;
-    const size_t h = blockIdx.x / kMergeParts;
-    const int d0 = (blockIdx.x % kMergeParts) * DH;
-    attn_merge_heads<DH>(a.part + h * sst * a.pst + d0, HD - d0, a.pst, sst, S, 1, a.out + h * HD + d0, lds,
-                         lds + 2 * S);
+    const int per = kAttnChunk * a.chunks;
+    const int S = (a.T - (a.t_begin & ~7) + per - 1) / per;  // this query's splits
+    const size_t h = blockIdx.x;
+    attn_merge_head<HD>(a.part + h * sst * a.pst, a.pst, S, a.out + h * HD, lds, lds + 2 * S);
 }
 
 // ── Prompt attention in one pass per block of queries ────────────────────
@@ -800,17 +836,26 @@ void launch_attention(const AttnArgs& a0, hipStream_t s) {
         LARQL_HIP_CHECK(hipGetLastError());
         return;
     }
-    a.S = a.batch ? attn_prompt_splits(a.T, a.batch, a.window) : attn_splits(a.T, a.t_begin);
+    // A decode step's workgroup takes several chunks in turn where there are more than two
+    // workgroups per CU: fewer partials to merge, the query prepared once for all of them.  Four
+    // 8B-shape layers and the head at position 16384 / 30000: 358 / 471 us with a chunk per
+    // workgroup, 326 / 393 with one workgroup per CU, 305 / 346 with two, 316 / 383 with four.
+    const int chunks = attn_splits(a.T, a.t_begin);
+    a.chunks = a.batch ? 1 : std::max(1, (chunks * a.num_kv + 2 * current_device_cus() - 1) / (2 * current_device_cus()));
+    a.S = a.batch ? attn_prompt_splits(a.T, a.batch, a.window) : (chunks + a.chunks - 1) / a.chunks;
     a.pst = attn_partial_stride(a.hd);
     if (2 * static_cast<size_t>(a.S) * sizeof(float) + 32 > static_cast<size_t>(kMergeLdsMax))
         fail(LARQL_HIP_ERR_UNSUPPORTED, "attention: too many position splits");
     const int nz = a.batch ? a.batch : 1;
     const size_t lds = merge_lds_bytes(a.S);
     const dim3 grid(a.S, a.num_kv, nz), block(kAttnThreads);
-    if (!dispatch_head_dim<32>(a.hd, [&](auto h) { attn_decode_kernel<decltype(h)::value><<<grid, block, 0, s>>>(a); }))
+    if (!dispatch_head_dim<32>(a.hd, [&](auto h) {
+            if (a.chunks > 1) attn_decode_kernel<decltype(h)::value, true><<<grid, block, 0, s>>>(a);
+            else attn_decode_kernel<decltype(h)::value, false><<<grid, block, 0, s>>>(a);
+        }))
         fail(LARQL_HIP_ERR_UNSUPPORTED, "attention: head_dim");
     LARQL_HIP_CHECK(hipGetLastError());
-    const dim3 g2(a.num_q * kMergeParts, 1, nz);
+    const dim3 g2(a.num_q, 1, nz);
     dispatch_head_dim<32>(a.hd, [&](auto h) { attn_combine_kernel<decltype(h)::value><<<g2, block, lds, s>>>(a); });
     LARQL_HIP_CHECK(hipGetLastError());
 }

@@ -350,6 +350,15 @@ def test_prefill_q8_q4_0_layers(hip, seq, formats, variant):
     assert e_ref <= tol and e_step <= tol and e_next <= tol
 
 
+@pytest.mark.parametrize("T0,hd,nq,nkv,window", [(4094, 64, 8, 8, 0), (4160, 64, 8, 8, 0), (8300, 32, 16, 8, 0),
+                                                 (9000, 96, 8, 8, 8500), (4500, 128, 16, 16, 0)])
+def test_decode_long_cache(hip, T0, hd, nq, nkv, window):
+    """Positions from which an attention workgroup takes more than one 64-position chunk (4096 on
+    at 8 kv heads, 2048 at 16): the last position with one, a first chunk of the next pair, a last
+    workgroup with fewer chunks than the others, a window that starts inside a chunk."""
+    run_sequence(hip, T0=T0, n_tokens=3, n_layers=1, hidden=512, inter=512, nq=nq, nkv=nkv, hd=hd, window=window)
+
+
 def test_prefill_wide_ffn_residual(hip):
     """An FFN wider than the row kernels hold (inter > 16384): the residual adds of a layer without
     post-norms, position by position against the oracle."""
