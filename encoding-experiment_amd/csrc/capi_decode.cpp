@@ -880,13 +880,25 @@ struct PromptProj {
     const float* packed = nullptr;
     const float* quantized = nullptr;
 
-    // A new input row block at X (the same buffer with other contents included).
-    void input() { packed = quantized = nullptr; }
-    void pack(const float* X, size_t K, larql::GemmRowStats& st, bool have_stats) {
+    // A new input: X's rows (the same buffer with other contents included), packed already or not.
+    void input(const float* X, bool is_packed) {
+        packed = is_packed ? X : nullptr;
+        quantized = nullptr;
+    }
+    void pack(const float* X, size_t K, larql::GemmRowStats& st) {
         st.xp = xp;
         if (packed == X) return;
-        if (!have_stats) larql::launch_gemm_row_stats(X, M, K, st, s);
-        larql::launch_gemm_x_pack(X, M, K, st, s);
+        if (K <= static_cast<size_t>(larql::kFusedRowMax)) {
+            larql::ResidRows r;
+            r.hin = X;
+            r.st = st;
+            r.m = static_cast<int>(M);
+            r.n = static_cast<int>(K);
+            larql::launch_resid_norm_stats_rows(r, s);
+        } else {
+            larql::launch_gemm_row_stats(X, M, K, st, s);
+            larql::launch_gemm_x_pack(X, M, K, st, s);
+        }
         packed = X;
     }
     void quantize(const float* X, size_t K) {
@@ -894,10 +906,11 @@ struct PromptProj {
         larql::launch_quantize_q8(X, K, M, q8, q8s, s);
         quantized = X;
     }
-    // One projection (input rows w.cols apart) -> Y rows ldy apart.  st: the rows' statistics,
-    // computed if have_stats.  defer: K-split partial products left to the caller.
+    // One projection (input rows w.cols apart) -> Y rows ldy apart.  st: the place of the rows'
+    // statistics, computed if the rows are packed.  defer: K-split partial products left to the
+    // caller.
     void run(const DevWeight& w, bool is_down, const float* X, float* Y, size_t ldy, larql::GemmRowStats st,
-             bool have_stats, larql::GemmSplits* defer = nullptr) {
+             larql::GemmSplits* defer = nullptr) {
         if (takes_q8(w, is_down)) {
             quantize(X, w.cols);
             if (ldy != w.rows) larql::launch_int_gemm(w, nullptr, q8, q8s, Y, nullptr, M, ldy, s);
@@ -906,7 +919,7 @@ struct PromptProj {
             if (defer) *defer = {nullptr, 1};
             return;
         }
-        pack(X, w.cols, st, have_stats);
+        pack(X, w.cols, st);
         larql::launch_gemm_f32(w, X, Y, M, spl, split_n, s, ldy, &st, defer);
     }
 };
@@ -918,6 +931,7 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
     auto& kv = c->kv;
     kv_ensure_model(c, m, M);
     const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim, ldmax = m->qkv_dim;
+    const size_t qd_max = m->q_dim;
     const PromptLayout lay = prompt_layout(m, M);
     float* base = static_cast<float*>(larql::ensure(c, m->prompt, lay.total() * sizeof(float)));
     float *H0 = base, *H1 = H0 + M * hidden, *XN = H1 + M * hidden, *QKV = XN + M * lay.wide, *ATT = QKV + M * ldmax;
@@ -928,22 +942,71 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
     const larql::GemmRowStats att_st = larql::gemm_row_stats_at(ST + lay.st_h, M, qmax);
     const larql::GemmRowStats act_st = larql::gemm_row_stats_at(ST + lay.st_h + lay.st_q, M, inter);
     PromptProj pj{M, SPL, lay.split, XP, reinterpret_cast<int8_t*>(Q8), Q8S, s};
-    larql::launch_copy_f32(dx, H0, M * hidden, s);
-    bool xn_ready = false;  // XN holds this layer's normed input and xn_st its statistics
+    // Row kernels between the projections (residual add, norms, the next GEMM's statistics and
+    // packed operands in one launch) where a row fits them
+    const bool fused = std::max({hidden, qd_max, inter}) <= static_cast<size_t>(larql::kFusedRowMax);
+    auto qkv_f32 = [&](const LayerDev& L) {  // the Q8-input projections read the normed rows themselves
+        return L.split_qkv ? takes_q8(L.wq, false) || takes_q8(L.wk, false) || takes_q8(L.wv, false) : takes_q8(L.qkv, false);
+    };
+    auto qkv_packed = [&](const LayerDev& L) {
+        return L.split_qkv ? !(takes_q8(L.wq, false) && takes_q8(L.wk, false) && takes_q8(L.wv, false))
+                           : !takes_q8(L.qkv, false);
+    };
+    // hin (+ P) -> hout, and the rows normed by (w, off, eps): f32 rows for Q8-input projections,
+    // packed ones for the others
+    auto rows = [&](const float* hin, const float* P, const larql::GemmSplits& sp, bool post, const float* pw, float poff,
+                    double peps, float scale, float* hout, bool norm, const float* w, float off, double eps, bool want_f32,
+                    bool want_packed) {
+        larql::ResidRows r;
+        r.P = P && sp.splits > 1 ? sp.part : P;
+        r.pstride = M * hidden;
+        r.splits = P ? sp.splits : 1;
+        r.hin = hin;
+        r.post = post;
+        r.pw = pw;
+        r.poff = poff;
+        r.eps = peps;
+        r.scale = scale;
+        r.hout = hout;
+        r.norm = norm;
+        r.w = w;
+        r.off = off;
+        r.norm_eps = eps;
+        if (norm) {
+            r.xn = want_f32 ? XN : nullptr;
+            if (want_packed) {
+                r.st = xn_st;
+                r.st.xp = XP;
+            }
+        }
+        r.m = static_cast<int>(M);
+        r.n = static_cast<int>(hidden);
+        larql::launch_resid_norm_stats_rows(r, s);
+        pj.input(XN, norm && want_packed);
+    };
+    const float* Hin = dx;  // the layer's input rows
+    if (fused) {
+        const LayerDev& L = m->layers[0];
+        rows(dx, nullptr, {}, false, nullptr, 0.f, 0.0, 1.0f, nullptr, true, L.input_norm, L.norm_offset, L.eps, qkv_f32(L),
+             qkv_packed(L));
+    }
     for (size_t l = 0; l < m->layers.size(); l++) {
         const LayerDev& L = m->layers[l];
+        const LayerDev* nx = l + 1 < m->layers.size() ? &m->layers[l + 1] : nullptr;
+        float* Hout = nx ? H0 : dout;
         // this layer's [q | k | v] rows, ld floats apart, and attention rows qd apart
         const size_t qd = static_cast<size_t>(L.nq) * L.hd, kvd = static_cast<size_t>(L.nkv) * L.hd, ld = qd + 2 * kvd;
-        if (!xn_ready) larql::launch_rmsnorm_rows(H0, L.input_norm, L.norm_offset, XN, M, hidden, L.eps, s);
-        pj.input();
-        if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
-            pj.run(L.wq, false, XN, QKV, ld, xn_st, xn_ready);
-            pj.run(L.wk, false, XN, QKV + qd, ld, xn_st, xn_ready);
-            pj.run(L.wv, false, XN, QKV + qd + kvd, ld, xn_st, xn_ready);
-        } else {
-            pj.run(L.qkv, false, XN, QKV, ld, xn_st, xn_ready);
+        if (!fused) {
+            larql::launch_rmsnorm_rows(Hin, L.input_norm, L.norm_offset, XN, M, hidden, L.eps, s);
+            pj.input(XN, false);
         }
-        xn_ready = false;
+        if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
+            pj.run(L.wq, false, XN, QKV, ld, xn_st);
+            pj.run(L.wk, false, XN, QKV + qd, ld, xn_st);
+            pj.run(L.wv, false, XN, QKV + qd + kvd, ld, xn_st);
+        } else {
+            pj.run(L.qkv, false, XN, QKV, ld, xn_st);
+        }
         if (L.v_norm) larql::launch_vnorm_rows(QKV + qd + kvd, M, ld, L.nkv, L.hd, L.eps, s);
         const float2* rope = rope_table(c, L.rope_base, L.rdim, s);
         larql::launch_rope_kv_rows(QKV, M, 0, qd, kvd, L.hd, L.rdim, rope, kv.k[l], kv.v[l], L.nkv, s);
@@ -967,57 +1030,67 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
         at.softcap = pa.softcap;
         larql::launch_attention(at, s);
         const float scale = L.layer_scalar != 0.0f ? L.layer_scalar : 1.0f;
-        // the split sums of wo and down, the residual adds, the next norm and the row
-        // statistics of the next GEMM's input: one row kernel after each projection, unless
-        // the projection's output is normed before its residual add
-        const bool fused = !L.post_norms && hidden <= larql::kFusedRowMax && inter <= larql::kFusedRowMax;
-        larql::GemmSplits sp{};
-        pj.input();
-        pj.run(L.wo, false, ATT, G, hidden, att_st, false, fused ? &sp : nullptr);
+        const float* fnorm = L.post_norms ? L.pre_ffn_norm : L.post_attn_norm;
+        const float foff = L.post_norms && !L.pre_ffn_norm ? 0.0f : L.norm_offset;
+        larql::GemmSplits sp{nullptr, 1};
+        pj.input(ATT, false);
+        pj.run(L.wo, false, ATT, G, hidden, att_st, fused ? &sp : nullptr);
         if (fused) {
-            larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H0, 1.0f, H1,
-                                                L.post_attn_norm, L.norm_offset, XN, M, hidden, L.eps, xn_st, s);
-        } else if (L.post_norms) {
-            larql::launch_resid_norm_rows(H0, G, L.post_attn_norm, L.norm_offset, 1.0f, H1, M, hidden, L.eps, s);
-            larql::launch_rmsnorm_rows(H1, L.pre_ffn_norm, L.pre_ffn_norm ? L.norm_offset : 0.0f, XN, M, hidden, L.eps, s);
+            rows(Hin, G, sp, L.post_norms, L.post_attn_norm, L.norm_offset, L.eps, 1.0f, H1, true, fnorm, foff, L.eps,
+                 L.split_gu, !L.split_gu);
         } else {
-            larql::launch_add_rows(H0, G, H1, M * hidden, s);
-            larql::launch_rmsnorm_rows(H1, L.post_attn_norm, L.norm_offset, XN, M, hidden, L.eps, s);
+            if (L.post_norms)
+                larql::launch_resid_norm_rows(Hin, G, L.post_attn_norm, L.norm_offset, 1.0f, H1, M, hidden, L.eps, s);
+            else
+                larql::launch_add_rows(Hin, G, H1, M * hidden, s);
+            larql::launch_rmsnorm_rows(H1, fnorm, foff, XN, M, hidden, L.eps, s);
+            pj.input(XN, false);
         }
-        pj.input();
-        bool act_ready = false;  // act_st holds ACT's statistics
+        const float* U = nullptr;  // up rows apart from the gate rows in G
+        sp = {nullptr, 1};
         if (L.split_gu) {
-            float* U = G + M * inter;
+            float* up = G + M * inter;
+            U = up;
             pj.quantize(XN, hidden);
             if (L.gate.format == LARQL_Q4_0 && L.up.format == LARQL_Q4_0) {
-                larql::launch_q4_0_matvec_pair(L.gate, L.up, pj.q8, pj.q8s, G, U, M, s);
+                larql::launch_q4_0_matvec_pair(L.gate, L.up, pj.q8, pj.q8s, G, up, M, s);
             } else {
-                pj.run(L.gate, false, XN, G, inter, xn_st, fused);
-                pj.run(L.up, false, XN, U, inter, xn_st, fused);
+                pj.run(L.gate, false, XN, G, inter, xn_st);
+                pj.run(L.up, false, XN, up, inter, xn_st);
             }
+        } else {
+            pj.run(L.gateup, false, XN, G, 2 * inter, xn_st, fused ? &sp : nullptr);
+        }
+        const bool down_q8 = takes_q8(L.down, true);
+        if (fused) {
+            larql::GemmRowStats st{};
+            if (!down_q8) {
+                st = act_st;
+                st.xp = XP;
+            }
+            larql::launch_gated_stats_rows(sp.splits > 1 ? sp.part : G, M * 2 * inter, sp.splits, U,
+                                           down_q8 ? ACT : nullptr, M, inter, L.act, st, s);
+        } else if (U) {
             larql::launch_gated_mul(G, U, ACT, M * inter, L.act, s);
         } else {
-            pj.run(L.gateup, false, XN, G, 2 * inter, xn_st, fused);
-            if (fused) larql::launch_gated_pair_stats_rows(G, ACT, M, inter, L.act, act_st, s);
-            else larql::launch_gated_pair_rows(G, ACT, M * inter, L.act, s);
-            act_ready = fused;
+            larql::launch_gated_pair_rows(G, ACT, M * inter, L.act, s);
         }
-        pj.input();
-        pj.run(L.down, true, ACT, G, hidden, act_st, act_ready, fused ? &sp : nullptr);
-        const LayerDev* nx = l + 1 < m->layers.size() ? &m->layers[l + 1] : nullptr;
+        pj.input(ACT, fused && !down_q8);
+        sp = {nullptr, 1};
+        pj.run(L.down, true, ACT, G, hidden, act_st, fused ? &sp : nullptr);
         if (fused) {
-            larql::launch_resid_norm_stats_rows(sp.splits > 1 ? sp.part : G, M * hidden, sp.splits, H1, scale, H0,
-                                                nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f,
-                                                nx ? XN : nullptr, M, hidden, nx ? nx->eps : 0.0, xn_st, s);
-            xn_ready = nx != nullptr;
+            rows(H1, G, sp, L.post_norms, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, L.eps, scale, Hout,
+                 nx != nullptr, nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f, nx ? nx->eps : 0.0,
+                 nx && qkv_f32(*nx), nx && qkv_packed(*nx));
         } else if (L.post_norms) {
-            larql::launch_resid_norm_rows(H1, G, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, scale, H0, M,
+            larql::launch_resid_norm_rows(H1, G, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, scale, Hout, M,
                                           hidden, L.eps, s);
         } else {
-            larql::launch_add_rows(H1, G, H0, M * hidden, s, scale);
+            larql::launch_add_rows(H1, G, Hout, M * hidden, s, scale);
         }
+        Hin = H0;
     }
-    larql::launch_copy_f32(H0, dout, M * hidden, s);
+    if (m->layers.empty()) larql::launch_copy_f32(dx, dout, M * hidden, s);
     kv.current_len = M;
 }
 

@@ -69,17 +69,36 @@ void launch_gated_mul(const float* G, const float* U, float* act, size_t n, int 
 // act[i] = act(GU[2i]) * GU[2i + 1]; kind 0 = SiLU, 1 = GELU-tanh.
 void launch_gated_pair_rows(const float* GU, float* act, size_t n, int kind, hipStream_t s);
 // Fused forms of the prompt pass, per row of n floats (n a multiple of 32, at most
-// kFusedRowMax: the row is held in LDS), each value
-// as the separate kernels compute it: hout = (hin + the projection row, its `splits`
-// partial products summed in split order, pstride floats apart) * scale; then, with xn,
-// xn = hout / rms(hout) * (off + w) and xn's GEMM row statistics into st.
+// kFusedRowMax: the row is held in LDS), each value as the separate kernels compute it.
 constexpr int kFusedRowMax = 16384;
-void launch_resid_norm_stats_rows(const float* P, size_t pstride, int splits, const float* hin, float scale,
-                                  float* hout, const float* w, float off, float* xn, size_t m, size_t n, double eps,
-                                  const GemmRowStats& st, hipStream_t s);
-// act rows (m x n) as launch_gated_pair_rows, with their GEMM row statistics into st.
-void launch_gated_pair_stats_rows(const float* GU, float* act, size_t m, size_t n, int kind, const GemmRowStats& st,
-                                  hipStream_t s);
+struct ResidRows {
+    // the projection row, its `splits` partial products summed in split order, pstride floats
+    // apart (null: h = hin)
+    const float* P = nullptr;
+    size_t pstride = 0;
+    int splits = 1;
+    const float* hin = nullptr;
+    // post-norm layers: the projection normed (weight pw, null for none) before the residual add
+    bool post = false;
+    const float* pw = nullptr;
+    float poff = 0.f;
+    double eps = 0.0;
+    float scale = 1.0f;     // h = (hin + y) * scale
+    float* hout = nullptr;  // h, if wanted
+    // x = h / rms(h) * (off + w) (w null: no weight), or h itself
+    bool norm = false;
+    const float* w = nullptr;
+    float off = 0.f;
+    double norm_eps = 0.0;
+    float* xn = nullptr;    // x (norm only), if wanted
+    GemmRowStats st{};      // x's GEMM row statistics and packed operands, if wanted
+    int m = 0, n = 0;
+};
+void launch_resid_norm_stats_rows(const ResidRows& a, hipStream_t s);
+// act(gate) * up rows (m x n) from interleaved pairs (K-split partial products pstride floats
+// apart) or, with U, separate rows: to act and with st, each if wanted.
+void launch_gated_stats_rows(const float* G, size_t pstride, int splits, const float* U, float* act, size_t m, size_t n,
+                             int kind, const GemmRowStats& st, hipStream_t s);
 void launch_f32_to_f16(const float* src, __half* dst, size_t n, hipStream_t s);
 
 }  // namespace larql

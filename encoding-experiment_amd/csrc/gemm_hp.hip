@@ -15,52 +15,17 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "gemm_hp.h"
 #include "larql_hip_internal.h"
 
 namespace larql {
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-
 constexpr int kPkWaves = 4;             // waves per workgroup, side by side along N
 constexpr int kPkR = 4;                 // 16-row weight tiles per wave
 constexpr int kPkRows = 16 * kPkR * kPkWaves;  // 256 weight rows per workgroup
 constexpr int kPkThreads = 64 * kPkWaves;
-
-// v - (f32) the low / high f16 half of h2, one v_fma_mix_f32 (the half widened inside the
-// instruction; written out because the compiler otherwise emits a conversion and a subtract)
-__device__ __forceinline__ float sub_f16_lo(float v, uint32_t h2) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(v));
-    return r;
-}
-__device__ __forceinline__ float sub_f16_hi(float v, uint32_t h2) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(v));
-    return r;
-}
-
-// {a, b} -> hi pair {fp16(a), fp16(b)} and lo pair {fp16(a - hi_a), fp16(b - hi_b)}
-__device__ __forceinline__ void hp_split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
-    const float la = sub_f16_lo(a, hi), lb = sub_f16_hi(b, hi);
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){la, lb}, f16x2));
-}
-
-// Eight f32 values -> their hi and lo operands.
-__device__ __forceinline__ void hp_split8(const float (&v)[8], v4u& hi, v4u& lo) {
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) hp_split2(v[2 * i], v[2 * i + 1], h[i], l[i]);
-    hi = v4u{h[0], h[1], h[2], h[3]};
-    lo = v4u{l[0], l[1], l[2], l[3]};
-}
 
 // One workgroup per row: the row's exponent and (with xs) scaled sub-block sums
 // (gemm_row_stats).
@@ -70,10 +35,8 @@ __global__ __launch_bounds__(256) void row_exp_kernel(const float* __restrict__ 
                    xs ? xs + static_cast<size_t>(blockIdx.x) * (K / 32) : nullptr);
 }
 
-// X [M x K] -> XP[token tile][k-step][hi, lo][64 lanes][16 B]: lane 16 g + i holds elements
-// 8 g .. 8 g + 7 of the k-step (one 32-element sub-block) of token i times its power of two, in
-// the order the nibbles of a weight dword unpack, (0, 2), (4, 6), (1, 3), (5, 7).  Tokens past M
-// are zeros.  Grid (K / 128, token tiles); wave w = k-step w of the workgroup's four.
+// X [M x K] -> the packed operands (hp_packed_at), each token times its power of two; tokens past
+// M are zeros.  Grid (K / 128, token tiles); wave w = k-step w of the workgroup's four.
 __global__ __launch_bounds__(256) void x_pack_kernel(const float* __restrict__ X, const int* __restrict__ xe,
                                                      v4u* __restrict__ XP, int M, int K) {
     const int lane = threadIdx.x & 63, ks = blockIdx.x * 4 + (threadIdx.x >> 6), g = lane >> 4;
@@ -87,7 +50,7 @@ __global__ __launch_bounds__(256) void x_pack_kernel(const float* __restrict__ X
     for (int k = 0; k < 8; k++) e[k] = m < M ? e[k] * sc : 0.0f;
     v4u hi, lo;
     hp_split8(e, hi, lo);
-    v4u* o = XP + ((static_cast<size_t>(blockIdx.y) * (K / 32) + ks) * 2) * 64 + lane;
+    v4u* o = XP + hp_packed_at(m, 4 * ks + g, K);
     o[0] = hi;
     o[64] = lo;
 }

@@ -14,6 +14,7 @@
 //     (LI/src/residual.rs:86-110) and the layer scalar.  These kernels also serve the
 //     decode step (one row).
 #include "decode.h"
+#include "gemm_hp.h"
 #include "matvec_common.h"
 
 namespace larql {
@@ -117,13 +118,20 @@ __global__ void gated_mul_kernel(const float* __restrict__ G, const float* __res
 // chunk and two workgroup barriers instead of a dependent load per element.
 constexpr int kRowChunk = 16;  // elements per thread per chunk
 
-// The row's exponent (every thread gets it; thread 0 stores it) and, with xs, its scaled
-// sub-block sums from the row in LDS: the arithmetic of gemm_row_stats, whose maximum is
-// order-free and whose sums run per sub-block in one thread.  m: this thread's max |x|;
-// wm: one float per wave.
+// Workgroup -> row, the 16 rows of a token tile on one XCD (workgroup i runs on XCD i % 8): the
+// packed operands of a tile share 128-byte lines, which that XCD's L2 then fills whole.  Grids
+// are whole groups of 128 rows.
+__device__ __forceinline__ int tile_row() {
+    const int j = static_cast<int>(blockIdx.x) >> 3;
+    return ((j >> 4) * 8 + (static_cast<int>(blockIdx.x) & 7)) * 16 + (j & 15);
+}
+
+// The statistics of row r (n floats in LDS, written by all threads) into st: its exponent and,
+// with st.xs, its scaled sub-block sums, the arithmetic of gemm_row_stats, whose maximum is
+// order-free and whose sums run per sub-block in one thread; with st.xp the row packed.  m:
+// this thread's max |x|; wm: one float per wave.
 template <int NT>
-__device__ __forceinline__ void lds_row_stats(const float* row, int n, float m, float* wm, int* __restrict__ e,
-                                              float* __restrict__ xs) {
+__device__ __forceinline__ void lds_row_out(const float* row, int n, int r, float m, float* wm, const GemmRowStats& st) {
     const int t = threadIdx.x;
     m = wave_max(m);
     if ((t & 63) == 0) wm[t >> 6] = m;
@@ -132,8 +140,13 @@ __device__ __forceinline__ void lds_row_stats(const float* row, int n, float m, 
 #pragma unroll
     for (int k = 1; k < NT / 64; k++) m = fmaxf(m, wm[k]);
     const int ev = (m > 0.f && m <= 3.4e38f) ? min(120, max(-120, 14 - ilogbf(m))) : 0;
-    if (t == 0) *e = ev;
-    if (!xs) return;
+    if (t == 0) st.xe[r] = ev;
+    if (st.xp) {
+        const float sc = ldexpf(1.0f, ev);
+        for (int e8 = t; e8 < n / 8; e8 += NT) hp_pack8(row + 8 * e8, sc, reinterpret_cast<v4u*>(st.xp) + hp_packed_at(r, e8, n));
+    }
+    if (!st.xs) return;
+    float* xs = st.xs + static_cast<size_t>(r) * (n / 32);
     const double sc = ldexp(1.0, ev - 5);
     for (int j = t; j < n / 32; j += NT) {
         const float4* p = reinterpret_cast<const float4*>(row + 32 * j);
@@ -148,105 +161,173 @@ __device__ __forceinline__ void lds_row_stats(const float* row, int n, float m, 
     }
 }
 
-// Grid M rows; 256 threads.  The residual step after a projection and the next
-// projection's input, per row of n floats, in the arithmetic of the separate kernels:
-//   y = the projection row, its `splits` partial products summed in split order (split z
-//       at P + z pstride; splits 1: P is the row itself)             (sum_splits_kernel);
-//   hout = (hin + y) * scale                                          (add_rows_kernel);
-//   and with xn: xn = (hout * (1 / rms(hout))) * (off + w)            (rmsnorm_rows_kernel,
-//   the f64 sum of squares over the same 256 threads, element i in thread i % 256, in the
-//   same order) with its row statistics for the next GEMM             (gemm_row_stats).
-__global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(
-    const float* __restrict__ P, size_t pstride, int splits, const float* __restrict__ hin, float scale,
-    float* __restrict__ hout, const float* __restrict__ w, float off, float* __restrict__ xn, int n, double eps,
-    int* __restrict__ xe, float* __restrict__ xs) {
+// f64 sum of ss over the 256 threads.
+__device__ __forceinline__ double block_sum_d(double ss, double* red) {
+    ss = wave_sum_d(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// The step between two projections, per row of n floats (256 threads), in the arithmetic of the
+// separate kernels:
+//   y = the projection row, its partial products summed in split order (sum_splits_kernel),
+//       four splits' loads at a time;
+//   POST: y = (y / rms(y)) * (poff + pw)                             (resid_norm_rows_kernel);
+//   h = (hin + y) * scale, or hin itself without a projection        (add_rows_kernel);
+//   x = norm ? (h * (1 / rms(h))) * (off + w) : h                    (rmsnorm_rows_kernel; every
+//       f64 sum of squares over the same 256 threads, element i in thread i % 256, in the same
+//       order);
+// h to hout, x to xn (each if given), and x's statistics and packed operands (if st.xe).
+template <bool POST>
+__global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(ResidRows a) {
     __shared__ __align__(16) float row[kFusedRowMax];
-    __shared__ double red[4];
+    __shared__ double red[2][4];
     __shared__ float wm[4];
-    const int t = threadIdx.x;
-    const size_t r = static_cast<size_t>(blockIdx.x) * n;
+    const int t = threadIdx.x, ri = tile_row(), n = a.n;
+    if (ri >= a.m) return;
+    const size_t r = static_cast<size_t>(ri) * n;
     double ss = 0.0;
+    float m = 0.f;
     float w0[kRowChunk];  // the norm weights of the first chunk, requested with its rows
     for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
-        float a[kRowChunk], h[kRowChunk];
+        float y[kRowChunk], h[kRowChunk];
 #pragma unroll
         for (int q = 0; q < kRowChunk; q++) {
             const size_t i = r + min(c0 + t + 256 * q, n - 1);
-            a[q] = P[i];
-            h[q] = hin[i];
+            y[q] = a.P ? a.P[i] : 0.f;
+            h[q] = POST ? 0.f : a.hin[i];
         }
         if (c0 == 0) {
 #pragma unroll
-            for (int q = 0; q < kRowChunk; q++) w0[q] = w && xn ? w[min(t + 256 * q, n - 1)] : 0.f;
+            for (int q = 0; q < kRowChunk; q++) w0[q] = a.w ? a.w[min(t + 256 * q, n - 1)] : 0.f;
         }
-        for (int z = 1; z < splits; z++) {
+        for (int z = 1; z < a.splits; z += 4) {
+            float v[4][kRowChunk];
 #pragma unroll
-            for (int q = 0; q < kRowChunk; q++) a[q] += P[z * pstride + r + min(c0 + t + 256 * q, n - 1)];
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int q = 0; q < kRowChunk; q++)
+                    v[k][q] = a.P[min(z + k, a.splits - 1) * a.pstride + r + min(c0 + t + 256 * q, n - 1)];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (z + k < a.splits)
+#pragma unroll
+                    for (int q = 0; q < kRowChunk; q++) y[q] += v[k][q];
         }
 #pragma unroll
         for (int q = 0; q < kRowChunk; q++) {
             const int i = c0 + t + 256 * q;
             if (i < n) {
-                const float hv = (h[q] + a[q]) * scale;
-                hout[r + i] = hv;
+                const float hv = POST ? y[q] : (a.P ? (h[q] + y[q]) * a.scale : h[q]);
+                if (!POST && a.hout) a.hout[r + i] = hv;
                 row[i] = hv;
                 ss += static_cast<double>(hv) * hv;
+                m = fmaxf(m, fabsf(hv));
             }
         }
     }
-    if (!xn) return;  // (uniform)
-    ss = wave_sum_d(ss);
-    if ((t & 63) == 0) red[t >> 6] = ss;
-    __syncthreads();
-    const double tot = (red[0] + red[1]) + (red[2] + red[3]);
-    const float inv = 1.0f / static_cast<float>(sqrt(tot / static_cast<double>(n) + eps));
+    if constexpr (POST) {  // (a thread's own elements of `row` throughout)
+        const double tot = block_sum_d(ss, red[0]);
+        const float inv = 1.0f / static_cast<float>(sqrt(tot / static_cast<double>(n) + a.eps));
+        ss = 0.0, m = 0.f;
+        for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
+            float h[kRowChunk], wv[kRowChunk];
+#pragma unroll
+            for (int q = 0; q < kRowChunk; q++) {
+                const int i = min(c0 + t + 256 * q, n - 1);
+                h[q] = a.hin[r + i];
+                wv[q] = a.pw ? a.pw[i] : 0.f;
+            }
+#pragma unroll
+            for (int q = 0; q < kRowChunk; q++) {
+                const int i = c0 + t + 256 * q;
+                if (i < n) {
+                    const float nv = a.pw ? (row[i] * inv) * (a.poff + wv[q]) : row[i] * inv;
+                    const float hv = (h[q] + nv) * a.scale;
+                    if (a.hout) a.hout[r + i] = hv;
+                    row[i] = hv;
+                    ss += static_cast<double>(hv) * hv;
+                    m = fmaxf(m, fabsf(hv));
+                }
+            }
+        }
+    }
+    if (!a.norm && !a.st.xe) return;  // (uniform)
+    if (a.norm) {
+        const double tot = block_sum_d(ss, red[1]);
+        const float inv = 1.0f / static_cast<float>(sqrt(tot / static_cast<double>(n) + a.norm_eps));
+        m = 0.f;
+        for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
+            float wv[kRowChunk];
+#pragma unroll
+            for (int q = 0; q < kRowChunk; q++) wv[q] = c0 == 0 ? w0[q] : (a.w ? a.w[min(c0 + t + 256 * q, n - 1)] : 0.f);
+#pragma unroll
+            for (int q = 0; q < kRowChunk; q++) {
+                const int i = c0 + t + 256 * q;
+                if (i < n) {  // (the thread's own elements of `row`: no barrier needed)
+                    const float x = a.w ? (row[i] * inv) * (a.off + wv[q]) : row[i] * inv;
+                    if (a.xn) a.xn[r + i] = x;
+                    row[i] = x;
+                    m = fmaxf(m, fabsf(x));
+                }
+            }
+        }
+    }
+    if (a.st.xe) lds_row_out<256>(row, n, ri, m, wm, a.st);
+}
+
+// act = act(gate) * up over a row of n outputs (1024 threads), from gate/up rows with the pairs
+// interleaved (as gated_pair_rows_kernel; K-split partial products summed in split order) or, with
+// U, from separate rows (gated_mul_kernel); to act if given, with its statistics and packed
+// operands for the down projection.
+__global__ __launch_bounds__(1024) void gated_stats_rows_kernel(const float* __restrict__ G, size_t pstride, int splits,
+                                                                const float* __restrict__ U, float* __restrict__ act,
+                                                                int M, int n, int kind, GemmRowStats st) {
+    constexpr int kChunk = 8;
+    __shared__ __align__(16) float row[kFusedRowMax];
+    __shared__ float wm[16];
+    const int t = threadIdx.x, ri = tile_row();
+    if (ri >= M) return;
+    const size_t r = static_cast<size_t>(ri) * n;
     float m = 0.f;
-    for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
-        float wv[kRowChunk];
+    for (int c0 = 0; c0 < n; c0 += 1024 * kChunk) {
+        float2 v[kChunk];
+        if (U) {
 #pragma unroll
-        for (int q = 0; q < kRowChunk; q++) wv[q] = c0 == 0 ? w0[q] : (w ? w[min(c0 + t + 256 * q, n - 1)] : 0.f);
+            for (int q = 0; q < kChunk; q++) {
+                const size_t i = r + min(c0 + t + 1024 * q, n - 1);
+                v[q] = make_float2(G[i], U[i]);
+            }
+        } else {
 #pragma unroll
-        for (int q = 0; q < kRowChunk; q++) {
-            const int i = c0 + t + 256 * q;
-            if (i < n) {  // (the thread's own elements of `row`: no barrier needed)
-                const float x = w ? (row[i] * inv) * (off + wv[q]) : row[i] * inv;
-                xn[r + i] = x;
+            for (int q = 0; q < kChunk; q++) v[q] = reinterpret_cast<const float2*>(G)[r + min(c0 + t + 1024 * q, n - 1)];
+            for (int z = 1; z < splits; z += 2) {
+                float2 p[2][kChunk];
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int q = 0; q < kChunk; q++)
+                        p[k][q] = reinterpret_cast<const float2*>(G + min(z + k, splits - 1) * pstride)[r + min(c0 + t + 1024 * q, n - 1)];
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+                    if (z + k < splits)
+#pragma unroll
+                        for (int q = 0; q < kChunk; q++) v[q].x += p[k][q].x, v[q].y += p[k][q].y;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kChunk; q++) {
+            const int i = c0 + t + 1024 * q;
+            if (i < n) {
+                const float x = gated_act(kind, v[q].x, v[q].y);
+                if (act) act[r + i] = x;
                 row[i] = x;
                 m = fmaxf(m, fabsf(x));
             }
         }
     }
-    lds_row_stats<256>(row, n, m, wm, xe + blockIdx.x, xs ? xs + static_cast<size_t>(blockIdx.x) * (n / 32) : nullptr);
-}
-
-// Grid M rows; 1024 threads.  act = act(gate) * up over a row of n outputs from the
-// gate/up row (pairs interleaved, as gated_pair_rows_kernel), with act's row statistics
-// for the down GEMM.
-__global__ __launch_bounds__(1024) void gated_pair_stats_rows_kernel(const float* __restrict__ GU,
-                                                                     float* __restrict__ act, int n, int kind,
-                                                                     int* __restrict__ xe, float* __restrict__ xs) {
-    __shared__ __align__(16) float row[kFusedRowMax];
-    __shared__ float wm[16];
-    const int t = threadIdx.x;
-    const size_t r = static_cast<size_t>(blockIdx.x) * n;
-    const float2* gu = reinterpret_cast<const float2*>(GU) + r;
-    float m = 0.f;
-    for (int c0 = 0; c0 < n; c0 += 1024 * kRowChunk) {
-        float2 v[kRowChunk];
-#pragma unroll
-        for (int q = 0; q < kRowChunk; q++) v[q] = gu[min(c0 + t + 1024 * q, n - 1)];
-#pragma unroll
-        for (int q = 0; q < kRowChunk; q++) {
-            const int i = c0 + t + 1024 * q;
-            if (i < n) {
-                const float a = gated_act(kind, v[q].x, v[q].y);
-                act[r + i] = a;
-                row[i] = a;
-                m = fmaxf(m, fabsf(a));
-            }
-        }
-    }
-    lds_row_stats<1024>(row, n, m, wm, xe + blockIdx.x, xs ? xs + static_cast<size_t>(blockIdx.x) * (n / 32) : nullptr);
+    if (st.xe) lds_row_out<1024>(row, n, ri, m, wm, st);
 }
 
 unsigned blocks(size_t n) { return static_cast<unsigned>((n + 255) / 256); }
@@ -297,24 +378,26 @@ void launch_gated_mul(const float* G, const float* U, float* act, size_t n, int 
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
-void launch_resid_norm_stats_rows(const float* P, size_t pstride, int splits, const float* hin, float scale,
-                                  float* hout, const float* w, float off, float* xn, size_t m, size_t n, double eps,
-                                  const GemmRowStats& st, hipStream_t s) {
-    if (m == 0) return;
-    if (splits < 1 || n % 32 != 0 || n > static_cast<size_t>(kFusedRowMax) || (xn && !st.xe))
+static dim3 tile_rows_grid(size_t m) { return dim3(static_cast<unsigned>((m + 127) / 128 * 128)); }
+
+void launch_resid_norm_stats_rows(const ResidRows& a, hipStream_t s) {
+    if (a.m == 0) return;
+    if (a.m > 0x7FFFFF00 || a.splits < 1 || a.n % 32 != 0 || a.n > kFusedRowMax || !a.hin || (a.post && !a.P) ||
+        (a.st.xp && !a.st.xe))
         fail(LARQL_HIP_ERR_INVALID, "fused residual and norm rows: bad arguments");
-    resid_norm_stats_rows_kernel<<<dim3(static_cast<unsigned>(m)), dim3(256), 0, s>>>(
-        P, pstride, splits, hin, scale, hout, w, off, xn, static_cast<int>(n), eps, st.xe, st.xs);
+    if (a.post) resid_norm_stats_rows_kernel<true><<<tile_rows_grid(a.m), dim3(256), 0, s>>>(a);
+    else resid_norm_stats_rows_kernel<false><<<tile_rows_grid(a.m), dim3(256), 0, s>>>(a);
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
-void launch_gated_pair_stats_rows(const float* GU, float* act, size_t m, size_t n, int kind, const GemmRowStats& st,
-                                  hipStream_t s) {
+void launch_gated_stats_rows(const float* G, size_t pstride, int splits, const float* U, float* act, size_t m, size_t n,
+                             int kind, const GemmRowStats& st, hipStream_t s) {
     if (m == 0) return;
-    if (n % 32 != 0 || n > static_cast<size_t>(kFusedRowMax) || !st.xe)
+    if (m > 0x7FFFFF00 || splits < 1 || (U && splits != 1) || n % 32 != 0 || n > static_cast<size_t>(kFusedRowMax) ||
+        (st.xp && !st.xe))
         fail(LARQL_HIP_ERR_INVALID, "fused gated rows: bad arguments");
-    gated_pair_stats_rows_kernel<<<dim3(static_cast<unsigned>(m)), dim3(1024), 0, s>>>(GU, act, static_cast<int>(n),
-                                                                                       kind, st.xe, st.xs);
+    gated_stats_rows_kernel<<<tile_rows_grid(m), dim3(1024), 0, s>>>(G, pstride, splits, U, act, static_cast<int>(m),
+                                                                   static_cast<int>(n), kind, st);
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
