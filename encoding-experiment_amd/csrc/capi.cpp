@@ -297,6 +297,19 @@ extern "C" int larql_hip_q4k_matvec(larql_hip_ctx* c, const uint8_t* q4k_data, s
     });
 }
 
+// m activation rows through a Q4_K weight: the matvec, the f32-accuracy GEMM for small batches,
+// the fp16 GEMM.
+static void q4k_rows(larql_hip_ctx* c, const DevWeight& w, const float* x, float* out, size_t m, hipStream_t s) {
+    if (larql::gemm_f32_small_batch(w, m)) {
+        const size_t pf = larql::gemm_f32_part_floats(w, m, true);
+        float* part = static_cast<float*>(larql::ensure(c, c->gemm_x16, pf * sizeof(float)));
+        larql::launch_gemm_f32(w, x, out, m, part, pf, s, 0, nullptr, nullptr, true);
+        return;
+    }
+    void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, larql::q4k_gemm_ws_bytes(m, w.cols)) : nullptr;
+    larql::launch_q4k_matvec(w, x, out, m, ws, s);
+}
+
 extern "C" int larql_hip_q4k_matmul(larql_hip_ctx* c, const uint8_t* q4k_data, size_t q4k_len, const float* x,
                                     size_t m, float* out, size_t num_rows, size_t hidden) {
     return guarded(c, [&] {
@@ -304,8 +317,7 @@ extern "C" int larql_hip_q4k_matmul(larql_hip_ctx* c, const uint8_t* q4k_data, s
         const DevWeight& w = larql::cached_weight(c, LARQL_Q4_K, q4k_data, q4k_len, nullptr, num_rows, hidden);
         const float* dx = stage_upload(c, c->stage_in, x, m * hidden);
         float* dout = static_cast<float*>(larql::ensure(c, c->stage_out, m * num_rows * sizeof(float)));
-        void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, larql::q4k_gemm_ws_bytes(m, hidden)) : nullptr;
-        larql::launch_q4k_matvec(w, dx, dout, m, ws, c->stream);
+        q4k_rows(c, w, dx, dout, m, c->stream);
         download(c, out, dout, m * num_rows * sizeof(float));
     });
 }
@@ -487,8 +499,7 @@ extern "C" int larql_hip_matvec_dev(larql_hip_ctx* c, uint64_t handle, const voi
         hipStream_t s = pick_stream(c, stream);
         switch (w.format) {
             case LARQL_Q4_K: {
-                void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, larql::q4k_gemm_ws_bytes(m, w.cols)) : nullptr;
-                larql::launch_q4k_matvec(w, static_cast<const float*>(x), out, m, ws, s);
+                q4k_rows(c, w, static_cast<const float*>(x), out, m, s);
                 break;
             }
             case LARQL_Q4_KF:  // one matvec per activation row

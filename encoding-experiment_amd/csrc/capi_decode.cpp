@@ -888,17 +888,7 @@ struct PromptProj {
     void pack(const float* X, size_t K, larql::GemmRowStats& st) {
         st.xp = xp;
         if (packed == X) return;
-        if (K <= static_cast<size_t>(larql::kFusedRowMax)) {
-            larql::ResidRows r;
-            r.hin = X;
-            r.st = st;
-            r.m = static_cast<int>(M);
-            r.n = static_cast<int>(K);
-            larql::launch_resid_norm_stats_rows(r, s);
-        } else {
-            larql::launch_gemm_row_stats(X, M, K, st, s);
-            larql::launch_gemm_x_pack(X, M, K, st, s);
-        }
+        larql::launch_gemm_pack_rows(X, M, K, st, s);
         packed = X;
     }
     void quantize(const float* X, size_t K) {

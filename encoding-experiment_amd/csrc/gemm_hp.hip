@@ -14,6 +14,7 @@
 // while each wave turns its own weight rows into operands in registers.
 #include <type_traits>
 
+#include "decode.h"
 #include "device_common.h"
 #include "gemm_hp.h"
 #include "larql_hip_internal.h"
@@ -151,8 +152,7 @@ struct PkArgs {
 // exact in f32; only the split's 2^-22 is lost), a fresh accumulator per super-block, added into
 // the total times d.  The min term follows the K loop: the sub-block sums X_j 2^(e - 5) against
 // -32 dmin m_j per row, both as fp16 pairs (three products), 32 sub-blocks per k-step.  A lane's
-// 16-byte nibble load holds one sub-block, transposed across the lane groups.  Weights need dmin
-// below ~136 (fp16 range of 32 dmin m_j); d has no limit.
+// 16-byte nibble load holds one sub-block, transposed across the lane groups.
 //
 // Q6_K: w = d sc (q - 32) per 16-element group; sc (q - 32) reaches 4096, past fp16's exact
 // integers, so it is split exactly, hi = fp16(sc (q - 32)) and lo the rest (at most 1): three
@@ -438,7 +438,20 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                     v4u, __builtin_amdgcn_raw_buffer_load_b128(rh, hl + static_cast<uint32_t>(sbc) * 256u, ho[j], 0));
 #pragma unroll
             for (int j = 0; j < kPkR; j++) {
-                const float nd = sv ? -32.0f * h2f(hd[j].x >> 16) : 0.f;
+                // -32 dmin m_j (32: small minima keep their low parts above fp16's smallest step);
+                // a row with |dmin| past fp16's range of that takes -dmin m_j / 16 and its sums
+                // 2^-9 times as large for the time being
+                const float dmin = sv ? h2f(hd[j].x >> 16) : 0.f;
+                float nd = -32.0f * dmin, back = 1.0f;
+                const bool wide = __builtin_amdgcn_ballot_w64(fabsf(dmin) >= 128.0f) != 0;
+                if (wide) {
+                    float mx = fabsf(dmin);
+                    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                    if (mx >= 128.0f) nd = -0.0625f * dmin, back = 512.0f;
+#pragma unroll
+                    for (int i = 0; i < TT; i++) acc[j][i] *= 1.0f / back;
+                }
                 float cm[8];
 #pragma unroll
                 for (int k = 0; k < 8; k++)
@@ -452,6 +465,10 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                     acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, Bh, acc[j][i], 0, 0, 0);
                     acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, Bl, acc[j][i], 0, 0, 0);
                     acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, Bh, acc[j][i], 0, 0, 0);
+                }
+                if (wide) {
+#pragma unroll
+                    for (int i = 0; i < TT; i++) acc[j][i] *= back;
                 }
             }
         }
@@ -476,11 +493,44 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
         }
 }
 
+// The dot of weight row `row` (Q4_K) and x as a plain f32 sum: for a token with an infinite
+// element, whose packed operands give NaN although its products with nonzero weights are
+// infinite.
+__device__ __forceinline__ float q4k_plain_dot(const uint8_t* qs, const uint4* hdr, const float* x, int row, int K) {
+    const size_t S = static_cast<size_t>(K) / 256;
+    float acc = 0.f;
+#pragma unroll 1
+    for (size_t sb = 0; sb < S; sb++) {
+        const uint4 h = hdr[q4k_hdr_index(row, sb, S)];
+        const float d = h2f(h.x & 0xFFFFu), dmin = h2f(h.x >> 16);
+#pragma unroll 1
+        for (int j = 0; j < 8; j++) {
+            const float sc = d * static_cast<float>(((j < 4 ? h.y : h.z) >> (8 * (j & 3))) & 0x3Fu);
+            const float mn = dmin * static_cast<float>((h.w >> (8 * (j & 3) + 4 * (j >> 2))) & 0xFu);
+            const uint8_t* q = qs + q4k_sub_offset(row, sb, j, S);
+#pragma unroll 1
+            for (int b = 0; b < 16; b++) {
+                const float* xe = x + 256 * sb + 32 * j + 2 * b;
+                acc = fmaf(fmaf(sc, static_cast<float>(q[b] & 15), -mn), xe[0], acc);
+                acc = fmaf(fmaf(sc, static_cast<float>(q[b] >> 4), -mn), xe[1], acc);
+            }
+        }
+    }
+    return acc;
+}
+
 // Y = sum over the splits of the partial products, in split order (deterministic); four
-// splits' loads at a time.  N a multiple of 4 and 16-byte rows: four columns per thread.
-template <int V>
+// splits' loads at a time.  N a multiple of V and rows aligned to V floats: V columns per thread.
+// PLAIN: an output that is not finite is summed again from the f32 inputs (q4k_plain_dot).
+struct PlainRows {
+    const uint8_t* qs;
+    const uint4* hdr;
+    const float* X;
+    int K;
+};
+template <int V, bool PLAIN>
 __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict__ Y, size_t n, int splits, int N,
-                                  int ldy) {
+                                  int ldy, PlainRows pl) {
     const size_t i = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) * V;
     if (i >= n) return;
     typedef float fv __attribute__((ext_vector_type(V)));
@@ -493,7 +543,14 @@ __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict
         for (int k = 0; k < 4; k++)
             if (z + k < splits) a += v[k];
     }
-    *reinterpret_cast<fv*>(Y + (i / N) * ldy + i % N) = a;
+    const size_t r = i / N, col = i % N;
+    if constexpr (PLAIN) {
+#pragma unroll
+        for (int k = 0; k < V; k++)
+            if (!(fabsf(a[k]) <= 3.4028235e38f))
+                a[k] = q4k_plain_dot(pl.qs, pl.hdr, pl.X + r * pl.K, static_cast<int>(col) + k, pl.K);
+    }
+    *reinterpret_cast<fv*>(Y + r * ldy + col) = a;
 }
 
 // Token tiles per workgroup (the fewest workgroups of at most four, evenly filled) and K-splits
@@ -504,21 +561,21 @@ __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict
 // 1) m N floats at ~5 TB/s, and a launch).
 struct PkPlan {
     int tt, splits, sb_per;
+    double ns;  // the modelled time of the GEMM and its sums
 };
 PkPlan pk_plan(const DevWeight& w, size_t m) {
     const int S = static_cast<int>((w.cols + 255) / 256);
     const long most = w.format == LARQL_Q4_K ? 4 : 3;  // (four would spill in the others)
     const long cus = current_device_cus(), mt = static_cast<long>((m + 15) / 16), gy = (mt + most - 1) / most;
-    PkPlan best{static_cast<int>((mt + gy - 1) / gy), 1, S};
+    PkPlan best{static_cast<int>((mt + gy - 1) / gy), 1, S, -1.0};
     constexpr double kUnit[5] = {0, 2200, 3000, 3600, 4100};  // ns
     const double unit = kUnit[best.tt] * (w.format == LARQL_Q6_K ? 1.5 : 1.0);
     const long wgs = static_cast<long>((w.rows + kPkRows - 1) / kPkRows) * ((mt + best.tt - 1) / best.tt);
-    double best_cost = -1.0;
     for (int s = 1; s <= 16 && s <= S; s++) {
         const int per = (S + s - 1) / s, eff = (S + per - 1) / per;
         double cost = static_cast<double>((wgs * eff + cus - 1) / cus) * per * unit;
         if (eff > 1) cost += 3000.0 + (eff + 1) * static_cast<double>(m) * static_cast<double>(w.rows) * 0.0008;
-        if (best_cost < 0 || cost < best_cost) best.splits = eff, best.sb_per = per, best_cost = cost;
+        if (best.ns < 0 || cost < best.ns) best.splits = eff, best.sb_per = per, best.ns = cost;
     }
     return best;
 }
@@ -536,9 +593,9 @@ size_t gemm_x_pack_floats(size_t m, size_t cols) { return (m + 15) / 16 * 16 * c
 
 // workspace: the K-split partials (when split), and for a caller without row statistics and packed
 // rows those
-size_t gemm_f32_part_floats(const DevWeight& w, size_t m) {
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain) {
     const PkPlan p = pk_plan(w, m);
-    return align4(p.splits > 1 ? p.splits * m * w.rows : 0) + align4(gemm_row_stats_floats(m, w.cols)) +
+    return align4(p.splits > 1 || plain ? p.splits * m * w.rows : 0) + align4(gemm_row_stats_floats(m, w.cols)) +
            gemm_x_pack_floats(m, w.cols) + 4;
 }
 
@@ -572,8 +629,36 @@ void launch_gemm_x_pack(const float* X, size_t m, size_t cols, const GemmRowStat
     }
 }
 
+void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s) {
+    if (cols > static_cast<size_t>(kFusedRowMax)) {
+        launch_gemm_row_stats(X, m, cols, st, s);
+        launch_gemm_x_pack(X, m, cols, st, s);
+        return;
+    }
+    if (m > 0x7FFFFF00) fail(LARQL_HIP_ERR_INVALID, "GEMM operand packing: too many tokens");
+    ResidRows r;
+    r.hin = X;
+    r.st = st;
+    r.m = static_cast<int>(m);
+    r.n = static_cast<int>(cols);
+    launch_resid_norm_stats_rows(r, s);
+}
+
+// Q4_K batches small enough that this GEMM beats the fp16 one (prefill.hip), whose workgroups
+// are 256 tokens whatever the batch: ~2.2 us per super-block of K and round of 80-row
+// workgroups, against the plan's time and its two other launches.  Measured [14336 x 4096]: 6
+// tokens 22.6 against 39.5 us, 64 tokens 41 against 42, 96 tokens 49 against 45; [4096 x 14336]:
+// 6 tokens 30 against 125, 192 tokens 83 against 145; [10240 x 2560]: 32 tokens 22 against 28,
+// 64 tokens 31 against 28.
+bool gemm_f32_small_batch(const DevWeight& w, size_t m) {
+    if (w.format != LARQL_Q4_K || m < 2 || m > 512) return false;
+    const size_t wgs = ((w.rows_pad / 16 + 4) / 5) * ((m + 255) / 256), cus = static_cast<size_t>(current_device_cus());
+    const double other = 6500.0 + static_cast<double>((wgs + cus - 1) / cus) * static_cast<double>(w.cols / 256) * 2200.0;
+    return 1.45 * pk_plan(w, m).ns + 8000.0 < other;
+}
+
 void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
-                     hipStream_t s, size_t ldy, const GemmRowStats* pre, GemmSplits* defer) {
+                     hipStream_t s, size_t ldy, const GemmRowStats* pre, GemmSplits* defer, bool plain) {
     if (ldy == 0) ldy = w.rows;
     if (ldy < w.rows || ldy > 0x7FFFFFFF) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: bad output row stride");
     if (defer && ldy != w.rows) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: deferred split sums need dense output rows");
@@ -583,20 +668,22 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     if (m == 0) return;
     if (m > 0x7FFFFFFF / w.cols) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: too many tokens");
     const PkPlan p = pk_plan(w, m);
-    if (!part || part_floats < gemm_f32_part_floats(w, m)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: workspace too small");
-    float* at = part + align4(p.splits > 1 ? p.splits * m * w.rows : 0);
+    if (plain && (w.format != LARQL_Q4_K || defer)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: plain sums of Q4_K outputs only");
+    if (!part || part_floats < gemm_f32_part_floats(w, m, plain)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: workspace too small");
+    const bool parts = p.splits > 1 || plain;  // the GEMM writes partial products, summed after it
+    float* at = part + align4(parts ? p.splits * m * w.rows : 0);
     GemmRowStats st;
     if (pre) {
         st = *pre;
     } else {
         st = gemm_row_stats_at(at, m, w.cols);
         if (w.format != LARQL_Q4_K) st.xs = nullptr;
-        launch_gemm_row_stats(X, m, w.cols, st, s);
     }
     if (!st.xp) {
         const uintptr_t xp = reinterpret_cast<uintptr_t>(at + align4(gemm_row_stats_floats(m, w.cols)));
         st.xp = reinterpret_cast<float*>((xp + 15) & ~uintptr_t{15});
-        launch_gemm_x_pack(X, m, w.cols, st, s);
+        if (pre) launch_gemm_x_pack(X, m, w.cols, st, s);
+        else launch_gemm_pack_rows(X, m, w.cols, st, s);
     }
     PkArgs a{};
     a.qs = w.qs;
@@ -604,7 +691,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     a.XP = reinterpret_cast<const v4u*>(st.xp);
     a.xe = st.xe;
     a.xs = st.xs;
-    a.Y = p.splits > 1 ? part : Y;
+    a.Y = parts ? part : Y;
     a.ypart = m * w.rows;
     a.M = static_cast<int>(m);
     a.N = static_cast<int>(w.rows);
@@ -612,7 +699,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     a.ntiles = static_cast<int>(w.rows_pad / 16);
     a.mtiles = static_cast<int>((m + 15) / 16);
     a.sb_per = p.sb_per;
-    a.ldy = static_cast<int>(p.splits > 1 ? w.rows : ldy);
+    a.ldy = static_cast<int>(parts ? w.rows : ldy);
     a.gx = static_cast<int>((w.rows + kPkRows - 1) / kPkRows);
     a.gy = (a.mtiles + p.tt - 1) / p.tt;
     a.gz = p.splits;
@@ -633,13 +720,18 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     else fmt(std::integral_constant<int, LARQL_Q4_0>{});
     LARQL_HIP_CHECK(hipGetLastError());
     if (defer) *defer = {p.splits > 1 ? part : nullptr, p.splits};
-    if (p.splits > 1 && !defer) {
+    if (parts && !defer) {
         const size_t n = m * w.rows;
         const int N = static_cast<int>(w.rows), ld = static_cast<int>(ldy);
-        if (N % 4 == 0 && ld % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0)
-            sum_splits_kernel<4><<<dim3(static_cast<unsigned>((n / 4 + 255) / 256)), dim3(256), 0, s>>>(part, Y, n, p.splits, N, ld);
-        else
-            sum_splits_kernel<1><<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s>>>(part, Y, n, p.splits, N, ld);
+        const PlainRows pl{w.qs, w.hdr, X, static_cast<int>(w.cols)};
+        auto sum = [&](auto v) {
+            constexpr int V = decltype(v)::value;
+            const dim3 g(static_cast<unsigned>((n / V + 255) / 256)), b(256);
+            if (plain) sum_splits_kernel<V, true><<<g, b, 0, s>>>(part, Y, n, p.splits, N, ld, pl);
+            else sum_splits_kernel<V, false><<<g, b, 0, s>>>(part, Y, n, p.splits, N, ld, pl);
+        };
+        if (N % 4 == 0 && ld % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0) sum(std::integral_constant<int, 4>{});
+        else sum(std::integral_constant<int, 1>{});
         LARQL_HIP_CHECK(hipGetLastError());
     }
 }

@@ -286,10 +286,16 @@ struct GemmSplits {
 // Y rows are ldy floats apart (0: w.rows), so a projection can fill a column slice.  part:
 // workspace of gemm_f32_part_floats.  pre: X's row statistics, already computed, and its packed
 // operands if xp is set (for Q4_K weights with the sub-block sums).  defer: leave the split
-// partial products unsummed (ldy = w.rows).
-size_t gemm_f32_part_floats(const DevWeight& w, size_t m);
+// partial products unsummed (ldy = w.rows).  plain (Q4_K): outputs that are not finite are summed
+// again from the f32 inputs (the packed operands of a row with an infinite element are NaN).
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain = false);
+// The row statistics and packed operands of X, in one launch where a row fits it.
+void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s);
+// Q4_K weights and batches for which launch_gemm_f32 is faster than launch_q4k_gemm.
+bool gemm_f32_small_batch(const DevWeight& w, size_t m);
 void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
-                     hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr, GemmSplits* defer = nullptr);
+                     hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr, GemmSplits* defer = nullptr,
+                     bool plain = false);
 // Q4_0 or Q8_0 weights (cols a multiple of 128) x any number of Q8 rows, block order as the
 // matvecs (gemm_int.hip); w2 / out2: a second weight of the same format and shape in the same
 // launch.  Output rows ldo floats apart (0: w.rows).

@@ -153,7 +153,8 @@ int larql_hip_q4k_matvec(larql_hip_ctx* ctx, const uint8_t* q4k_data, size_t q4k
 
 /* Prefill projection: out[m][num_rows] = x[m][hidden] . deq(Q4_K)^T for m tokens at once —
  * the per-position q4k_matvec loop of the Metal prefill (LC/src/metal/prefill.rs:21-110,
- * trait prefill_q4 LC/src/backend.rs:143-152) as one MFMA GEMM (fp16 operands, f32 sums).
+ * trait prefill_q4 LC/src/backend.rs:143-152) as one MFMA GEMM (fp16 operands, f32 sums;
+ * small batches the f32-accuracy GEMM).
  * m = 1 is the matvec. */
 int larql_hip_q4k_matmul(larql_hip_ctx* ctx, const uint8_t* q4k_data, size_t q4k_len, const float* x, size_t m,
                          float* out, size_t num_rows, size_t hidden);
@@ -186,7 +187,7 @@ int larql_hip_quantize_weights(larql_hip_ctx* ctx, int format, const float* x, s
 /* ── device-resident fast path (device pointers; enqueue on `stream`) ──── */
 
 /* One matvec with a registered weight.  For LARQL_Q4_K / LARQL_Q6_K `x` is f32
- * [m][cols] and x_scales is unused (m > 1: Q4_K runs the fp16-operand prefill GEMM, Q6_K
+ * [m][cols] and x_scales is unused (m > 1: Q4_K runs the fp16-operand prefill GEMM, small batches and Q6_K
  * the f32-accuracy GEMM of the prompt pass); for LARQL_Q4_0 / LARQL_Q8_0 `x` is int8 [m][cols] and x_scales f32
  * [m][cols/32], any m (each output row in the single-row order, bit for bit).
  * out is f32 [m][rows].

@@ -130,3 +130,73 @@ def test_q6k_gemm_rows_match_matvec_oracle(hip, rows, cols, m, scaled):
     finally:
         hip.release_weight(h)
         hip.forget_host(q6k)
+
+
+def _q4k_values(b, rows, cols):
+    """d, dmin, scales, mins and codes of 148-byte blocks -> f64 weights."""
+    b = b.reshape(-1, 148)
+    d, dmin = (b[:, i:i + 2].copy().view(np.float16).astype(np.float64) for i in (0, 2))
+    sc = (b[:, 4:12] & 63).astype(np.float64)
+    mn = np.concatenate([b[:, 16:20] & 15, b[:, 16:20] >> 4], 1).astype(np.float64)
+    q = np.stack([b[:, 20:] & 15, b[:, 20:] >> 4], -1).reshape(-1, 8, 32).astype(np.float64)
+    return (q * (d * sc)[..., None] - (dmin * mn)[..., None]).reshape(rows, cols)
+
+
+# 2 .. 64 tokens, odd row counts, one super-block, K split over up to 16 workgroups, rows of more
+# than 16384 (packed by the separate kernels); the larger shapes are those the small-batch route takes
+@pytest.mark.parametrize("rows,cols,m", [(300, 4096, 2), (4096, 4096, 16), (1000, 2560, 17), (257, 14336, 33),
+                                         (4096, 8192, 48), (130, 4352, 64), (64, 17408, 5), (14336, 4096, 6)])
+def test_q4k_small_batch_rows(hip, rows, cols, m):
+    """Small batches of Q4_K (matvec_dev, the f32-accuracy GEMM): every output against the f64
+    product of the dequantized weights, within 1e-5 of the row's largest (f32 sums: 2^-24 per term,
+    random signs, K <= 17408 -> ~1e-6).  One token scaled by 1e6 and one by 1e-20 (each row has its
+    own power of two), and super-blocks with a minimum scale of 300, past the range of the usual
+    fp16 minimum operand."""
+    torch = pytest.importorskip("torch")
+    print(f"[q4k small] rows={rows} cols={cols} m={m}", flush=True)
+    b = oracle.quantize_q4_k(oracle.gauss(95, rows * cols, 0.0, 0.02)).reshape(-1, 148).copy()
+    b[5::97, 2:4] = np.array([300.0], np.float16).view(np.uint8)
+    x = oracle.gauss(96, m * cols).reshape(m, cols).copy()
+    x[0] *= np.float32(1e6)
+    x[m - 1] *= np.float32(1e-20)
+    h = hip.register_weight(larql_hip.Q4_K, b.reshape(-1), rows, cols)
+    try:
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dx, dy, m=m)
+        hip.synchronize()
+        got = dy.cpu().numpy().reshape(m, rows).astype(np.float64)
+        ref = x.astype(np.float64) @ _q4k_values(b, rows, cols).T
+        e = np.max(np.abs(got - ref), 1) / np.max(np.abs(ref), 1)
+        print(f"  worst row {np.max(e):.2e}", flush=True)
+        assert np.max(e) <= 1e-5
+    finally:
+        hip.release_weight(h)
+
+
+def test_q4k_small_batch_infinite_elements(hip):
+    """A token with one infinite element: every output is that infinity times the sign of its weight
+    (as the f32 sum gives it), the other tokens' outputs are unaffected; a NaN makes its token NaN."""
+    torch = pytest.importorskip("torch")
+    rows, cols, m = 4096, 4096, 4
+    b = oracle.quantize_q4_k(oracle.gauss(97, rows * cols, 0.0, 0.02))
+    W = _q4k_values(b, rows, cols)
+    x = oracle.gauss(98, m * cols).reshape(m, cols).copy()
+    x[1, 77] = np.inf
+    x[2, 1000] = np.nan
+    h = hip.register_weight(larql_hip.Q4_K, b, rows, cols)
+    try:
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dx, dy, m=m)
+        hip.synchronize()
+        got = dy.cpu().numpy().reshape(m, rows)
+        clear = np.abs(W[:, 77]) > 1e-6   # (a weight at the rounding of zero may have either sign)
+        assert clear.mean() > 0.99
+        np.testing.assert_array_equal(got[1][clear], np.sign(W[clear, 77]) * np.inf)
+        assert np.all(np.isnan(got[2]))
+        for t in (0, 3):
+            ref = x[t].astype(np.float64) @ W.T
+            assert np.max(np.abs(got[t] - ref)) <= 1e-5 * np.max(np.abs(ref))
+    finally:
+        hip.release_weight(h)
