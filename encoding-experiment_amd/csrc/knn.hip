@@ -11,6 +11,7 @@
 // The f32 scores are single fma chains over k from +0 per (feature, query), the
 // oracle's canonical order, so scores and therefore top-k indices are bit-exact.
 #include "device_common.h"
+#include "f32_lane.h"
 #include "knn.h"
 
 #include <algorithm>
@@ -25,8 +26,6 @@ namespace larql {
 namespace {
 
 constexpr int kThreads = 256;
-
-typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 // ── f32 scores ─────────────────────────────────────────────────────────────
 // A lane owns NF features and walks k in order, so a score is one fma chain held in one
@@ -43,29 +42,6 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 // 1.86 for 64, 3.46 for 128.
 constexpr int kF32Stage = 32;
 
-// A query block of a k: QW consecutive floats at a wave-uniform address, read with scalar loads.
-typedef const float __attribute__((address_space(4))) * scalar_f32_ptr;
-
-// XT[b][k][QW] = the QW queries of block b at k: X[QW b + i][k] for existing queries and
-// k < K, else +0 (b < Qp / QW, k < Kp).
-__global__ void queries_t_kernel(const float* __restrict__ X, float* __restrict__ XT, int Q, int K, int Kp, int Qp,
-                                 int qw) {
-    __shared__ float t[32][33];
-    const int nk = (Kp + 31) / 32, k0 = 32 * static_cast<int>(blockIdx.x % nk), q0 = 32 * static_cast<int>(blockIdx.x / nk);
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int q = q0 + ty + 8 * i, k = k0 + tx;
-        t[ty + 8 * i][tx] = (q < Q && k < K) ? X[static_cast<size_t>(q) * K + k] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int k = k0 + ty + 8 * i, q = q0 + tx;
-        if (k < Kp && q < Qp) XT[(static_cast<size_t>(q / qw) * Kp + k) * qw + q % qw] = t[tx][ty + 8 * i];
-    }
-}
-
 // Four float4 of a lane's staged row (chunks 4 HALF .. 4 HALF + 3), read and waited for in
 // one block: the compiler does not see the loads that fill the ring, so its own LDS reads
 // would wait for every one of them.
@@ -79,12 +55,6 @@ __device__ __forceinline__ void ring_read4(uint32_t a, floatx4_t (&v)[4]) {
         : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
         : "v"(a0), "v"(a1), "v"(a2), "v"(a3)
         : "memory");
-}
-
-// At most N vector memory operations of the wave still in flight.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 template <int QW, int NF, int NW, int ND>
@@ -1021,8 +991,7 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
     const float* XT = X;  // one query of a whole row: as it lies
     if (gate_scores_f32_ws_floats(K, Q)) {
         if (!ws) fail(LARQL_HIP_ERR_INVALID, "gate scores: no workspace for the queries");
-        queries_t_kernel<<<dim3(((Kp + 31) / 32) * ((Qp + 31) / 32)), dim3(256), 0, s>>>(X, ws, Q, K, Kp, Qp, p.qw);
-        LARQL_HIP_CHECK(hipGetLastError());
+        launch_queries_t(X, static_cast<size_t>(K), 1, ws, Q, K, Kp, Qp, p.qw, s);
         XT = ws;
     }
     auto go = [&](auto qw, auto nf, auto nw, auto nd) {

@@ -52,6 +52,32 @@ def test_matmul_bit_exact(hip, m, k, n):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (m, k, n)
 
 
+@pytest.mark.parametrize("k", [1, 4, 15, 16, 17, 31, 33, 48, 100])
+@pytest.mark.parametrize("q,rows", [(1, 64), (2, 65), (3, 63), (5, 130), (9, 70), (17, 129), (33, 64), (65, 200)])
+def test_matmul_lanes_bit_exact(hip, q, rows, k):
+    """Products in lanes: every split of the smaller side over waves and workgroups, rows at the
+    edges of 64, k at the edges of 16 and of stages of 32, either side the larger, both layouts
+    of B, operands at a 4-byte offset (rows that are not 16-byte aligned)."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(q * 1000 + rows + k)
+    small, big = _rand(rng, q, k), _rand(rng, rows, k)
+    ref = _ref_transb(small, big)
+    for m, n, a, b, want in ((q, rows, small, big, ref), (rows, q, big, small, ref.T)):
+        for tb in (True, False):
+            bb = b if tb else np.ascontiguousarray(b.T)
+            for off in (0, 1):
+                da = torch.empty(a.size + off, device="cuda")[off:]
+                db = torch.empty(bb.size + off, device="cuda")[off:]
+                da.copy_(torch.from_numpy(a.reshape(-1)))
+                db.copy_(torch.from_numpy(bb.reshape(-1)))
+                out = torch.full((m * n,), 7.0, device="cuda")
+                torch.cuda.synchronize()
+                hip.matmul_dev(da, db, out, m, k, n, transpose_b=tb)
+                torch.cuda.synchronize()
+                got = out.cpu().numpy().reshape(m, n)
+                assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(want).view(np.uint32)), (m, n, tb, off)
+
+
 def test_matmul_edge_cases(hip):
     """k = 0 gives zeros; special values propagate as the chain propagates them; a
     batch equals its calls in order; mismatched inner dimensions raise."""
