@@ -46,9 +46,9 @@ __global__ __launch_bounds__(256) void x_pack_kernel(const float* __restrict__ X
     const float* p = X + static_cast<size_t>(mc) * K + 32 * ks + 8 * g;
     const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + 4);
     const float sc = m < M ? ldexpf(1.0f, xe[mc]) : 0.0f;
-    float e[8] = {a.x, a.z, b.x, b.z, a.y, a.w, b.y, b.w};
+    float e[8] = {a.x, b.x, a.z, b.z, a.y, b.y, a.w, b.w};
 #pragma unroll
-    for (int k = 0; k < 8; k++) e[k] = m < M ? e[k] * sc : 0.0f;
+    for (int k = 0; k < 8; k++) e[k] = m < M ? e[k] * (k < 4 ? sc : sc * 0.0625f) : 0.0f;
     v4u hi, lo;
     hp_split8(e, hi, lo);
     v4u* o = XP + hp_packed_at(m, 4 * ks + g, K);
@@ -108,11 +108,19 @@ __device__ __forceinline__ void read_a(uint32_t a, int t, v4u (&h)[TT], v4u (&l)
     }
 }
 
-// Two codes (bytes of `codes` chosen by sel) as fp16 integers times s: 0x64 above a code byte is
-// fp16 1024 + q, and fma(1024 + q, s, -1024 s) = s q exactly while |s q| <= 2048.
-__device__ __forceinline__ uint32_t sq_pair(uint32_t codes, uint32_t sel, f16x2 s, f16x2 ns) {
-    const f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, codes, sel));
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(b, s, ns));
+// The eight codes of a nibble dword as fp16 pairs, code times 2^-24 (elements 0, 4, 2, 6) or 2^-20
+// (1, 5, 3, 7): a nibble in the low byte of a half is a subnormal, kept by the matrix cores.
+__device__ __forceinline__ void nibble_pairs(uint32_t w, f16x2 (&o)[4]) {
+    const uint32_t w8 = w >> 8;
+    o[0] = __builtin_bit_cast(f16x2, w & 0x000F000Fu);
+    o[1] = __builtin_bit_cast(f16x2, w8 & 0x000F000Fu);
+    o[2] = __builtin_bit_cast(f16x2, w & 0x00F000F0u);
+    o[3] = __builtin_bit_cast(f16x2, w8 & 0x00F000F0u);
+}
+
+__device__ __forceinline__ half8 operand8(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+    return __builtin_bit_cast(half8, v4u{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                         __builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)});
 }
 
 // 4 x 4 transpose of a lane's dwords across the four lane groups: lane group g gets dword g of
@@ -136,10 +144,11 @@ struct PkArgs {
     int M, N, K, ntiles, mtiles, sb_per, ldy, gx, gy, gz;
 };
 
-// Bound: issue, MFMA plus the VALU between (2.3 per MFMA at four token tiles, 9 at one), which add
+// Bound: issue, MFMA plus the VALU between (1.9 per MFMA at four token tiles, 7.5 at one), which add
 // up at any number of waves.  Measured, Q4_K [28672 x 4096] with the two launches before it: 512
-// tokens 250 us (482 TFLOP/s; 311 us for the GEMM alone when each workgroup split f32 tokens into
-// pairs itself and one wave per SIMD waited for its own loads and LDS reads), 24 tokens 35 us.
+// tokens 230 us (523 TFLOP/s; 311 us for the GEMM alone when each workgroup split f32 tokens into
+// pairs itself and one wave per SIMD waited for its own loads and LDS reads; 250 with the codes
+// made fp16 integers by a byte permute and an fma per pair), 24 tokens 35 us.
 //
 // 16 TT tokens x 256 weight rows per workgroup: wave w owns 64 rows (kPkR tiles), all waves
 // share the token operands.  A unit is 128 k (half a super-block, four k-steps of one 32-element
@@ -148,7 +157,8 @@ struct PkArgs {
 //
 // Q4_K: w = d s_j q - dmin m_j, so per super-block and token
 //   sum_k x_k w_k = d sum_j s_j (sum_{k in j} x_k q_k) - dmin sum_j m_j X_j,  X_j = sum_{k in j} x_k.
-// s_j q <= 945 is an exact fp16 integer, the weight operand of both products (x hi and lo, both
+// s_j q <= 945 (times 2^-24: the codes are read as fp16 subnormals, an and-mask per two of them)
+// is exact in fp16, the weight operand of both products (x hi and lo, both
 // exact in f32; only the split's 2^-22 is lost), a fresh accumulator per super-block, added into
 // the total times d.  The min term follows the K loop: the sub-block sums X_j 2^(e - 5) against
 // -32 dmin m_j per row, both as fp16 pairs (three products), 32 sub-blocks per k-step.  A lane's
@@ -158,11 +168,13 @@ struct PkArgs {
 // integers, so it is split exactly, hi = fp16(sc (q - 32)) and lo the rest (at most 1): three
 // products per super-block accumulator (the dropped x_lo w_lo is ~2^-23 of it).
 //
-// Q4_0: w = d (q - 8) per 32-element block: q - 8 as fp16, a fresh accumulator per k-step, added
+// Q4_0: w = d (q - 8) per 32-element block: q - 8 (times 2^-24) in fp16, a fresh accumulator per k-step, added
 // into the total times d.
 template <int FMT, int TT>
 __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     constexpr bool kQ4K = FMT == LARQL_Q4_K, kQ6K = FMT == LARQL_Q6_K;
+    // an operand's unit: codes times 2^-24; Q6_K weights at a quarter
+    constexpr float kUnit = kQ6K ? 4.0f : 16777216.0f;
     // weight loads per wave of a unit of each parity
     constexpr int kWLoads0 = (kQ6K ? 4 : 2) * kPkR, kWLoads1 = 2 * kPkR;
     __shared__ __align__(1024) v4u As[2][TT * 8 * 64];
@@ -307,46 +319,42 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
 #pragma unroll
             for (int j = 0; j < kPkR; j++) {
                 const uint32_t word = n[j][t];
-                uint32_t lo = word & 0x0F0F0F0Fu, hi = (word >> 4) & 0x0F0F0F0Fu;
                 half8 B, Bl;
                 if constexpr (kQ4K) {
-                    // s = scale of sub-block 4h + t (both halves), ns = -1024 s
+                    // the scale of sub-block 4h + t in both halves
                     const f16x2 sv =
                         __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, s6[j], 0x04000400u + 0x00010001u * t)) -
                         f16x2{1024.0f16, 1024.0f16};
-                    const f16x2 ns = sv * f16x2{-1024.0f16, -1024.0f16};
-                    B = __builtin_bit_cast(half8, v4u{sq_pair(lo, 0x04010400u, sv, ns), sq_pair(lo, 0x04030402u, sv, ns),
-                                                      sq_pair(hi, 0x04010400u, sv, ns), sq_pair(hi, 0x04030402u, sv, ns)});
+                    f16x2 q[4];
+                    nibble_pairs(word, q);
+                    B = operand8(q[0] * sv, q[1] * sv, q[2] * sv, q[3] * sv);
                 } else if constexpr (kQ6K) {
                     const uint32_t hb = nh[j][t] >> (4 * (g & 1));
-                    lo |= (hb & 0x03030303u) << 4;
-                    hi |= ((hb >> 2) & 0x03030303u) << 4;
-                    // the scale of this lane's 16-element group: byte 2 h + g / 2 of lane group t's word
+                    const uint32_t lo = (word & 0x0F0F0F0Fu) | ((hb & 0x03030303u) << 4);
+                    const uint32_t hi = ((word >> 4) & 0x0F0F0F0Fu) | (((hb >> 2) & 0x03030303u) << 4);
+                    // the scale of this lane's 16-element group: byte 2 h + g / 2 of lane group t's
+                    // word; even elements at a quarter, odd ones at four times the weight
                     const int scw = __builtin_amdgcn_ds_bpermute(4 * (16 * t + c), static_cast<int>(sc6[j]));
                     const _Float16 sf = static_cast<_Float16>(static_cast<int8_t>(scw >> (16 * h + 8 * (g >> 1))));
-                    const f16x2 sv = {sf, sf};
-                    uint32_t bh[4], bl[4];
-                    auto pr = [&](uint32_t codes, uint32_t sel, uint32_t& oh, uint32_t& ol) __attribute__((always_inline)) {
+                    const f16x2 se = f16x2{sf, sf} * f16x2{0.25f16, 0.25f16}, so = f16x2{sf, sf} * f16x2{4.0f16, 4.0f16};
+                    f16x2 bh[4], bl[4];
+                    auto pr = [&](uint32_t codes, uint32_t sel, f16x2 sv, f16x2& oh, f16x2& ol) __attribute__((always_inline)) {
                         const f16x2 q = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, codes, sel)) -
                                         f16x2{1056.0f16, 1056.0f16};
-                        const f16x2 p = q * sv;
-                        oh = __builtin_bit_cast(uint32_t, p);
-                        ol = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, sv, -p));
+                        oh = q * sv;
+                        ol = __builtin_elementwise_fma(q, sv, -oh);
                     };
-                    pr(lo, 0x04010400u, bh[0], bl[0]);
-                    pr(lo, 0x04030402u, bh[1], bl[1]);
-                    pr(hi, 0x04010400u, bh[2], bl[2]);
-                    pr(hi, 0x04030402u, bh[3], bl[3]);
-                    B = __builtin_bit_cast(half8, v4u{bh[0], bh[1], bh[2], bh[3]});
-                    Bl = __builtin_bit_cast(half8, v4u{bl[0], bl[1], bl[2], bl[3]});
+                    pr(lo, 0x04020400u, se, bh[0], bl[0]);
+                    pr(lo, 0x04030401u, se, bh[1], bl[1]);
+                    pr(hi, 0x04020400u, so, bh[2], bl[2]);
+                    pr(hi, 0x04030401u, so, bh[3], bl[3]);
+                    B = operand8(bh[0], bh[1], bh[2], bh[3]);
+                    Bl = operand8(bl[0], bl[1], bl[2], bl[3]);
                 } else {
-                    auto pr = [](uint32_t codes, uint32_t sel) __attribute__((always_inline)) {
-                        return __builtin_bit_cast(
-                            uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, codes, sel)) -
-                                          f16x2{1032.0f16, 1032.0f16});
-                    };
-                    B = __builtin_bit_cast(half8, v4u{pr(lo, 0x04010400u), pr(lo, 0x04030402u), pr(hi, 0x04010400u),
-                                                      pr(hi, 0x04030402u)});
+                    constexpr _Float16 u8e = 0x1p-21f16, u8o = 0x1p-17f16;  // code 8
+                    f16x2 q[4];
+                    nibble_pairs(word, q);
+                    B = operand8(q[0] - f16x2{u8e, u8e}, q[1] - f16x2{u8e, u8e}, q[2] - f16x2{u8o, u8o}, q[3] - f16x2{u8o, u8o});
                 }
                 constexpr bool kSuper = kQ4K || kQ6K;  // an accumulator per super-block, else per block
                 const bool fresh = kSuper ? (h == 0 && t == 0) : true;
@@ -366,7 +374,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
             if constexpr (!kQ4K && !kQ6K) {  // the blocks' sums times d (row c)
 #pragma unroll
                 for (int j = 0; j < kPkR; j++) {
-                    const float d = h2f(w.h[j][t >> 1] >> (16 * (t & 1)));
+                    const float d = h2f(w.h[j][t >> 1] >> (16 * (t & 1))) * kUnit;
 #pragma unroll
                     for (int i = 0; i < TT; i++)
 #pragma unroll
@@ -377,7 +385,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
         if constexpr ((kQ4K || kQ6K) && h == 1) {  // the super-block's sum times d (row c)
 #pragma unroll
             for (int j = 0; j < kPkR; j++) {
-                const float d = dsb[j];
+                const float d = dsb[j] * kUnit;
 #pragma unroll
                 for (int i = 0; i < TT; i++)
 #pragma unroll

@@ -321,8 +321,10 @@ def test_prefill_q8_q4_0_layers(hip, seq, formats, variant):
     another order than the decode kernel's, so an activation next to a rounding tie may take the
     neighbouring Q8 code: a step of max|x| / 127 in one of 512 elements, ~3 sigma / 127 of sqrt(512)
     sigma = 1e-3 of that input, and half a dozen quantized inputs over the two layers add in
-    quadrature: 3e-3 of the output's scale."""
-    tol = 3e-3
+    quadrature: 3e-3 of the output's scale.  A post-norm layer norms each branch's output before its
+    residual add, which scales a flip's share of a weak branch up with it: decoding such a model
+    step by step is itself up to 8.3e-3 from the oracle (seeds 78 .. 82); twice that."""
+    tol = 1.7e-2 if variant else 3e-3
     n_layers, hidden, inter, nq, nkv, hd = 2, 512, 1024, 8, 2, 64
     print(f"[prefill q8] seq={seq} formats={formats} variant={variant}", flush=True)
     m = SmallModel(n_layers, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=78, formats=formats, variant=variant)
