@@ -24,7 +24,8 @@ using larql::fail;
 
 struct LayerDev {
     // Q|K|V fused by rows and gate/up interleaved by rows when each pair shares a format;
-    // otherwise separate weights (mixed Q4_K / Q6_K projections, as in Q4_K_M files)
+    // otherwise separate weights (mixed Q4_K / Q6_K projections, as in Q4_K_M files), where Q and
+    // K of one format are still one weight, wq = Q|K with wk empty
     DevWeight qkv, wo, gateup, down;
     DevWeight wq, wk, wv, gate, up;
     bool split_qkv = false, split_gu = false;
@@ -243,10 +244,16 @@ larql_hip_model* build_model(larql_hip_ctx* c, const larql_pipeline_layer* layer
             d.split_qkv = form(L.wq, qd, hidden) != form(L.wk, kvd, hidden) ||
                           form(L.wq, qd, hidden) != form(L.wv, kvd, hidden);
             if (d.split_qkv) {
-                d.wq = build_weight(c, m, L.wq.format, hidden, {{L.wq.data, L.wq.len, qd, L.wq.scales}}, false,
-                                    on_device);
-                d.wk = build_weight(c, m, L.wk.format, hidden, {{L.wk.data, L.wk.len, kvd, L.wk.scales}}, false,
-                                    on_device);
+                if (form(L.wq, qd, hidden) == form(L.wk, kvd, hidden)) {
+                    d.wq = build_weight(c, m, L.wq.format, hidden,
+                                        {{L.wq.data, L.wq.len, qd, L.wq.scales}, {L.wk.data, L.wk.len, kvd, L.wk.scales}},
+                                        false, on_device);
+                } else {
+                    d.wq = build_weight(c, m, L.wq.format, hidden, {{L.wq.data, L.wq.len, qd, L.wq.scales}}, false,
+                                        on_device);
+                    d.wk = build_weight(c, m, L.wk.format, hidden, {{L.wk.data, L.wk.len, kvd, L.wk.scales}}, false,
+                                        on_device);
+                }
                 d.wv = build_weight(c, m, L.wv.format, hidden, {{L.wv.data, L.wv.len, kvd, L.wv.scales}}, false,
                                     on_device);
             } else {
@@ -514,9 +521,9 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
                 larql::launch_mv(w, a, s);
             }
         };
-        if (L.split_qkv) {  // three launches into the [q | k | v] buffer
+        if (L.split_qkv) {  // two or three launches into the [q | k | v] buffer
             qkv_proj(L.wq, m->qkv);
-            qkv_proj(L.wk, m->qkv + qd);
+            if (L.wk.rows) qkv_proj(L.wk, m->qkv + qd);
             qkv_proj(L.wv, m->qkv + qd + kvd);
         } else {
             qkv_proj(L.qkv, m->qkv);
@@ -661,7 +668,7 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
             const LayerDev* Ln = l + 1 < m->layers.size() ? &m->layers[l + 1] : nullptr;
             const int d_groups = q4k_mfma(L.down) ? larql::q4k_mfma_groups(L.down, 0) : 0;
             prenormed = Ln && q4k_mfma(L.down) &&
-                        (Ln->split_qkv ? takes_psum(Ln->wq, d_groups) && takes_psum(Ln->wk, d_groups) &&
+                        (Ln->split_qkv ? takes_psum(Ln->wq, d_groups) && (!Ln->wk.rows || takes_psum(Ln->wk, d_groups)) &&
                                              takes_psum(Ln->wv, d_groups)
                                        : takes_psum(Ln->qkv, d_groups));
             if (prenormed) {
@@ -811,7 +818,10 @@ PromptLayout prompt_layout(const larql_hip_model* m, size_t M) {
     for (const LayerDev& L : m->layers) {
         if (!larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd))
             part_n = m->part_per_split * larql::attn_prompt_splits(1, static_cast<int>(M), 0) * M;
-        if (L.split_qkv) need(L.wq, false), need(L.wk, false), need(L.wv, false);
+        if (L.split_qkv) {
+            need(L.wq, false), need(L.wv, false);
+            if (L.wk.rows) need(L.wk, false);
+        }
         else need(L.qkv, false);
         need(L.wo, false), need(L.down, true);
         if (L.split_gu) need(L.gate, false), need(L.up, false);
@@ -850,7 +860,8 @@ static bool prompt_batchable(const larql_hip_model* m, size_t M) {
         if (L.split_gu ? !(takes_q8(L.gate, false) && takes_q8(L.up, false) && ok(L.gate, false) && ok(L.up, false))
                        : L.gateup.format != LARQL_Q4_K)
             return false;
-        if (L.split_qkv ? !(ok(L.wq, false) && ok(L.wk, false) && ok(L.wv, false)) : !ok(L.qkv, false)) return false;
+        if (L.split_qkv ? !(ok(L.wq, false) && (!L.wk.rows || ok(L.wk, false)) && ok(L.wv, false)) : !ok(L.qkv, false))
+            return false;
         one_pass &= larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd);
     }
     if (!any_int) return true;
@@ -936,10 +947,11 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
     // packed operands in one launch) where a row fits them
     const bool fused = std::max({hidden, qd_max, inter}) <= static_cast<size_t>(larql::kFusedRowMax);
     auto qkv_f32 = [&](const LayerDev& L) {  // the Q8-input projections read the normed rows themselves
-        return L.split_qkv ? takes_q8(L.wq, false) || takes_q8(L.wk, false) || takes_q8(L.wv, false) : takes_q8(L.qkv, false);
+        return L.split_qkv ? takes_q8(L.wq, false) || (L.wk.rows && takes_q8(L.wk, false)) || takes_q8(L.wv, false)
+                           : takes_q8(L.qkv, false);
     };
     auto qkv_packed = [&](const LayerDev& L) {
-        return L.split_qkv ? !(takes_q8(L.wq, false) && takes_q8(L.wk, false) && takes_q8(L.wv, false))
+        return L.split_qkv ? !(takes_q8(L.wq, false) && (!L.wk.rows || takes_q8(L.wk, false)) && takes_q8(L.wv, false))
                            : !takes_q8(L.qkv, false);
     };
     // hin (+ P) -> hout, and the rows normed by (w, off, eps): f32 rows for Q8-input projections,
@@ -992,7 +1004,7 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
         }
         if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
             pj.run(L.wq, false, XN, QKV, ld, xn_st);
-            pj.run(L.wk, false, XN, QKV + qd, ld, xn_st);
+            if (L.wk.rows) pj.run(L.wk, false, XN, QKV + qd, ld, xn_st);
             pj.run(L.wv, false, XN, QKV + qd + kvd, ld, xn_st);
         } else {
             pj.run(L.qkv, false, XN, QKV, ld, xn_st);

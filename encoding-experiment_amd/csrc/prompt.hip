@@ -17,6 +17,8 @@
 #include "gemm_hp.h"
 #include "matvec_common.h"
 
+#include <type_traits>
+
 namespace larql {
 
 namespace {
@@ -116,7 +118,6 @@ __global__ void gated_mul_kernel(const float* __restrict__ G, const float* __res
 // steps, and each thread's loads of a chunk are issued together (indices clamped into
 // the row, so no load sits under a branch), so a row costs one round trip to memory per
 // chunk and two workgroup barriers instead of a dependent load per element.
-constexpr int kRowChunk = 16;  // elements per thread per chunk
 
 // Workgroup -> row, the 16 rows of a token tile on one XCD (workgroup i runs on XCD i % 8): the
 // packed operands of a tile share 128-byte lines, which that XCD's L2 then fills whole.  Grids
@@ -161,63 +162,68 @@ __device__ __forceinline__ void lds_row_out(const float* row, int n, int r, floa
     }
 }
 
-// f64 sum of ss over the 256 threads.
+// f64 sum of ss over the NT threads, wave by wave.
+template <int NT>
 __device__ __forceinline__ double block_sum_d(double ss, double* red) {
     ss = wave_sum_d(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
-    return (red[0] + red[1]) + (red[2] + red[3]);
+    double tot = red[0];
+#pragma unroll
+    for (int k = 1; k < NT / 64; k++) tot += red[k];
+    return tot;
 }
 
-// The step between two projections, per row of n floats (256 threads), in the arithmetic of the
-// separate kernels:
+// The step between two projections, per row of n floats, in the arithmetic of the separate
+// kernels (f64 sums of squares in another order):
 //   y = the projection row, its partial products summed in split order (sum_splits_kernel),
-//       four splits' loads at a time;
+//       several splits' loads at a time;
 //   POST: y = (y / rms(y)) * (poff + pw)                             (resid_norm_rows_kernel);
 //   h = (hin + y) * scale, or hin itself without a projection        (add_rows_kernel);
-//   x = norm ? (h * (1 / rms(h))) * (off + w) : h                    (rmsnorm_rows_kernel; every
-//       f64 sum of squares over the same 256 threads, element i in thread i % 256, in the same
-//       order);
+//   x = norm ? (h * (1 / rms(h))) * (off + w) : h                    (rmsnorm_rows_kernel);
 // h to hout, x to xn (each if given), and x's statistics and packed operands (if st.xe).
-template <bool POST>
-__global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(ResidRows a) {
+// NT threads: 256 where there are rows enough to fill the GPU, else 1024 (fewer elements per thread
+// to wait for in turn: 9.3 -> 7.3 us per launch at 24 rows of 4096; 11.2 -> 13.0 at 512 rows).
+template <int NT, bool POST>
+__global__ __launch_bounds__(NT) void resid_norm_stats_rows_kernel(ResidRows a) {
+    constexpr int kRowChunk = 4096 / NT, kZ = NT == 256 ? 4 : 8;  // elements per thread and chunk, splits' loads together
     __shared__ __align__(16) float row[kFusedRowMax];
-    __shared__ double red[2][4];
-    __shared__ float wm[4];
+    __shared__ double red[2][NT / 64];
+    __shared__ float wm[NT / 64];
     const int t = threadIdx.x, ri = tile_row(), n = a.n;
     if (ri >= a.m) return;
     const size_t r = static_cast<size_t>(ri) * n;
     double ss = 0.0;
     float m = 0.f;
     float w0[kRowChunk];  // the norm weights of the first chunk, requested with its rows
-    for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
+    for (int c0 = 0; c0 < n; c0 += NT * kRowChunk) {
         float y[kRowChunk], h[kRowChunk];
 #pragma unroll
         for (int q = 0; q < kRowChunk; q++) {
-            const size_t i = r + min(c0 + t + 256 * q, n - 1);
+            const size_t i = r + min(c0 + t + NT * q, n - 1);
             y[q] = a.P ? a.P[i] : 0.f;
             h[q] = POST ? 0.f : a.hin[i];
         }
         if (c0 == 0) {
 #pragma unroll
-            for (int q = 0; q < kRowChunk; q++) w0[q] = a.w ? a.w[min(t + 256 * q, n - 1)] : 0.f;
+            for (int q = 0; q < kRowChunk; q++) w0[q] = a.w ? a.w[min(t + NT * q, n - 1)] : 0.f;
         }
-        for (int z = 1; z < a.splits; z += 4) {
-            float v[4][kRowChunk];
+        for (int z = 1; z < a.splits; z += kZ) {
+            float v[kZ][kRowChunk];
 #pragma unroll
-            for (int k = 0; k < 4; k++)
+            for (int k = 0; k < kZ; k++)
 #pragma unroll
                 for (int q = 0; q < kRowChunk; q++)
-                    v[k][q] = a.P[min(z + k, a.splits - 1) * a.pstride + r + min(c0 + t + 256 * q, n - 1)];
+                    v[k][q] = a.P[min(z + k, a.splits - 1) * a.pstride + r + min(c0 + t + NT * q, n - 1)];
 #pragma unroll
-            for (int k = 0; k < 4; k++)
+            for (int k = 0; k < kZ; k++)
                 if (z + k < a.splits)
 #pragma unroll
                     for (int q = 0; q < kRowChunk; q++) y[q] += v[k][q];
         }
 #pragma unroll
         for (int q = 0; q < kRowChunk; q++) {
-            const int i = c0 + t + 256 * q;
+            const int i = c0 + t + NT * q;
             if (i < n) {
                 const float hv = POST ? y[q] : (a.P ? (h[q] + y[q]) * a.scale : h[q]);
                 if (!POST && a.hout) a.hout[r + i] = hv;
@@ -228,20 +234,20 @@ __global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(ResidRows a)
         }
     }
     if constexpr (POST) {  // (a thread's own elements of `row` throughout)
-        const double tot = block_sum_d(ss, red[0]);
+        const double tot = block_sum_d<NT>(ss, red[0]);
         const float inv = 1.0f / static_cast<float>(sqrt(tot / static_cast<double>(n) + a.eps));
         ss = 0.0, m = 0.f;
-        for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
+        for (int c0 = 0; c0 < n; c0 += NT * kRowChunk) {
             float h[kRowChunk], wv[kRowChunk];
 #pragma unroll
             for (int q = 0; q < kRowChunk; q++) {
-                const int i = min(c0 + t + 256 * q, n - 1);
+                const int i = min(c0 + t + NT * q, n - 1);
                 h[q] = a.hin[r + i];
                 wv[q] = a.pw ? a.pw[i] : 0.f;
             }
 #pragma unroll
             for (int q = 0; q < kRowChunk; q++) {
-                const int i = c0 + t + 256 * q;
+                const int i = c0 + t + NT * q;
                 if (i < n) {
                     const float nv = a.pw ? (row[i] * inv) * (a.poff + wv[q]) : row[i] * inv;
                     const float hv = (h[q] + nv) * a.scale;
@@ -255,16 +261,16 @@ __global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(ResidRows a)
     }
     if (!a.norm && !a.st.xe) return;  // (uniform)
     if (a.norm) {
-        const double tot = block_sum_d(ss, red[1]);
+        const double tot = block_sum_d<NT>(ss, red[1]);
         const float inv = 1.0f / static_cast<float>(sqrt(tot / static_cast<double>(n) + a.norm_eps));
         m = 0.f;
-        for (int c0 = 0; c0 < n; c0 += 256 * kRowChunk) {
+        for (int c0 = 0; c0 < n; c0 += NT * kRowChunk) {
             float wv[kRowChunk];
 #pragma unroll
-            for (int q = 0; q < kRowChunk; q++) wv[q] = c0 == 0 ? w0[q] : (a.w ? a.w[min(c0 + t + 256 * q, n - 1)] : 0.f);
+            for (int q = 0; q < kRowChunk; q++) wv[q] = c0 == 0 ? w0[q] : (a.w ? a.w[min(c0 + t + NT * q, n - 1)] : 0.f);
 #pragma unroll
             for (int q = 0; q < kRowChunk; q++) {
-                const int i = c0 + t + 256 * q;
+                const int i = c0 + t + NT * q;
                 if (i < n) {  // (the thread's own elements of `row`: no barrier needed)
                     const float x = a.w ? (row[i] * inv) * (a.off + wv[q]) : row[i] * inv;
                     if (a.xn) a.xn[r + i] = x;
@@ -274,7 +280,7 @@ __global__ __launch_bounds__(256) void resid_norm_stats_rows_kernel(ResidRows a)
             }
         }
     }
-    if (a.st.xe) lds_row_out<256>(row, n, ri, m, wm, a.st);
+    if (a.st.xe) lds_row_out<NT>(row, n, ri, m, wm, a.st);
 }
 
 // act = act(gate) * up over a row of n outputs (1024 threads), from gate/up rows with the pairs
@@ -385,8 +391,13 @@ void launch_resid_norm_stats_rows(const ResidRows& a, hipStream_t s) {
     if (a.m > 0x7FFFFF00 || a.splits < 1 || a.n % 32 != 0 || a.n > kFusedRowMax || !a.hin || (a.post && !a.P) ||
         (a.st.xp && !a.st.xe))
         fail(LARQL_HIP_ERR_INVALID, "fused residual and norm rows: bad arguments");
-    if (a.post) resid_norm_stats_rows_kernel<true><<<tile_rows_grid(a.m), dim3(256), 0, s>>>(a);
-    else resid_norm_stats_rows_kernel<false><<<tile_rows_grid(a.m), dim3(256), 0, s>>>(a);
+    auto go = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        if (a.post) resid_norm_stats_rows_kernel<NT, true><<<tile_rows_grid(a.m), dim3(NT), 0, s>>>(a);
+        else resid_norm_stats_rows_kernel<NT, false><<<tile_rows_grid(a.m), dim3(NT), 0, s>>>(a);
+    };
+    if (a.m >= current_device_cus()) go(std::integral_constant<int, 256>{});
+    else go(std::integral_constant<int, 1024>{});
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
