@@ -39,9 +39,10 @@ __device__ __forceinline__ long pack64(uint32_t lo, uint32_t hi) {
 }
 
 struct IgArgs {
-    const uint8_t* qs[2];  // up to two weights of one shape and their scales and outputs
-    const void* sc[2];
-    float* out[2];
+    const void* qs[kIntGemmMats];  // weights of one shape and their scales
+    const void* sc[kIntGemmMats];
+    float* out;                    // of the first weight; the others' ostep floats apart
+    ptrdiff_t ostep;
     const int8_t* X8;  // [M][K] codes
     const float* XS;   // [M][K / 32] scales
     int M, N, nb, ntiles, ldo, gx, gy, gz;
@@ -67,8 +68,8 @@ __global__ __launch_bounds__(kIgThreads) void int_gemm_kernel(IgArgs a) {
     if (grp >= a.gx * a.gz) return;
     const int bx = grp % a.gx, bz = grp / a.gx;
     const int t0 = by * 16 * TT, nt0 = (bx * kIgWaves + wave) * R;
-    const uint8_t* qs = a.qs[bz];
-    float* out = a.out[bz];
+    const uint8_t* qs = static_cast<const uint8_t*>(a.qs[bz]);
+    float* out = a.out + bz * a.ostep;
 
     // raw buffer loads (the launcher keeps the weights below 2 GiB): lane part + uniform part
     const uint32_t qbytes = static_cast<uint32_t>(a.ntiles) * 16u * (kQ40 ? static_cast<uint32_t>(K / 2) : static_cast<uint32_t>(K));
@@ -261,34 +262,12 @@ bool int_gemm_takes(const DevWeight& w) {
            w.rows_pad * w.cols <= 0x7FFFFFFF;
 }
 
-void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
-                     float* out2, size_t m, size_t ldo, hipStream_t s) {
-    if (m == 0) return;
-    if (ldo == 0) ldo = w.rows;
-    if (!int_gemm_takes(w) || (w2 && (w2->format != w.format || w2->rows != w.rows || w2->cols != w.cols)))
-        fail(LARQL_HIP_ERR_INVALID, "int GEMM: Q4_0 or Q8_0 weights of one shape, cols a multiple of 128");
-    if (ldo < w.rows || ldo > 0x7FFFFFFF || m > 0x7FFFFFFF / w.cols) fail(LARQL_HIP_ERR_INVALID, "int GEMM: bad sizes");
-    IgArgs a{};
-    a.qs[0] = w.qs;
-    a.sc[0] = w.d;
-    a.out[0] = out;
-    if (w2) {
-        a.qs[1] = w2->qs;
-        a.sc[1] = w2->d;
-        a.out[1] = out2;
-    }
-    a.X8 = q8x;
-    a.XS = q8s;
-    a.M = static_cast<int>(m);
-    a.N = static_cast<int>(w.rows);
-    a.nb = static_cast<int>(w.cols / 32);
-    a.ntiles = static_cast<int>(w.rows_pad / 16);
-    a.ldo = static_cast<int>(ldo);
-    a.gz = w2 ? 2 : 1;
+namespace {
+void launch_ig(IgArgs& a, int fmt, hipStream_t s) {
     // Token tiles and weight tiles per wave: the least modelled time, rounds of workgroups over
     // the CUs times a workgroup's VALU issue per block (16 per 16 x 16 tile, ~12 to unpack a
     // weight tile, ~30 of loop, staging and waits)
-    const long cus = current_device_cus(), mt = static_cast<long>((m + 15) / 16);
+    const long cus = current_device_cus(), mt = (static_cast<long>(a.M) + 15) / 16;
     int TT = 1, R = 1;
     double best = -1;
     for (int r = 1; r <= 2; r++)
@@ -300,9 +279,55 @@ void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x,
     a.gx = (a.ntiles + 4 * R - 1) / (4 * R);
     a.gy = static_cast<int>((mt + TT - 1) / TT);
     const unsigned grid = static_cast<unsigned>((static_cast<long>(a.gx) * a.gz + 7) / 8 * 8 * a.gy);
-    if (w.format == LARQL_Q4_0) launch_fmt<LARQL_Q4_0>(a, TT, R, grid, s);
+    if (fmt == LARQL_Q4_0) launch_fmt<LARQL_Q4_0>(a, TT, R, grid, s);
     else launch_fmt<LARQL_Q8_0>(a, TT, R, grid, s);
     LARQL_HIP_CHECK(hipGetLastError());
+}
+}  // namespace
+
+void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
+                     float* out2, size_t m, size_t ldo, hipStream_t s) {
+    if (m == 0) return;
+    if (ldo == 0) ldo = w.rows;
+    if (!int_gemm_takes(w) || (w2 && (w2->format != w.format || w2->rows != w.rows || w2->cols != w.cols)))
+        fail(LARQL_HIP_ERR_INVALID, "int GEMM: Q4_0 or Q8_0 weights of one shape, cols a multiple of 128");
+    if (ldo < w.rows || ldo > 0x7FFFFFFF || m > 0x7FFFFFFF / w.cols) fail(LARQL_HIP_ERR_INVALID, "int GEMM: bad sizes");
+    IgArgs a{};
+    a.qs[0] = w.qs;
+    a.sc[0] = w.d;
+    a.out = out;
+    if (w2) {
+        a.qs[1] = w2->qs;
+        a.sc[1] = w2->d;
+        a.ostep = out2 - out;
+    }
+    a.X8 = q8x;
+    a.XS = q8s;
+    a.M = static_cast<int>(m);
+    a.N = static_cast<int>(w.rows);
+    a.nb = static_cast<int>(w.cols / 32);
+    a.ntiles = static_cast<int>(w.rows_pad / 16);
+    a.ldo = static_cast<int>(ldo);
+    a.gz = w2 ? 2 : 1;
+    launch_ig(a, w.format, s);
+}
+
+void launch_int_gemm_q4_layers(const void* const* nib, const void* const* scales, int layers, const int8_t* X8,
+                               const float* XS, float* S, int F, int K, int Q, hipStream_t s) {
+    if (layers < 1 || layers > kIntGemmMats || K % 128) fail(LARQL_HIP_ERR_INVALID, "int GEMM: bad layers");
+    IgArgs a{};
+    for (int l = 0; l < layers; l++) a.qs[l] = nib[l], a.sc[l] = scales[l];
+    a.out = S;
+    a.ostep = static_cast<ptrdiff_t>(Q) * F;
+    a.X8 = X8;
+    a.XS = XS;
+    a.M = Q;
+    a.N = F;
+    a.nb = K / 32;
+    a.ntiles = static_cast<int>(pad_rows(static_cast<size_t>(F)) / 16);
+    a.ldo = F;
+    a.gz = layers;
+    launch_ig(a, LARQL_Q4_0, s);
 }
 
 }  // namespace larql

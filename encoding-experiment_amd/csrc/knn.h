@@ -21,7 +21,9 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
                             hipStream_t s);
 size_t gate_scores_f32_ws_floats(int K, int Q);
 // S[l][q][f] = sum_b (float)isum * (f16(scale) * XS[q][b]) in block order (Q4_0 x Q8).
-// XA / XSP: work buffers of q4_xa_bytes / q4_xsp_bytes (the queries as MFMA operands).
+// XA / XSP: work buffers of q4_xa_bytes / q4_xsp_bytes (the queries as MFMA operands), unused
+// where gate_scores_q4_direct.
+bool gate_scores_q4_direct(int n_layers, int F, int K, int Q);
 void launch_gate_scores_q4(const KnnLayers& nibbles, const KnnLayers& scales, int n_layers, const int8_t* X8,
                            const float* XS, uint4* XA, float* XSP, float* S, int F, int K, int Q, hipStream_t s);
 size_t q4_xa_bytes(int K, int Q);

@@ -1025,9 +1025,21 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
+// The int GEMM (gemm_int.hip, tiles of 16 .. 64 queries, the codes staged as they lie) for few
+// queries or walks too small for the 128 x 128 tiles to fill the GPU.  Scores of 34 x [10240 x
+// 2560]: 1 query 178 against 266 us, 32 queries 219 against 281, 64 queries 355 against 352, 256
+// queries 1143 against 1001; 6 x [3000 x 1152]: 1 query 14 against 21 us, 256 queries 46 against 60.
+bool gate_scores_q4_direct(int n_layers, int F, int K, int Q) {
+    if (K % 128 || static_cast<size_t>(F) * K > 0x7FFFFFFF) return false;
+    const long wgs = static_cast<long>((F + kQ4TileF - 1) / kQ4TileF) * ((Q + 8 * kQ4TileG - 1) / (8 * kQ4TileG)) * n_layers;
+    return Q <= 32 || wgs < 2L * current_device_cus();
+}
+
 void launch_gate_scores_q4(const KnnLayers& nib, const KnnLayers& scales, int n_layers, const int8_t* X8,
                            const float* XS, uint4* XA, float* XSP, float* S, int F, int K, int Q, hipStream_t s) {
     if (K % 64) fail(LARQL_HIP_ERR_INVALID, "gate scores: Q4_0 hidden must be a multiple of 64");
+    if (gate_scores_q4_direct(n_layers, F, K, Q))
+        return launch_int_gemm_q4_layers(nib.p, scales.p, n_layers, X8, XS, S, F, K, Q, s);
     const int ng = (Q + 7) / 8;
     const size_t nxa = static_cast<size_t>(K / 64) * ng * 64;
     q4_xa_kernel<<<dim3(static_cast<unsigned>((nxa + 255) / 256)), dim3(256), 0, s>>>(X8, XS, XA, XSP, K, Q, ng);

@@ -300,6 +300,10 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
 // Q4_0 or Q8_0 weights (cols a multiple of 128) x any number of Q8 rows, block order as the
 // matvecs (gemm_int.hip); w2 / out2: a second weight of the same format and shape in the same
 // launch.  Output rows ldo floats apart (0: w.rows).
+// launch_int_gemm_q4_layers: S[l][q][f] over up to kIntGemmMats Q4_0 matrices [F x K].
+constexpr int kIntGemmMats = LARQL_HIP_KNN_MAX_LAYERS;
+void launch_int_gemm_q4_layers(const void* const* nib, const void* const* scales, int layers, const int8_t* X8,
+                               const float* XS, float* S, int F, int K, int Q, hipStream_t s);
 bool int_gemm_takes(const DevWeight& w);
 void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
                      float* out2, size_t m, size_t ldo, hipStream_t s);

@@ -94,7 +94,9 @@ def test_gate_scores_f32_query_counts_bit_exact(hip, nq, features, hidden):
             hip.release_weight(h)
 
 
-@pytest.mark.parametrize("features,hidden,nq,k", [(10240, 2560, 6, 32), (1000, 2560, 130, 17), (64, 64, 2, 64)])
+# hidden a multiple of 128 (the int GEMM; its tiles' edges) or of 64 only (the 128 x 128 tiles)
+@pytest.mark.parametrize("features,hidden,nq,k", [(10240, 2560, 6, 32), (1000, 2560, 130, 17), (64, 64, 2, 64),
+                                                  (129, 384, 17, 32), (70, 128, 49, 5), (300, 192, 65, 32)])
 def test_gate_knn_q4_bit_exact(hip, features, hidden, nq, k):
     print(f"[knn q4] F={features} K={hidden} nq={nq} k={k}", flush=True)
     gate = oracle.gauss(31, features * hidden, 0.0, 0.02)
