@@ -322,11 +322,6 @@ extern "C" int larql_hip_q4k_matmul(larql_hip_ctx* c, const uint8_t* q4k_data, s
     });
 }
 
-static float* f32_ws(larql_hip_ctx* c, size_t m, size_t k, size_t n, int transpose_b) {
-    const size_t f = larql::f32_matmul_ws_floats(m, k, n, transpose_b != 0);
-    return f ? static_cast<float*>(larql::ensure(c, c->knn_xpad, f * sizeof(float))) : nullptr;
-}
-
 extern "C" int larql_hip_matmul(larql_hip_ctx* c, const float* a, size_t m, size_t k, const float* b, size_t n,
                                 int transpose_b, float* out) {
     return guarded(c, [&] {
@@ -335,7 +330,7 @@ extern "C" int larql_hip_matmul(larql_hip_ctx* c, const float* a, size_t m, size
         const float* da = k ? stage_upload(c, c->stage_in, a, m * k) : nullptr;
         const float* db = k ? stage_upload(c, c->stage_in2, b, n * k) : nullptr;
         float* dc = static_cast<float*>(larql::ensure(c, c->stage_out, m * n * sizeof(float)));
-        larql::launch_f32_matmul(da, db, dc, m, k, n, transpose_b != 0, f32_ws(c, m, k, n, transpose_b), c->stream);
+        larql::launch_f32_matmul(da, db, dc, m, k, n, transpose_b != 0, c->stream);
         download(c, out, dc, m * n * sizeof(float));
     });
 }
@@ -345,7 +340,7 @@ extern "C" int larql_hip_matmul_dev(larql_hip_ctx* c, const float* a, size_t m, 
     return guarded(c, [&] {
         if (m == 0 || n == 0) return;
         if (!out || (k > 0 && (!a || !b))) fail(LARQL_HIP_ERR_INVALID, "null pointer");
-        larql::launch_f32_matmul(a, b, out, m, k, n, transpose_b != 0, f32_ws(c, m, k, n, transpose_b), pick_stream(c, stream));
+        larql::launch_f32_matmul(a, b, out, m, k, n, transpose_b != 0, pick_stream(c, stream));
     });
 }
 

@@ -44,16 +44,17 @@ KnnPlan plan_layers(larql_hip_ctx* c, const uint64_t* handles, size_t n_layers) 
     return p;
 }
 
-// Scores [n_layers][nq][F] into `scores` (device).
+// Scores [n_layers][nq][F] into `scores` (device; own_scores: a work buffer of the context).
 void run_scores(larql_hip_ctx* c, const KnnPlan& p, size_t n_layers, const float* queries, size_t nq, float* scores,
-                hipStream_t s) {
+                hipStream_t s, bool own_scores) {
     if (!queries || !scores || nq == 0) fail(LARQL_HIP_ERR_INVALID, "gate KNN: null queries/scores or nq == 0");
     if (nq > 0x7FFFFFFF / static_cast<size_t>(p.K)) fail(LARQL_HIP_ERR_INVALID, "gate KNN: too many queries");
     const int Q = static_cast<int>(nq);
     if (p.format == LARQL_F32) {
-        const size_t nws = larql::gate_scores_f32_ws_floats(p.K, Q);
+        // (scores into the caller's buffer use no work buffer of the context where none is needed)
+        const size_t nws = larql::gate_scores_f32_ws_floats(p.K, Q, own_scores);
         float* ws = nws ? static_cast<float*>(larql::ensure(c, c->knn_xpad, nws * sizeof(float))) : nullptr;
-        larql::launch_gate_scores_f32(p.a, static_cast<int>(n_layers), queries, ws, scores, p.F, p.K, Q, s);
+        larql::launch_gate_scores_f32(p.a, static_cast<int>(n_layers), queries, ws, nws, scores, p.F, p.K, Q, s);
     } else {
         int8_t* q8 = static_cast<int8_t*>(larql::ensure(c, c->knn_q8, nq * p.K));
         float* q8s = static_cast<float*>(larql::ensure(c, c->knn_q8s, nq * (p.K / 32) * sizeof(float)));
@@ -100,7 +101,7 @@ extern "C" int larql_hip_gate_scores_dev(larql_hip_ctx* c, const uint64_t* handl
                                          const float* queries, size_t nq, float* scores, void* stream) {
     return guarded(c, [&] {
         const KnnPlan p = plan_layers(c, handles, n_layers);
-        run_scores(c, p, n_layers, queries, nq, scores, pick_stream(c, stream));
+        run_scores(c, p, n_layers, queries, nq, scores, pick_stream(c, stream), false);
     });
 }
 
@@ -113,7 +114,7 @@ extern "C" int larql_hip_gate_knn_dev(larql_hip_ctx* c, const uint64_t* handles,
         if (!idx || !scores) fail(LARQL_HIP_ERR_INVALID, "gate KNN: null outputs");
         hipStream_t s = pick_stream(c, stream);
         float* S = static_cast<float*>(larql::ensure(c, c->knn_scores, n_layers * nq * p.F * sizeof(float)));
-        run_scores(c, p, n_layers, queries, nq, S, s);
+        run_scores(c, p, n_layers, queries, nq, S, s, true);
         topk_any(c, S, n_layers * nq, static_cast<size_t>(p.F), p.F, top_k, 0, idx, scores, s);
     });
 }
@@ -143,7 +144,7 @@ extern "C" int larql_hip_gate_knn(larql_hip_ctx* c, int format, const void* gate
         float* dq = static_cast<float*>(larql::ensure(c, c->stage_in, qbytes));
         LARQL_HIP_CHECK(hipMemcpyAsync(dq, queries, qbytes, hipMemcpyHostToDevice, c->stream));
         float* S = static_cast<float*>(larql::ensure(c, c->knn_scores, nq * p.F * sizeof(float)));
-        run_scores(c, p, 1, dq, nq, S, c->stream);
+        run_scores(c, p, 1, dq, nq, S, c->stream, true);
         uint32_t* di = static_cast<uint32_t*>(larql::ensure(c, c->knn_idx, nq * top_k * sizeof(uint32_t)));
         float* dv = static_cast<float*>(larql::ensure(c, c->knn_val, nq * top_k * sizeof(float)));
         topk_any(c, S, nq, static_cast<size_t>(p.F), p.F, top_k, 0, di, dv, c->stream);

@@ -8,7 +8,8 @@
 // its own order, within f32 rounding of this one.
 //
 // Two forms: lanes (a chain per lane, the other side's values as scalar operands), and 256 x 64
-// tiles for large products whose larger side is k-major.
+// tiles for large products.
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.h"
@@ -22,11 +23,14 @@ namespace {
 constexpr int kGThreads = 256;
 constexpr int kGTileR = 256, kGTileC = 64, kGKs = 16;
 
-// Workgroup tile: 256 "rows" (operand R, k-major: element k of row r at k ldr + r) x 64 "columns"
-// (operand C, k-minor), thread tile 8 x 8, K in LDS stages of 16 (double-buffered, the next stage's
-// global loads held in registers while the current one is consumed); out[c][r].  Loads are scalar
-// and predicated (any K, any alignment); rows and columns past the matrix are clamped duplicates,
-// never stored.
+// Workgroup tile: 256 "rows" (operand R) x 64 "columns" (operand C), thread tile 8 x 8,
+// K in LDS stages of 16 (double-buffered, the next stage's global loads held in registers
+// while the current one is consumed).  Each operand may be k-minor in memory (a row of K
+// floats per row / column) or k-major (a row of the other dimension per k); the LDS tiles
+// are k-major either way.  The launcher puts the larger of m and n on the 256 side and
+// stores C transposed when it swaps them.  Loads are scalar and predicated (any K, any
+// alignment); rows and columns past the matrix are clamped duplicates, never stored.
+template <bool R_KMAJOR, bool C_KMAJOR, bool OUT_T>
 __global__ __launch_bounds__(kGThreads) void f32_gemm_kernel(const float* __restrict__ R, size_t ldr,
                                                              const float* __restrict__ Cm, size_t ldc,
                                                              float* __restrict__ out, size_t ldo, int Rn, int Cn,
@@ -37,37 +41,61 @@ __global__ __launch_bounds__(kGThreads) void f32_gemm_kernel(const float* __rest
     const int r0 = blockIdx.y * kGTileR, c0 = blockIdx.x * kGTileC;
     const int tr = tid & 31, tc = tid >> 5;  // rows r0 + 8 tr .., columns c0 + 8 tc ..
 
-    // R stage: thread = (rows r0 + 4 (tid & 63) .. + 3, k 4 (tid >> 6) .. + 3)
+    // R stage: k-minor, thread = row r0 + tid, 16 consecutive k; k-major, thread =
+    // (rows r0 + 4 (tid & 63) .. + 3, k 4 (tid >> 6) .. + 3)
     float rv[16];
     auto rload = [&](int k0) __attribute__((always_inline)) {
-        const int rr = 4 * (tid & 63), kk = 4 * (tid >> 6);
+        if constexpr (!R_KMAJOR) {
+            const float* p = R + static_cast<size_t>(min(r0 + tid, Rn - 1)) * ldr;
 #pragma unroll
-        for (int a = 0; a < 4; a++)
+            for (int i = 0; i < 16; i++) rv[i] = k0 + i < K ? p[k0 + i] : 0.f;
+        } else {
+            const int rr = 4 * (tid & 63), kk = 4 * (tid >> 6);
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int k = k0 + kk + a;
-                rv[4 * a + b] = k < K ? R[static_cast<size_t>(k) * ldr + min(r0 + rr + b, Rn - 1)] : 0.f;
-            }
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const int k = k0 + kk + a;
+                    rv[4 * a + b] = k < K ? R[static_cast<size_t>(k) * ldr + min(r0 + rr + b, Rn - 1)] : 0.f;
+                }
+        }
     };
     auto rstore = [&](int buf) __attribute__((always_inline)) {
-        const int rr = 4 * (tid & 63), kk = 4 * (tid >> 6);
+        if constexpr (!R_KMAJOR) {
 #pragma unroll
-        for (int a = 0; a < 4; a++)
-            *reinterpret_cast<float4*>(&Rs[buf][kk + a][rr]) =
-                make_float4(rv[4 * a], rv[4 * a + 1], rv[4 * a + 2], rv[4 * a + 3]);
+            for (int i = 0; i < 16; i++) Rs[buf][i][tid] = rv[i];
+        } else {
+            const int rr = 4 * (tid & 63), kk = 4 * (tid >> 6);
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+                *reinterpret_cast<float4*>(&Rs[buf][kk + a][rr]) =
+                    make_float4(rv[4 * a], rv[4 * a + 1], rv[4 * a + 2], rv[4 * a + 3]);
+        }
     };
-    // C stage: thread = (column c0 + (tid & 63), k 4 (tid >> 6) .. + 3)
+    // C stage: k-minor, thread = (column c0 + (tid & 63), k 4 (tid >> 6) .. + 3); k-major,
+    // thread = (columns c0 + 4 (tid & 15) .. + 3, k tid >> 4)
     float cv[4];
     auto cload = [&](int k0) __attribute__((always_inline)) {
-        const float* p = Cm + static_cast<size_t>(min(c0 + (tid & 63), Cn - 1)) * ldc;
-        const int kk = k0 + 4 * (tid >> 6);
+        if constexpr (!C_KMAJOR) {
+            const float* p = Cm + static_cast<size_t>(min(c0 + (tid & 63), Cn - 1)) * ldc;
+            const int kk = k0 + 4 * (tid >> 6);
 #pragma unroll
-        for (int i = 0; i < 4; i++) cv[i] = kk + i < K ? p[kk + i] : 0.f;
+            for (int i = 0; i < 4; i++) cv[i] = kk + i < K ? p[kk + i] : 0.f;
+        } else {
+            const int k = k0 + (tid >> 4), cc = 4 * (tid & 15);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                cv[i] = k < K ? Cm[static_cast<size_t>(k) * ldc + min(c0 + cc + i, Cn - 1)] : 0.f;
+        }
     };
     auto cstore = [&](int buf) __attribute__((always_inline)) {
-        const int kk = 4 * (tid >> 6);
+        if constexpr (!C_KMAJOR) {
+            const int kk = 4 * (tid >> 6);
 #pragma unroll
-        for (int i = 0; i < 4; i++) Cs[buf][kk + i][tid & 63] = cv[i];
+            for (int i = 0; i < 4; i++) Cs[buf][kk + i][tid & 63] = cv[i];
+        } else {
+            *reinterpret_cast<float4*>(&Cs[buf][tid >> 4][4 * (tid & 15)]) = make_float4(cv[0], cv[1], cv[2], cv[3]);
+        }
     };
 
     float acc[8][8];
@@ -120,34 +148,15 @@ __global__ __launch_bounds__(kGThreads) void f32_gemm_kernel(const float* __rest
         for (int j = 0; j < 8; j++) {
             const int c = c0 + tc * 8 + j;
             if (c >= Cn) continue;
-            out[static_cast<size_t>(c) * ldo + r] = acc[i][j];
+            if constexpr (OUT_T) out[static_cast<size_t>(c) * ldo + r] = acc[i][j];
+            else out[static_cast<size_t>(r) * ldo + c] = acc[i][j];
         }
     }
 }
 
 // ── few rows on one side, or too few tiles to fill the GPU ────────────────
-// XT[b][k][QW] = the QW queries of block b at k: element k of query QW b + i (at
-// X + q sq + k sk) for existing queries and k < K, else +0 (b < Qp / QW, k < Kp).
-__global__ void queries_t_kernel(const float* __restrict__ X, size_t sq, size_t sk, float* __restrict__ XT, int Q,
-                                 int K, int Kp, int Qp, int qw) {
-    __shared__ float t[32][33];
-    const int nk = (Kp + 31) / 32, k0 = 32 * static_cast<int>(blockIdx.x % nk), q0 = 32 * static_cast<int>(blockIdx.x / nk);
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int q = q0 + ty + 8 * i, k = k0 + tx;
-        t[ty + 8 * i][tx] = (q < Q && k < K) ? X[q * sq + k * sk] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int k = k0 + ty + 8 * i, q = q0 + tx;
-        if (k < Kp && q < Qp) XT[(static_cast<size_t>(q / qw) * Kp + k) * qw + q % qw] = t[tx][ty + 8 * i];
-    }
-}
-
 // The larger of m and n ("rows") goes over the lanes, one fma chain each, the other side's QW values
-// at a k come as scalar operands (XT, scalar loads): 64 rows x QW NW columns per workgroup, so a
+// at a k come as scalar operands (scalar loads of X as it lies): 64 rows x QW NW columns per workgroup, so a
 // product fills the GPU with waves where 256 x 64 tiles would leave most CUs idle.  K_MAJOR rows
 // (element k of row r at k ld + r) are read as they lie, a 256-byte line per k, 16 k ahead.
 // Others are staged by global_load_lds, E floats a lane (4 where rows are 16-byte aligned, else 1),
@@ -156,8 +165,8 @@ __global__ void queries_t_kernel(const float* __restrict__ X, size_t sq, size_t 
 // different banks.  The ring is read and waited for in one asm block, since the compiler does not
 // track by stage the loads that fill it.
 // Bound: the chains' and the scalar loads' latency in few waves, fp32 VALU issue in many.  One row
-// by [10240 x 2560] 71 us (755 in tiles: 40 of them), 7 by [12000 x 2600] 126 (903), by [2600 x
-// 12000] 119 (541), 16 by [1000 x 2000] 87 (575), 512 by [12000 x 2600] 685 us, 47 TFLOP/s (1317).
+// by [10240 x 2560] 71 us (755 in tiles: 40 of them), 7 by [12000 x 2600] 116 (903), by [2600 x
+// 12000] 119 (541), 16 by [1000 x 2000] 48 (575), 512 by [12000 x 2600] 836 us, 38 TFLOP/s (1317).
 constexpr int kLaneNd = 3;
 
 template <int E>
@@ -201,32 +210,37 @@ __device__ __forceinline__ void load_lds(const float* src, float* dst) {
     else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
-template <int QW, int NW, bool K_MAJOR, bool OUT_T, int E>
+template <int QW, int NW, bool K_MAJOR, bool X_KMAJOR, bool OUT_T, int E>
 __global__ __launch_bounds__(64 * NW) void f32_lane_gemm_kernel(const float* __restrict__ G, size_t ld,
-                                                                const float* __restrict__ XT, float* __restrict__ out,
-                                                                size_t ldo, int R, int K, int Q) {
+                                                                const float* __restrict__ X, size_t ldx,
+                                                                float* __restrict__ out, size_t ldo, int R, int K, int Q) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = blockIdx.x * 64, q0 = (blockIdx.y * NW + wave) * QW;
-    const scalar_f32_ptr xt =
-        (scalar_f32_ptr)(reinterpret_cast<uintptr_t>(XT) + sizeof(float) * (static_cast<size_t>(q0) * K));
+    // (waves past the last column repeat the last QW of the Q >= QW: the same values again)
+    const int r0 = blockIdx.x * 64, q0 = min((static_cast<int>(blockIdx.y) * NW + wave) * QW, Q - QW);
+    // column q0 + q at k: X k-minor, x[q ldx + k]; k-major, x[k ldx + q]
+    const scalar_f32_ptr x = (scalar_f32_ptr)(reinterpret_cast<uintptr_t>(X) +
+                                              sizeof(float) * (X_KMAJOR ? static_cast<size_t>(q0) : q0 * ldx));
     float acc[QW];
 #pragma unroll
     for (int q = 0; q < QW; q++) acc[q] = 0.f;
-    // n k from k0 on (n <= 16) whose values this lane holds
+    // 16 k (or n < 16) from k0 on, whose values of its row the lane holds
     auto full = [&](int k0, const float (&v)[16]) __attribute__((always_inline)) {
-        const scalar_f32_ptr x = xt + static_cast<size_t>(k0) * QW;
+        if constexpr (X_KMAJOR) {
 #pragma unroll
-        for (int i = 0; i < 16; i++)
+            for (int i = 0; i < 16; i++)
 #pragma unroll
-            for (int q = 0; q < QW; q++) acc[q] = fmaf(v[i], x[i * QW + q], acc[q]);
+                for (int q = 0; q < QW; q++) acc[q] = fmaf(v[i], x[static_cast<size_t>(k0 + i) * ldx + q], acc[q]);
+        } else {
+            lane_fma16<QW>(acc, v, x, ldx, k0);
+        }
     };
     auto part = [&](int k0, int n, const float (&v)[16]) __attribute__((always_inline)) {
-        const scalar_f32_ptr x = xt + static_cast<size_t>(k0) * QW;
 #pragma unroll
         for (int i = 0; i < 15; i++)
             if (i < n)
 #pragma unroll
-                for (int q = 0; q < QW; q++) acc[q] = fmaf(v[i], x[i * QW + q], acc[q]);
+                for (int q = 0; q < QW; q++)
+                    acc[q] = fmaf(v[i], X_KMAJOR ? x[static_cast<size_t>(k0 + i) * ldx + q] : x[q * ldx + k0 + i], acc[q]);
     };
     if constexpr (K_MAJOR) {
         const float* p = G + min(r0 + lane, R - 1);
@@ -300,23 +314,34 @@ __global__ __launch_bounds__(64 * NW) void f32_lane_gemm_kernel(const float* __r
     const int r = r0 + lane;
     if (r >= R) return;
 #pragma unroll
-    for (int q = 0; q < QW; q++)
-        if (q0 + q < Q) {
-            if constexpr (OUT_T) out[static_cast<size_t>(r) * ldo + q0 + q] = acc[q];
-            else out[static_cast<size_t>(q0 + q) * ldo + r] = acc[q];
-        }
+    for (int q = 0; q < QW; q++) {
+        if constexpr (OUT_T) out[static_cast<size_t>(r) * ldo + q0 + q] = acc[q];
+        else out[static_cast<size_t>(q0 + q) * ldo + r] = acc[q];
+    }
+}
+
+template <bool RK, bool CK, bool OT>
+void launch_gemm(const float* R, size_t ldr, const float* Cm, size_t ldc, float* out, size_t ldo, size_t Rn,
+                 size_t Cn, size_t K, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>((Cn + kGTileC - 1) / kGTileC),
+                    static_cast<unsigned>((Rn + kGTileR - 1) / kGTileR));
+    f32_gemm_kernel<RK, CK, OT><<<grid, dim3(kGThreads), 0, s>>>(R, ldr, Cm, ldc, out, ldo, static_cast<int>(Rn),
+                                                                 static_cast<int>(Cn), static_cast<int>(K));
+    LARQL_HIP_CHECK(hipGetLastError());
 }
 
 // Whether the lanes' form runs a product of `rows` x `q` (rows >= q) whose rows are k-minor or
-// k-major.  The tiles take k-minor rows a float at a time per thread, 24 TFLOP/s at their best (512
-// x [12000 x 2600]: 1317 us); k-major ones keep the tiles where most CUs get one (300 x [2600 x
-// 12000], 235 tiles: 540 us, 609 in lanes; 100 x [2600 x 12000], 94 tiles: 541 us, 353 in lanes).
+// k-major.  The tiles take k-minor rows a float at a time per thread: lanes up to two tiles per
+// CU (512 x [12000 x 2600], 376 tiles: 836 us in lanes, 1317 in tiles); k-major rows below three
+// tiles for four CUs (100 x [2600 x 12000], 94 tiles: 353 us in lanes, 541 in tiles; 300 columns,
+// 235 tiles: 609 and 540).
 bool lane_form(size_t rows, size_t q, size_t k, bool k_major) {
     const size_t tiles = (rows + kGTileR - 1) / kGTileR * ((q + kGTileC - 1) / kGTileC);
-    return k > 0 && (!k_major || 4 * tiles < 3 * static_cast<size_t>(current_device_cus()));
+    const size_t cus = static_cast<size_t>(current_device_cus());
+    return k > 0 && (k_major ? 4 * tiles < 3 * cus : tiles < 2 * cus);
 }
 
-// Columns per wave and waves per workgroup.
+// Columns per wave (at most q) and waves per workgroup.
 struct LanePlan {
     int qw, nw;
 };
@@ -326,24 +351,19 @@ LanePlan lane_plan(size_t q) {
     if (q <= 32) return {4, 8};
     return {8, 8};
 }
-size_t lane_qp(size_t q) {
-    const LanePlan p = lane_plan(q);
-    const size_t b = static_cast<size_t>(p.qw) * p.nw;
-    return (q + b - 1) / b * b;
-}
-
-template <bool KM, bool OT, int E>
-void launch_lane(const float* G, size_t ld, const float* XT, float* out, size_t ldo, int R, int K, int Q, hipStream_t s) {
+template <bool KM, bool XK, bool OT, int E>
+void launch_lane(const float* G, size_t ld, const float* X, size_t ldx, float* out, size_t ldo, int R, int K, int Q, hipStream_t s) {
     const LanePlan p = lane_plan(static_cast<size_t>(Q));
     const unsigned gx = static_cast<unsigned>((R + 63) / 64);
-    const size_t blocks = lane_qp(static_cast<size_t>(Q)) / (p.qw * p.nw);
+    const size_t per = static_cast<size_t>(p.qw) * p.nw, blocks = (Q + per - 1) / per;
     auto go = [&](auto qw, auto nw) {
         constexpr int QW = decltype(qw)::value, NW = decltype(nw)::value;
         for (size_t y = 0; y < blocks; y += 65535) {  // (grid y is at most 65535)
-            const size_t q0 = y * QW * NW;
-            f32_lane_gemm_kernel<QW, NW, KM, OT, E>
+            // (a last launch of fewer than QW columns starts earlier: the same values again)
+            const size_t q0 = std::min(y * per, static_cast<size_t>(Q - QW));
+            f32_lane_gemm_kernel<QW, NW, KM, XK, OT, E>
                 <<<dim3(gx, static_cast<unsigned>(blocks - y < 65535 ? blocks - y : 65535)), dim3(64 * NW), 0, s>>>(
-                    G, ld, XT + q0 * K, out + (OT ? q0 : q0 * ldo), ldo, R, K, Q - static_cast<int>(q0));
+                    G, ld, X + (XK ? q0 : q0 * ldx), ldx, out + (OT ? q0 : q0 * ldo), ldo, R, K, Q - static_cast<int>(q0));
         }
     };
     using std::integral_constant;
@@ -363,19 +383,8 @@ void launch_lane(const float* G, size_t ld, const float* XT, float* out, size_t 
 
 }  // namespace
 
-void launch_queries_t(const float* X, size_t sq, size_t sk, float* XT, int Q, int K, int Kp, int Qp, int qw,
-                      hipStream_t s) {
-    queries_t_kernel<<<dim3(((Kp + 31) / 32) * ((Qp + 31) / 32)), dim3(256), 0, s>>>(X, sq, sk, XT, Q, K, Kp, Qp, qw);
-    LARQL_HIP_CHECK(hipGetLastError());
-}
-
-size_t f32_matmul_ws_floats(size_t m, size_t k, size_t n, bool transpose_b) {
-    const size_t rows = m > n ? m : n, q = m > n ? n : m;
-    return q > 1 && lane_form(rows, q, k, m <= n && !transpose_b) ? k * lane_qp(q) : 0;
-}
-
 void launch_f32_matmul(const float* A, const float* B, float* C, size_t m, size_t k, size_t n, bool transpose_b,
-                       float* ws, hipStream_t s) {
+                       hipStream_t s) {
     if (m == 0 || n == 0) return;
     if (m > 0x7FFFFFFFu || n > 0x7FFFFFFFu || k > 0x7FFFFFFFu || (m + kGTileR - 1) / kGTileR > 65535 ||
         (n + kGTileR - 1) / kGTileR > 65535)
@@ -383,31 +392,27 @@ void launch_f32_matmul(const float* A, const float* B, float* C, size_t m, size_
     const bool swap = m > n;  // A's rows over the lanes
     const size_t rows = swap ? m : n, q = swap ? n : m;
     if (lane_form(rows, q, k, !swap && !transpose_b)) {
-        // the scalar side's element k of column i: A [m][k], B [n][k] or B [k][n]
-        const float* X = swap ? B : A;
-        const size_t sq = swap && !transpose_b ? 1 : k, sk = swap && !transpose_b ? n : 1;
-        const float* XT = X;  // one column lies as it is needed
         const int R = static_cast<int>(rows), K = static_cast<int>(k), Q = static_cast<int>(q);
-        if (q > 1) {
-            if (!ws) fail(LARQL_HIP_ERR_INVALID, "matmul: no workspace");
-            launch_queries_t(X, sq, sk, ws, Q, K, K, static_cast<int>(lane_qp(q)), lane_plan(q).qw, s);
-            XT = ws;
-        }
         const float* G = swap ? A : B;
         const bool al16 = k % 4 == 0 && reinterpret_cast<uintptr_t>(G) % 16 == 0;
-        if (!swap && !transpose_b) launch_lane<true, false, 1>(G, n, XT, C, n, R, K, Q, s);
-        else if (!swap && al16) launch_lane<false, false, 4>(G, k, XT, C, n, R, K, Q, s);
-        else if (!swap) launch_lane<false, false, 1>(G, k, XT, C, n, R, K, Q, s);
-        else if (al16) launch_lane<false, true, 4>(G, k, XT, C, n, R, K, Q, s);
-        else launch_lane<false, true, 1>(G, k, XT, C, n, R, K, Q, s);
+        if (!swap && !transpose_b) launch_lane<true, false, false, 1>(B, n, A, k, C, n, R, K, Q, s);
+        else if (!swap && al16) launch_lane<false, false, false, 4>(B, k, A, k, C, n, R, K, Q, s);
+        else if (!swap) launch_lane<false, false, false, 1>(B, k, A, k, C, n, R, K, Q, s);
+        else if (transpose_b && al16) launch_lane<false, false, true, 4>(A, k, B, k, C, n, R, K, Q, s);
+        else if (transpose_b) launch_lane<false, false, true, 1>(A, k, B, k, C, n, R, K, Q, s);
+        else if (al16) launch_lane<false, true, true, 4>(A, k, B, n, C, n, R, K, Q, s);
+        else launch_lane<false, true, true, 1>(A, k, B, n, C, n, R, K, Q, s);
         return;
     }
-    // B [k][n], the larger side, as rows, A's rows as columns, C stored as it lies (for k = 0, zeros,
-    // also where B is not so: nothing is loaded)
-    const dim3 grid(static_cast<unsigned>((m + kGTileC - 1) / kGTileC), static_cast<unsigned>((n + kGTileR - 1) / kGTileR));
-    f32_gemm_kernel<<<grid, dim3(kGThreads), 0, s>>>(B, n, A, k, C, n, static_cast<int>(n), static_cast<int>(m),
-                                                     static_cast<int>(k));
-    LARQL_HIP_CHECK(hipGetLastError());
+    // A [m][k] is k-minor; B is [n][k] (k-minor, transpose_b) or [k][n] (k-major).  The
+    // larger of m and n goes on the 256 side; C [m][n] is stored transposed when n is there.
+    if (transpose_b) {
+        if (m >= n) launch_gemm<false, false, false>(A, k, B, k, C, n, m, n, k, s);
+        else launch_gemm<false, false, true>(B, k, A, k, C, n, n, m, k, s);
+    } else {
+        if (m >= n) launch_gemm<false, true, false>(A, k, B, n, C, n, m, n, k, s);
+        else launch_gemm<true, false, true>(B, n, A, k, C, n, n, m, k, s);
+    }
 }
 
 }  // namespace larql

@@ -9,7 +9,7 @@ namespace larql {
 
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-// A query block of a k: QW consecutive floats at a wave-uniform address, read with scalar loads.
+// Floats at wave-uniform addresses, read with scalar loads.
 typedef const float __attribute__((address_space(4))) * scalar_f32_ptr;
 
 // At most N vector memory operations of the wave still in flight.
@@ -18,9 +18,18 @@ __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// The scalar operands' layout: XT[b][k][qw] = element k of query qw b + i (at X + q sq + k sk) for
-// q < Q and k < K, else +0; b < Qp / qw, k < Kp (f32_gemm.hip).
-void launch_queries_t(const float* X, size_t sq, size_t sk, float* XT, int Q, int K, int Kp, int Qp, int qw,
-                      hipStream_t s);
+// acc[q] += v[i] x_q[k0 + i] for i = 0 .. 15 in order, x_q the row q (< QW) at X + q sq of a k-minor
+// matrix: 16 consecutive floats per row as scalar operands, four rows' chains side by side.
+template <int QW>
+__device__ __forceinline__ void lane_fma16(float (&acc)[QW], const float (&v)[16], scalar_f32_ptr X, size_t sq, int k0) {
+    constexpr int G = QW < 4 ? QW : 4;
+#pragma unroll
+    for (int q0 = 0; q0 < QW; q0 += G) {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int q = q0; q < q0 + G; q++) acc[q] = fmaf(v[i], X[q * sq + k0 + i], acc[q]);
+    }
+}
 
 }  // namespace larql

@@ -15,11 +15,11 @@ struct KnnLayers {
 
 // S[l][q][f] = G_l[f, :] . X[q, :], one fma chain over k from +0 per element.
 // Gate rows lie f32_row_stride(K) floats apart, padded with -0 (a padded term leaves a
-// chain as it is); X [Q][K] is dense.  ws: gate_scores_f32_ws_floats(K, Q) floats (the
-// queries k-major; none for one query whose rows need no padding).
-void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, float* S, int F, int K, int Q,
-                            hipStream_t s);
-size_t gate_scores_f32_ws_floats(int K, int Q);
+// chain as it is); X [Q][K] is dense.  ws: gate_scores_f32_ws_floats floats, the queries padded
+// or, if may_transpose and it pays, k-major (none where neither).
+void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, size_t ws_floats, float* S, int F,
+                            int K, int Q, hipStream_t s);
+size_t gate_scores_f32_ws_floats(int K, int Q, bool may_transpose);
 // S[l][q][f] = sum_b (float)isum * (f16(scale) * XS[q][b]) in block order (Q4_0 x Q8).
 // XA / XSP: work buffers of q4_xa_bytes / q4_xsp_bytes (the queries as MFMA operands), unused
 // where gate_scores_q4_direct.

@@ -30,17 +30,36 @@ constexpr int kThreads = 256;
 // ── f32 scores ─────────────────────────────────────────────────────────────
 // A lane owns NF features and walks k in order, so a score is one fma chain held in one
 // register; a wave serves QW queries, whose values at one k come as scalar operands
-// (XT[block][k][query], read through the scalar cache: one v_fmac_f32 v, s, v per term and no LDS
-// traffic for the queries).  The gate rows are staged by global_load_lds: 64 NF rows x 32 k
+// (read through the scalar cache as they lie: one v_fmac_f32 v, s, v per term and no LDS traffic for
+// the queries).  The gate rows are staged by global_load_lds: 64 NF rows x 32 k
 // per stage, a ring of ND stages, whole 128-byte lines per row, no registers in flight.
 // Chunk j (4 k) of row r sits in slot j ^ (r & 7) of the row's eight, so eight consecutive
 // lanes reading the same chunk of their rows touch eight different bank groups.  The NW
 // waves of a workgroup share the staged rows and serve QW queries each.
 // Bound: HBM for few queries (34 x [10240 x 2560], 3.57 GB: 587 us for one query, 6.1 TB/s,
 // against 4.8 ms in a 64 x 256 tile that computes 256 queries whatever their number), the
-// scalar loads' latency and fp32 VALU issue for more: 636 us for 2, 838 for 8, 1.22 ms for 32,
+// scalar loads' latency and fp32 VALU issue for more: 608 us for 2, 700 for 8, 1.15 ms for 32,
 // 1.86 for 64, 3.46 for 128.
 constexpr int kF32Stage = 32;
+
+// XT[b][k][QW] = the QW queries of block b at k: X[QW b + i][k] for existing queries and k < K, else +0 (b < Qp / QW, k < Kp).
+__global__ void queries_t_kernel(const float* __restrict__ X, float* __restrict__ XT, int Q,
+                                 int K, int Kp, int Qp, int qw) {
+    __shared__ float t[32][33];
+    const int nk = (Kp + 31) / 32, k0 = 32 * static_cast<int>(blockIdx.x % nk), q0 = 32 * static_cast<int>(blockIdx.x / nk);
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int q = q0 + ty + 8 * i, k = k0 + tx;
+        t[ty + 8 * i][tx] = (q < Q && k < K) ? X[static_cast<size_t>(q) * K + k] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int k = k0 + ty + 8 * i, q = q0 + tx;
+        if (k < Kp && q < Qp) XT[(static_cast<size_t>(q / qw) * Kp + k) * qw + q % qw] = t[tx][ty + 8 * i];
+    }
+}
 
 // Four float4 of a lane's staged row (chunks 4 HALF .. 4 HALF + 3), read and waited for in
 // one block: the compiler does not see the loads that fill the ring, so its own LDS reads
@@ -57,14 +76,16 @@ __device__ __forceinline__ void ring_read4(uint32_t a, floatx4_t (&v)[4]) {
         : "memory");
 }
 
-template <int QW, int NF, int NW, int ND>
-__global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, const float* __restrict__ XT,
+template <int QW, int NF, int NW, int ND, bool XT>
+__global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, const float* __restrict__ X,
                                                                   float* __restrict__ S, int F, int K, int Q) {
     constexpr int kRows = 64 * NF, kPer = 8 * NF / NW;  // rows per stage; load instructions per wave and stage
     static_assert(kPer * NW == 8 * NF, "the waves split a stage's loads evenly");
     __shared__ __align__(128) float4 ring[ND][kRows * 8];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int f0 = blockIdx.x * kRows, q0 = (blockIdx.y * NW + wave) * QW, l = blockIdx.z;
+    // (waves past the last query repeat the last QW of the Q >= QW, the same scores again; XT: padding)
+    const int f0 = blockIdx.x * kRows, qb = (static_cast<int>(blockIdx.y) * NW + wave) * QW, l = blockIdx.z;
+    const int q0 = XT ? qb : min(qb, Q - QW);
     const float* __restrict__ G = static_cast<const float*>(g.p[l]);
     // load instruction i of the wave: rows 8 (kPer wave + i) .. + 7, eight lanes a row
     const float* gp[kPer];
@@ -96,26 +117,27 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
 #pragma unroll
     for (int d = 0; d < ND - 1; d++) gload(min(d, last), d);
     int slot = 0;
-    const scalar_f32_ptr xt = (scalar_f32_ptr)(reinterpret_cast<uintptr_t>(XT) + sizeof(float) * (static_cast<size_t>(q0) * K));
+    const scalar_f32_ptr xq = (scalar_f32_ptr)(reinterpret_cast<uintptr_t>(X) + sizeof(float) * (static_cast<size_t>(q0) * K));
+    // (XT: block q0 / QW of the k-major queries starts at the same offset)
     // 16 k of the stage in slot `slot`
     auto half = [&](int k0, auto hc) __attribute__((always_inline)) {
         constexpr int H = decltype(hc)::value;
-        floatx4_t v[NF][4];
 #pragma unroll
-        for (int f = 0; f < NF; f++)
-            ring_read4<H>(mine + static_cast<uint32_t>(slot) * (kRows * 128u) + 8192u * f, v[f]);
-        scalar_f32_ptr x = xt + static_cast<size_t>(k0 + 16 * H) * QW;
+        for (int f = 0; f < NF; f++) {
+            floatx4_t r[4];
+            ring_read4<H>(mine + static_cast<uint32_t>(slot) * (kRows * 128u) + 8192u * f, r);
+            float v[16];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+            for (int i = 0; i < 16; i++) v[i] = r[i >> 2][i & 3];
+            if constexpr (XT) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
+                for (int i = 0; i < 16; i++)
 #pragma unroll
-                for (int q = 0; q < QW; q++) {
-                    const float xv = x[(4 * j + e) * QW + q];
-#pragma unroll
-                    for (int f = 0; f < NF; f++) acc[f][q] = fmaf(v[f][j][e], xv, acc[f][q]);
-                }
+                    for (int q = 0; q < QW; q++) acc[f][q] = fmaf(v[i], xq[static_cast<size_t>(k0 + 16 * H + i) * QW + q], acc[f][q]);
+            } else {
+                lane_fma16<QW>(acc[f], v, xq, K, k0 + 16 * H);
             }
+        }
     };
     for (int st = 0; st < ns; st++) {
         // stage st has landed (this wave's loads, then everyone's), and every wave is past
@@ -135,14 +157,14 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
         if (fo >= F) continue;
 #pragma unroll
         for (int q = 0; q < QW; q++)
-            if (q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + fo] = acc[f][q];
+            if (!XT || q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + fo] = acc[f][q];
     }
 }
 
 // More than 128 queries: the chains are bound by fp32 VALU issue and the scalar operands of the
 // kernel above do not arrive fast enough (7.4 ms for 256), so the queries go through LDS as
-// well: 5.33 ms for 256 at 34 x [10240 x 2560], 85 TFLOP/s (5.51 with a thread's eight queries
-// adjacent and the queries transposed on their way into LDS).  A thread tile of 8 features x 16
+// well: 5.50 ms for 256 at 34 x [10240 x 2560], 83 TFLOP/s (5.69 with a thread's eight queries
+// adjacent).  A thread tile of 8 features x 16
 // queries took 5.82 ms (two waves per SIMD).
 // Workgroup tile: 64 features x 256 queries, thread tile 8 x 8 (64 accumulators); K in
 // double-buffered LDS stages of 16, the next stage's global loads in registers meanwhile.  A
@@ -150,7 +172,7 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
 // contiguous.
 constexpr int kF32TileF = 64, kF32TileQ = 256, kF32Ks = 16;
 
-__global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLayers g, const float* __restrict__ XT,
+__global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLayers g, const float* __restrict__ X,
                                                                         float* __restrict__ S, int F, int K, int Q) {
     __shared__ float Gs[2][kF32Ks][kF32TileF];
     __shared__ float Xs[2][kF32Ks][kF32TileQ];
@@ -159,21 +181,21 @@ __global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLa
     const int f0 = blockIdx.x * kF32TileF, q0 = blockIdx.y * kF32TileQ;
     const int tid = threadIdx.x;
     const int tq = tid & 31, tf = tid >> 5;  // queries q0 + 128 i + 4 tq .., features f0 + 8 tf ..
-    // global -> LDS: G row f0 + (tid & 63), k-quarter tid >> 6; XT rows (tid >> 6) + 4 i
-    const int lf = tid & 63, lk = 4 * (tid >> 6), xq = 4 * (tid & 63), xk = tid >> 6;
+    // global -> LDS: G row f0 + (tid & 63), k-quarter tid >> 6; X row q0 + tid, all 16 k
+    const int lf = tid & 63, lk = 4 * (tid >> 6);
     const float* gp = G + static_cast<size_t>(min(f0 + lf, F - 1)) * K + lk;
-    const float* xp = XT + static_cast<size_t>(q0) * K + static_cast<size_t>(xk) * kF32TileQ + xq;
+    const float* xp = X + static_cast<size_t>(min(q0 + tid, Q - 1)) * K;
     floatx4_t gr, xr[4];
     auto gload = [&](int k0) __attribute__((always_inline)) {
         gr = *reinterpret_cast<const floatx4_t*>(gp + k0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) xr[i] = *reinterpret_cast<const floatx4_t*>(xp + static_cast<size_t>(k0 + 4 * i) * kF32TileQ);
+        for (int i = 0; i < 4; i++) xr[i] = *reinterpret_cast<const floatx4_t*>(xp + k0 + 4 * i);
     };
     auto lstore = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; i++) Gs[b][lk + i][lf] = gr[i];
 #pragma unroll
-        for (int i = 0; i < 4; i++) *reinterpret_cast<floatx4_t*>(&Xs[b][xk + 4 * i][xq]) = xr[i];
+        for (int i = 0; i < 16; i++) Xs[b][i][tid] = xr[i >> 2][i & 3];
     };
     float acc[8][8];
 #pragma unroll
@@ -955,7 +977,7 @@ __global__ __launch_bounds__(64 * kWWaves) void topk_wave_kernel(const float* __
 
 }  // namespace
 
-// Queries per wave (qw) and waves per workgroup (nw) of a walk of Q queries.  Few queries per
+// Queries per wave (qw, at most Q) and waves per workgroup (nw) of a walk of Q queries.  Few queries per
 // wave and more waves: a wave waits for its scalar loads every 16 k, and only other waves can
 // issue meanwhile (8 queries of one wave 1.78 ms, of four waves 0.84; 32 of four waves 1.87,
 // of eight 1.22; 64 of four waves 3.1, of eight 1.86).  Above 128 the tile kernel: 128 queries
@@ -971,34 +993,41 @@ F32Plan f32_plan(int Q) {
     if (Q <= 128) return {Q <= 64 ? 8 : 16, 8};
     return {kF32TileQ, 1};  // the tile kernel
 }
-int f32_qp(int Q) {
-    const F32Plan p = f32_plan(Q);
-    const int b = p.qw * p.nw;
-    return (Q + b - 1) / b * b;
-}
 }  // namespace
 
-size_t gate_scores_f32_ws_floats(int K, int Q) {
-    const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
-    return Q == 1 && Kp == K ? 0 : static_cast<size_t>(Kp) * f32_qp(Q);
+// Queries k-major in a workspace, where one is given: above 32 queries a wave's 8 or 16 are then
+// one contiguous run per k (64 queries 1.86 against 2.31 ms as they lie, 128 queries 3.46 against
+// 4.49, 5.17 in tiles; 32 queries 1.22 against 1.15).
+static bool f32_transposed(int Q) { return Q > 32 && Q <= 128; }
+
+size_t gate_scores_f32_ws_floats(int K, int Q, bool may_transpose) {
+    const size_t Kp = f32_row_stride(static_cast<size_t>(K));
+    if (may_transpose && f32_transposed(Q)) return Kp * 128;
+    return Kp == static_cast<size_t>(K) ? 0 : Kp * Q;
 }
 
-void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, float* S, int F, int K, int Q,
-                            hipStream_t s) {
+void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, size_t ws_floats, float* S, int F,
+                            int K, int Q, hipStream_t s) {
     const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
-    const F32Plan p = f32_plan(Q);
-    const int Qp = f32_qp(Q);
-    const float* XT = X;  // one query of a whole row: as it lies
-    if (gate_scores_f32_ws_floats(K, Q)) {
-        if (!ws) fail(LARQL_HIP_ERR_INVALID, "gate scores: no workspace for the queries");
-        launch_queries_t(X, static_cast<size_t>(K), 1, ws, Q, K, Kp, Qp, p.qw, s);
-        XT = ws;
+    F32Plan p = f32_plan(Q);
+    const bool xt = f32_transposed(Q) && ws && ws_floats >= static_cast<size_t>(Kp) * 128;
+    if (!xt && Q > 64 && Q <= 128) p = {8, 8};
+    const int per = p.qw * p.nw, gy = (Q + per - 1) / per;
+    if (xt) {
+        const int Qp = gy * per;
+        queries_t_kernel<<<dim3(((Kp + 31) / 32) * ((Qp + 31) / 32)), dim3(256), 0, s>>>(X, ws, Q, K, Kp, Qp, p.qw);
+        LARQL_HIP_CHECK(hipGetLastError());
+        X = ws;
+    } else if (Kp != K) {  // rows of the device gate are f32_row_stride(K) apart; the queries padded to match
+        if (!ws || ws_floats < static_cast<size_t>(Kp) * Q) fail(LARQL_HIP_ERR_INVALID, "gate scores: no workspace for the queries");
+        launch_pad_rows_f32(X, ws, static_cast<size_t>(Q), static_cast<size_t>(K), static_cast<size_t>(Kp), 0.0f, s);
+        X = ws;
     }
-    auto go = [&](auto qw, auto nf, auto nw, auto nd) {
+    auto go = [&](auto qw, auto nf, auto nw, auto nd, auto tr) {
         constexpr int QW = decltype(qw)::value, NF = decltype(nf)::value, NW = decltype(nw)::value,
                       ND = decltype(nd)::value;
-        const dim3 grid((F + 64 * NF - 1) / (64 * NF), Qp / (QW * NW), n_layers);
-        gate_scores_f32_kernel<QW, NF, NW, ND><<<grid, dim3(64 * NW), 0, s>>>(g, XT, S, F, Kp, Q);
+        const dim3 grid((F + 64 * NF - 1) / (64 * NF), gy, n_layers);
+        gate_scores_f32_kernel<QW, NF, NW, ND, decltype(tr)::value><<<grid, dim3(64 * NW), 0, s>>>(g, X, S, F, Kp, Q);
     };
     using std::integral_constant;
     const integral_constant<int, 1> c1;
@@ -1006,21 +1035,24 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
     const integral_constant<int, 4> c4;
     const integral_constant<int, 8> c8;
     const integral_constant<int, 16> c16;
+    const integral_constant<bool, false> direct;
+    const integral_constant<bool, true> kmajor;
     if (p.qw == kF32TileQ) {
-        const dim3 grid((F + kF32TileF - 1) / kF32TileF, Qp / kF32TileQ, n_layers);
-        gate_scores_f32_tile_kernel<<<grid, dim3(kThreads), 0, s>>>(g, XT, S, F, Kp, Q);
+        const dim3 grid((F + kF32TileF - 1) / kF32TileF, gy, n_layers);
+        gate_scores_f32_tile_kernel<<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
     } else if (p.nw == 1) {
-        if (p.qw == 1) go(c1, c1, c1, c4);
-        else go(c2, c1, c1, c4);
+        if (p.qw == 1) go(c1, c1, c1, c4, direct);
+        else go(c2, c1, c1, c4, direct);
     } else if (p.qw == 2) {
-        if (p.nw == 2) go(c2, c1, c2, c4);
-        else go(c2, c1, c4, c4);
+        if (p.nw == 2) go(c2, c1, c2, c4, direct);
+        else go(c2, c1, c4, c4, direct);
     } else if (p.qw == 4) {
-        if (p.nw == 4) go(c4, c1, c4, c4);
-        else go(c4, c1, c8, c4);
+        if (p.nw == 4) go(c4, c1, c4, c4, direct);
+        else go(c4, c1, c8, c4, direct);
     } else {
-        if (p.qw == 8) go(c8, c1, c8, c4);
-        else go(c16, c1, c8, c4);
+        if (p.qw == 8 && xt) go(c8, c1, c8, c4, kmajor);
+        else if (p.qw == 8) go(c8, c1, c8, c4, direct);
+        else go(c16, c1, c8, c4, kmajor);
     }
     LARQL_HIP_CHECK(hipGetLastError());
 }

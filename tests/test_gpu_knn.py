@@ -41,7 +41,8 @@ def oracle_knn_q4(q4, queries, features, hidden, k):
 
 
 @pytest.mark.parametrize("features,hidden,nq,k", [(1000, 2560, 37, 32), (10240, 2560, 8, 32), (64, 256, 300, 64),
-                                                  (130, 64, 3, 1)])
+                                                  (130, 64, 3, 1), (130, 48, 100, 8), (200, 30, 65, 5),
+                                                  (64, 32, 128, 32)])
 def test_gate_knn_f32_bit_exact(hip, features, hidden, nq, k):
     print(f"[knn f32] F={features} K={hidden} nq={nq} k={k}", flush=True)
     gate = oracle.gauss(11, features * hidden, 0.0, 0.02).reshape(features, hidden)
@@ -73,7 +74,8 @@ def test_gate_scores_f32_bit_exact(hip):
 @pytest.mark.parametrize("nq", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 257])
 @pytest.mark.parametrize("features,hidden", [(1, 16), (65, 48), (130, 30), (64, 100)])
 def test_gate_scores_f32_query_counts_bit_exact(hip, nq, features, hidden):
-    """Every split of the queries over waves and workgroups (their edges), rows whose last stage
+    """Scores into the caller's buffer: every split of the queries over waves and workgroups (their
+    edges; gate_knn's own splits of 33 .. 128 queries are above), rows whose last stage
     of 32 holds 16 or fewer real k, padded rows, partial feature blocks: the oracle's chain bit
     for bit, over two layers."""
     torch = pytest.importorskip("torch")
