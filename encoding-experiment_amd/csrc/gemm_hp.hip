@@ -145,10 +145,11 @@ struct PkArgs {
 };
 
 // Bound: issue, MFMA plus the VALU between (1.9 per MFMA at four token tiles, 7.5 at one), which add
-// up at any number of waves.  Measured, Q4_K [28672 x 4096] with the two launches before it: 512
-// tokens 230 us (523 TFLOP/s; 311 us for the GEMM alone when each workgroup split f32 tokens into
-// pairs itself and one wave per SIMD waited for its own loads and LDS reads; 250 with the codes
-// made fp16 integers by a byte permute and an fma per pair), 24 tokens 35 us.
+// up at any number of waves.  Measured, Q4_K [28672 x 4096] (kernel trace): 512 tokens 258 us (466
+// TFLOP/s; 311 us when each workgroup split f32 tokens into pairs itself and one wave per SIMD
+// waited for its own loads and LDS reads), 24 tokens 30 us (the call 83 us on the fp16 GEMM).  Two
+// 8B-shape layers at 512 tokens took 1205 us with the codes made fp16 integers by a byte permute and
+// an fma per pair, 1133 with the masks.
 //
 // 16 TT tokens x 256 weight rows per workgroup: wave w owns 64 rows (kPkR tiles), all waves
 // share the token operands.  A unit is 128 k (half a super-block, four k-steps of one 32-element
