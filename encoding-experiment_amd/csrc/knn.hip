@@ -172,6 +172,7 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
 // contiguous.
 constexpr int kF32TileF = 64, kF32TileQ = 256, kF32Ks = 16;
 
+template <bool XT>
 __global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLayers g, const float* __restrict__ X,
                                                                         float* __restrict__ S, int F, int K, int Q) {
     __shared__ float Gs[2][kF32Ks][kF32TileF];
@@ -184,18 +185,27 @@ __global__ __launch_bounds__(kThreads, 3) void gate_scores_f32_tile_kernel(KnnLa
     // global -> LDS: G row f0 + (tid & 63), k-quarter tid >> 6; X row q0 + tid, all 16 k
     const int lf = tid & 63, lk = 4 * (tid >> 6);
     const float* gp = G + static_cast<size_t>(min(f0 + lf, F - 1)) * K + lk;
-    const float* xp = X + static_cast<size_t>(min(q0 + tid, Q - 1)) * K;
+    // (XT: the block's k-major queries, rows (tid >> 6) + 4 i, four queries a thread)
+    const int xq = 4 * (tid & 63), xk = tid >> 6;
+    const float* xp = XT ? X + static_cast<size_t>(q0) * K + static_cast<size_t>(xk) * kF32TileQ + xq
+                         : X + static_cast<size_t>(min(q0 + tid, Q - 1)) * K;
     floatx4_t gr, xr[4];
     auto gload = [&](int k0) __attribute__((always_inline)) {
         gr = *reinterpret_cast<const floatx4_t*>(gp + k0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) xr[i] = *reinterpret_cast<const floatx4_t*>(xp + k0 + 4 * i);
+        for (int i = 0; i < 4; i++)
+            xr[i] = *reinterpret_cast<const floatx4_t*>(xp + (XT ? static_cast<size_t>(k0 + 4 * i) * kF32TileQ : k0 + 4 * i));
     };
     auto lstore = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; i++) Gs[b][lk + i][lf] = gr[i];
 #pragma unroll
-        for (int i = 0; i < 16; i++) Xs[b][i][tid] = xr[i >> 2][i & 3];
+        for (int i = 0; i < 4; i++) {
+            if constexpr (XT) *reinterpret_cast<floatx4_t*>(&Xs[b][xk + 4 * i][xq]) = xr[i];
+            else
+#pragma unroll
+                for (int e = 0; e < 4; e++) Xs[b][4 * i + e][tid] = xr[i][e];
+        }
     };
     float acc[8][8];
 #pragma unroll
@@ -997,12 +1007,14 @@ F32Plan f32_plan(int Q) {
 
 // Queries k-major in a workspace, where one is given: above 32 queries a wave's 8 or 16 are then
 // one contiguous run per k (64 queries 1.86 against 2.31 ms as they lie, 128 queries 3.46 against
-// 4.49, 5.17 in tiles; 32 queries 1.22 against 1.15).
-static bool f32_transposed(int Q) { return Q > 32 && Q <= 128; }
+// 4.49, 5.17 in tiles; 32 queries 1.22 against 1.15), and a tile's stage is copied as it lies (256
+// queries 5.50 against 5.62).
+static bool f32_transposed(int Q) { return Q > 32; }
+static size_t f32_transposed_floats(size_t Kp, int Q) { return Kp * (Q <= 128 ? 128 : (static_cast<size_t>(Q) + 255) / 256 * 256); }
 
 size_t gate_scores_f32_ws_floats(int K, int Q, bool may_transpose) {
     const size_t Kp = f32_row_stride(static_cast<size_t>(K));
-    if (may_transpose && f32_transposed(Q)) return Kp * 128;
+    if (may_transpose && f32_transposed(Q)) return f32_transposed_floats(Kp, Q);
     return Kp == static_cast<size_t>(K) ? 0 : Kp * Q;
 }
 
@@ -1010,7 +1022,7 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
                             int K, int Q, hipStream_t s) {
     const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
     F32Plan p = f32_plan(Q);
-    const bool xt = f32_transposed(Q) && ws && ws_floats >= static_cast<size_t>(Kp) * 128;
+    const bool xt = f32_transposed(Q) && ws && ws_floats >= f32_transposed_floats(static_cast<size_t>(Kp), Q);
     if (!xt && Q > 64 && Q <= 128) p = {8, 8};
     const int per = p.qw * p.nw, gy = (Q + per - 1) / per;
     if (xt) {
@@ -1039,7 +1051,8 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
     const integral_constant<bool, true> kmajor;
     if (p.qw == kF32TileQ) {
         const dim3 grid((F + kF32TileF - 1) / kF32TileF, gy, n_layers);
-        gate_scores_f32_tile_kernel<<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
+        if (xt) gate_scores_f32_tile_kernel<true><<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
+        else gate_scores_f32_tile_kernel<false><<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
     } else if (p.nw == 1) {
         if (p.qw == 1) go(c1, c1, c1, c4, direct);
         else go(c2, c1, c1, c4, direct);
