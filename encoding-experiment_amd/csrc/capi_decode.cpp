@@ -455,15 +455,24 @@ bool takes_q8(const DevWeight& w, bool is_down) {
     return w.format == LARQL_Q8_0 || (w.format == LARQL_Q4_0 && !is_down);
 }
 
-// The model's Q8 activation: quantize_to_q8 of x[n], or of its norm when norm_w is given.
-void quantize_input(larql_hip_model* m, const float* x, size_t n, const float* norm_w, float off, double eps,
+// The Q8 activation of `rows` input rows, and where a norm before it goes.
+struct Q8Rows {
+    size_t rows;
+    float* xn;
+    int8_t* q8;
+    float* q8s;
+};
+Q8Rows step_q8(const larql_hip_model* m) { return {1, m->xn, m->q8, m->q8s}; }
+
+// quantize_to_q8 of the rows x[n], or of their norms when norm_w is given.
+void quantize_input(const Q8Rows& q, const float* x, size_t n, const float* norm_w, float off, double eps,
                     hipStream_t s) {
     const float* src = x;
     if (norm_w) {
-        larql::launch_rmsnorm_rows(x, norm_w, off, m->xn, 1, n, eps, s);
-        src = m->xn;
+        larql::launch_rmsnorm_rows(x, norm_w, off, q.xn, q.rows, n, eps, s);
+        src = q.xn;
     }
-    larql::launch_quantize_q8(src, n, 1, m->q8, m->q8s, s);
+    larql::launch_quantize_q8(src, n, q.rows, q.q8, q.q8s, s);
 }
 
 // Weights whose m = 1 matvec is the Q4_K MFMA kernel (the producer / consumer epilogues).
@@ -471,10 +480,12 @@ bool q4k_mfma(const DevWeight& w) { return w.format == LARQL_Q4_K || w.format ==
 // A Q4_K MFMA consumer able to take n producer partial sums.
 bool takes_psum(const DevWeight& w, int n) { return q4k_mfma(w) && n <= larql::q4k_mfma_max_psum(w, 0); }
 
-// out = W . (the model's Q8 activation), blocks accumulated in order (bit-exact int dots).
-void int_proj(const DevWeight& w, larql_hip_model* m, float* out, hipStream_t s) {
-    if (w.format == LARQL_Q8_0) larql::launch_q8_matvec(w, m->q8, m->q8s, out, 1, s);
-    else larql::launch_q4_0_matvec(w, m->q8, m->q8s, out, 1, s);
+// out = W . (the Q8 activation) per row, blocks accumulated in order (bit-exact int dots); output
+// rows w.rows floats apart, or ldo (weights of int_gemm_takes).
+void int_proj(const DevWeight& w, const Q8Rows& q, float* out, hipStream_t s, size_t ldo = 0) {
+    if (ldo && ldo != w.rows && q.rows > 1) larql::launch_int_gemm(w, nullptr, q.q8, q.q8s, out, nullptr, q.rows, ldo, s);
+    else if (w.format == LARQL_Q8_0) larql::launch_q8_matvec(w, q.q8, q.q8s, out, q.rows, s);
+    else larql::launch_q4_0_matvec(w, q.q8, q.q8s, out, q.rows, s);
 }
 
 // Prompt-attention options of prefill_q4 / full_pipeline_q4 (use_qk_norm, softcap); a
@@ -502,9 +513,9 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
         bool have_q8 = false;
         auto qkv_proj = [&](const DevWeight& w, float* out) {
             if (takes_q8(w, false)) {
-                if (!have_q8) quantize_input(m, hin, m->hidden, L.input_norm, L.norm_offset, L.eps, s);
+                if (!have_q8) quantize_input(step_q8(m), hin, m->hidden, L.input_norm, L.norm_offset, L.eps, s);
                 have_q8 = true;
-                int_proj(w, m, out, s);
+                int_proj(w, step_q8(m), out, s);
             } else {
                 larql::MvArgs a;
                 a.x = hin;
@@ -552,8 +563,8 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
         const bool o_q8 = takes_q8(L.wo, false);
         if (L.post_norms || o_q8) {
             if (o_q8) {
-                quantize_input(m, m->attn, qd, nullptr, 0.f, L.eps, s);
-                int_proj(L.wo, m, m->otmp, s);
+                quantize_input(step_q8(m), m->attn, qd, nullptr, 0.f, L.eps, s);
+                int_proj(L.wo, step_q8(m), m->otmp, s);
             } else {
                 larql::MvArgs o;
                 o.x = m->attn;
@@ -611,12 +622,12 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
             g.norm_offset = foff;
         }
         if (g_q8 || u_q8) {  // gate and up apart, then act(gate) * up
-            quantize_input(m, m->h1, m->hidden, fnorm, foff, L.eps, s);
+            quantize_input(step_q8(m), m->h1, m->hidden, fnorm, foff, L.eps, s);
             float* outs[2] = {m->gtmp, m->utmp};
             const DevWeight* ws[2] = {&L.gate, &L.up};
             for (int i = 0; i < 2; i++) {
                 if (takes_q8(*ws[i], false)) {
-                    int_proj(*ws[i], m, outs[i], s);
+                    int_proj(*ws[i], step_q8(m), outs[i], s);
                 } else {
                     larql::MvArgs gi = g;
                     gi.out = outs[i];
@@ -644,8 +655,8 @@ void enqueue_layers(larql_hip_ctx* c, larql_hip_model* m, const float* x0, int T
             if (L.down.format == LARQL_Q4_0) {  // f32 activation (the reference's q4_f32_matvec)
                 larql::launch_q4_0_f32_matvec(L.down, m->act, m->otmp, s);
             } else if (L.down.format == LARQL_Q8_0) {
-                quantize_input(m, m->act, m->inter, nullptr, 0.f, L.eps, s);
-                int_proj(L.down, m, m->otmp, s);
+                quantize_input(step_q8(m), m->act, m->inter, nullptr, 0.f, L.eps, s);
+                int_proj(L.down, step_q8(m), m->otmp, s);
             } else {
                 larql::MvArgs d;
                 d.x = m->act;
@@ -788,177 +799,222 @@ extern "C" int larql_hip_decode_token(larql_hip_ctx* c, const larql_pipeline_lay
     });
 }
 
-// A projection the batched prompt pass runs over all positions: the Q8-input formats on the
-// ordered int GEMM, the others (and Q4_0 as the down projection) on the f32-accuracy GEMM.
-static bool batched_proj(const DevWeight& w, bool is_down) {
-    return takes_q8(w, is_down) ? larql::int_gemm_takes(w) : larql::gemm_f32_takes(w);
+// The batched prompt pass takes layers with gate/up fused in Q4_K and every other projection Q4_K
+// or Q6_K (Q4_K and Q4_K_M files).
+static bool prompt_batchable(const larql_hip_model* m) {
+    auto ok = [](const DevWeight& w) { return w.format == LARQL_Q4_K || w.format == LARQL_Q6_K; };
+    for (const LayerDev& L : m->layers) {
+        if (L.split_gu || L.gateup.format != LARQL_Q4_K || !ok(L.wo) || !ok(L.down)) return false;
+        if (L.split_qkv ? !(ok(L.wq) && (!L.wk.rows || ok(L.wk)) && ok(L.wv)) : !ok(L.qkv)) return false;
+    }
+    return true;
+}
+
+// Layers whose projections are all Q8_0 / Q4_0: a block of positions runs through each layer at
+// once, with the bits of the steps (Q / K / V of two formats need the int GEMM's column slices).
+static bool prompt_q8(const larql_hip_model* m) {
+    auto slice = [](const DevWeight& w) { return takes_q8(w, false) && larql::int_gemm_takes(w); };
+    for (const LayerDev& L : m->layers) {
+        if (!takes_q8(L.wo, false) || !(takes_q8(L.down, true) || L.down.format == LARQL_Q4_0)) return false;
+        if (!L.split_gu || !takes_q8(L.gate, false) || !takes_q8(L.up, false)) return false;
+        if (L.split_qkv ? !(slice(L.wq) && (!L.wk.rows || slice(L.wk)) && slice(L.wv)) : !takes_q8(L.qkv, false)) return false;
+    }
+    return true;
+}
+
+static size_t a4(size_t n) { return (n + 3) & ~size_t{3}; }
+
+// A prompt of prompt_q8 layers, kQ8Block positions at a time through all layers: per position the
+// launches of enqueue_layers over all rows of the block, so the hidden states and the cache are
+// those of decoding token by token, bit for bit (a projection's Q8 codes flip at a rounding tie
+// on any other order of sums: up to 5e-3 of the output over two layers).  The work buffer holds
+// one block whatever the prompt's length.
+constexpr size_t kQ8Block = 1024;
+constexpr size_t kQ8PartFloats = size_t{16} << 20;  // attention partials of one launch
+static void run_prompt_q8(larql_hip_ctx* c, larql_hip_model* m, const float* dx, size_t M, float* dout, hipStream_t s,
+                          const PromptAttn& pa) {
+    auto& kv = c->kv;
+    kv_ensure_model(c, m, M);
+    const size_t hidden = m->hidden, inter = m->inter, nb = std::min(M, kQ8Block);
+    const size_t wide = std::max({hidden, m->q_dim, inter});
+    const size_t part_q = m->part_per_split * larql::attn_prompt_splits(1, static_cast<int>(M), 0);  // of one query, at most
+    const size_t qb = std::min(nb, std::max<size_t>(1, kQ8PartFloats / part_q));  // queries per attention launch
+    size_t xp_n = 0;  // the Q4_0 down projection's permuted input
+    for (const LayerDev& L : m->layers)
+        if (L.down.format == LARQL_Q4_0) xp_n = larql::q4_0_f32_rows_ws_floats(nb, inter);
+    const size_t sizes[] = {nb * hidden, nb * hidden, nb * hidden, nb * hidden, nb * m->qkv_dim, nb * m->q_dim,
+                            nb * inter,  nb * inter,  nb * inter,  (nb * wide + 3) / 4, nb * (wide / 32), part_q * qb, xp_n};
+    constexpr int kRegions = sizeof(sizes) / sizeof(sizes[0]);
+    size_t total = 0;
+    for (size_t n : sizes) total += a4(n);
+    float* at = static_cast<float*>(larql::ensure(c, m->prompt, total * sizeof(float)));
+    float* r[kRegions];
+    for (int i = 0; i < kRegions; i++) r[i] = at, at += a4(sizes[i]);
+    float *H0 = r[0], *H1 = r[1], *OT = r[3], *QKV = r[4], *ATT = r[5], *G = r[6], *U = r[7], *ACT = r[8];
+    float *PART = r[11], *XP = xp_n ? r[12] : nullptr;
+    for (size_t p0 = 0; p0 < M; p0 += nb) {
+        const size_t n = std::min(nb, M - p0);
+        const Q8Rows q{n, r[2], reinterpret_cast<int8_t*>(r[9]), r[10]};
+        const float* hin = dx + p0 * hidden;
+        for (size_t l = 0; l < m->layers.size(); l++) {
+            const LayerDev& L = m->layers[l];
+            const size_t qd = static_cast<size_t>(L.nq) * L.hd, kvd = static_cast<size_t>(L.nkv) * L.hd, ld = qd + 2 * kvd;
+            float* hout = l + 1 < m->layers.size() ? H0 : dout + p0 * hidden;
+            quantize_input(q, hin, hidden, L.input_norm, L.norm_offset, L.eps, s);
+            if (L.split_qkv) {
+                int_proj(L.wq, q, QKV, s, ld);
+                if (L.wk.rows) int_proj(L.wk, q, QKV + qd, s, ld);
+                int_proj(L.wv, q, QKV + qd + kvd, s, ld);
+            } else {
+                int_proj(L.qkv, q, QKV, s);
+            }
+            if (L.v_norm) larql::launch_vnorm_rows(QKV + qd + kvd, n, ld, L.nkv, L.hd, L.eps, s);
+            larql::AttnArgs at{};
+            at.rope = rope_table(c, L.rope_base, L.rdim, s);
+            larql::launch_rope_kv_rows(QKV, n, p0, qd, kvd, L.hd, L.rdim, at.rope, kv.k[l], kv.v[l], L.nkv, s);
+            at.kc = kv.k[l];
+            at.vc = kv.v[l];
+            at.part = PART;
+            at.num_q = L.nq;
+            at.num_kv = L.nkv;
+            at.hd = L.hd;
+            at.rdim = L.rdim;
+            at.scale = L.attn_scale;
+            at.window = L.window;
+            at.qkv_ld = static_cast<int>(ld);
+            at.qk_norm = pa.qk_norm;
+            at.softcap = pa.softcap;
+            at.as_steps = true;
+            // runs of queries whose step takes one chunk per workgroup; others as the step itself
+            auto begin = [&](size_t T) { return L.window > 0 && T > static_cast<size_t>(L.window) ? static_cast<int>(T) - L.window : 0; };
+            auto one_chunk = [&](size_t T) { return larql::attn_step_chunks(static_cast<int>(T), begin(T), L.nkv) == 1; };
+            for (size_t i = 0; i < n;) {
+                size_t cnt = 0;
+                while (cnt < qb && i + cnt < n && one_chunk(p0 + i + cnt + 1)) cnt++;
+                at.qkv = QKV + i * ld;
+                at.out = ATT + i * qd;
+                at.T = static_cast<int>(p0 + i + 1);
+                at.t_begin = begin(p0 + i + 1);
+                at.batch = static_cast<int>(cnt);
+                larql::launch_attention(at, s);
+                i += std::max<size_t>(cnt, 1);
+            }
+            quantize_input(q, ATT, qd, nullptr, 0.f, L.eps, s);
+            int_proj(L.wo, q, OT, s);
+            if (L.post_norms)
+                larql::launch_resid_norm_rows(hin, OT, L.post_attn_norm, L.norm_offset, 1.0f, H1, n, hidden, L.eps, s);
+            else
+                larql::launch_add_rows(hin, OT, H1, n * hidden, s);
+            const float* fnorm = L.post_norms ? (L.pre_ffn_norm ? L.pre_ffn_norm : m->ones) : L.post_attn_norm;
+            quantize_input(q, H1, hidden, fnorm, L.post_norms && !L.pre_ffn_norm ? 0.0f : L.norm_offset, L.eps, s);
+            if (L.gate.format == LARQL_Q4_0 && L.up.format == LARQL_Q4_0) {
+                larql::launch_q4_0_matvec_pair(L.gate, L.up, q.q8, q.q8s, G, U, n, s);
+            } else {
+                int_proj(L.gate, q, G, s);
+                int_proj(L.up, q, U, s);
+            }
+            larql::launch_gated_mul(G, U, ACT, n * inter, L.act, s);
+            if (L.down.format == LARQL_Q4_0) {  // f32 activation
+                larql::launch_q4_0_f32_matvec(L.down, ACT, OT, s, n, XP);
+            } else {
+                quantize_input(q, ACT, inter, nullptr, 0.f, L.eps, s);
+                int_proj(L.down, q, OT, s);
+            }
+            const float scale = L.layer_scalar != 0.0f ? L.layer_scalar : 1.0f;
+            if (L.post_norms)
+                larql::launch_resid_norm_rows(H1, OT, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, scale, hout,
+                                              n, hidden, L.eps, s);
+            else
+                larql::launch_add_rows(H1, OT, hout, n * hidden, s, scale);
+            hin = hout;
+        }
+    }
+    kv.current_len = M;
 }
 
 // Floats of the batched prompt pass's work buffer, in the order of its regions.
 namespace {
-size_t a4(size_t n) { return (n + 3) & ~size_t{3}; }
-
 struct PromptLayout {
-    size_t wide, gw, rows, split, st_h, st_q, st_a, xp, q8, q8s;
-    size_t total() const { return rows + a4(split) + st_h + st_q + st_a + xp + q8 + q8s; }
+    size_t gw, rows, split, st_h, st_q, st_a, xp;
+    size_t total() const { return rows + a4(split) + st_h + st_q + st_a + xp; }
 };
 
 PromptLayout prompt_layout(const larql_hip_model* m, size_t M) {
     PromptLayout p{};
     const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim;
-    p.wide = std::max({hidden, qmax, inter});
     p.gw = std::max(hidden, 2 * inter);
     size_t part_n = 0;  // partials of attention shapes without the one-pass prompt kernel
-    bool any_int = false;
-    // GEMM workspace: K-split partial products (and operands it packs itself)
-    auto need = [&](const DevWeight& w, bool is_down) {
-        if (takes_q8(w, is_down)) any_int = true;
-        else p.split = std::max(p.split, larql::gemm_f32_part_floats(w, M));
-    };
+    auto need = [&](const DevWeight& w) { p.split = std::max(p.split, larql::gemm_f32_part_floats(w, M)); };
     for (const LayerDev& L : m->layers) {
         if (!larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd))
             part_n = m->part_per_split * larql::attn_prompt_splits(1, static_cast<int>(M), 0) * M;
         if (L.split_qkv) {
-            need(L.wq, false), need(L.wv, false);
-            if (L.wk.rows) need(L.wk, false);
+            need(L.wq), need(L.wv);
+            if (L.wk.rows) need(L.wk);
+        } else {
+            need(L.qkv);
         }
-        else need(L.qkv, false);
-        need(L.wo, false), need(L.down, true);
-        if (L.split_gu) need(L.gate, false), need(L.up, false);
-        else need(L.gateup, false);
+        need(L.wo), need(L.gateup), need(L.down);
     }
-    p.rows = a4(2 * M * hidden + M * p.wide + M * m->qkv_dim + M * qmax + M * p.gw + M * inter + part_n);
+    p.rows = a4(3 * M * hidden + M * m->qkv_dim + M * qmax + M * p.gw + M * inter + part_n);
     // row statistics of the normed hidden rows, of the attention rows and of the activation
     // rows (separate regions: a producer may still read the previous GEMM's partial products),
-    // the packed operands and the Q8 codes of one input
+    // and the packed operands of one input
     p.st_h = a4(larql::gemm_row_stats_floats(M, hidden));
     p.st_q = a4(larql::gemm_row_stats_floats(M, qmax));
     p.st_a = a4(larql::gemm_row_stats_floats(M, inter));
-    p.xp = larql::gemm_x_pack_floats(M, p.wide);
-    if (any_int) {
-        p.q8 = a4((M * p.wide + 3) / 4);
-        p.q8s = a4(M * (p.wide / 32));
-    }
+    p.xp = larql::gemm_x_pack_floats(M, std::max({hidden, qmax, inter}));
     return p;
 }
-}  // namespace
 
-// The batched prompt pass takes layers whose projections are Q4_K, Q6_K, Q8_0 or Q4_0, with
-// gate/up fused in Q4_K or both Q8-input (Q4_K, Q4_K_M and Q8_0 / Q4_0 files); others run
-// position by position.  So do Q8_0 / Q4_0 prompts that position by position need no more
-// than a step's buffers and batched would not fit: past 31-bit row blocks, attention shapes that
-// hold every query's partials at more than 4096 positions, or a work buffer beyond the free memory.
-static bool prompt_batchable(const larql_hip_model* m, size_t M) {
-    bool any_int = false;
-    auto ok = [&](const DevWeight& w, bool is_down) {
-        any_int |= w.format == LARQL_Q4_0 || w.format == LARQL_Q8_0;
-        return batched_proj(w, is_down);
-    };
-    bool one_pass = true;
-    for (const LayerDev& L : m->layers) {
-        if (!ok(L.wo, false) || !ok(L.down, true)) return false;
-        if (L.split_gu ? !(takes_q8(L.gate, false) && takes_q8(L.up, false) && ok(L.gate, false) && ok(L.up, false))
-                       : L.gateup.format != LARQL_Q4_K)
-            return false;
-        if (L.split_qkv ? !(ok(L.wq, false) && (!L.wk.rows || ok(L.wk, false)) && ok(L.wv, false)) : !ok(L.qkv, false))
-            return false;
-        one_pass &= larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd);
-    }
-    if (!any_int) return true;
-    if (M > 0x7FFFFFFF / std::max({m->hidden, 2 * m->inter, m->qkv_dim}) || (!one_pass && M > 4096)) return false;
-    const size_t bytes = prompt_layout(m, M).total() * sizeof(float);
-    if (bytes <= m->prompt.n || bytes <= (size_t{1} << 30)) return true;
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return bytes + (size_t{1} << 30) <= free_b;
-}
-
-namespace {
-
-// The prompt pass's projections of M positions: the GEMM workspaces, and which form of the
-// current input rows they hold (packed operands and row statistics, or Q8 codes).
+// The prompt pass's projections of M positions: the GEMM workspaces, and whose rows' packed
+// operands xp holds.
 struct PromptProj {
     size_t M;
     float* spl;
     size_t split_n;
-    float* xp;     // packed operands of the current input
-    int8_t* q8;    // its quantize_to_q8 codes and scales
-    float* q8s;
+    float* xp;
     hipStream_t s;
     const float* packed = nullptr;
-    const float* quantized = nullptr;
 
     // A new input: X's rows (the same buffer with other contents included), packed already or not.
-    void input(const float* X, bool is_packed) {
-        packed = is_packed ? X : nullptr;
-        quantized = nullptr;
-    }
-    void pack(const float* X, size_t K, larql::GemmRowStats& st) {
-        st.xp = xp;
-        if (packed == X) return;
-        larql::launch_gemm_pack_rows(X, M, K, st, s);
-        packed = X;
-    }
-    void quantize(const float* X, size_t K) {
-        if (quantized == X) return;
-        larql::launch_quantize_q8(X, K, M, q8, q8s, s);
-        quantized = X;
-    }
+    void input(const float* X, bool is_packed) { packed = is_packed ? X : nullptr; }
     // One projection (input rows w.cols apart) -> Y rows ldy apart.  st: the place of the rows'
-    // statistics, computed if the rows are packed.  defer: K-split partial products left to the
-    // caller.
-    void run(const DevWeight& w, bool is_down, const float* X, float* Y, size_t ldy, larql::GemmRowStats st,
+    // statistics, computed if the rows are not packed.  defer: K-split partial products left to
+    // the caller.
+    void run(const DevWeight& w, const float* X, float* Y, size_t ldy, larql::GemmRowStats st,
              larql::GemmSplits* defer = nullptr) {
-        if (takes_q8(w, is_down)) {
-            quantize(X, w.cols);
-            if (ldy != w.rows) larql::launch_int_gemm(w, nullptr, q8, q8s, Y, nullptr, M, ldy, s);
-            else if (w.format == LARQL_Q8_0) larql::launch_q8_matvec(w, q8, q8s, Y, M, s);
-            else larql::launch_q4_0_matvec(w, q8, q8s, Y, M, s);
-            if (defer) *defer = {nullptr, 1};
-            return;
+        st.xp = xp;
+        if (packed != X) {
+            larql::launch_gemm_pack_rows(X, M, w.cols, st, s);
+            packed = X;
         }
-        pack(X, w.cols, st);
         larql::launch_gemm_f32(w, X, Y, M, spl, split_n, s, ldy, &st, defer);
     }
 };
-
 }  // namespace
 
 static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, size_t M, float* dout, hipStream_t s,
-                       const PromptAttn& pa = {}) {
+                       const PromptAttn& pa) {
     auto& kv = c->kv;
     kv_ensure_model(c, m, M);
     const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim, ldmax = m->qkv_dim;
-    const size_t qd_max = m->q_dim;
     const PromptLayout lay = prompt_layout(m, M);
     float* base = static_cast<float*>(larql::ensure(c, m->prompt, lay.total() * sizeof(float)));
-    float *H0 = base, *H1 = H0 + M * hidden, *XN = H1 + M * hidden, *QKV = XN + M * lay.wide, *ATT = QKV + M * ldmax;
+    float *H0 = base, *H1 = H0 + M * hidden, *XN = H1 + M * hidden, *QKV = XN + M * hidden, *ATT = QKV + M * ldmax;
     float *G = ATT + M * qmax, *ACT = G + M * lay.gw, *PART = ACT + M * inter, *SPL = base + lay.rows;
     float* ST = SPL + a4(lay.split);
-    float *XP = ST + lay.st_h + lay.st_q + lay.st_a, *Q8 = XP + lay.xp, *Q8S = Q8 + lay.q8;
     const larql::GemmRowStats xn_st = larql::gemm_row_stats_at(ST, M, hidden);
     const larql::GemmRowStats att_st = larql::gemm_row_stats_at(ST + lay.st_h, M, qmax);
     const larql::GemmRowStats act_st = larql::gemm_row_stats_at(ST + lay.st_h + lay.st_q, M, inter);
-    PromptProj pj{M, SPL, lay.split, XP, reinterpret_cast<int8_t*>(Q8), Q8S, s};
+    float* XP = ST + lay.st_h + lay.st_q + lay.st_a;
+    PromptProj pj{M, SPL, lay.split, XP, s};
     // Row kernels between the projections (residual add, norms, the next GEMM's statistics and
     // packed operands in one launch) where a row fits them
-    const bool fused = std::max({hidden, qd_max, inter}) <= static_cast<size_t>(larql::kFusedRowMax);
-    auto qkv_f32 = [&](const LayerDev& L) {  // the Q8-input projections read the normed rows themselves
-        return L.split_qkv ? takes_q8(L.wq, false) || (L.wk.rows && takes_q8(L.wk, false)) || takes_q8(L.wv, false)
-                           : takes_q8(L.qkv, false);
-    };
-    auto qkv_packed = [&](const LayerDev& L) {
-        return L.split_qkv ? !(takes_q8(L.wq, false) && (!L.wk.rows || takes_q8(L.wk, false)) && takes_q8(L.wv, false))
-                           : !takes_q8(L.qkv, false);
-    };
-    // hin (+ P) -> hout, and the rows normed by (w, off, eps): f32 rows for Q8-input projections,
-    // packed ones for the others
+    const bool fused = std::max({hidden, qmax, inter}) <= static_cast<size_t>(larql::kFusedRowMax);
+    // hin (+ P) -> hout, and the rows normed by (w, off, eps), packed
     auto rows = [&](const float* hin, const float* P, const larql::GemmSplits& sp, bool post, const float* pw, float poff,
-                    double peps, float scale, float* hout, bool norm, const float* w, float off, double eps, bool want_f32,
-                    bool want_packed) {
+                    double peps, float scale, float* hout, bool norm, const float* w, float off, double eps) {
         larql::ResidRows r;
         r.P = P && sp.splits > 1 ? sp.part : P;
         r.pstride = M * hidden;
@@ -975,22 +1031,18 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
         r.off = off;
         r.norm_eps = eps;
         if (norm) {
-            r.xn = want_f32 ? XN : nullptr;
-            if (want_packed) {
-                r.st = xn_st;
-                r.st.xp = XP;
-            }
+            r.st = xn_st;
+            r.st.xp = XP;
         }
         r.m = static_cast<int>(M);
         r.n = static_cast<int>(hidden);
         larql::launch_resid_norm_stats_rows(r, s);
-        pj.input(XN, norm && want_packed);
+        pj.input(XN, norm);
     };
     const float* Hin = dx;  // the layer's input rows
     if (fused) {
         const LayerDev& L = m->layers[0];
-        rows(dx, nullptr, {}, false, nullptr, 0.f, 0.0, 1.0f, nullptr, true, L.input_norm, L.norm_offset, L.eps, qkv_f32(L),
-             qkv_packed(L));
+        rows(dx, nullptr, {}, false, nullptr, 0.f, 0.0, 1.0f, nullptr, true, L.input_norm, L.norm_offset, L.eps);
     }
     for (size_t l = 0; l < m->layers.size(); l++) {
         const LayerDev& L = m->layers[l];
@@ -1003,11 +1055,11 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
             pj.input(XN, false);
         }
         if (L.split_qkv) {  // Q, K, V into their column ranges of the [q | k | v] rows
-            pj.run(L.wq, false, XN, QKV, ld, xn_st);
-            if (L.wk.rows) pj.run(L.wk, false, XN, QKV + qd, ld, xn_st);
-            pj.run(L.wv, false, XN, QKV + qd + kvd, ld, xn_st);
+            pj.run(L.wq, XN, QKV, ld, xn_st);
+            if (L.wk.rows) pj.run(L.wk, XN, QKV + qd, ld, xn_st);
+            pj.run(L.wv, XN, QKV + qd + kvd, ld, xn_st);
         } else {
-            pj.run(L.qkv, false, XN, QKV, ld, xn_st);
+            pj.run(L.qkv, XN, QKV, ld, xn_st);
         }
         if (L.v_norm) larql::launch_vnorm_rows(QKV + qd + kvd, M, ld, L.nkv, L.hd, L.eps, s);
         const float2* rope = rope_table(c, L.rope_base, L.rdim, s);
@@ -1036,10 +1088,9 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
         const float foff = L.post_norms && !L.pre_ffn_norm ? 0.0f : L.norm_offset;
         larql::GemmSplits sp{nullptr, 1};
         pj.input(ATT, false);
-        pj.run(L.wo, false, ATT, G, hidden, att_st, fused ? &sp : nullptr);
+        pj.run(L.wo, ATT, G, hidden, att_st, fused ? &sp : nullptr);
         if (fused) {
-            rows(Hin, G, sp, L.post_norms, L.post_attn_norm, L.norm_offset, L.eps, 1.0f, H1, true, fnorm, foff, L.eps,
-                 L.split_gu, !L.split_gu);
+            rows(Hin, G, sp, L.post_norms, L.post_attn_norm, L.norm_offset, L.eps, 1.0f, H1, true, fnorm, foff, L.eps);
         } else {
             if (L.post_norms)
                 larql::launch_resid_norm_rows(Hin, G, L.post_attn_norm, L.norm_offset, 1.0f, H1, M, hidden, L.eps, s);
@@ -1048,42 +1099,21 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
             larql::launch_rmsnorm_rows(H1, fnorm, foff, XN, M, hidden, L.eps, s);
             pj.input(XN, false);
         }
-        const float* U = nullptr;  // up rows apart from the gate rows in G
         sp = {nullptr, 1};
-        if (L.split_gu) {
-            float* up = G + M * inter;
-            U = up;
-            pj.quantize(XN, hidden);
-            if (L.gate.format == LARQL_Q4_0 && L.up.format == LARQL_Q4_0) {
-                larql::launch_q4_0_matvec_pair(L.gate, L.up, pj.q8, pj.q8s, G, up, M, s);
-            } else {
-                pj.run(L.gate, false, XN, G, inter, xn_st);
-                pj.run(L.up, false, XN, up, inter, xn_st);
-            }
-        } else {
-            pj.run(L.gateup, false, XN, G, 2 * inter, xn_st, fused ? &sp : nullptr);
-        }
-        const bool down_q8 = takes_q8(L.down, true);
+        pj.run(L.gateup, XN, G, 2 * inter, xn_st, fused ? &sp : nullptr);
         if (fused) {
-            larql::GemmRowStats st{};
-            if (!down_q8) {
-                st = act_st;
-                st.xp = XP;
-            }
-            larql::launch_gated_stats_rows(sp.splits > 1 ? sp.part : G, M * 2 * inter, sp.splits, U,
-                                           down_q8 ? ACT : nullptr, M, inter, L.act, st, s);
-        } else if (U) {
-            larql::launch_gated_mul(G, U, ACT, M * inter, L.act, s);
+            larql::GemmRowStats st = act_st;
+            st.xp = XP;
+            larql::launch_gated_stats_rows(sp.splits > 1 ? sp.part : G, M * 2 * inter, sp.splits, M, inter, L.act, st, s);
         } else {
             larql::launch_gated_pair_rows(G, ACT, M * inter, L.act, s);
         }
-        pj.input(ACT, fused && !down_q8);
+        pj.input(ACT, fused);
         sp = {nullptr, 1};
-        pj.run(L.down, true, ACT, G, hidden, act_st, fused ? &sp : nullptr);
+        pj.run(L.down, ACT, G, hidden, act_st, fused ? &sp : nullptr);
         if (fused) {
             rows(H1, G, sp, L.post_norms, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, L.eps, scale, Hout,
-                 nx != nullptr, nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f, nx ? nx->eps : 0.0,
-                 nx && qkv_f32(*nx), nx && qkv_packed(*nx));
+                 nx != nullptr, nx ? nx->input_norm : nullptr, nx ? nx->norm_offset : 0.0f, nx ? nx->eps : 0.0);
         } else if (L.post_norms) {
             larql::launch_resid_norm_rows(H1, G, L.post_ffn_norm, L.post_ffn_norm ? L.norm_offset : 0.0f, scale, Hout, M,
                                           hidden, L.eps, s);
@@ -1094,6 +1124,15 @@ static void run_prompt(larql_hip_ctx* c, larql_hip_model* m, const float* dx, si
     }
     if (m->layers.empty()) larql::launch_copy_f32(dx, dout, M * hidden, s);
     kv.current_len = M;
+}
+
+// A prompt from position 0: all positions at once where the layers allow it, else a step each.
+static void run_positions(larql_hip_ctx* c, larql_hip_model* m, const float* dx, size_t M, float* dout, hipStream_t s,
+                          const PromptAttn& pa = {}) {
+    if (M > 1 && prompt_batchable(m)) run_prompt(c, m, dx, M, dout, s, pa);
+    else if (M > 1 && prompt_q8(m)) run_prompt_q8(c, m, dx, M, dout, s, pa);
+    else
+        for (size_t p = 0; p < M; p++) run_decode(c, m, dx + p * m->hidden, dout + p * m->hidden, nullptr, s, pa);
 }
 
 extern "C" int larql_hip_prefill_q4(larql_hip_ctx* c, const larql_pipeline_layer* layers, size_t num_layers,
@@ -1113,11 +1152,7 @@ extern "C" int larql_hip_prefill_q4(larql_hip_ctx* c, const larql_pipeline_layer
         const float* dx = stage_upload(c, c->stage_in, x, seq_len * hidden);
         float* dout = static_cast<float*>(larql::ensure(c, c->stage_out, seq_len * hidden * sizeof(float)));
         const PromptAttn pa{use_qk_norm != 0, softcap};
-        if (seq_len > 1 && prompt_batchable(m, seq_len))
-            run_prompt(c, m, dx, seq_len, dout, c->stream, pa);
-        else
-            for (size_t p = 0; p < seq_len; p++)
-                run_decode(c, m, dx + p * hidden, dout + p * hidden, nullptr, c->stream, pa);
+        run_positions(c, m, dx, seq_len, dout, c->stream, pa);
         download(c, out, dout, seq_len * hidden * sizeof(float));
     });
 }
@@ -1146,11 +1181,7 @@ extern "C" int larql_hip_full_pipeline_q4(larql_hip_ctx* c, const larql_pipeline
         const float* dx = stage_upload(c, c->stage_in, x, seq_len * hidden);
         float* dout = static_cast<float*>(larql::ensure(c, c->stage_out, seq_len * hidden * sizeof(float)));
         const PromptAttn pa{use_qk_norm != 0, softcap};
-        if (seq_len > 1 && prompt_batchable(m, seq_len))
-            run_prompt(c, m, dx, seq_len, dout, c->stream, pa);
-        else
-            for (size_t p = 0; p < seq_len; p++)
-                run_decode(c, m, dx + p * hidden, dout + p * hidden, nullptr, c->stream, pa);
+        run_positions(c, m, dx, seq_len, dout, c->stream, pa);
         download(c, out, dout, seq_len * hidden * sizeof(float));
     });
 }
@@ -1279,11 +1310,7 @@ extern "C" int larql_hip_model_prefill_dev(larql_hip_ctx* c, larql_hip_model* m,
         hipStream_t s = pick_stream(c, stream);
         kv_ensure_model(c, m, seq_len);
         c->kv.current_len = 0;
-        if (seq_len > 1 && prompt_batchable(m, seq_len))
-            run_prompt(c, m, x_dev, seq_len, out_dev, s);
-        else
-            for (size_t p = 0; p < seq_len; p++)
-                run_decode(c, m, x_dev + p * m->hidden, out_dev + p * m->hidden, nullptr, s);
+        run_positions(c, m, x_dev, seq_len, out_dev, s);
     });
 }
 

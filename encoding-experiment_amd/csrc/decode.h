@@ -28,12 +28,17 @@ struct AttnArgs {
     // score s to tanh(s / softcap) * softcap before the softmax.
     int qk_norm = 0;
     float softcap = 0.f;
+    // Prompt mode with every query summed as its own decode step sums it, bit for bit (queries
+    // whose step takes one chunk per workgroup, attn_step_chunks).
+    bool as_steps = false;
 };
 
 void launch_attention(const AttnArgs& a, hipStream_t s);
 // Position splits of one query (T positions from t_begin) and the most over a prompt's
 // queries T0 .. T0 + batch - 1 (its partials stride).
 int attn_splits(int T, int t_begin);
+// 64-position chunks that a workgroup of a decode step takes in turn.
+int attn_step_chunks(int T, int t_begin, int num_kv);
 int attn_prompt_splits(int T0, int batch, int window);
 // Prompt mode in one pass per block of queries, without partials.
 bool attn_prompt_one_pass(int reps, int hd);
@@ -90,15 +95,14 @@ struct ResidRows {
     const float* w = nullptr;
     float off = 0.f;
     double norm_eps = 0.0;
-    float* xn = nullptr;    // x (norm only), if wanted
     GemmRowStats st{};      // x's GEMM row statistics and packed operands, if wanted
     int m = 0, n = 0;
 };
 void launch_resid_norm_stats_rows(const ResidRows& a, hipStream_t s);
 // act(gate) * up rows (m x n) from interleaved pairs (K-split partial products pstride floats
-// apart) or, with U, separate rows: to act and with st, each if wanted.
-void launch_gated_stats_rows(const float* G, size_t pstride, int splits, const float* U, float* act, size_t m, size_t n,
-                             int kind, const GemmRowStats& st, hipStream_t s);
+// apart), as statistics and packed operands.
+void launch_gated_stats_rows(const float* G, size_t pstride, int splits, size_t m, size_t n, int kind,
+                             const GemmRowStats& st, hipStream_t s);
 void launch_f32_to_f16(const float* src, __half* dst, size_t n, hipStream_t s);
 
 }  // namespace larql

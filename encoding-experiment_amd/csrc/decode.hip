@@ -30,8 +30,8 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 // Split-half RoPE of element d of head vector x (LI/src/attention/rope.rs:22-55):
 // pairs (i, i + rdim/2), dims >= rdim untouched.  cs[i] = (cos, sin) of pair i.
 __device__ __forceinline__ float rope_elem(const float* x, int d, int half, const float2* cs) {
-    if (d < half) return x[d] * cs[d].x - x[d + half] * cs[d].y;
-    if (d < 2 * half) return x[d - half] * cs[d - half].y + x[d] * cs[d - half].x;
+    if (d < half) return rope_low(x[d], x[d + half], cs[d]);
+    if (d < 2 * half) return rope_high(x[d - half], x[d], cs[d - half]);
     return x[d];
 }
 
@@ -133,18 +133,26 @@ __device__ __forceinline__ void attn_select_query(AttnArgs& a) {
 
 // o = sum_s e_s o_s / sum_s e_s l_s with e_s = exp(m_s - max_s m_s) for the HD dims of a query
 // head: its partial entry of split s at base + s pst = {o[HD], m, l}.  One workgroup; ml holds 2 S
-// floats of LDS.  The threads are G groups of HD / 2 (two dims each), group k taking the k-th of
-// G runs of splits, in order, the runs' sums added in order.
+// floats of LDS.  The threads are G groups of HD / 2 (two dims each), group k loading the k-th of
+// G runs of splits.  RUN, up to kMergeRun splits: the first group adds all of them in order, the
+// others' through LDS; else each group adds its run in order, and the runs' sums are added in order.
 // The loads of every (m, l) pair and of the first PF splits of each group's run are issued
-// together, so for S <= G PF (the splits of a decode step: 68 of head_dim 128) the merge waits
-// on memory once.
+// together, so for S <= G PF (68 splits of head_dim 128) the merge waits on memory once.
+constexpr int kMergeRun = 34;
 template <int HD>
+constexpr int merge_groups() { return kAttnThreads / (HD / 2); }
+// float2 of LDS of a merge: the splits' dims or the groups' sums
+template <int HD, bool RUN>
+constexpr int merge_stage() { return merge_groups<HD>() == 1 ? 1 : RUN ? kMergeRun * (HD / 2) : merge_groups<HD>() * (HD / 2); }
+
+template <int HD, bool RUN>
 __device__ __forceinline__ void attn_merge_head(const float* __restrict__ base, int pst, int S,
-                                                float* __restrict__ out, float* ml, float* inv_l) {
-    constexpr int H2 = HD / 2, G = kAttnThreads / H2, PF = G == 1 ? 34 : 17;
-    __shared__ float2 sums[G][H2];
+                                                float* __restrict__ out, float* ml, float* inv_l, float2* stage) {
+    constexpr int H2 = HD / 2, G = merge_groups<HD>();
+    constexpr int PF = G == 1 ? kMergeRun : RUN ? (kMergeRun + G - 1) / G : 17;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int grp = min(tid / H2, G - 1), d = 2 * (tid % H2);  // (threads past G H2 repeat others' work)
+    // (threads past the last group repeat others' work)
+    const int grp = min(tid / H2, G - 1), d2 = tid % H2;
     const int per = (S + G - 1) / G, s0 = min(grp * per, S), s1 = min(s0 + per, S);
     // the first (m, l) pair of each thread first: loads complete in order, so storing it
     // to LDS then waits for it alone, not for the prefetch behind it
@@ -152,7 +160,7 @@ __device__ __forceinline__ void attn_merge_head(const float* __restrict__ base, 
     const float2 ml0 = *reinterpret_cast<const float2*>(base + static_cast<size_t>(k0) * pst + HD);
     __builtin_amdgcn_sched_barrier(0);
     float2 ov[PF];
-    const float* src = base + d;
+    const float* src = base + 2 * d2;
     // unconditional loads (split clamped into range; a load under a condition becomes a branch,
     // and the loads would then wait one by one): splits past the run load data it does not use
 #pragma unroll
@@ -179,10 +187,27 @@ __device__ __forceinline__ void attn_merge_head(const float* __restrict__ base, 
         L = wave_sum_dpp(L);
         if (lane == 0) *inv_l = 1.0f / L;
     }
+    if constexpr (RUN && G > 1) {
+#pragma unroll
+        for (int u = 0; u < PF; u++)
+            if (s0 + u < s1) stage[(s0 + u) * H2 + d2] = ov[u];
+    }
     lds_barrier();
+    if (RUN && tid >= H2) return;
     float2 o = make_float2(0.f, 0.f);
-    {
-        // every weight read from LDS before the first is used; splits past the run keep o
+    if constexpr (RUN) {
+        // every weight (and dim) read from LDS before the first is used; splits past S keep o
+        float ev[kMergeRun];
+#pragma unroll
+        for (int u = 0; u < kMergeRun; u++) ev[u] = ml[2 * min(u, S - 1)];
+#pragma unroll
+        for (int u = 0; u < kMergeRun; u++) {
+            const float2 v = G > 1 ? stage[min(u, S - 1) * H2 + tid] : ov[G > 1 ? 0 : u];
+            const float x = fmaf(v.x, ev[u], o.x), y = fmaf(v.y, ev[u], o.y);
+            o.x = u < S ? x : o.x;
+            o.y = u < S ? y : o.y;
+        }
+    } else {
         float ev[PF];
 #pragma unroll
         for (int u = 0; u < PF; u++) ev[u] = ml[2 * min(s0 + u, S - 1)];
@@ -192,29 +217,29 @@ __device__ __forceinline__ void attn_merge_head(const float* __restrict__ base, 
             o.x = s0 + u < s1 ? x : o.x;
             o.y = s0 + u < s1 ? y : o.y;
         }
-    }
-    for (int s = s0 + PF; s < s1; s += 16) {  // splits past PF: sixteen loads in flight per round
-        float2 v[16];
+        for (int s = s0 + PF; s < s1; s += 16) {  // splits past PF: sixteen loads in flight per round
+            float2 v[16];
 #pragma unroll
-        for (int u = 0; u < 16; u++)
-            v[u] = *reinterpret_cast<const float2*>(src + static_cast<size_t>(min(s + u, s1 - 1)) * pst);
+            for (int u = 0; u < 16; u++)
+                v[u] = *reinterpret_cast<const float2*>(src + static_cast<size_t>(min(s + u, s1 - 1)) * pst);
 #pragma unroll
-        for (int u = 0; u < 16; u++)
-            if (s + u < s1) {
-                o.x = fmaf(v[u].x, ml[2 * (s + u)], o.x);
-                o.y = fmaf(v[u].y, ml[2 * (s + u)], o.y);
-            }
-    }
-    if constexpr (G > 1) {
-        sums[grp][tid % H2] = o;
-        lds_barrier();
-        if (tid >= H2) return;
-        o = sums[0][tid];
+            for (int u = 0; u < 16; u++)
+                if (s + u < s1) {
+                    o.x = fmaf(v[u].x, ml[2 * (s + u)], o.x);
+                    o.y = fmaf(v[u].y, ml[2 * (s + u)], o.y);
+                }
+        }
+        if constexpr (G > 1) {
+            stage[grp * H2 + d2] = o;
+            lds_barrier();
+            if (tid >= H2) return;
+            o = stage[tid];
 #pragma unroll
-        for (int k = 1; k < G; k++) o.x += sums[k][tid].x, o.y += sums[k][tid].y;
+            for (int k = 1; k < G; k++) o.x += stage[k * H2 + tid].x, o.y += stage[k * H2 + tid].y;
+        }
     }
     const float il = *inv_l;
-    *reinterpret_cast<float2*>(out + d) = make_float2(o.x * il, o.y * il);
+    *reinterpret_cast<float2*>(out + 2 * d2) = make_float2(o.x * il, o.y * il);
 }
 
 // LDS of one head's merge: S (m, l) pairs and its reciprocal sum.
@@ -488,7 +513,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
 // workgroups placed on one XCD and meeting in its L2 through an atomic arrival count) was
 // measured: 1.5405 against 1.5408 ms per 8B decode step, so the chain of memory round
 // trips, not the launch between them, sets the cost; the merge stays a launch.
-template <int HD>
+// RUN: no query has more than kMergeRun splits.
+template <int HD, bool RUN>
 __global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(AttnArgs a) {
     extern __shared__ float lds[];
     const int sst = a.S;  // partial stride per head
@@ -496,7 +522,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(AttnArgs a) 
     const int per = kAttnChunk * a.chunks;
     const int S = (a.T - (a.t_begin & ~7) + per - 1) / per;  // this query's splits
     const size_t h = blockIdx.x;
-    attn_merge_head<HD>(a.part + h * sst * a.pst, a.pst, S, a.out + h * HD, lds, lds + 2 * S);
+    const float* base = a.part + h * sst * a.pst;
+    float* o = a.out + h * HD;
+    __shared__ float2 stage[merge_stage<HD, true>() > merge_stage<HD, false>() || RUN ? merge_stage<HD, true>() : merge_stage<HD, false>()];
+    if (RUN || S <= kMergeRun) attn_merge_head<HD, true>(base, a.pst, S, o, lds, lds + 2 * S, stage);
+    else if constexpr (!RUN) attn_merge_head<HD, false>(base, a.pst, S, o, lds, lds + 2 * S, stage);
 }
 
 // ── Prompt attention in one pass per block of queries ────────────────────
@@ -809,6 +839,15 @@ int attn_prompt_splits(int T0, int batch, int window) {
 
 bool attn_prompt_one_pass(int reps, int hd) { return hd <= 256 && 16 % reps == 0; }
 
+// A decode step's workgroup takes several chunks in turn where there are more than two
+// workgroups per CU: fewer partials to merge, the query prepared once for all of them.  Four
+// 8B-shape layers and the head at position 16384 / 30000: 358 / 471 us with a chunk per
+// workgroup, 326 / 393 with one workgroup per CU, 305 / 346 with two, 316 / 383 with four.
+int attn_step_chunks(int T, int t_begin, int num_kv) {
+    const int cus = current_device_cus();
+    return std::max(1, (attn_splits(T, t_begin) * num_kv + 2 * cus - 1) / (2 * cus));
+}
+
 // f(std::integral_constant<int, hd>) for the instantiated head dims, the multiples of 32
 // from HD up to 512; false for any other hd.
 template <int HD, typename F>
@@ -825,7 +864,7 @@ void launch_attention(const AttnArgs& a0, hipStream_t s) {
     AttnArgs a = a0;
     const int reps = a.num_q / a.num_kv;
     if (!attn_supported(reps, a.hd)) fail(LARQL_HIP_ERR_UNSUPPORTED, "attention: head geometry");
-    if (a.batch && attn_prompt_one_pass(reps, a.hd)) {  // prompt mode: one pass per block of queries
+    if (a.batch && !a.as_steps && attn_prompt_one_pass(reps, a.hd)) {  // prompt mode: one pass per block of queries
         const int qpb = 4 * (16 / reps);
         const dim3 gp(static_cast<unsigned>((a.batch + qpb - 1) / qpb), a.num_kv), bp(kAttnThreads);
         if (!dispatch_head_dim<32>(a.hd, [&](auto h) {
@@ -836,12 +875,8 @@ void launch_attention(const AttnArgs& a0, hipStream_t s) {
         LARQL_HIP_CHECK(hipGetLastError());
         return;
     }
-    // A decode step's workgroup takes several chunks in turn where there are more than two
-    // workgroups per CU: fewer partials to merge, the query prepared once for all of them.  Four
-    // 8B-shape layers and the head at position 16384 / 30000: 358 / 471 us with a chunk per
-    // workgroup, 326 / 393 with one workgroup per CU, 305 / 346 with two, 316 / 383 with four.
     const int chunks = attn_splits(a.T, a.t_begin);
-    a.chunks = a.batch ? 1 : std::max(1, (chunks * a.num_kv + 2 * current_device_cus() - 1) / (2 * current_device_cus()));
+    a.chunks = a.batch ? 1 : attn_step_chunks(a.T, a.t_begin, a.num_kv);
     a.S = a.batch ? attn_prompt_splits(a.T, a.batch, a.window) : (chunks + a.chunks - 1) / a.chunks;
     a.pst = attn_partial_stride(a.hd);
     if (2 * static_cast<size_t>(a.S) * sizeof(float) + 32 > static_cast<size_t>(kMergeLdsMax))
@@ -856,7 +891,10 @@ void launch_attention(const AttnArgs& a0, hipStream_t s) {
         fail(LARQL_HIP_ERR_UNSUPPORTED, "attention: head_dim");
     LARQL_HIP_CHECK(hipGetLastError());
     const dim3 g2(a.num_q, 1, nz);
-    dispatch_head_dim<32>(a.hd, [&](auto h) { attn_combine_kernel<decltype(h)::value><<<g2, block, lds, s>>>(a); });
+    dispatch_head_dim<32>(a.hd, [&](auto h) {
+        if (a.S <= kMergeRun) attn_combine_kernel<decltype(h)::value, true><<<g2, block, lds, s>>>(a);
+        else attn_combine_kernel<decltype(h)::value, false><<<g2, block, lds, s>>>(a);
+    });
     LARQL_HIP_CHECK(hipGetLastError());
 }
 

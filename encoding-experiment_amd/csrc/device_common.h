@@ -7,14 +7,14 @@
 
 namespace larql {
 
-// IEEE binary16 -> binary32 (exact; subnormal inputs are decoded, as the
-// reference decoders LC/src/cpu/ops/q4_common.rs:426-442 and q4_dot.c:9-35 do).
 // Workgroup barrier for data exchanged through LDS only: the wave's LDS accesses complete,
 // then s_barrier.  __syncthreads() is also a workgroup-scope release, which waits for every
 // global load in flight (vmcnt(0)): in a kernel that keeps loads in flight across its
 // barriers (prefetch, or operands used after later LDS phases) that exposes their latency.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// IEEE binary16 -> binary32 (exact; subnormal inputs are decoded, as the
+// reference decoders LC/src/cpu/ops/q4_common.rs:426-442 and q4_dot.c:9-35 do).
 __device__ __forceinline__ float h2f(uint32_t bits16) {
     return __half2float(__ushort_as_half(static_cast<unsigned short>(bits16 & 0xFFFFu)));
 }
@@ -47,6 +47,11 @@ __device__ __forceinline__ float wave_max(float v) {
     for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
     return v;
 }
+
+// The two elements of a RoPE pair (x, y), cs = (cos, sin): x cos - y sin and y cos + x sin, each
+// one rounded product and one fma, so that every kernel that rotates a row gives the same bits.
+__device__ __forceinline__ float rope_low(float x, float y, float2 cs) { return __builtin_fmaf(x, cs.x, -(y * cs.y)); }
+__device__ __forceinline__ float rope_high(float x, float y, float2 cs) { return __builtin_fmaf(x, cs.y, y * cs.x); }
 
 // Row statistics of one token row for the f32-accuracy GEMMs, by a 256-thread workgroup
 // (all threads call it; it synchronises the workgroup): *e = the power of two that puts

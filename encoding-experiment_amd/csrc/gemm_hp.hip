@@ -1,5 +1,5 @@
 // f32-accuracy GEMMs of quantized weights: Y[M x N] = X[M x K] . deq(W)^T from f32 X, for the
-// chains of projections of the prompt pass and for small batches (Q4_K, Q6_K and Q4_0).
+// chains of projections of the prompt pass and for small batches (Q4_K and Q6_K).
 //
 // Every f32 activation x is split into two fp16 parts, hi = fp16(x) and lo = fp16(x - hi) (x -
 // hi exact in f32), x = hi + lo to ~2^-22, and the products run on v_mfma_f32_16x16x32_f16 with
@@ -134,8 +134,8 @@ __device__ __forceinline__ v4u transpose4(v4u q) {
 }
 
 struct PkArgs {
-    const uint8_t* qs;    // Q4_K / Q4_0 nibbles, Q6_K blocks
-    const uint8_t* hdr;   // Q4_K headers, Q4_0 f16 scales (Q6_K: unused)
+    const uint8_t* qs;    // Q4_K nibbles, Q6_K blocks
+    const uint8_t* hdr;   // Q4_K headers (Q6_K: unused)
     const v4u* XP;        // packed X (x_pack_kernel)
     const int* xe;        // row exponents
     const float* xs;      // scaled sub-block sums (Q4_K)
@@ -168,12 +168,10 @@ struct PkArgs {
 // Q6_K: w = d sc (q - 32) per 16-element group; sc (q - 32) reaches 4096, past fp16's exact
 // integers, so it is split exactly, hi = fp16(sc (q - 32)) and lo the rest (at most 1): three
 // products per super-block accumulator (the dropped x_lo w_lo is ~2^-23 of it).
-//
-// Q4_0: w = d (q - 8) per 32-element block: q - 8 (times 2^-24) in fp16, a fresh accumulator per k-step, added
-// into the total times d.
 template <int FMT, int TT>
 __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     constexpr bool kQ4K = FMT == LARQL_Q4_K, kQ6K = FMT == LARQL_Q6_K;
+    static_assert(kQ4K || kQ6K, "Q4_K or Q6_K");
     // an operand's unit: codes times 2^-24; Q6_K weights at a quarter
     constexpr float kUnit = kQ6K ? 4.0f : 16777216.0f;
     // weight loads per wave of a unit of each parity
@@ -191,10 +189,8 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     if (grp >= a.gx * a.gz) return;
     const int bx = grp % a.gx, bz = grp / a.gx;
     const int mt0 = by * TT, nt0 = (bx * kPkWaves + wave) * kPkR;
-    // split bz of K: super-blocks (Q4_0: 256 k) [bz sb_per, (bz + 1) sb_per), sums to Y[bz].
-    // Units of 128 k; a last half super-block may be missing (K % 256 == 128, Q4_0).
-    const int nu = K / 128;
-    const int u0 = 2 * bz * a.sb_per, u1 = min(nu, u0 + 2 * a.sb_per), last = u1 - 1;
+    // split bz of K: super-blocks [bz sb_per, (bz + 1) sb_per), two units of 128 k each, sums to Y[bz]
+    const int u0 = 2 * bz * a.sb_per, u1 = min(K / 128, u0 + 2 * a.sb_per), last = u1 - 1;
     float* Y = a.Y + bz * a.ypart;
 
     // raw buffer loads: the wave-uniform part of each offset in the scalar operand, the lane's in
@@ -202,7 +198,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     // whatever the weight's or X's size
     const int nks = K / 32;
     const uint32_t qtile = kQ6K ? static_cast<uint32_t>(K / 256) * static_cast<uint32_t>(kQ6Block) : 8u * K;
-    const uint32_t htile = kQ4K ? K : 32u * nks;  // headers 256 bytes, scales 512 bytes per super-block
+    const uint32_t htile = K;  // headers, 256 bytes per super-block (Q6_K: none)
     const int ntc = min(nt0, a.ntiles - 1), have = min(kPkR, a.ntiles - ntc), mhave = min(TT, a.mtiles - mt0);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<v4u*>(a.XP) + static_cast<size_t>(mt0) * nks * 128, 0,
@@ -210,19 +206,17 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(a.qs) + static_cast<size_t>(ntc) * qtile, 0, static_cast<int>(have * qtile), 0x00020000);
     const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(a.hdr) + static_cast<size_t>(ntc) * htile, 0, static_cast<int>(have * htile), 0x00020000);
+        const_cast<uint8_t*>(a.hdr) + static_cast<size_t>(ntc) * htile, 0, kQ4K ? static_cast<int>(have * htile) : 0, 0x00020000);
     uint32_t qo[kPkR], ho[kPkR];
 #pragma unroll
     for (int j = 0; j < kPkR; j++) {  // (tiles past the last re-read it; their rows are not stored)
         qo[j] = static_cast<uint32_t>(min(j, have - 1)) * qtile;
         ho[j] = static_cast<uint32_t>(min(j, have - 1)) * htile;
     }
-    // the lane's part: Q4_K and Q6_K tile-major (16 bytes a lane, header of row c), Q4_0 row-major
-    // (row c, block 4 u + g; the scales of row c's four blocks)
-    const uint32_t ql = kQ4K || kQ6K ? lane * 16u : static_cast<uint32_t>(c) * (K / 2) + 16u * g;
-    const uint32_t hl = kQ4K ? c * 16u : static_cast<uint32_t>(c) * (2u * nks);
+    // the lane's part: tile-major, 16 bytes a lane, the header of row c
+    const uint32_t ql = lane * 16u, hl = c * 16u;
     // load instruction n = wave 2 TT + i of a unit: token tile n / 8, KB n % 8 of its 8 KB (k-step
-    // t = (n % 8) / 2, part n % 2).  Q4_K, Q4_0: unit u is k-steps 4 u + t; Q6_K: 8 (u / 2) + 2 t +
+    // t = (n % 8) / 2, part n % 2).  Q4_K: unit u is k-steps 4 u + t; Q6_K: 8 (u / 2) + 2 t +
     // u % 2 (the sub-blocks whose codes one load of the block layout holds)
     uint32_t xo[2 * TT];
 #pragma unroll
@@ -240,7 +234,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     };
     struct Wu {
         v4u q[kPkR];
-        v2u h[kPkR];  // Q4_K: {d | dmin << 16, scales of the unit's sub-blocks}; Q4_0: four f16 scales; Q6_K: high bits
+        v2u h[kPkR];  // Q4_K: {d | dmin << 16, scales of the unit's sub-blocks}; Q6_K: high bits
     };
     // Q6_K: scales (int8 x 4 of the lane's 64 elements) and d of the super-block in progress and
     // of the one requested
@@ -258,7 +252,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                 const uint32_t hso = ho[j] + static_cast<uint32_t>(u >> 1) * 256u;
                 if constexpr (h) w.h[j].y = __builtin_amdgcn_raw_buffer_load_b32(rh, hl, hso + 8u, 0);
                 else w.h[j] = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(rh, hl, hso, 0));
-            } else if constexpr (kQ6K) {
+            } else {
                 const uint32_t bo = qo[j] + static_cast<uint32_t>(u >> 1) * static_cast<uint32_t>(kQ6Block);
                 w.q[j] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rq, ql, bo + h * 1024u, 2));
                 w.h[j] = __builtin_bit_cast(
@@ -267,11 +261,6 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                     sc6n[j] = __builtin_amdgcn_raw_buffer_load_b32(rq, lane * 4u, bo + static_cast<uint32_t>(kQ6Sc), 0);
                     d6n[j] = __builtin_amdgcn_raw_buffer_load_b16(rq, c * 2u, bo + static_cast<uint32_t>(kQ6D), 0);
                 }
-            } else {
-                w.q[j] = __builtin_bit_cast(
-                    v4u, __builtin_amdgcn_raw_buffer_load_b128(rq, ql, qo[j] + static_cast<uint32_t>(u) * 64u, 0));
-                w.h[j] = __builtin_bit_cast(
-                    v2u, __builtin_amdgcn_raw_buffer_load_b64(rh, hl, ho[j] + static_cast<uint32_t>(u) * 8u, 0));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -329,7 +318,7 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                     f16x2 q[4];
                     nibble_pairs(word, q);
                     B = operand8(q[0] * sv, q[1] * sv, q[2] * sv, q[3] * sv);
-                } else if constexpr (kQ6K) {
+                } else {
                     const uint32_t hb = nh[j][t] >> (4 * (g & 1));
                     const uint32_t lo = (word & 0x0F0F0F0Fu) | ((hb & 0x03030303u) << 4);
                     const uint32_t hi = ((word >> 4) & 0x0F0F0F0Fu) | (((hb >> 2) & 0x03030303u) << 4);
@@ -351,14 +340,8 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                     pr(hi, 0x04030401u, so, bh[3], bl[3]);
                     B = operand8(bh[0], bh[1], bh[2], bh[3]);
                     Bl = operand8(bl[0], bl[1], bl[2], bl[3]);
-                } else {
-                    constexpr _Float16 u8e = 0x1p-21f16, u8o = 0x1p-17f16;  // code 8
-                    f16x2 q[4];
-                    nibble_pairs(word, q);
-                    B = operand8(q[0] - f16x2{u8e, u8e}, q[1] - f16x2{u8e, u8e}, q[2] - f16x2{u8o, u8o}, q[3] - f16x2{u8o, u8o});
                 }
-                constexpr bool kSuper = kQ4K || kQ6K;  // an accumulator per super-block, else per block
-                const bool fresh = kSuper ? (h == 0 && t == 0) : true;
+                const bool fresh = h == 0 && t == 0;  // an accumulator per super-block
 #pragma unroll
                 for (int i = 0; i < TT; i++)
                     dp[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
@@ -372,18 +355,8 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                 for (int i = 0; i < TT; i++)
                     dp[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, al[i]), B, dp[j][i], 0, 0, 0);
             }
-            if constexpr (!kQ4K && !kQ6K) {  // the blocks' sums times d (row c)
-#pragma unroll
-                for (int j = 0; j < kPkR; j++) {
-                    const float d = h2f(w.h[j][t >> 1] >> (16 * (t & 1))) * kUnit;
-#pragma unroll
-                    for (int i = 0; i < TT; i++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) acc[j][i][r] = fmaf(d, dp[j][i][r], acc[j][i][r]);
-                }
-            }
         }
-        if constexpr ((kQ4K || kQ6K) && h == 1) {  // the super-block's sum times d (row c)
+        if constexpr (h == 1) {  // the super-block's sum times d (row c)
 #pragma unroll
             for (int j = 0; j < kPkR; j++) {
                 const float d = dsb[j] * kUnit;
@@ -412,12 +385,10 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
         compute(h, hc, w);
         load_w(min(u + 2, last), hc, w);
     };
-    int u = u0;
-    for (; u + 1 < u1; u += 2) {
+    for (int u = u0; u < u1; u += 2) {
         stage(u, std::integral_constant<int, 0>{}, w0);
         stage(u + 1, std::integral_constant<int, 1>{}, w1);
     }
-    if (u < u1) stage(u, std::integral_constant<int, 0>{}, w0);  // (Q4_0)
     wait_vmcnt<0>();  // nothing may land in LDS after the workgroup has ended
 
     if constexpr (kQ4K) {
@@ -573,8 +544,8 @@ struct PkPlan {
     double ns;  // the modelled time of the GEMM and its sums
 };
 PkPlan pk_plan(const DevWeight& w, size_t m) {
-    const int S = static_cast<int>((w.cols + 255) / 256);
-    const long most = w.format == LARQL_Q4_K ? 4 : 3;  // (four would spill in the others)
+    const int S = static_cast<int>(w.cols / 256);
+    const long most = w.format == LARQL_Q4_K ? 4 : 3;  // (four would spill for Q6_K)
     const long cus = current_device_cus(), mt = static_cast<long>((m + 15) / 16), gy = (mt + most - 1) / most;
     PkPlan best{static_cast<int>((mt + gy - 1) / gy), 1, S, -1.0};
     constexpr double kUnit[5] = {0, 2200, 3000, 3600, 4100};  // ns
@@ -592,11 +563,6 @@ PkPlan pk_plan(const DevWeight& w, size_t m) {
 size_t align4(size_t n) { return (n + 3) & ~size_t{3}; }
 
 }  // namespace
-
-bool gemm_f32_takes(const DevWeight& w) {
-    if (w.format == LARQL_Q4_0) return w.cols % 128 == 0;
-    return w.format == LARQL_Q4_K || w.format == LARQL_Q6_K;
-}
 
 size_t gemm_x_pack_floats(size_t m, size_t cols) { return (m + 15) / 16 * 16 * cols; }
 
@@ -671,7 +637,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     if (ldy == 0) ldy = w.rows;
     if (ldy < w.rows || ldy > 0x7FFFFFFF) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: bad output row stride");
     if (defer && ldy != w.rows) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: deferred split sums need dense output rows");
-    if (!gemm_f32_takes(w)) fail(LARQL_HIP_ERR_UNSUPPORTED, "f32 GEMM: Q4_K, Q6_K or Q4_0 (cols a multiple of 128)");
+    if (w.format != LARQL_Q4_K && w.format != LARQL_Q6_K) fail(LARQL_HIP_ERR_UNSUPPORTED, "f32 GEMM: Q4_K or Q6_K weights");
     if (pre && (!pre->xe || (w.format == LARQL_Q4_K && !pre->xs)))
         fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: incomplete row statistics");
     if (m == 0) return;
@@ -696,7 +662,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     }
     PkArgs a{};
     a.qs = w.qs;
-    a.hdr = w.format == LARQL_Q4_K ? reinterpret_cast<const uint8_t*>(w.hdr) : static_cast<const uint8_t*>(w.d);
+    a.hdr = reinterpret_cast<const uint8_t*>(w.hdr);
     a.XP = reinterpret_cast<const v4u*>(st.xp);
     a.xe = st.xe;
     a.xs = st.xs;
@@ -725,8 +691,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
         else if constexpr (decltype(f)::value == LARQL_Q4_K) go(f, std::integral_constant<int, 4>{});
     };
     if (w.format == LARQL_Q4_K) fmt(std::integral_constant<int, LARQL_Q4_K>{});
-    else if (w.format == LARQL_Q6_K) fmt(std::integral_constant<int, LARQL_Q6_K>{});
-    else fmt(std::integral_constant<int, LARQL_Q4_0>{});
+    else fmt(std::integral_constant<int, LARQL_Q6_K>{});
     LARQL_HIP_CHECK(hipGetLastError());
     if (defer) *defer = {p.splits > 1 ? part : nullptr, p.splits};
     if (parts && !defer) {

@@ -258,10 +258,9 @@ void launch_f32_matmul(const float* A, const float* B, float* C, size_t m, size_
 // MFMA operands.
 size_t q4k_gemm_ws_bytes(size_t m, size_t cols);
 void launch_q4k_gemm(const DevWeight& w, const float* X, float* Y, size_t m, void* ws, hipStream_t s);
-// The same product at f32 accuracy for Q4_K, Q6_K and Q4_0 weights (gemm_hp.hip: X as fp16
+// The same product at f32 accuracy for Q4_K and Q6_K weights (gemm_hp.hip: X as fp16
 // operand pairs scaled into range by per-token powers of two): ~1e-6 instead of ~1e-4, for
 // chains of projections (the batched prompt pass) and small batches.
-bool gemm_f32_takes(const DevWeight& w);
 // Row statistics of an input (row exponents xe; the scaled sub-block sums xs that Q4_K weights
 // use, m x cols / 32 floats from a 16-byte boundary), which a caller may fuse into the kernel
 // that produces the input, and its packed operands xp (gemm_x_pack_floats, 16-byte aligned;
@@ -313,8 +312,12 @@ void launch_q4_0_matvec_pair(const DevWeight& w1, const DevWeight& w2, const int
                              float* out1, float* out2, size_t m, hipStream_t s);
 void launch_q8_matvec(const DevWeight& w, const int8_t* q8x, const float* q8s, float* out,
                       size_t m, hipStream_t s);
-// Q4_0 weights x f32 activation (one row of x), the reference GPU's q4_f32_matvec.
-void launch_q4_0_f32_matvec(const DevWeight& w, const float* x, float* out, hipStream_t s);
+// Q4_0 weights x m f32 activation rows, the reference GPU's q4_f32_matvec; each output row in the
+// single-row order, bit for bit.  ws: q4_0_f32_rows_ws_floats of 16-byte aligned workspace for many
+// rows (null: row by row).
+void launch_q4_0_f32_matvec(const DevWeight& w, const float* x, float* out, hipStream_t s, size_t m = 1,
+                            float* ws = nullptr);
+size_t q4_0_f32_rows_ws_floats(size_t m, size_t cols);
 void launch_quantize_q8(const float* x, size_t n, size_t m, int8_t* q8, float* scales, hipStream_t s);
 // q4_vecmat: chunks of rows per partial (q4_vecmat_chunks) and the two-pass launch;
 // part holds chunks x cols floats.

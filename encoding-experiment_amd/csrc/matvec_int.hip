@@ -919,6 +919,8 @@ __global__ __launch_bounds__(1024) void q4_0_f32_mv_kernel(const uint8_t* __rest
     __shared__ float part[16][kQfRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int r0 = blockIdx.x * kQfRows;
+    x += blockIdx.y * (32 * static_cast<size_t>(nb));
+    out += blockIdx.y * static_cast<size_t>(rows);
     const int b = 64 * wave + lane;
     const bool on = b < nb;
     const int bc = on ? b : nb - 1;  // past the row's end: a real block, contributing 0
@@ -978,17 +980,167 @@ __global__ __launch_bounds__(1024) void q4_0_f32_mv_kernel(const uint8_t* __rest
         out[r0 + threadIdx.x] = v;
     }
 }
+
+// The same products for many rows of x (the prompt pass), every output the sum above, bit for bit.
+// v_mfma_f32_16x16x1_4b_f32 does one fma per output and block: a wave takes 16 weight rows x 16 rows
+// of x and four blocks of its 64 at a time, 32 of them chaining the blocks' 32 elements, so a
+// block's sum is the chain above.  The four blocks are 16 apart (q, q + 16, q + 32, q + 48) and the
+// q in bit-reversed order, so that the shuffles' tree is two adds inside the four and a four-deep
+// stack of partial sums.  Weight row = operand A (output rows 4 g + r of lane (g, c)), x = operand B
+// (column c): lane (b, i) holds block b of weight row i and of x row i.
+// Bound: MFMA issue (8 passes each) and the VALU between: [4096 x 14336], 96 rows 167 us, of which the
+// MFMAs are 78 and the VALU 62 (counters), against 306 us with a lane per block, an f32 fma per
+// weight and the shuffles, and 96 launches of the matvec for a row each; 271 us with x read as it lies
+// (16 bytes of each of 64 lines per load).
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kQrTile = 16;
+
+// The i-th group's first block, the 4-bit reversal of i.
+__device__ __forceinline__ int qr_group(int i) { return static_cast<int>(__brev(static_cast<unsigned>(i)) >> 28); }
+// The block of a 64-block run that lane group g holds in the i-th group (past the row's end: the last).
+__device__ __forceinline__ int qr_block(int wave, int i, int g, int nb) {
+    return min(64 * wave + qr_group(i) + 16 * g, nb - 1);
+}
+
+// XP[16 rows of x][run][group][float4 k][lane (g, c)] = float4 k of the lane's block of row c (past the
+// last row: the last), so that the loads of the kernel below are contiguous.  Grid (16 runs,
+// ceil(M / 16)), 512 threads.
+__global__ __launch_bounds__(512) void q4_0_f32_x_kernel(const float* __restrict__ X, float4* __restrict__ XP, int nb, int M) {
+    const int lane = threadIdx.x & 63, k = threadIdx.x >> 6;
+    const int b = qr_block(blockIdx.x >> 4, blockIdx.x & 15, lane >> 4, nb);
+    const float4* x = reinterpret_cast<const float4*>(
+        X + static_cast<size_t>(min(kQrTile * static_cast<int>(blockIdx.y) + (lane & 15), M - 1)) * (32 * static_cast<size_t>(nb)));
+    XP[(blockIdx.y * static_cast<size_t>(gridDim.x) + blockIdx.x) * 512 + threadIdx.x] = x[8 * b + k];
+}
+
+__global__ __launch_bounds__(1024) void q4_0_f32_rows_kernel(const uint8_t* __restrict__ qs,
+                                                             const uint16_t* __restrict__ d,
+                                                             const float4* __restrict__ XP, float* __restrict__ out,
+                                                             int rows, int nb, int M) {
+#pragma clang fp contract(off)
+    extern __shared__ uint4 qr_lds[];  // the waves' scales [64 blocks][16 rows] f16, then their sums
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int g = lane >> 4, c = lane & 15, r0 = blockIdx.x * kQrTile, t0 = blockIdx.y * kQrTile, b0 = 64 * wave;
+    uint16_t* sc = reinterpret_cast<uint16_t*>(qr_lds) + wave * (64 * kQrTile);
+    for (int i = lane; i < 64 * kQrTile; i += 64) {  // (row i / 64, block i % 64)
+        const size_t row = static_cast<size_t>(min(r0 + i / 64, rows - 1));
+        sc[(i % 64) * kQrTile + i / 64] = d[row * nb + min(b0 + i % 64, nb - 1)];
+    }
+    const uint4* wp = reinterpret_cast<const uint4*>(qs) + static_cast<size_t>(min(r0 + c, rows - 1)) * nb;
+    const float4* xp = XP + (blockIdx.y * static_cast<size_t>(nw) + wave) * (16 * 512) + lane;
+    uint4 wn = wp[qr_block(wave, 0, g, nb)];
+    float4 xv[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {  // (in order: the waits in the loop count the loads after the one they need)
+        xv[k] = xp[64 * k];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    f32x4 s0{}, s1{}, s2{}, s3{}, tot{};
+#pragma unroll 1
+    for (int i = 0; i < 16; i++) {
+        const int q = qr_group(i), ni = min(i + 1, 15);
+        const uint32_t wd[4] = {wn.x, wn.y, wn.z, wn.w};
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            lo[k] = wd[k] & 0x0F0F0F0Fu, hi[k] = (wd[k] >> 4) & 0x0F0F0F0Fu;
+            asm volatile("" : "+v"(lo[k]), "+v"(hi[k]));  // byte conversions, not field extracts
+        }
+        wn = wp[qr_block(wave, ni, g, nb)];
+        floatx16 acc{};
+        float xsum = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float4 x = xv[k];
+            const uint32_t l = lo[k >> 1] >> (16 * (k & 1)), h = hi[k >> 1] >> (16 * (k & 1));
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(ubyte0(l), x.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(ubyte0(h), x.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(ubyte1(l), x.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(ubyte1(h), x.w, acc, 0, 0, 0);
+            xsum = (((xsum + x.x) + x.y) + x.z) + x.w;
+            xv[k] = xp[512 * ni + 64 * k];  // the next blocks', once these are used up
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4 v[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const float xs = __shfl(xsum, 16 * b + c, 64);
+            const uint2 dd = *reinterpret_cast<const uint2*>(&sc[(q + 16 * b) * kQrTile + 4 * g]);
+            const float dr[4] = {h2f(dd.x), h2f(dd.x >> 16), h2f(dd.y), h2f(dd.y >> 16)};
+            const bool on = b0 + q + 16 * b < nb;
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[b][r] = on ? __builtin_fmaf(-8.0f, xs, acc[4 * b + r]) * dr[r] : 0.f;
+        }
+        f32x4 s = (v[0] + v[2]) + (v[1] + v[3]);
+        if (i & 1) {
+            s = s0 + s;
+            if (i & 2) {
+                s = s1 + s;
+                if (i & 4) {
+                    s = s2 + s;
+                    if (i & 8) tot = s3 + s;
+                    else s3 = s;
+                } else {
+                    s2 = s;
+                }
+            } else {
+                s1 = s;
+            }
+        } else {
+            s0 = s;
+        }
+    }
+    // the waves' sums in order: part[wave][x row][weight row]
+    __syncthreads();
+    f32x4* part = reinterpret_cast<f32x4*>(qr_lds);
+    part[(wave * kQrTile + c) * 4 + g] = tot;
+    __syncthreads();
+    const float* p = reinterpret_cast<const float*>(qr_lds);
+    for (int i = threadIdx.x; i < kQrTile * kQrTile; i += blockDim.x) {
+        float v = p[i];
+        for (int k = 1; k < nw; k++) v += p[k * (kQrTile * kQrTile) + i];
+        const int t = t0 + i / kQrTile, r = r0 + i % kQrTile;
+        if (t < M && r < rows) out[static_cast<size_t>(t) * rows + r] = v;
+    }
+}
 }  // namespace
 
-void launch_q4_0_f32_matvec(const DevWeight& w, const float* x, float* out, hipStream_t s) {
+size_t q4_0_f32_rows_ws_floats(size_t m, size_t cols) {
+    return (m + kQrTile - 1) / kQrTile * ((cols / 32 + 63) / 64) * (64 * 32 * kQrTile);
+}
+
+void launch_q4_0_f32_matvec(const DevWeight& w, const float* x, float* out, hipStream_t s, size_t m, float* ws) {
     if (w.format != LARQL_Q4_0) fail(LARQL_HIP_ERR_UNSUPPORTED, "q4_0 f32 matvec: Q4_0 weights only");
-    if (w.rows == 0) return;
+    if (w.rows == 0 || m == 0) return;
     const int nb = static_cast<int>(w.cols / 32);
     if (nb > 16 * 64) fail(LARQL_HIP_ERR_UNSUPPORTED, "q4_0 f32 matvec: rows longer than 32768");
-    const dim3 grid(static_cast<unsigned>((w.rows + kQfRows - 1) / kQfRows)), block(64 * ((nb + 63) / 64));
-    q4_0_f32_mv_kernel<<<grid, block, 0, s>>>(w.qs, static_cast<const uint16_t*>(w.d), x, out,
-                                             static_cast<int>(w.rows), nb);
-    LARQL_HIP_CHECK(hipGetLastError());
+    const unsigned nw = static_cast<unsigned>((nb + 63) / 64);
+    const uint16_t* d = static_cast<const uint16_t*>(w.d);
+    const int rows = static_cast<int>(w.rows);
+    for (size_t t = 0; t < m; t += 32768) {  // (grid y is at most 65535)
+        const unsigned n = static_cast<unsigned>(std::min<size_t>(m - t, 32768));
+        const float* xt = x + t * w.cols;
+        float* o = out + t * w.rows;
+        // a tile of the matrix cores costs the same for 1 .. 16 rows, the matvec grows with them: the
+        // tiles from about four rows per CU's weight-row tile on (two layers of a prompt of 4 / 8
+        // positions, [4096 x 14336]: 230 / 235 us against 236 / 302 row by row; [2560 x 10240], 4 / 8:
+        // 211 / 219 against 184 / 219)
+        const size_t rtiles = (w.rows + kQrTile - 1) / kQrTile;
+        if (ws && n * rtiles >= 4 * static_cast<size_t>(current_device_cus())) {
+            const unsigned tiles = (n + kQrTile - 1) / kQrTile;
+            float4* xp = reinterpret_cast<float4*>(ws);
+            q4_0_f32_x_kernel<<<dim3(16 * nw, tiles), dim3(512), 0, s>>>(xt, xp, nb, static_cast<int>(n));
+            LARQL_HIP_CHECK(hipGetLastError());
+            q4_0_f32_rows_kernel<<<dim3(static_cast<unsigned>(rtiles), tiles), dim3(64 * nw),
+                                   nw * 64 * kQrTile * sizeof(uint16_t), s>>>(w.qs, d, xp, o, rows, nb, static_cast<int>(n));
+        } else {
+            const dim3 grid((rows + kQfRows - 1) / kQfRows, n);
+            q4_0_f32_mv_kernel<<<grid, dim3(64 * nw), 0, s>>>(w.qs, d, xt, o, rows, nb);
+        }
+        LARQL_HIP_CHECK(hipGetLastError());
+    }
 }
 
 // 1..4 activation rows: the lane-group kernel (one pass over the weights); 5..8: the

@@ -87,8 +87,8 @@ __global__ void rope_kv_rows_kernel(const float* __restrict__ QKV, int M, int p0
     const float* k = row + q_dim + kvh * hd;
     const float2* cs = rope + static_cast<size_t>(pos) * half;
     float kr = k[d];
-    if (d < half) kr = k[d] * cs[d].x - k[d + half] * cs[d].y;
-    else if (d < 2 * half) kr = k[d - half] * cs[d - half].y + k[d] * cs[d - half].x;
+    if (d < half) kr = rope_low(k[d], k[d + half], cs[d]);
+    else if (d < 2 * half) kr = rope_high(k[d - half], k[d], cs[d - half]);
     kc[(static_cast<size_t>(pos) * num_kv + kvh) * hd + d] = __float2half_rn(kr);
     vc[((static_cast<size_t>(pos >> 3) * num_kv + kvh) * hd + d) * 8 + (pos & 7)] =
         __float2half_rn(row[q_dim + kv_dim + j]);
@@ -181,7 +181,7 @@ __device__ __forceinline__ double block_sum_d(double ss, double* red) {
 //   POST: y = (y / rms(y)) * (poff + pw)                             (resid_norm_rows_kernel);
 //   h = (hin + y) * scale, or hin itself without a projection        (add_rows_kernel);
 //   x = norm ? (h * (1 / rms(h))) * (off + w) : h                    (rmsnorm_rows_kernel);
-// h to hout, x to xn (each if given), and x's statistics and packed operands (if st.xe).
+// h to hout (if given), x as its statistics and packed operands (if st.xe).
 // NT threads: 256 where there are rows enough to fill the GPU, else 1024 (fewer elements per thread
 // to wait for in turn: 9.3 -> 7.3 us per launch at 24 rows of 4096; 11.2 -> 13.0 at 512 rows).
 template <int NT, bool POST>
@@ -273,7 +273,6 @@ __global__ __launch_bounds__(NT) void resid_norm_stats_rows_kernel(ResidRows a) 
                 const int i = c0 + t + NT * q;
                 if (i < n) {  // (the thread's own elements of `row`: no barrier needed)
                     const float x = a.w ? (row[i] * inv) * (a.off + wv[q]) : row[i] * inv;
-                    if (a.xn) a.xn[r + i] = x;
                     row[i] = x;
                     m = fmaxf(m, fabsf(x));
                 }
@@ -283,12 +282,10 @@ __global__ __launch_bounds__(NT) void resid_norm_stats_rows_kernel(ResidRows a) 
     if (a.st.xe) lds_row_out<NT>(row, n, ri, m, wm, a.st);
 }
 
-// act = act(gate) * up over a row of n outputs (1024 threads), from gate/up rows with the pairs
-// interleaved (as gated_pair_rows_kernel; K-split partial products summed in split order) or, with
-// U, from separate rows (gated_mul_kernel); to act if given, with its statistics and packed
-// operands for the down projection.
+// act(gate) * up over a row of n outputs (1024 threads) from gate/up rows with the pairs interleaved
+// (as gated_pair_rows_kernel; K-split partial products summed in split order): its statistics and
+// packed operands for the down projection.
 __global__ __launch_bounds__(1024) void gated_stats_rows_kernel(const float* __restrict__ G, size_t pstride, int splits,
-                                                                const float* __restrict__ U, float* __restrict__ act,
                                                                 int M, int n, int kind, GemmRowStats st) {
     constexpr int kChunk = 8;
     __shared__ __align__(16) float row[kFusedRowMax];
@@ -299,41 +296,32 @@ __global__ __launch_bounds__(1024) void gated_stats_rows_kernel(const float* __r
     float m = 0.f;
     for (int c0 = 0; c0 < n; c0 += 1024 * kChunk) {
         float2 v[kChunk];
-        if (U) {
 #pragma unroll
-            for (int q = 0; q < kChunk; q++) {
-                const size_t i = r + min(c0 + t + 1024 * q, n - 1);
-                v[q] = make_float2(G[i], U[i]);
-            }
-        } else {
+        for (int q = 0; q < kChunk; q++) v[q] = reinterpret_cast<const float2*>(G)[r + min(c0 + t + 1024 * q, n - 1)];
+        for (int z = 1; z < splits; z += 2) {
+            float2 p[2][kChunk];
 #pragma unroll
-            for (int q = 0; q < kChunk; q++) v[q] = reinterpret_cast<const float2*>(G)[r + min(c0 + t + 1024 * q, n - 1)];
-            for (int z = 1; z < splits; z += 2) {
-                float2 p[2][kChunk];
+            for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int k = 0; k < 2; k++)
+                for (int q = 0; q < kChunk; q++)
+                    p[k][q] = reinterpret_cast<const float2*>(G + min(z + k, splits - 1) * pstride)[r + min(c0 + t + 1024 * q, n - 1)];
 #pragma unroll
-                    for (int q = 0; q < kChunk; q++)
-                        p[k][q] = reinterpret_cast<const float2*>(G + min(z + k, splits - 1) * pstride)[r + min(c0 + t + 1024 * q, n - 1)];
+            for (int k = 0; k < 2; k++)
+                if (z + k < splits)
 #pragma unroll
-                for (int k = 0; k < 2; k++)
-                    if (z + k < splits)
-#pragma unroll
-                        for (int q = 0; q < kChunk; q++) v[q].x += p[k][q].x, v[q].y += p[k][q].y;
-            }
+                    for (int q = 0; q < kChunk; q++) v[q].x += p[k][q].x, v[q].y += p[k][q].y;
         }
 #pragma unroll
         for (int q = 0; q < kChunk; q++) {
             const int i = c0 + t + 1024 * q;
             if (i < n) {
                 const float x = gated_act(kind, v[q].x, v[q].y);
-                if (act) act[r + i] = x;
                 row[i] = x;
                 m = fmaxf(m, fabsf(x));
             }
         }
     }
-    if (st.xe) lds_row_out<1024>(row, n, ri, m, wm, st);
+    lds_row_out<1024>(row, n, ri, m, wm, st);
 }
 
 unsigned blocks(size_t n) { return static_cast<unsigned>((n + 255) / 256); }
@@ -401,14 +389,13 @@ void launch_resid_norm_stats_rows(const ResidRows& a, hipStream_t s) {
     LARQL_HIP_CHECK(hipGetLastError());
 }
 
-void launch_gated_stats_rows(const float* G, size_t pstride, int splits, const float* U, float* act, size_t m, size_t n,
-                             int kind, const GemmRowStats& st, hipStream_t s) {
+void launch_gated_stats_rows(const float* G, size_t pstride, int splits, size_t m, size_t n, int kind,
+                             const GemmRowStats& st, hipStream_t s) {
     if (m == 0) return;
-    if (m > 0x7FFFFF00 || splits < 1 || (U && splits != 1) || n % 32 != 0 || n > static_cast<size_t>(kFusedRowMax) ||
-        (st.xp && !st.xe))
+    if (m > 0x7FFFFF00 || splits < 1 || n % 32 != 0 || n > static_cast<size_t>(kFusedRowMax) || !st.xe)
         fail(LARQL_HIP_ERR_INVALID, "fused gated rows: bad arguments");
-    gated_stats_rows_kernel<<<tile_rows_grid(m), dim3(1024), 0, s>>>(G, pstride, splits, U, act, static_cast<int>(m),
-                                                                   static_cast<int>(n), kind, st);
+    gated_stats_rows_kernel<<<tile_rows_grid(m), dim3(1024), 0, s>>>(G, pstride, splits, static_cast<int>(m),
+                                                                     static_cast<int>(n), kind, st);
     LARQL_HIP_CHECK(hipGetLastError());
 }
 

@@ -304,31 +304,35 @@ def test_decode_q8_attention_q4_0_ffn(hip, formats, variant):
     run_sequence(hip, T0=21, n_tokens=2, n_layers=2, formats=formats, variant=variant)
 
 
-# Formats of Q8_0 / Q4_0 layers: all projections, separate Q / K / V beside Q4_K, gate and up in
-# different formats with a Q8_0 down.
+# Q8_0 / Q4_0 layers, as (seq, formats, variant, geometry): all projections, Q / K / V and gate / up in
+# two formats, a Q8_0 down, post-norms; layers mixed with Q4_K and Q6_K (position by position).
 Q8_ATTN_Q4_FFN = {n: "q8_0" for n in ("wq", "wk", "wv", "wo")} | {n: "q4_0" for n in ("gate", "up", "down")}
-Q8_PROMPTS = [(2, Q8_ATTN_Q4_FFN, None), (17, Q8_ATTN_Q4_FFN, None), (49, Q8_ATTN_Q4_FFN, None),
-              (18, {"wq": "q8_0", "wv": "q8_0", "wk": "q6_k", "down": "q4_0"}, None),
-              (33, {"wq": "q8_0", "wo": "q4_0", "gate": "q8_0", "up": "q4_0", "down": "q8_0"}, None),
-              (16, {"gate": "q8_0", "up": "q8_0", "down": "q6_k"}, None),
-              (20, Q8_ATTN_Q4_FFN, dict(has_post_norms=True, norm_offset=1.0, activation="gelu_tanh", layer_scalar=0.5))]
+POST_NORMS = dict(has_post_norms=True, norm_offset=1.0, activation="gelu_tanh", layer_scalar=0.5)
+Q8_PROMPTS = [(2, {}, None, {}), (17, {}, None, {}), (49, {}, None, {}), (70, {}, None, {}),
+              (18, {"wv": "q4_0"}, None, {}), (18, {"wk": "q4_0", "up": "q8_0"}, None, {}),
+              (33, {"wo": "q4_0", "gate": "q8_0", "down": "q8_0"}, None, {}), (20, {}, POST_NORMS, {}),
+              (20, {}, POST_NORMS | dict(ffn_norm_weights=False, has_v_norm=True, rotary_dim=32), {}),
+              (18, {"wk": "q6_k", "gate": "q4_k", "up": "q4_k"}, None, {}),
+              # a sliding window; rows of one block past a 64-block run; rows of more than 16384;
+              # head_dim 256 and 8 query heads per kv head
+              (90, {}, None, dict(window=37)), (21, {}, None, dict(inter=2080)), (9, {}, None, dict(inter=16640, hidden=256)),
+              (70, {}, None, dict(nq=8, nkv=1, hd=32)), (66, {}, None, dict(nq=2, nkv=1, hd=256)),
+              # more positions than run through a layer at once; positions whose decode step takes
+              # two chunks per attention workgroup
+              (1031, {}, None, dict(hidden=256, inter=512, nq=4, nkv=2)),
+              (530, {}, None, dict(hidden=256, inter=256, nq=64, nkv=64, hd=32))]
 
 
-@pytest.mark.parametrize("seq,formats,variant", Q8_PROMPTS)
-def test_prefill_q8_q4_0_layers(hip, seq, formats, variant):
-    """prefill_q4 of Q8_0 / Q4_0 layers, every position at once: against the oracle layers and
-    against decoding the prompt token by token, then the next decode_token.  The attention sums in
-    another order than the decode kernel's, so an activation next to a rounding tie may take the
-    neighbouring Q8 code: a step of max|x| / 127 in one of 512 elements, ~3 sigma / 127 of sqrt(512)
-    sigma = 1e-3 of that input, and half a dozen quantized inputs over the two layers add in
-    quadrature: 3e-3 of the output's scale.  A post-norm layer norms each branch's output before its
-    residual add, which scales a flip's share of a weak branch up with it: decoding such a model
-    step by step is itself up to 8.3e-3 from the oracle (seeds 78 .. 82); twice that."""
-    tol = 1.7e-2 if variant else 3e-3
-    n_layers, hidden, inter, nq, nkv, hd = 2, 512, 1024, 8, 2, 64
-    print(f"[prefill q8] seq={seq} formats={formats} variant={variant}", flush=True)
-    m = SmallModel(n_layers, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=78, formats=formats, variant=variant)
-    layers = m.hip_layers(10000.0)
+@pytest.mark.parametrize("seq,formats,variant,geom", Q8_PROMPTS)
+def test_prefill_q8_q4_0_layers(hip, seq, formats, variant, geom):
+    """prefill_q4 of Q8_0 / Q4_0 layers, a block of positions at once: every hidden state and the next
+    decode_token are those of decoding the prompt token by token, bit for bit."""
+    g = dict(n_layers=2, hidden=512, inter=1024, nq=8, nkv=2, hd=64) | geom
+    window = g.pop("window", 0)
+    hidden, inter, nq, nkv, hd = (g[k] for k in ("hidden", "inter", "nq", "nkv", "hd"))
+    print(f"[prefill q8] seq={seq} formats={formats} variant={variant} {geom}", flush=True)
+    m = SmallModel(**g, cap=seq + 2, seed=78, formats=Q8_ATTN_Q4_FFN | formats, variant=variant)
+    layers = m.hip_layers(10000.0, window)
     x = np.stack([oracle.gauss(8100 + p, hidden) for p in range(seq)])
     args = (hidden, inter, nq * hd, nkv * hd)
     hip.reset_kv_cache()
@@ -339,17 +343,42 @@ def test_prefill_q8_q4_0_layers(hip, seq, formats, variant):
     hip.reset_kv_cache()
     step = np.stack([hip.decode_token(layers, x[p], *args, nq, nkv, hd, 10000.0) for p in range(seq)])
     after_step = hip.decode_token(layers, nxt, *args, nq, nkv, hd, 10000.0)
-    ref = []
     for p in range(seq):
-        h = x[p].copy()
+        assert np.array_equal(got[p].view(np.uint32), step[p].view(np.uint32)), (p, rel_err(got[p], step[p]))
+    assert np.array_equal(after.view(np.uint32), after_step.view(np.uint32))
+
+
+@pytest.mark.parametrize("qk_norm,softcap", [(True, 0.0), (False, 1.5), (True, 1.5)])
+def test_prefill_q8_q4_0_attention_options(hip, qk_norm, softcap):
+    """use_qk_norm and softcap of a Q8_0 / Q4_0 prompt: position p is the last position of the prompt cut
+    there, bit for bit (one position is a decode step with the same options), and follows the
+    oracle's layers: their sums' order may flip a Q8 code next to a tie (3e-3 of the output: a step of
+    max|x| / 127, ~3 sigma / 127 of sqrt(512) sigma, 1e-3 of its input, half a dozen quantized inputs
+    in quadrature)."""
+    n_layers, hidden, inter, nq, nkv, hd, seq = 2, 512, 1024, 8, 2, 64, 70
+    print(f"[prefill q8 options] qk_norm={qk_norm} softcap={softcap}", flush=True)
+    m = SmallModel(n_layers, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=84, formats=Q8_ATTN_Q4_FFN,
+                   variant=dict(attn_scale=0.25))
+    for L in m.layers:
+        L.update(qk_norm=qk_norm, softcap=softcap, attn_scale=0.25)
+    layers = m.hip_layers(10000.0)
+    for hl in layers:
+        hl.attn_scale = 0.25
+    x = np.stack([oracle.gauss(880 + p, hidden) for p in range(seq)])
+
+    def prompt(n):
+        hip.reset_kv_cache()
+        return hip.prefill_q4(layers, x[:n], hidden, inter, nq * hd, nkv * hd, n, nq, nkv, hd, 10000.0,
+                              use_qk_norm=qk_norm, softcap=softcap)
+
+    got = prompt(seq)
+    for n in (1, 2, 16, 64, 65):
+        assert np.array_equal(prompt(n).view(np.uint32), got[:n].view(np.uint32)), n
+    for p in range(seq):
+        ref = x[p].copy()
         for L in m.layers:
-            h = oracle.decode_layer(L, h, p, hidden, inter, nq, nkv, hd, 10000.0)
-        ref.append(h)
-    e_ref = max(rel_err(got[p], ref[p]) for p in range(seq))
-    e_step = max(rel_err(got[p], step[p].astype(np.float64)) for p in range(seq))
-    e_next = rel_err(after, after_step.astype(np.float64))
-    print(f"  oracle {e_ref:.2e}, step by step {e_step:.2e}, next token {e_next:.2e}", flush=True)
-    assert e_ref <= tol and e_step <= tol and e_next <= tol
+            ref = oracle.decode_layer(L, ref, p, hidden, inter, nq, nkv, hd, 10000.0)
+        assert rel_err(got[p], ref) <= 3e-3, p
 
 
 @pytest.mark.parametrize("T0,hd,nq,nkv,window", [(4094, 64, 8, 8, 0), (4160, 64, 8, 8, 0), (8300, 32, 16, 8, 0),
