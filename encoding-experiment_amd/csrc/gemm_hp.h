@@ -44,9 +44,8 @@ __device__ __forceinline__ void hp_split8(const float (&v)[8], v4u& hi, v4u& lo)
 }
 
 // Packed operands XP[token tile][k-step][hi, lo][64 lanes][16 B]: lane 16 g + i of k-step ks
-// holds elements 32 ks + 8 g .. + 7 of token i of the tile times the token's power of two, the
-// odd ones divided by 16, in the order masks of a weight dword give its nibbles, (0, 4), (2, 6),
-// (1, 5), (3, 7): an odd element's nibble is left in place, 16 times its code.  The index of
+// holds elements 32 ks + 8 g .. + 7 of token i of the tile times the token's power of two, in the
+// order masks of a weight dword give its nibbles, (0, 4), (2, 6), (1, 5), (3, 7).  The index of
 // the hi part of token m's eight elements e8 = 4 ks + g; the lo part is 64 further.
 __device__ __forceinline__ size_t hp_packed_at(int m, int e8, int K) {
     return ((static_cast<size_t>(m >> 4) * (K / 32) + (e8 >> 2)) * 2) * 64 + 16 * (e8 & 3) + (m & 15);
@@ -55,8 +54,7 @@ __device__ __forceinline__ size_t hp_packed_at(int m, int e8, int K) {
 // Eight elements x[0 .. 7] times sc -> packed at o.
 __device__ __forceinline__ void hp_pack8(const float* x, float sc, v4u* o) {
     const floatx4 a = *reinterpret_cast<const floatx4*>(x), b = *reinterpret_cast<const floatx4*>(x + 4);
-    const float so = sc * 0.0625f;
-    const float e[8] = {a.x * sc, b.x * sc, a.z * sc, b.z * sc, a.y * so, b.y * so, a.w * so, b.w * so};
+    const float e[8] = {a.x * sc, b.x * sc, a.z * sc, b.z * sc, a.y * sc, b.y * sc, a.w * sc, b.w * sc};
     v4u hi, lo;
     hp_split8(e, hi, lo);
     o[0] = hi;

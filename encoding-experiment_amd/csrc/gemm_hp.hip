@@ -2,7 +2,8 @@
 // chains of projections of the prompt pass and for small batches (Q4_K and Q6_K).
 //
 // Every f32 activation x is split into two fp16 parts, hi = fp16(x) and lo = fp16(x - hi) (x -
-// hi exact in f32), x = hi + lo to ~2^-22, and the products run on v_mfma_f32_16x16x32_f16 with
+// hi exact in f32), x = hi + lo to ~2^-22 of x or 2^-40 of the row's largest element, whichever is
+// more (lo's smallest step), and the products run on v_mfma_f32_16x16x32_f16 with
 // f32 accumulation against fp16 weight operands that are exact integers.  Single fp16 operands
 // (2^-11) compounded past the 1e-3 bar through 8 and 16 layers; bf16 pairs (2^-16 per product)
 // doubled the error.  fp16's range is made safe per token: the row statistics hold the power of
@@ -48,7 +49,7 @@ __global__ __launch_bounds__(256) void x_pack_kernel(const float* __restrict__ X
     const float sc = m < M ? ldexpf(1.0f, xe[mc]) : 0.0f;
     float e[8] = {a.x, b.x, a.z, b.z, a.y, b.y, a.w, b.w};
 #pragma unroll
-    for (int k = 0; k < 8; k++) e[k] = m < M ? e[k] * (k < 4 ? sc : sc * 0.0625f) : 0.0f;
+    for (int k = 0; k < 8; k++) e[k] = m < M ? e[k] * sc : 0.0f;
     v4u hi, lo;
     hp_split8(e, hi, lo);
     v4u* o = XP + hp_packed_at(m, 4 * ks + g, K);
@@ -109,7 +110,7 @@ __device__ __forceinline__ void read_a(uint32_t a, int t, v4u (&h)[TT], v4u (&l)
 }
 
 // The eight codes of a nibble dword as fp16 pairs, code times 2^-24 (elements 0, 4, 2, 6) or 2^-20
-// (1, 5, 3, 7): a nibble in the low byte of a half is a subnormal, kept by the matrix cores.
+// (1, 5, 3, 7): a nibble in the low byte of a half is a subnormal, exact in an fp16 product.
 __device__ __forceinline__ void nibble_pairs(uint32_t w, f16x2 (&o)[4]) {
     const uint32_t w8 = w >> 8;
     o[0] = __builtin_bit_cast(f16x2, w & 0x000F000Fu);
@@ -144,12 +145,13 @@ struct PkArgs {
     int M, N, K, ntiles, mtiles, sb_per, ldy, gx, gy, gz;
 };
 
-// Bound: issue, MFMA plus the VALU between (1.9 per MFMA at four token tiles, 7.5 at one), which add
-// up at any number of waves.  Measured, Q4_K [28672 x 4096] (kernel trace): 512 tokens 258 us (466
+// Measured, Q4_K [28672 x 4096] (kernel trace): 512 tokens 258 us (466
 // TFLOP/s; 311 us when each workgroup split f32 tokens into pairs itself and one wave per SIMD
-// waited for its own loads and LDS reads), 24 tokens 30 us (the call 83 us on the fp16 GEMM).  Two
-// 8B-shape layers at 512 tokens took 1205 us with the codes made fp16 integers by a byte permute and
-// an fma per pair, 1133 with the masks.
+// waited for its own loads and LDS reads), 24 tokens 30 us (the call 83 us on the fp16 GEMM).  The
+// codes by masks take 13 VALU per eight weights; made fp16 integers by a byte permute and an fma per
+// pair, 14 (two 8B-shape layers, 512 tokens: 1137 us against 1164; bit-identical).  Left subnormal
+// (11 VALU), the codes cost the sums of the matrix cores three bits: 1.9e-6 from 64 bits at K =
+// 4096 against 2.3e-7, at the same speed.
 //
 // 16 TT tokens x 256 weight rows per workgroup: wave w owns 64 rows (kPkR tiles), all waves
 // share the token operands.  A unit is 128 k (half a super-block, four k-steps of one 32-element
@@ -158,8 +160,7 @@ struct PkArgs {
 //
 // Q4_K: w = d s_j q - dmin m_j, so per super-block and token
 //   sum_k x_k w_k = d sum_j s_j (sum_{k in j} x_k q_k) - dmin sum_j m_j X_j,  X_j = sum_{k in j} x_k.
-// s_j q <= 945 (times 2^-24: the codes are read as fp16 subnormals, an and-mask per two of them)
-// is exact in fp16, the weight operand of both products (x hi and lo, both
+// s_j q <= 945 is exact in fp16, the weight operand of both products (x hi and lo, both
 // exact in f32; only the split's 2^-22 is lost), a fresh accumulator per super-block, added into
 // the total times d.  The min term follows the K loop: the sub-block sums X_j 2^(e - 5) against
 // -32 dmin m_j per row, both as fp16 pairs (three products), 32 sub-blocks per k-step.  A lane's
@@ -172,8 +173,8 @@ template <int FMT, int TT>
 __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
     constexpr bool kQ4K = FMT == LARQL_Q4_K, kQ6K = FMT == LARQL_Q6_K;
     static_assert(kQ4K || kQ6K, "Q4_K or Q6_K");
-    // an operand's unit: codes times 2^-24; Q6_K weights at a quarter
-    constexpr float kUnit = kQ6K ? 4.0f : 16777216.0f;
+    // an operand's unit: Q4_K s_j q times 2^-14, Q6_K weights at a quarter
+    constexpr float kUnit = kQ6K ? 4.0f : 16384.0f;
     // weight loads per wave of a unit of each parity
     constexpr int kWLoads0 = (kQ6K ? 4 : 2) * kPkR, kWLoads1 = 2 * kPkR;
     __shared__ __align__(1024) v4u As[2][TT * 8 * 64];
@@ -317,27 +318,29 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
                         f16x2{1024.0f16, 1024.0f16};
                     f16x2 q[4];
                     nibble_pairs(word, q);
-                    B = operand8(q[0] * sv, q[1] * sv, q[2] * sv, q[3] * sv);
+                    // (2^10 times, so that no operand but zero is subnormal; odd codes are 16 times theirs)
+                    const f16x2 se = sv * f16x2{1024.0f16, 1024.0f16}, so = sv * f16x2{64.0f16, 64.0f16};
+                    B = operand8(q[0] * se, q[1] * se, q[2] * so, q[3] * so);
                 } else {
                     const uint32_t hb = nh[j][t] >> (4 * (g & 1));
                     const uint32_t lo = (word & 0x0F0F0F0Fu) | ((hb & 0x03030303u) << 4);
                     const uint32_t hi = ((word >> 4) & 0x0F0F0F0Fu) | (((hb >> 2) & 0x03030303u) << 4);
                     // the scale of this lane's 16-element group: byte 2 h + g / 2 of lane group t's
-                    // word; even elements at a quarter, odd ones at four times the weight
+                    // word, the weights at a quarter
                     const int scw = __builtin_amdgcn_ds_bpermute(4 * (16 * t + c), static_cast<int>(sc6[j]));
                     const _Float16 sf = static_cast<_Float16>(static_cast<int8_t>(scw >> (16 * h + 8 * (g >> 1))));
-                    const f16x2 se = f16x2{sf, sf} * f16x2{0.25f16, 0.25f16}, so = f16x2{sf, sf} * f16x2{4.0f16, 4.0f16};
+                    const f16x2 sv = f16x2{sf, sf} * f16x2{0.25f16, 0.25f16};
                     f16x2 bh[4], bl[4];
-                    auto pr = [&](uint32_t codes, uint32_t sel, f16x2 sv, f16x2& oh, f16x2& ol) __attribute__((always_inline)) {
+                    auto pr = [&](uint32_t codes, uint32_t sel, f16x2& oh, f16x2& ol) __attribute__((always_inline)) {
                         const f16x2 q = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, codes, sel)) -
                                         f16x2{1056.0f16, 1056.0f16};
                         oh = q * sv;
                         ol = __builtin_elementwise_fma(q, sv, -oh);
                     };
-                    pr(lo, 0x04020400u, se, bh[0], bl[0]);
-                    pr(lo, 0x04030401u, se, bh[1], bl[1]);
-                    pr(hi, 0x04020400u, so, bh[2], bl[2]);
-                    pr(hi, 0x04030401u, so, bh[3], bl[3]);
+                    pr(lo, 0x04020400u, bh[0], bl[0]);
+                    pr(lo, 0x04030401u, bh[1], bl[1]);
+                    pr(hi, 0x04020400u, bh[2], bl[2]);
+                    pr(hi, 0x04030401u, bh[3], bl[3]);
                     B = operand8(bh[0], bh[1], bh[2], bh[3]);
                     Bl = operand8(bl[0], bl[1], bl[2], bl[3]);
                 }

@@ -200,3 +200,75 @@ def test_q4k_small_batch_infinite_elements(hip):
             assert np.max(np.abs(got[t] - ref)) <= 1e-5 * np.max(np.abs(ref))
     finally:
         hip.release_weight(h)
+
+
+@pytest.mark.parametrize("cols,m", [(4096, 4), (14336, 17), (2048, 40)])
+def test_q4k_f32_gemm_keeps_f32_accuracy(hip, cols, m):
+    """Ordinary tokens and weights through the f32-accuracy GEMM: 4e-7 of the output's norm (the pair's
+    2^-22, and f32 sums: a few 2^-24 of terms about three times the weights, whose codes and minima
+    are multiplied apart).  Operands below fp16's normal range cost the matrix cores' sums 1.9e-6 at
+    4096."""
+    torch = pytest.importorskip("torch")
+    rows = 512
+    b = oracle.quantize_q4_k(oracle.gauss(103, rows * cols, 0.0, 0.02))
+    x = oracle.gauss(104, m * cols).reshape(m, cols)
+    h = hip.register_weight(larql_hip.Q4_K, b, rows, cols)
+    try:
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dx, dy, m=m)
+        hip.synchronize()
+        ref = x.astype(np.float64) @ _q4k_values(b, rows, cols).T
+        e = np.linalg.norm(dy.cpu().numpy().reshape(m, rows) - ref) / np.linalg.norm(ref)
+        print(f"[f32 gemm] cols={cols} m={m}: {e:.2e}", flush=True)
+        assert e <= 4e-7
+    finally:
+        hip.release_weight(h)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("col", [518, 519])
+def test_f32_gemm_rows_with_an_outlier(hip, fmt, col):
+    """A token whose largest element (1e6, ordinary ones ~1) meets only zero weights: the elements are
+    held to 2^-24 in units that put the largest in [2^14, 2^15), here 2^-19, at even and odd
+    positions alike, so the error grows over the same token's without it by 2^-19 / sqrt(12) =
+    5.5e-7 of the output's norm; twice that."""
+    torch = pytest.importorskip("torch")
+    rows, cols, m = 256, 4096, 4
+    w = oracle.gauss(101, rows * cols, 0.0, 0.02)
+    sb, e = divmod(col, 256)
+    if fmt == "q4_k":
+        b = oracle.quantize_q4_k(w).reshape(rows, cols // 256, 148).copy()
+        b[:, :, 2:4] = 0                                    # no minima (their sums have a step of their own)
+        b[:, sb, 20 + e // 2] &= 0x0F if e % 2 else 0xF0    # code 0
+        W = _q4k_values(b, rows, cols)
+    else:
+        b = oracle.quantize_q6_k(w).reshape(rows, cols // 256, 210).copy()
+        b[:, sb, e // 2] &= 0x0F if e % 2 else 0xF0         # code 32: nibble 0, high bits 2
+        b[:, sb, 128 + e // 4] = (b[:, sb, 128 + e // 4] & (0xFF ^ (3 << (2 * (e % 4))))) | (2 << (2 * (e % 4)))
+        p = b.reshape(-1, 210)
+        q = np.stack([p[:, :128] & 15, p[:, :128] >> 4], -1).reshape(-1, 256).astype(np.float64)
+        q += 16.0 * np.stack([(p[:, 128:192] >> (2 * i)) & 3 for i in range(4)], -1).reshape(-1, 256) - 32.0
+        d = p[:, 208:210].copy().view(np.float16).astype(np.float64)
+        W = (q.reshape(-1, 16, 16) * (p[:, 192:208].copy().view(np.int8) * d)[..., None]).reshape(rows, cols)
+    assert np.all(W[:, col] == 0)
+    x = oracle.gauss(102, m * cols).reshape(m, cols).copy()
+    h = hip.register_weight(larql_hip.Q4_K if fmt == "q4_k" else larql_hip.Q6_K, b.reshape(-1), rows, cols)
+
+    def error():
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dx, dy, m=m)
+        hip.synchronize()
+        ref = x.astype(np.float64) @ W.T
+        return np.linalg.norm(dy.cpu().numpy().reshape(m, rows) - ref) / np.linalg.norm(ref)
+
+    try:
+        x[:, col] = 1.0
+        plain = error()
+        x[:, col] = 1e6
+        outlier = error()
+        print(f"[outlier] {fmt} col={col}: {plain:.2e} -> {outlier:.2e}", flush=True)
+        assert outlier <= plain + 1.1e-6
+    finally:
+        hip.release_weight(h)
