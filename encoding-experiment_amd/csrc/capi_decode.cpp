@@ -728,7 +728,8 @@ uint64_t f32_bits(float v) {
 }
 
 // Cache key of a trait-call model: every field of every layer that build_model reads
-// (weights and norm vectors by pointer, length and sampled content; the scalars by value).
+// (weights, Q8_0 scales and norm vectors by pointer, length and sampled content; the scalars by
+// value).
 std::vector<uint64_t> layers_key(const larql_pipeline_layer* layers, size_t n, size_t hidden, size_t inter) {
     std::vector<uint64_t> k{n, hidden, inter};
     auto vec = [&](const float* v) {
@@ -737,11 +738,21 @@ std::vector<uint64_t> layers_key(const larql_pipeline_layer* layers, size_t n, s
     };
     for (size_t l = 0; l < n; l++) {
         const larql_pipeline_layer& L = layers[l];
-        for (const larql_quant_weight* w : {&L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down}) {
+        const size_t qd = L.num_q_heads * L.head_dim, kvd = L.num_kv_heads * L.head_dim;
+        const struct {
+            const larql_quant_weight* w;
+            size_t n;  // elements
+        } weights[] = {{&L.wq, qd * hidden},     {&L.wk, kvd * hidden},   {&L.wv, kvd * hidden},  {&L.wo, hidden * qd},
+                       {&L.gate, inter * hidden}, {&L.up, inter * hidden}, {&L.down, hidden * inter}};
+        for (const auto& [w, n] : weights) {
             k.push_back(reinterpret_cast<uint64_t>(w->data));
             k.push_back(w->len);
             k.push_back(static_cast<uint64_t>(w->format));
             k.push_back(w->data ? larql::host_fingerprint(w->data, w->len) : 0);
+            if (w->format == LARQL_Q8_0) {  // (a shorter buffer is refused when the model is built)
+                k.push_back(reinterpret_cast<uint64_t>(w->scales));
+                k.push_back(w->scales && w->len >= n ? larql::host_fingerprint(w->scales, n / 32 * sizeof(float)) : 0);
+            }
         }
         vec(L.input_norm);
         vec(L.post_attn_norm);

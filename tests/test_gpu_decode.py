@@ -348,6 +348,37 @@ def test_prefill_q8_q4_0_layers(hip, seq, formats, variant, geom):
     assert np.array_equal(after.view(np.uint32), after_step.view(np.uint32))
 
 
+def test_trait_calls_follow_changed_q8_scales(hip):
+    """Q8_0 codes are normalised by their block's maximum, so weights that differ by a factor have the same
+    codes and other scales: prefill_q4 and decode_token after scales changed in place, and with
+    another scale array for the same codes, are those of a context that never saw the old ones."""
+    n_layers, hidden, inter, nq, nkv, hd, seq = 1, 256, 512, 4, 2, 64, 3
+    m = SmallModel(n_layers, hidden, inter, nq, nkv, hd, cap=seq + 2, seed=91, formats=Q8_ATTN_Q4_FFN)
+    x = np.stack([oracle.gauss(890 + p, hidden) for p in range(seq + 1)])
+    args = (hidden, inter, nq * hd, nkv * hd)
+
+    def outputs(be):
+        be.reset_kv_cache()
+        layers = m.hip_layers(10000.0)
+        return np.vstack([be.prefill_q4(layers, x[:seq], *args, seq, nq, nkv, hd, 10000.0),
+                          be.decode_token(layers, x[seq], *args, nq, nkv, hd, 10000.0)])
+
+    def fresh():
+        be = larql_hip.HipBackend(0, strict=True)
+        try:
+            return outputs(be)
+        finally:
+            be.close()
+
+    first = outputs(hip)
+    m.layers[0]["wo_s"] *= np.float32(1.5)
+    second = outputs(hip)
+    assert np.array_equal(second, fresh()) and not np.array_equal(first, second)
+    m.layers[0]["wv_s"] = (m.layers[0]["wv_s"] * np.float32(0.5)).copy()
+    third = outputs(hip)
+    assert np.array_equal(third, fresh()) and not np.array_equal(second, third)
+
+
 @pytest.mark.parametrize("qk_norm,softcap", [(True, 0.0), (False, 1.5), (True, 1.5)])
 def test_prefill_q8_q4_0_attention_options(hip, qk_norm, softcap):
     """use_qk_norm and softcap of a Q8_0 / Q4_0 prompt: position p is the last position of the prompt cut
