@@ -476,46 +476,96 @@ __global__ __launch_bounds__(kPkThreads, 2) void pk_gemm_kernel(PkArgs a) {
         }
 }
 
-// The dot of weight row `row` (Q4_K) and x as a plain f32 sum: for a token with an infinite
-// element, whose packed operands give NaN although its products with nonzero weights are
-// infinite.
-__device__ __forceinline__ float q4k_plain_dot(const uint8_t* qs, const uint4* hdr, const float* x, int row, int K) {
-    const size_t S = static_cast<size_t>(K) / 256;
-    float acc = 0.f;
-#pragma unroll 1
-    for (size_t sb = 0; sb < S; sb++) {
-        const uint4 h = hdr[q4k_hdr_index(row, sb, S)];
-        const float d = h2f(h.x & 0xFFFFu), dmin = h2f(h.x >> 16);
-#pragma unroll 1
-        for (int j = 0; j < 8; j++) {
-            const float sc = d * static_cast<float>(((j < 4 ? h.y : h.z) >> (8 * (j & 3))) & 0x3Fu);
-            const float mn = dmin * static_cast<float>((h.w >> (8 * (j & 3) + 4 * (j >> 2))) & 0xFu);
-            const uint8_t* q = qs + q4k_sub_offset(row, sb, j, S);
-#pragma unroll 1
-            for (int b = 0; b < 16; b++) {
-                const float* xe = x + 256 * sb + 32 * j + 2 * b;
-                acc = fmaf(fmaf(sc, static_cast<float>(q[b] & 15), -mn), xe[0], acc);
-                acc = fmaf(fmaf(sc, static_cast<float>(q[b] >> 4), -mn), xe[1], acc);
-            }
-        }
-    }
-    return acc;
-}
-
-// Y = sum over the splits of the partial products, in split order (deterministic); four
-// splits' loads at a time.  N a multiple of V and rows aligned to V floats: V columns per thread.
-// PLAIN: an output that is not finite is summed again from the f32 inputs (q4k_plain_dot).
+// Weights of the token rows whose outputs are summed again from the f32 inputs: a token with an
+// infinite or NaN element, whose packed operands give NaN although its products with nonzero
+// weights are infinite, or one whose sum overflows on the way.
 struct PlainRows {
     const uint8_t* qs;
     const uint4* hdr;
     const float* X;
     int K;
 };
+
+__device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
+
+// Scale and minimum of sub-block j under header h (Q4_K).
+__device__ __forceinline__ float2 q4k_sub_scale(const uint4& h, int j) {
+    return make_float2(h2f(h.x & 0xFFFFu) * static_cast<float>(((j < 4 ? h.y : h.z) >> (8 * (j & 3))) & 0x3Fu),
+                       h2f(h.x >> 16) * static_cast<float>((h.w >> (8 * (j & 3) + 4 * (j >> 2))) & 0xFu));
+}
+
+// Products of the elements of x (row `x`, the wave's) that are not finite with V weight rows from
+// `col` on, summed; the finite elements change nothing.  found: whether there is one; odd: whether a
+// scale or minimum of the lane's weight rows is not finite (its rows need every product).  `live`: the
+// lane's outputs count.  All lanes of the wave call it.
+template <int V>
+__device__ __forceinline__ void q4k_infinite_products(const PlainRows& pl, const float* x, int col, bool live, float (&t)[V],
+                                                      bool& found, bool& odd) {
+    const int lane = threadIdx.x & 63, S = pl.K / 256;
+    found = odd = false;
+#pragma unroll
+    for (int k = 0; k < V; k++) t[k] = 0.f;
+    const float4* xp = reinterpret_cast<const float4*>(x) + lane;
+    float4 next = xp[0];
+    for (int sb = 0; sb < S; sb++) {
+        const float v[4] = {next.x, next.y, next.z, next.w};
+        next = xp[64 * min(sb + 1, S - 1)];
+#pragma unroll
+        for (int k = 0; k < V; k++) {
+            const uint32_t dm = pl.hdr[q4k_hdr_index(col + k, sb, S)].x;
+            odd |= (dm & 0x7C00u) == 0x7C00u || (dm & 0x7C000000u) == 0x7C000000u;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            for (uint64_t at = __builtin_amdgcn_ballot_w64(not_finite(v[e])); at; at &= at - 1) {
+                const int src = __builtin_ctzll(at), el = 4 * src + e, j = el >> 5;
+                const float xv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[e]), src));
+                found = true;
+                bool done = true;
+#pragma unroll
+                for (int k = 0; k < V; k++) {
+                    const float2 sc = q4k_sub_scale(pl.hdr[q4k_hdr_index(col + k, sb, S)], j);
+                    const uint32_t b = pl.qs[q4k_sub_offset(col + k, sb, j, S) + ((el & 31) >> 1)];
+                    t[k] = fmaf(fmaf(sc.x, static_cast<float>(el & 1 ? b >> 4 : b & 15u), -sc.y), xv, t[k]);
+                    done &= isnan(t[k]);
+                }
+                if (!__builtin_amdgcn_ballot_w64(live && !done)) return;  // (NaN stays NaN)
+            }
+        }
+    }
+}
+
+// The dot of weight row `row` and x as a plain f32 sum, by the whole wave (a sub-block per lane).
+__device__ __forceinline__ float q4k_plain_dot(const PlainRows& pl, const float* x, int row) {
+    const int S = pl.K / 256;
+    float acc = 0.f;
+    for (int b = threadIdx.x & 63; b < 8 * S; b += 64) {
+        const int sb = b >> 3, j = b & 7;
+        const float2 sc = q4k_sub_scale(pl.hdr[q4k_hdr_index(row, sb, S)], j);
+        const uint4 q = *reinterpret_cast<const uint4*>(pl.qs + q4k_sub_offset(row, sb, j, S));
+        const float* xe = x + 32 * b;
+#pragma unroll 1
+        for (int k = 0; k < 4; k++) {
+            uint32_t w = k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w;
+#pragma unroll
+            for (int i = 0; i < 8; i++, w >>= 4)
+                acc = fmaf(fmaf(sc.x, static_cast<float>(w & 15u), -sc.y), xe[8 * k + i], acc);
+        }
+    }
+    return wave_sum(acc);
+}
+
+// Y = sum over the splits of the partial products, in split order (deterministic); four
+// splits' loads at a time.  N a multiple of V and rows aligned to V floats: V columns per thread.
+// PLAIN: an output that is not finite is summed again from the f32 inputs, by its wave: one infinite
+// token of six, [14336 x 4096], 31 us the call (21 without; 1300 with a thread's serial sum for each
+// output), of four, [4096 x 14336], 55 us (25; 4550).
 template <int V, bool PLAIN>
 __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict__ Y, size_t n, int splits, int N,
                                   int ldy, PlainRows pl) {
-    const size_t i = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) * V;
-    if (i >= n) return;
+    const size_t i0 = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) * V;
+    if (!PLAIN && i0 >= n) return;
+    const size_t i = PLAIN ? (i0 < n ? i0 : n - V) : i0;  // (PLAIN: the last wave stays whole)
     typedef float fv __attribute__((ext_vector_type(V)));
     fv a = *reinterpret_cast<const fv*>(P + i);
     for (int z = 1; z < splits; z += 4) {
@@ -528,10 +578,30 @@ __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict
     }
     const size_t r = i / N, col = i % N;
     if constexpr (PLAIN) {
+        bool bad = false;
 #pragma unroll
-        for (int k = 0; k < V; k++)
-            if (!(fabsf(a[k]) <= 3.4028235e38f))
-                a[k] = q4k_plain_dot(pl.qs, pl.hdr, pl.X + r * pl.K, static_cast<int>(col) + k, pl.K);
+        for (int k = 0; k < V; k++) bad |= not_finite(a[k]);
+        uint64_t left = __builtin_amdgcn_ballot_w64(bad);
+        while (left) {  // a token row of the wave at a time
+            const uint32_t ru = __builtin_amdgcn_readlane(static_cast<uint32_t>(r), __builtin_ctzll(left));
+            const float* x = pl.X + static_cast<size_t>(ru) * pl.K;
+            const bool mine = bad && static_cast<uint32_t>(r) == ru;
+            left &= ~__builtin_amdgcn_ballot_w64(mine);
+            float t[V];
+            bool found, odd;
+            q4k_infinite_products<V>(pl, x, static_cast<int>(col), mine, t, found, odd);
+#pragma unroll
+            for (int k = 0; k < V; k++) {
+                if (mine && found && !odd && not_finite(a[k])) a[k] = t[k];
+                uint64_t each = __builtin_amdgcn_ballot_w64(mine && (!found || odd) && not_finite(a[k]));
+                for (; each; each &= each - 1) {
+                    const int src = __builtin_ctzll(each);
+                    const float y = q4k_plain_dot(pl, x, __builtin_amdgcn_readlane(static_cast<int>(col) + k, src));
+                    if ((threadIdx.x & 63) == src) a[k] = y;
+                }
+            }
+        }
+        if (i0 >= n) return;
     }
     *reinterpret_cast<fv*>(Y + r * ldy + col) = a;
 }

@@ -272,3 +272,74 @@ def test_f32_gemm_rows_with_an_outlier(hip, fmt, col):
         assert outlier <= plain + 1.1e-6
     finally:
         hip.release_weight(h)
+
+
+@pytest.mark.parametrize("rows,cols,m", [(4096, 4096, 4), (257, 14336, 5), (130, 4352, 3)])
+def test_q4k_small_batch_nonfinite_sums(hip, rows, cols, m):
+    """Tokens whose packed operands overflow, rows of any width: several infinities of either sign (each
+    output their products' sum: an infinity, or NaN where they disagree or meet a zero weight), a token
+    of infinities only, one whose largest element is next to f32's limit (finite outputs), beside
+    ordinary ones."""
+    torch = pytest.importorskip("torch")
+    b = oracle.quantize_q4_k(oracle.gauss(105, rows * cols, 0.0, 0.02))
+    W = _q4k_values(b, rows, cols)
+    x = oracle.gauss(106, m * cols).reshape(m, cols).copy()
+    x[0, [3, 700]] = np.inf
+    x[1, [9, 256]], x[1, 1029] = -np.inf, np.inf
+    x[2, 77] = np.float32(3.4025e38)
+    if m > 3:
+        x[3] = np.inf
+    h = hip.register_weight(larql_hip.Q4_K, b, rows, cols)
+    try:
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+        hip.matvec_dev(h, dx, dy, m=m)
+        hip.synchronize()
+        got = dy.cpu().numpy().reshape(m, rows)
+        for t in range(m):
+            inf = np.flatnonzero(np.isinf(x[t]))
+            if inf.size:
+                clear = np.all(np.abs(W[:, inf]) > 1e-6, 1) if inf.size < 9 else np.ones(rows, bool)
+                with np.errstate(invalid="ignore"):
+                    want = np.sum(np.sign(np.float32(W[:, inf])) * x[t, inf], 1)
+                np.testing.assert_array_equal(got[t][clear], want[clear].astype(np.float32))
+            else:   # (the plain sum's order: 2^-24 per term, random signs)
+                ref = x[t].astype(np.float64) @ W.T
+                assert np.max(np.abs(got[t] - ref)) <= 1e-5 * np.max(np.abs(ref)), t
+    finally:
+        hip.release_weight(h)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_q4k_small_batch_with_one_nonfinite_token_is_no_slow_path(hip, value):
+    """One infinite or NaN token among six costs its share of a pass over the weights' scales, not a
+    serial sum per output (30 times the call): less than three times the ordinary call."""
+    torch = pytest.importorskip("torch")
+    rows, cols, m = 14336, 4096, 6
+    h = hip.register_weight(larql_hip.Q4_K, oracle.quantize_q4_k(oracle.gauss(107, rows * cols, 0.0, 0.02)), rows, cols)
+    stream = torch.cuda.Stream()
+    out = torch.empty(m * rows, device="cuda", dtype=torch.float32)
+
+    def us(x):
+        dx = torch.from_numpy(x).cuda()
+        torch.cuda.synchronize()
+        best = np.inf
+        for _ in range(5):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record(stream)
+            for _ in range(10):
+                hip.matvec_dev(h, dx, out, m=m, stream=stream)
+            b.record(stream)
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best
+
+    try:
+        x = oracle.gauss(108, m * cols).reshape(m, cols).copy()
+        plain = us(x)
+        x[2, 1500] = value
+        other = us(x)
+        print(f"[nonfinite token] {value}: {plain:.1f} -> {other:.1f} us", flush=True)
+        assert other <= 3 * plain
+    finally:
+        hip.release_weight(h)
