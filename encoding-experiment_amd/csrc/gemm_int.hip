@@ -263,27 +263,43 @@ bool int_gemm_takes(const DevWeight& w) {
 }
 
 namespace {
-void launch_ig(IgArgs& a, int fmt, hipStream_t s) {
-    // Token tiles and weight tiles per wave: the least modelled time, rounds of workgroups over
-    // the CUs times a workgroup's VALU issue per block (16 per 16 x 16 tile, ~12 to unpack a
-    // weight tile, ~30 of loop, staging and waits)
-    const long cus = current_device_cus(), mt = (static_cast<long>(a.M) + 15) / 16;
-    int TT = 1, R = 1;
+// Token tiles and weight tiles per wave: the least modelled time, rounds of workgroups over
+// the CUs times a workgroup's VALU issue per block (16 per 16 x 16 tile, ~12 to unpack a
+// weight tile, ~30 of loop, staging and waits)
+struct IgPlan {
+    int TT, R;
+    long rounds;
+};
+IgPlan ig_plan(long ntiles, size_t m, int mats) {
+    const long cus = current_device_cus(), mt = (static_cast<long>(m) + 15) / 16;
+    IgPlan p{1, 1, 1};
     double best = -1;
     for (int r = 1; r <= 2; r++)
         for (int t = 1; t <= 4; t++) {
-            const long wgs = (a.ntiles + 4L * r - 1) / (4L * r) * ((mt + t - 1) / t) * a.gz;
+            const long wgs = (ntiles + 4L * r - 1) / (4L * r) * ((mt + t - 1) / t) * mats;
             const double cost = static_cast<double>((wgs + cus - 1) / cus) * (r * (16.0 * t + 12.0) + 30.0);
-            if (best < 0 || cost < best) best = cost, TT = t, R = r;
+            if (best < 0 || cost < best) best = cost, p = {t, r, (wgs + cus - 1) / cus};
         }
+    return p;
+}
+
+void launch_ig(IgArgs& a, int fmt, hipStream_t s) {
+    const auto [TT, R, rounds] = ig_plan(a.ntiles, static_cast<size_t>(a.M), a.gz);
     a.gx = (a.ntiles + 4 * R - 1) / (4 * R);
-    a.gy = static_cast<int>((mt + TT - 1) / TT);
+    a.gy = ((a.M + 15) / 16 + TT - 1) / TT;
     const unsigned grid = static_cast<unsigned>((static_cast<long>(a.gx) * a.gz + 7) / 8 * 8 * a.gy);
     if (fmt == LARQL_Q4_0) launch_fmt<LARQL_Q4_0>(a, TT, R, grid, s);
     else launch_fmt<LARQL_Q8_0>(a, TT, R, grid, s);
     LARQL_HIP_CHECK(hipGetLastError());
 }
 }  // namespace
+
+// Measured, rows 2048 .. 20000 (one matrix or two), 9 .. 33 activation rows: a line in the workgroup's
+// tiles per block and round.
+double int_gemm_us(const DevWeight& w, size_t m, int mats) {
+    const IgPlan p = ig_plan(static_cast<long>(w.rows_pad / 16), m, mats);
+    return 3.4 + static_cast<double>(w.cols / 32) * static_cast<double>(p.rounds) * (p.R * (16 * p.TT + 12) + 12.5) * 0.0031;
+}
 
 void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
                      float* out2, size_t m, size_t ldo, hipStream_t s) {

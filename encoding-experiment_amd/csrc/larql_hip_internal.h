@@ -303,6 +303,8 @@ constexpr int kIntGemmMats = LARQL_HIP_KNN_MAX_LAYERS;
 void launch_int_gemm_q4_layers(const void* const* nib, const void* const* scales, int layers, const int8_t* X8,
                                const float* XS, float* S, int F, int K, int Q, hipStream_t s);
 bool int_gemm_takes(const DevWeight& w);
+// The modelled time of m rows through one weight (or `mats` of its shape in one launch), microseconds.
+double int_gemm_us(const DevWeight& w, size_t m, int mats);
 void launch_int_gemm(const DevWeight& w, const DevWeight* w2, const int8_t* q8x, const float* q8s, float* out,
                      float* out2, size_t m, size_t ldo, hipStream_t s);
 void launch_q4_0_matvec(const DevWeight& w, const int8_t* q8x, const float* q8s, float* out,

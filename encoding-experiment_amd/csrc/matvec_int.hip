@@ -875,12 +875,30 @@ void launch_int_mv_batched(const DevWeight& w, const int8_t* q8x, const float* q
 }
 
 // One launch of the int GEMM instead of passes of up to 8 rows (a pass streams the weights
-// again).  Weights of fewer than 8192 rows are worth it above 16 activation rows: their few
-// workgroups leave one wave per SIMD, and a wave's chain of blocks then takes as long as two
-// passes (Q8_0 [4096 x 4096]: 16 rows 15.8 us in two passes, 20.1 in the GEMM; 64 rows 63.5
-// against 20.0; Q4_0 [14336 x 4096]: 9 rows 20.8 against 20.2, 128 rows 204 against 65 us).
-bool int_gemm_pays(const DevWeight& w, size_t m) {
-    return m > (w.rows >= 8192 ? 8u : 16u) && int_gemm_takes(w) && m <= 0x7FFFFFFF / w.cols;
+// again), where its modelled time is the shorter.  A wave of the GEMM is a chain over all blocks of
+// its row, so few workgroups take as long as many, and passes of 8 rows are cheap next to it up to
+// two or three of them (Q8_0 [8192 x 4096], 16 rows: 16.7 us in two passes, 20.5 in the GEMM; 17 rows
+// 25.0 and 21.4; two Q4_0 [10240 x 4096], 16 rows 27.9 and 33.4; 33 rows 62.8 and 56).  A pass of 8: its own
+// chain, or the weight's bytes at ~5.7 TB/s (Q8_0), and more workgroups than the GPU holds at once
+// (Q4_0, from ~24000 rows on); a single row left over: its bytes.  Of 1242 measured calls of 9 .. 48
+// rows two come out slower than by passes, by 4%.
+// Rows too long for 8 x images in LDS go through in passes of 4 or fewer: the GEMM from 8192
+// weight rows on, and above 16 activation rows below (Q8_0, 9 rows of [8192 x 8192]: 47 us in passes,
+// 36 in the GEMM; of [4096 x 8192] 30 in passes, 17 rows 50 and 37).
+bool int_gemm_pays(const DevWeight& w, size_t m, int mats = 1) {
+    if (m <= 8 || !int_gemm_takes(w) || m > 0x7FFFFFFF / w.cols) return false;
+    const size_t nb = w.cols / 32;
+    if (8 * nb * (32 + sizeof(float)) > kLdsLimit) return m > (w.rows >= 8192 ? 8u : 16u);
+    const bool q40 = w.format == LARQL_Q4_0;
+    const double rows = static_cast<double>(w.rows) * mats, blocks = static_cast<double>(nb);
+    const double mb = rows * blocks * (q40 ? 18 : 36) * 1e-6;
+    const double chain = q40 ? (2.3 + 0.079 * blocks) * std::max(1.0, rows / 24576.0)
+                             : std::max(2.5 + 0.047 * blocks, 1.0 + 0.175 * mb);
+    const size_t left = m % 8;
+    double passes = static_cast<double>(m / 8) * chain;
+    if (left == 1) passes += 1.5 + mb / 5.2;
+    else if (left) passes += q40 ? chain * (0.55 + 0.05625 * static_cast<double>(left)) : chain;
+    return int_gemm_us(w, m, mats) < passes;
 }
 
 }  // namespace
@@ -895,7 +913,7 @@ void launch_q4_0_matvec_pair(const DevWeight& w1, const DevWeight& w2, const int
                              float* out1, float* out2, size_t m, hipStream_t s) {
     if (w1.format != LARQL_Q4_0 || w2.format != LARQL_Q4_0 || w1.rows != w2.rows || w1.cols != w2.cols)
         fail(LARQL_HIP_ERR_INVALID, "q4_0 matvec pair: two Q4_0 matrices of one shape");
-    if (int_gemm_pays(w1, m)) return launch_int_gemm(w1, &w2, q8x, q8s, out1, out2, m, 0, s);
+    if (int_gemm_pays(w1, m, 2)) return launch_int_gemm(w1, &w2, q8x, q8s, out1, out2, m, 0, s);
     launch_int_mv_batched<LARQL_Q4_0>(w1, q8x, q8s, out1, m, s, &w2, out2);
 }
 

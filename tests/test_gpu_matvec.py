@@ -383,3 +383,59 @@ def test_read_floor_other_formats_explicit_shapes(hip):
     m = wq.copy()
     m[12345] ^= 0x04
     assert bin(folds(m)[0] ^ base[0]).count("1") == 1
+
+
+@pytest.mark.parametrize("fmt,rows,cols,m", [("q8_0", 8192, 4096, 16), ("q8_0", 8192, 5120, 9), ("q4_0", 20000, 5120, 9),
+                                             ("pair", 10240, 4096, 16), ("pair", 14336, 2560, 12)])
+def test_int_matvec_rows_not_slower_than_in_passes(hip, fmt, rows, cols, m):
+    """9 .. 17 activation rows in one call cost no more than the same rows in calls of up to 8 (the passes
+    that the int GEMM replaces where it is the faster: it took a quarter more here); 10% for noise."""
+    torch = pytest.importorskip("torch")
+    stream = torch.cuda.Stream()
+    g = torch.Generator(device="cuda").manual_seed(7)
+    n = rows * cols
+
+    def weight():
+        if fmt == "q8_0":
+            q = torch.randint(-127, 128, (n,), dtype=torch.int8, device="cuda", generator=g)
+            s = torch.rand(n // 32, device="cuda", generator=g) * 1e-3
+            torch.cuda.synchronize()
+            return hip.register_weight_device(larql_hip.Q8_0, q, n, rows, cols, s)
+        b = torch.randint(0, 256, (n // 32, 18), dtype=torch.uint8, device="cuda", generator=g)
+        b[:, 1] = 0x1C   # f16 scales of ordinary size
+        torch.cuda.synchronize()
+        return hip.register_weight_device(larql_hip.Q4_0, b.reshape(-1), b.numel(), rows, cols)
+
+    ws = [weight() for _ in range(2 if fmt == "pair" else 1)]
+    x = torch.randn(m, cols, device="cuda", generator=g)
+    x8 = torch.randint(-127, 128, (m, cols), dtype=torch.int8, device="cuda", generator=g)
+    xs = torch.rand(m, cols // 32, device="cuda", generator=g)
+    outs = [torch.empty(m, rows, device="cuda") for _ in ws]
+
+    def call(r0, r1):
+        if fmt == "pair":
+            hip.pair_batch_dev(ws[0], ws[1], x[r0:r1], r1 - r0, outs[0][r0:r1], outs[1][r0:r1], stream=stream)
+        else:
+            hip.matvec_dev(ws[0], x8[r0:r1], outs[0][r0:r1], m=r1 - r0, x_scales=xs[r0:r1], stream=stream)
+
+    def us(step):
+        best = np.inf
+        for _ in range(6):
+            torch.cuda.synchronize()
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record(stream)
+            for _ in range(20):
+                for r0 in range(0, m, step):
+                    call(r0, min(m, r0 + step))
+            b.record(stream)
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    try:
+        passes, one = us(8), us(m)
+        print(f"[int rows] {fmt} {rows}x{cols} m={m}: {one:.1f} us, in passes {passes:.1f}", flush=True)
+        assert one <= 1.1 * passes
+    finally:
+        for h in ws:
+            hip.release_weight(h)
