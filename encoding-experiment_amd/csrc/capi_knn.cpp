@@ -52,7 +52,7 @@ void run_scores(larql_hip_ctx* c, const KnnPlan& p, size_t n_layers, const float
     const int Q = static_cast<int>(nq);
     if (p.format == LARQL_F32) {
         // (scores into the caller's buffer use no work buffer of the context where none is needed)
-        const size_t nws = larql::gate_scores_f32_ws_floats(p.K, Q, own_scores);
+        const size_t nws = larql::gate_scores_f32_ws_floats(static_cast<int>(n_layers), p.F, p.K, Q, own_scores);
         float* ws = nws ? static_cast<float*>(larql::ensure(c, c->knn_xpad, nws * sizeof(float))) : nullptr;
         larql::launch_gate_scores_f32(p.a, static_cast<int>(n_layers), queries, ws, nws, scores, p.F, p.K, Q, s);
     } else {

@@ -19,7 +19,7 @@ struct KnnLayers {
 // or, if may_transpose and it pays, k-major (none where neither).
 void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, size_t ws_floats, float* S, int F,
                             int K, int Q, hipStream_t s);
-size_t gate_scores_f32_ws_floats(int K, int Q, bool may_transpose);
+size_t gate_scores_f32_ws_floats(int n_layers, int F, int K, int Q, bool may_transpose);
 // S[l][q][f] = sum_b (float)isum * (f16(scale) * XS[q][b]) in block order (Q4_0 x Q8).
 // XA / XSP: work buffers of q4_xa_bytes / q4_xsp_bytes (the queries as MFMA operands), unused
 // where gate_scores_q4_direct.

@@ -987,43 +987,58 @@ __global__ __launch_bounds__(64 * kWWaves) void topk_wave_kernel(const float* __
 
 }  // namespace
 
-// Queries per wave (qw, at most Q) and waves per workgroup (nw) of a walk of Q queries.  Few queries per
-// wave and more waves: a wave waits for its scalar loads every 16 k, and only other waves can
-// issue meanwhile (8 queries of one wave 1.78 ms, of four waves 0.84; 32 of four waves 1.87,
-// of eight 1.22; 64 of four waves 3.1, of eight 1.86).  Above 128 the tile kernel: 128 queries
-// cost 3.46 ms here and 4.9 there, 256 7.4 ms here and 5.3 there.
+// Queries per wave (qw, at most Q) and waves per workgroup (nw) of a walk of Q queries over `blocks`
+// workgroups of 64 features (all layers).  Few queries per wave and more waves: a wave waits for its
+// scalar loads every 16 k, and only other waves can issue meanwhile (34 x [10240 x 2560]: 8 queries of
+// one wave 1.78 ms, of four waves 0.70; 32 of four waves 1.87, of eight 1.15; 64 of four waves 3.1, of
+// eight 1.86).
+// 65 .. 128 queries: 16 of a wave where they come k-major (xt), else 8, except that walks of 1.5 to 2
+// workgroups per CU take the tile kernel: it computes 256 queries whatever their number, but its
+// workgroups all run at once (3 x [10240 x 1088], 480 workgroups, 128 queries: 206 us against 231 in
+// waves of 8; 6 x [3000 x 1152], 282: 214 against 163; 2 x [10240 x 2560], 320: 466 against 352; 34 layers,
+// 5440: 4.9 ms against 4.49 of 8 and 3.46 of 16).  Above 128 the tile kernel (256 queries of 34 layers 5.5 ms
+// against 7.4).
 namespace {
 struct F32Plan {
     int qw, nw;
 };
-F32Plan f32_plan(int Q) {
+F32Plan f32_plan(int Q, long blocks, bool xt) {
+    const long cus = current_device_cus();
     if (Q <= 2) return {Q, 1};
     if (Q <= 8) return {2, Q <= 4 ? 2 : 4};
     if (Q <= 32) return {4, Q <= 16 ? 4 : 8};
-    if (Q <= 128) return {Q <= 64 ? 8 : 16, 8};
+    if (Q <= 64) return {8, 8};
+    if (Q <= 128 && xt) return {16, 8};
+    if (Q <= 128 && (2 * blocks <= 3 * cus || blocks > 2 * cus)) return {8, 8};
     return {kF32TileQ, 1};  // the tile kernel
 }
-}  // namespace
+long f32_blocks(int n_layers, int F) { return (F + 63L) / 64 * n_layers; }
 
 // Queries k-major in a workspace, where one is given: above 32 queries a wave's 8 or 16 are then
 // one contiguous run per k (64 queries 1.86 against 2.31 ms as they lie, 128 queries 3.46 against
 // 4.49, 5.17 in tiles; 32 queries 1.22 against 1.15), and a tile's stage is copied as it lies (256
-// queries 5.50 against 5.62).
-static bool f32_transposed(int Q) { return Q > 32; }
-static size_t f32_transposed_floats(size_t Kp, int Q) { return Kp * (Q <= 128 ? 128 : (static_cast<size_t>(Q) + 255) / 256 * 256); }
+// queries 5.50 against 5.62).  In walks of fewer than two workgroups per CU the launch that transposes
+// costs more than it gives: with the top-k, 100 queries of 6 x [3000 x 1152] (282 workgroups) 236 us with
+// it and waves of 16, 176 without and of 8; of 3 x [10240 x 1088] (480) 229 and, in tiles, 220; 128 of
+// 8 x [4000 x 1024] (504) 187 and 213, 256 of 4 x [8000 x 1500] (500) 325 and 336.
+bool f32_transposed(int n_layers, int F, int Q) {
+    return Q > 32 && 10 * f32_blocks(n_layers, F) * ((Q + kF32TileQ - 1) / kF32TileQ) >= 19L * current_device_cus();
+}
+size_t f32_transposed_floats(size_t Kp, int Q) { return Kp * (Q <= 128 ? 128 : (static_cast<size_t>(Q) + 255) / 256 * 256); }
+}  // namespace
 
-size_t gate_scores_f32_ws_floats(int K, int Q, bool may_transpose) {
+size_t gate_scores_f32_ws_floats(int n_layers, int F, int K, int Q, bool may_transpose) {
     const size_t Kp = f32_row_stride(static_cast<size_t>(K));
-    if (may_transpose && f32_transposed(Q)) return f32_transposed_floats(Kp, Q);
+    if (may_transpose && f32_transposed(n_layers, F, Q)) return f32_transposed_floats(Kp, Q);
     return Kp == static_cast<size_t>(K) ? 0 : Kp * Q;
 }
 
 void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, float* ws, size_t ws_floats, float* S, int F,
                             int K, int Q, hipStream_t s) {
     const int Kp = static_cast<int>(f32_row_stride(static_cast<size_t>(K)));
-    F32Plan p = f32_plan(Q);
-    const bool xt = f32_transposed(Q) && ws && ws_floats >= f32_transposed_floats(static_cast<size_t>(Kp), Q);
-    if (!xt && Q > 64 && Q <= 128) p = {8, 8};
+    const bool xt =
+        f32_transposed(n_layers, F, Q) && ws && ws_floats >= f32_transposed_floats(static_cast<size_t>(Kp), Q);
+    const F32Plan p = f32_plan(Q, f32_blocks(n_layers, F), xt);
     const int per = p.qw * p.nw, gy = (Q + per - 1) / per;
     if (xt) {
         const int Qp = gy * per;

@@ -96,6 +96,69 @@ def test_gate_scores_f32_query_counts_bit_exact(hip, nq, features, hidden):
             hip.release_weight(h)
 
 
+@pytest.mark.parametrize("nq", [33, 64, 65, 100, 128, 129, 257])
+@pytest.mark.parametrize("features,hidden", [(1400, 48), (1345, 30)])
+def test_gate_knn_f32_large_walk_bit_exact(hip, nq, features, hidden):
+    """Walks of more than two workgroups of 64 features per CU, whose queries are put k-major first: every
+    score of 24 layers (two gates in turn; k beyond the selection kernels ranks whole rows), bit for
+    bit the oracle's chain."""
+    torch = pytest.importorskip("torch")
+    print(f"[knn f32 walk] F={features} K={hidden} nq={nq}", flush=True)
+    layers = 24
+    gates = [oracle.gauss(63 + l, features * hidden, 0.0, 0.02).reshape(features, hidden) for l in range(2)]
+    queries = oracle.gauss(65, nq * hidden).reshape(nq, hidden)
+    hs = [hip.register_weight(larql_hip.F32, g, features, hidden) for g in gates]
+    try:
+        dq = torch.from_numpy(queries).cuda()
+        idx = torch.empty(layers, nq, features, dtype=torch.int32, device="cuda")
+        val = torch.empty(layers, nq, features, device="cuda")
+        hip.gate_knn_dev(hs * (layers // 2), dq, nq, features, idx, val)
+        hip.synchronize()
+        i, v = idx.cpu().numpy(), val.cpu().numpy()
+        for l in range(2):
+            ref = np.stack([oracle.gate_scores_f32(gates[l], q, features, hidden) for q in queries])
+            order = np.argsort(-np.abs(ref), axis=1, kind="stable")
+            want = np.take_along_axis(ref, order, 1)
+            for m in range(l, layers, 2):
+                np.testing.assert_array_equal(i[m], order)
+                np.testing.assert_array_equal(v[m].view(np.uint32), want.view(np.uint32))
+    finally:
+        for h in hs:
+            hip.release_weight(h)
+
+
+@pytest.mark.parametrize("layers,features,hidden", [(3, 10240, 1088), (8, 4000, 1024), (6, 3000, 1152)])
+def test_gate_scores_f32_of_128_queries_cost_no_more_than_of_256(hip, layers, features, hidden):
+    """A tile of 256 queries computes all of them whatever their number, so 128 are never worth more."""
+    torch = pytest.importorskip("torch")
+    gate = torch.randn(features, hidden, device="cuda") * 0.02
+    torch.cuda.synchronize()
+    hs = [hip.register_weight_device(larql_hip.F32, gate, gate.numel() * 4, features, hidden) for _ in range(layers)]
+    stream = torch.cuda.Stream()
+    x, sc = torch.randn(256, hidden, device="cuda"), torch.empty(layers * 256 * features, device="cuda")
+
+    def us(nq):
+        best = np.inf
+        for _ in range(6):
+            torch.cuda.synchronize()
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record(stream)
+            for _ in range(40):
+                hip.gate_scores_dev(hs, x, nq, sc, stream=stream)
+            b.record(stream)
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 25)
+        return best
+
+    try:
+        half, full = us(128), us(256)
+        print(f"[scores f32] {layers} x [{features} x {hidden}]: 128 queries {half:.1f} us, 256 {full:.1f}", flush=True)
+        assert half <= full
+    finally:
+        for h in hs:
+            hip.release_weight(h)
+
+
 # hidden a multiple of 128 (the int GEMM; its tiles' edges) or of 64 only (the 128 x 128 tiles)
 @pytest.mark.parametrize("features,hidden,nq,k", [(10240, 2560, 6, 32), (1000, 2560, 130, 17), (64, 64, 2, 64),
                                                   (129, 384, 17, 32), (70, 128, 49, 5), (300, 192, 65, 32)])
