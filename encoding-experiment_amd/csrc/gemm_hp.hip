@@ -637,6 +637,11 @@ size_t align4(size_t n) { return (n + 3) & ~size_t{3}; }
 
 }  // namespace
 
+// Q4_K operands of 2 GiB and more (X in f32, the nibbles), which the GEMM refuses.
+static bool q4k_gemm_above_2gib(const DevWeight& w, size_t m) {
+    return w.format == LARQL_Q4_K && (m > 0x7FFFFFFF / (4 * w.cols) || w.rows_pad > 0x7FFFFFFF / (w.cols / 2));
+}
+
 size_t gemm_x_pack_floats(size_t m, size_t cols) { return (m + 15) / 16 * 16 * cols; }
 
 // workspace: the K-split partials (when split), and for a caller without row statistics and packed
@@ -699,7 +704,7 @@ void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowS
 // 6 tokens 30 against 125, 192 tokens 83 against 145; [10240 x 2560]: 32 tokens 22 against 28,
 // 64 tokens 31 against 28.
 bool gemm_f32_small_batch(const DevWeight& w, size_t m) {
-    if (w.format != LARQL_Q4_K || m < 2 || m > 512) return false;
+    if (w.format != LARQL_Q4_K || m < 2 || m > 512 || q4k_gemm_above_2gib(w, m)) return false;
     const size_t wgs = ((w.rows_pad / 16 + 4) / 5) * ((m + 255) / 256), cus = static_cast<size_t>(current_device_cus());
     const double other = 6500.0 + static_cast<double>((wgs + cus - 1) / cus) * static_cast<double>(w.cols / 256) * 2200.0;
     return 1.45 * pk_plan(w, m).ns + 8000.0 < other;
@@ -715,6 +720,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
         fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: incomplete row statistics");
     if (m == 0) return;
     if (m > 0x7FFFFFFF / w.cols) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: too many tokens");
+    if (q4k_gemm_above_2gib(w, m)) fail(LARQL_HIP_ERR_UNSUPPORTED, "f32 GEMM: operands above 2 GiB");
     const PkPlan p = pk_plan(w, m);
     if (plain && (w.format != LARQL_Q4_K || defer)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: plain sums of Q4_K outputs only");
     if (!part || part_floats < gemm_f32_part_floats(w, m, plain)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: workspace too small");

@@ -343,3 +343,24 @@ def test_q4k_small_batch_with_one_nonfinite_token_is_no_slow_path(hip, value):
         assert other <= 3 * plain
     finally:
         hip.release_weight(h)
+
+
+@pytest.mark.parametrize("m", [6, 700])
+def test_q4k_batches_above_2gib_are_refused(hip, m):
+    """Q4_K weights whose nibbles fill 2 GiB: both GEMMs of several rows say so, whatever the batch."""
+    torch = pytest.importorskip("torch")
+    rows, cols = 1048577, 4096
+    raw = torch.zeros(rows * (cols // 256) * 148, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    h = hip.register_weight_device(larql_hip.Q4_K, raw, raw.numel(), rows, cols)
+    del raw
+    try:
+        x = torch.ones(m, cols, device="cuda")
+        out = torch.empty(m, rows, device="cuda")
+        torch.cuda.synchronize()
+        with pytest.raises(larql_hip.LarqlHipError, match="2 GiB"):
+            hip.matvec_dev(h, x, out, m=m)
+    finally:
+        hip.synchronize()
+        hip.release_weight(h)
+        torch.cuda.empty_cache()
