@@ -5,6 +5,7 @@
 // failure into a negative status plus a message (larql_hip_last_error).  Nothing in
 // here falls back to a CPU computation: a failure is reported, and the caller decides
 // (the reference callers fall back to the CPU backend on None, LV/src/index/gate.rs:684-704).
+#include <algorithm>
 #include <atomic>
 #include <hip/hip_runtime.h>
 
@@ -297,17 +298,27 @@ extern "C" int larql_hip_q4k_matvec(larql_hip_ctx* c, const uint8_t* q4k_data, s
     });
 }
 
+// Workspace of a batch of m > 1 rows of a Q4_K weight: no less than any smaller batch's (whose K
+// splits may take more), so that it grows only with m.
+static size_t q4k_rows_ws(const DevWeight& w, size_t m) {
+    auto need = [&](size_t n) {
+        return larql::gemm_f32_small_batch(w, n) ? larql::gemm_f32_part_floats(w, n, true) * sizeof(float)
+                                                 : larql::q4k_gemm_ws_bytes(n, w.cols);
+    };
+    // (the fp16 GEMM's grows with m by itself)
+    for (; w.ws_m < std::min(m, larql::kSmallBatchMax); w.ws_m++) w.ws_bytes = std::max(w.ws_bytes, need(w.ws_m + 1));
+    return std::max(w.ws_bytes, need(m));
+}
+
 // m activation rows through a Q4_K weight: the matvec, the f32-accuracy GEMM for small batches,
 // the fp16 GEMM.
 static void q4k_rows(larql_hip_ctx* c, const DevWeight& w, const float* x, float* out, size_t m, hipStream_t s) {
-    if (larql::gemm_f32_small_batch(w, m)) {
-        const size_t pf = larql::gemm_f32_part_floats(w, m, true);
-        float* part = static_cast<float*>(larql::ensure(c, c->gemm_x16, pf * sizeof(float)));
-        larql::launch_gemm_f32(w, x, out, m, part, pf, s, 0, nullptr, nullptr, true);
-        return;
-    }
-    void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, larql::q4k_gemm_ws_bytes(m, w.cols)) : nullptr;
-    larql::launch_q4k_matvec(w, x, out, m, ws, s);
+    void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, q4k_rows_ws(w, m)) : nullptr;
+    if (larql::gemm_f32_small_batch(w, m))
+        larql::launch_gemm_f32(w, x, out, m, static_cast<float*>(ws), larql::gemm_f32_part_floats(w, m, true), s, 0, nullptr,
+                               nullptr, true);
+    else
+        larql::launch_q4k_matvec(w, x, out, m, ws, s);
 }
 
 extern "C" int larql_hip_q4k_matmul(larql_hip_ctx* c, const uint8_t* q4k_data, size_t q4k_len, const float* x,

@@ -704,7 +704,7 @@ void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowS
 // 6 tokens 30 against 125, 192 tokens 83 against 145; [10240 x 2560]: 32 tokens 22 against 28,
 // 64 tokens 31 against 28.
 bool gemm_f32_small_batch(const DevWeight& w, size_t m) {
-    if (w.format != LARQL_Q4_K || m < 2 || m > 512 || q4k_gemm_above_2gib(w, m)) return false;
+    if (w.format != LARQL_Q4_K || m < 2 || m > kSmallBatchMax || q4k_gemm_above_2gib(w, m)) return false;
     const size_t wgs = ((w.rows_pad / 16 + 4) / 5) * ((m + 255) / 256), cus = static_cast<size_t>(current_device_cus());
     const double other = 6500.0 + static_cast<double>((wgs + cus - 1) / cus) * static_cast<double>(w.cols / 256) * 2200.0;
     return 1.45 * pk_plan(w, m).ns + 8000.0 < other;

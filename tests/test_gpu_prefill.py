@@ -364,3 +364,44 @@ def test_q4k_batches_above_2gib_are_refused(hip, m):
         hip.synchronize()
         hip.release_weight(h)
         torch.cuda.empty_cache()
+
+
+def test_q4k_batch_workspace_grows_only_with_the_batch(hip):
+    """A context whose largest batch of a Q4_K weight has run allocates nothing for smaller ones, though
+    their K splits differ, so they record into a HIP graph; three replays with eager work between
+    them give the eager results."""
+    torch = pytest.importorskip("torch")
+    rows, cols, sizes = 14336, 4096, (2, 16, 33, 48, 64, 96)
+    be = larql_hip.HipBackend(0, strict=True)
+    h = be.register_weight(larql_hip.Q4_K, oracle.quantize_q4_k(oracle.gauss(109, rows * cols, 0.0, 0.02)), rows, cols)
+    try:
+        x = torch.from_numpy(oracle.gauss(110, 512 * cols).reshape(512, cols)).cuda()
+        out, ref = (torch.empty(512, rows, device="cuda") for _ in range(2))
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        be.matvec_dev(h, x, out, m=512, stream=side)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for m in sizes:
+            be.matvec_dev(h, x, ref, m=m, stream=side)
+            torch.cuda.synchronize()
+            assert torch.cuda.mem_get_info()[0] == free, m
+        for m in sizes:
+            print(f"[q4k graph] m={m}", flush=True)
+            be.matvec_dev(h, x, ref, m=m, stream=side)
+            torch.cuda.synchronize()
+            want = ref[:m].clone()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                be.matvec_dev(h, x, out, m=m, stream=side)
+            for _ in range(3):
+                out.fill_(7.0)
+                be.matvec_dev(h, x, ref, m=64, stream=side)
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out[:m], want)
+            del graph
+    finally:
+        be.synchronize()
+        be.close()
