@@ -955,7 +955,7 @@ PromptLayout prompt_layout(const larql_hip_model* m, size_t M) {
     const size_t hidden = m->hidden, inter = m->inter, qmax = m->q_dim;
     p.gw = std::max(hidden, 2 * inter);
     size_t part_n = 0;  // partials of attention shapes without the one-pass prompt kernel
-    auto need = [&](const DevWeight& w) { p.split = std::max(p.split, larql::gemm_f32_part_floats(w, M)); };
+    auto need = [&](const DevWeight& w) { p.split = std::max(p.split, larql::gemm_f32_part_floats(w, M, false, true)); };
     for (const LayerDev& L : m->layers) {
         if (!larql::attn_prompt_one_pass(L.nq / L.nkv, L.hd))
             part_n = m->part_per_split * larql::attn_prompt_splits(1, static_cast<int>(M), 0) * M;

@@ -644,12 +644,12 @@ static bool q4k_gemm_above_2gib(const DevWeight& w, size_t m) {
 
 size_t gemm_x_pack_floats(size_t m, size_t cols) { return (m + 15) / 16 * 16 * cols; }
 
-// workspace: the K-split partials (when split), and for a caller without row statistics and packed
-// rows those
-size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain) {
+// workspace: the K-split partials (when split), and for a caller without packed rows those and
+// their statistics
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain, bool packed) {
     const PkPlan p = pk_plan(w, m);
-    return align4(p.splits > 1 || plain ? p.splits * m * w.rows : 0) + align4(gemm_row_stats_floats(m, w.cols)) +
-           gemm_x_pack_floats(m, w.cols) + 4;
+    const size_t parts = align4(p.splits > 1 || plain ? p.splits * m * w.rows : 0);
+    return packed ? parts + 4 : parts + align4(gemm_row_stats_floats(m, w.cols)) + gemm_x_pack_floats(m, w.cols) + 4;
 }
 
 size_t gemm_row_stats_floats(size_t m, size_t cols) { return m + 4 + m * (cols / 32); }
@@ -723,7 +723,7 @@ void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, flo
     if (q4k_gemm_above_2gib(w, m)) fail(LARQL_HIP_ERR_UNSUPPORTED, "f32 GEMM: operands above 2 GiB");
     const PkPlan p = pk_plan(w, m);
     if (plain && (w.format != LARQL_Q4_K || defer)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: plain sums of Q4_K outputs only");
-    if (!part || part_floats < gemm_f32_part_floats(w, m, plain)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: workspace too small");
+    if (!part || part_floats < gemm_f32_part_floats(w, m, plain, pre && pre->xp)) fail(LARQL_HIP_ERR_INVALID, "f32 GEMM: workspace too small");
     const bool parts = p.splits > 1 || plain;  // the GEMM writes partial products, summed after it
     float* at = part + align4(parts ? p.splits * m * w.rows : 0);
     GemmRowStats st;

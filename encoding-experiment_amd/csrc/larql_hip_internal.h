@@ -289,7 +289,8 @@ struct GemmSplits {
 // operands if xp is set (for Q4_K weights with the sub-block sums).  defer: leave the split
 // partial products unsummed (ldy = w.rows).  plain (Q4_K): outputs that are not finite are summed
 // again from the f32 inputs (the packed operands of a row with an infinite element are NaN).
-size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain = false);
+// packed: the caller brings pre with xp.
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain = false, bool packed = false);
 // The row statistics and packed operands of X, in one launch where a row fits it.
 void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s);
 // Q4_K weights and batches (at most kSmallBatchMax rows) for which launch_gemm_f32 is faster than

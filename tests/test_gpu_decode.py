@@ -421,6 +421,32 @@ def test_decode_long_cache(hip, T0, hd, nq, nkv, window):
     run_sequence(hip, T0=T0, n_tokens=3, n_layers=1, hidden=512, inter=512, nq=nq, nkv=nkv, hd=hd, window=window)
 
 
+def test_prefill_work_buffer_holds_one_packed_input(hip):
+    """The work buffer of a Q4_K prompt: per position the rows of its steps, one packed input and the row
+    statistics, grown by a quarter.  A second packed input would be a fifth more."""
+    torch = pytest.importorskip("torch")
+    hidden, inter, nq, nkv, hd, seq = 256, 16384, 4, 2, 64, 2048
+    m = SmallModel(1, hidden, inter, nq, nkv, hd, cap=2, seed=92)
+    be = larql_hip.HipBackend(0, strict=True)
+    try:
+        model = be.model(m.hip_layers(10000.0), hidden, inter)
+        x = torch.randn(seq, hidden, device="cuda")
+        out = torch.empty(seq, hidden, device="cuda")
+        model.prefill_dev(x[:2], 2, out)   # the cache of 4096 positions
+        be.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        model.prefill_dev(x, seq, out)
+        be.synchronize()
+        used = free - torch.cuda.mem_get_info()[0]
+        floats = (3 * hidden + (nq + 2 * nkv) * hd + nq * hd + 2 * inter + 2 * inter + (2 * hidden + inter) // 32 + 4
+                  + 16 * hidden)   # K splits of the down projection, at most
+        print(f"[prefill buffer] {used / 2**20:.0f} MiB for {seq * floats * 4 / 2**20:.0f} MiB of rows", flush=True)
+        assert used <= 1.25 * 4 * seq * floats + (8 << 20)
+        model.close()
+    finally:
+        be.close()
+
+
 def test_prefill_wide_ffn_residual(hip):
     """An FFN wider than the row kernels hold (inter > 16384): the residual adds of a layer without
     post-norms, position by position against the oracle."""
