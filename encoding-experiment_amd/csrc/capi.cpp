@@ -298,27 +298,23 @@ extern "C" int larql_hip_q4k_matvec(larql_hip_ctx* c, const uint8_t* q4k_data, s
     });
 }
 
-// Workspace of a batch of m > 1 rows of a Q4_K weight: no less than any smaller batch's (whose K
-// splits may take more), so that it grows only with m.
-static size_t q4k_rows_ws(const DevWeight& w, size_t m) {
-    auto need = [&](size_t n) {
-        return larql::gemm_f32_small_batch(w, n) ? larql::gemm_f32_part_floats(w, n, true) * sizeof(float)
-                                                 : larql::q4k_gemm_ws_bytes(n, w.cols);
-    };
-    // (the fp16 GEMM's grows with m by itself)
-    for (; w.ws_m < std::min(m, larql::kSmallBatchMax); w.ws_m++) w.ws_bytes = std::max(w.ws_bytes, need(w.ws_m + 1));
-    return std::max(w.ws_bytes, need(m));
-}
-
 // m activation rows through a Q4_K weight: the matvec, the f32-accuracy GEMM for small batches,
-// the fp16 GEMM.
+// the fp16 GEMM.  The workspace is no less than any smaller batch's (whose K splits may take more),
+// so that it grows only with m.
 static void q4k_rows(larql_hip_ctx* c, const DevWeight& w, const float* x, float* out, size_t m, hipStream_t s) {
-    void* ws = m > 1 ? larql::ensure(c, c->gemm_x16, q4k_rows_ws(w, m)) : nullptr;
-    if (larql::gemm_f32_small_batch(w, m))
-        larql::launch_gemm_f32(w, x, out, m, static_cast<float*>(ws), larql::gemm_f32_part_floats(w, m, true), s, 0, nullptr,
-                               nullptr, true);
-    else
-        larql::launch_q4k_matvec(w, x, out, m, ws, s);
+    if (m <= 1) return larql::launch_q4k_matvec(w, x, out, m, nullptr, s);
+    // (tiles of 16 rows, whole ones kept with the weight: inside one the splits only fall with the
+    // rows, so its first batch's splits bound it; the fp16 GEMM's workspace grows with m by itself)
+    auto tile = [&](size_t t, size_t rows) {
+        return larql::gemm_f32_small_batch(w, std::max<size_t>(2, 16 * t + 1), rows) * sizeof(float);
+    };
+    const size_t n = std::min(m, larql::kSmallBatchMax);
+    for (; w.ws_tiles < n / 16; w.ws_tiles++) w.ws_bytes = std::max(w.ws_bytes, tile(w.ws_tiles, 16 * (w.ws_tiles + 1)));
+    const size_t part = larql::gemm_f32_small_batch(w, m);
+    const size_t own = std::max(part ? part * sizeof(float) : larql::q4k_gemm_ws_bytes(m, w.cols), n % 16 ? tile(n / 16, n) : 0);
+    void* ws = larql::ensure(c, c->gemm_x16, std::max(w.ws_bytes, own));
+    if (part) larql::launch_gemm_f32(w, x, out, m, static_cast<float*>(ws), part, s, 0, nullptr, nullptr, true);
+    else larql::launch_q4k_matvec(w, x, out, m, ws, s);
 }
 
 extern "C" int larql_hip_q4k_matmul(larql_hip_ctx* c, const uint8_t* q4k_data, size_t q4k_len, const float* x,

@@ -13,6 +13,7 @@
 // Two launches: x_pack_kernel writes X once as ready-made operands (1 KB per 16 tokens, k-step
 // of 32 and part), and the GEMM streams them into LDS by buffer loads that need no registers,
 // while each wave turns its own weight rows into operands in registers.
+#include <algorithm>
 #include <type_traits>
 
 #include "decode.h"
@@ -646,10 +647,12 @@ size_t gemm_x_pack_floats(size_t m, size_t cols) { return (m + 15) / 16 * 16 * c
 
 // workspace: the K-split partials (when split), and for a caller without packed rows those and
 // their statistics
-size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain, bool packed) {
-    const PkPlan p = pk_plan(w, m);
+static size_t part_floats_of(const PkPlan& p, const DevWeight& w, size_t m, bool plain, bool packed) {
     const size_t parts = align4(p.splits > 1 || plain ? p.splits * m * w.rows : 0);
     return packed ? parts + 4 : parts + align4(gemm_row_stats_floats(m, w.cols)) + gemm_x_pack_floats(m, w.cols) + 4;
+}
+size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain, bool packed) {
+    return part_floats_of(pk_plan(w, m), w, m, plain, packed);
 }
 
 size_t gemm_row_stats_floats(size_t m, size_t cols) { return m + 4 + m * (cols / 32); }
@@ -703,11 +706,12 @@ void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowS
 // tokens 22.6 against 39.5 us, 64 tokens 41 against 42, 96 tokens 49 against 45; [4096 x 14336]:
 // 6 tokens 30 against 125, 192 tokens 83 against 145; [10240 x 2560]: 32 tokens 22 against 28,
 // 64 tokens 31 against 28.
-bool gemm_f32_small_batch(const DevWeight& w, size_t m) {
-    if (w.format != LARQL_Q4_K || m < 2 || m > kSmallBatchMax || q4k_gemm_above_2gib(w, m)) return false;
+size_t gemm_f32_small_batch(const DevWeight& w, size_t m, size_t rows) {
+    if (w.format != LARQL_Q4_K || m < 2 || m > kSmallBatchMax || q4k_gemm_above_2gib(w, m)) return 0;
     const size_t wgs = ((w.rows_pad / 16 + 4) / 5) * ((m + 255) / 256), cus = static_cast<size_t>(current_device_cus());
     const double other = 6500.0 + static_cast<double>((wgs + cus - 1) / cus) * static_cast<double>(w.cols / 256) * 2200.0;
-    return 1.45 * pk_plan(w, m).ns + 8000.0 < other;
+    const PkPlan p = pk_plan(w, m);
+    return 1.45 * p.ns + 8000.0 < other ? part_floats_of(p, w, std::max(m, rows), true, false) : 0;
 }
 
 void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,

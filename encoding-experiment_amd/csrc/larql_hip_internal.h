@@ -77,8 +77,8 @@ struct DevWeight {
     size_t host_len = 0;
     uint64_t host_fp = 0;    // sampled content fingerprint of the host bytes
     uint64_t handle = 0;
-    // the largest workspace of this weight's batches of up to ws_m rows (Q4_K, q4k_rows)
-    mutable size_t ws_m = 1, ws_bytes = 0;
+    // the workspace of this weight's batches of up to 16 ws_tiles rows (Q4_K, q4k_rows)
+    mutable size_t ws_tiles = 0, ws_bytes = 0;
 };
 
 // FNV-1a over the whole buffer when it is small, else over 64 evenly spaced
@@ -293,10 +293,10 @@ struct GemmSplits {
 size_t gemm_f32_part_floats(const DevWeight& w, size_t m, bool plain = false, bool packed = false);
 // The row statistics and packed operands of X, in one launch where a row fits it.
 void launch_gemm_pack_rows(const float* X, size_t m, size_t cols, const GemmRowStats& st, hipStream_t s);
-// Q4_K weights and batches (at most kSmallBatchMax rows) for which launch_gemm_f32 is faster than
-// launch_q4k_gemm.
+// Q4_K weights and batches (at most kSmallBatchMax rows) for which launch_gemm_f32 (plain) is faster
+// than launch_q4k_gemm: its workspace (for `rows` rows in the same K splits, if more), else 0.
 constexpr size_t kSmallBatchMax = 512;
-bool gemm_f32_small_batch(const DevWeight& w, size_t m);
+size_t gemm_f32_small_batch(const DevWeight& w, size_t m, size_t rows = 0);
 void launch_gemm_f32(const DevWeight& w, const float* X, float* Y, size_t m, float* part, size_t part_floats,
                      hipStream_t s, size_t ldy = 0, const GemmRowStats* pre = nullptr, GemmSplits* defer = nullptr,
                      bool plain = false);
