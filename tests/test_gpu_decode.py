@@ -413,11 +413,17 @@ def test_prefill_q8_q4_0_attention_options(hip, qk_norm, softcap):
 
 
 @pytest.mark.parametrize("T0,hd,nq,nkv,window", [(4094, 64, 8, 8, 0), (4160, 64, 8, 8, 0), (8300, 32, 16, 8, 0),
-                                                 (9000, 96, 8, 8, 8500), (4500, 128, 16, 16, 0)])
+                                                 (9000, 96, 8, 8, 8500), (4500, 128, 16, 16, 0),
+                                                 (4200, 128, 32, 8, 0), (8300, 256, 8, 4, 0), (4160, 32, 64, 8, 0),
+                                                 (4300, 64, 48, 8, 0), (8300, 320, 8, 4, 0), (4200, 512, 8, 8, 0),
+                                                 (2175, 128, 4, 2, 0), (2300, 256, 4, 2, 0), (2300, 512, 2, 1, 0),
+                                                 (4500, 384, 2, 1, 0)])
 def test_decode_long_cache(hip, T0, hd, nq, nkv, window):
     """Positions from which an attention workgroup takes more than one 64-position chunk (4096 on
     at 8 kv heads, 2048 at 16): the last position with one, a first chunk of the next pair, a last
-    workgroup with fewer chunks than the others, a window that starts inside a chunk."""
+    workgroup with fewer chunks than the others, a window that starts inside a chunk; four, six and
+    eight query heads per kv head (several heads per wave), head_dim 256 and above; and merges of
+    34 and 35 splits (added by one group of threads, by several) and of more with one or two groups."""
     run_sequence(hip, T0=T0, n_tokens=3, n_layers=1, hidden=512, inter=512, nq=nq, nkv=nkv, hd=hd, window=window)
 
 

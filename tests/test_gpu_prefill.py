@@ -148,14 +148,17 @@ def _q4k_values(b, rows, cols):
                                          (4096, 8192, 48), (130, 4352, 64), (64, 17408, 5), (14336, 4096, 6)])
 def test_q4k_small_batch_rows(hip, rows, cols, m):
     """Small batches of Q4_K (matvec_dev, the f32-accuracy GEMM): every output against the f64
-    product of the dequantized weights, within 1e-5 of the row's largest (f32 sums: 2^-24 per term,
-    random signs, K <= 17408 -> ~1e-6).  One token scaled by 1e6 and one by 1e-20 (each row has its
+    product of the dequantized weights.  One token scaled by 1e6 and one by 1e-20 (each row has its
     own power of two), and super-blocks with a minimum scale of 300, past the range of the usual
-    fp16 minimum operand."""
+    fp16 minimum operand.  The weight rows with such a block and the others are compared apart, each
+    with the rms of its own outputs: 4e-6 (an error of 2.3e-7 of the norm, normal over up to 14336
+    outputs, and f32 sums; for the former, whose outputs are the few large minima, 1e-5)."""
     torch = pytest.importorskip("torch")
     print(f"[q4k small] rows={rows} cols={cols} m={m}", flush=True)
     b = oracle.quantize_q4_k(oracle.gauss(95, rows * cols, 0.0, 0.02)).reshape(-1, 148).copy()
     b[5::97, 2:4] = np.array([300.0], np.float16).view(np.uint8)
+    large = np.zeros(rows, bool)
+    large[np.arange(5, rows * (cols // 256), 97) // (cols // 256)] = True
     x = oracle.gauss(96, m * cols).reshape(m, cols).copy()
     x[0] *= np.float32(1e6)
     x[m - 1] *= np.float32(1e-20)
@@ -167,9 +170,11 @@ def test_q4k_small_batch_rows(hip, rows, cols, m):
         hip.synchronize()
         got = dy.cpu().numpy().reshape(m, rows).astype(np.float64)
         ref = x.astype(np.float64) @ _q4k_values(b, rows, cols).T
-        e = np.max(np.abs(got - ref), 1) / np.max(np.abs(ref), 1)
-        print(f"  worst row {np.max(e):.2e}", flush=True)
-        assert np.max(e) <= 1e-5
+        assert not np.all(large)
+        for which, bar in ((~large, 4e-6), (large, 1e-5)):
+            e = np.max(np.abs(got - ref)[:, which], 1) / np.sqrt(np.mean(ref[:, which] ** 2, 1))
+            print(f"  {which.sum()} weight rows: {np.max(e):.2e}", flush=True)
+            assert np.max(e) <= bar
     finally:
         hip.release_weight(h)
 
