@@ -374,35 +374,35 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
         qop[i] = op;
     }
     auto new_row = [&]() __attribute__((always_inline)) {
-    if (owner) {
-        if (fresh && t0 + 16 * wave + c == pos) {
+        if (owner) {
+            if (fresh && t0 + 16 * wave + c == pos) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) cur.k[ks] = *reinterpret_cast<const v4u*>(&knew[32 * ks + 8 * g]);
-        }
-        // the block holding pos: the new value at pos (prompt mode: the cached one), zeros
-        // above it (beyond this query)
+                for (int ks = 0; ks < KS; ks++) cur.k[ks] = *reinterpret_cast<const v4u*>(&knew[32 * ks + 8 * g]);
+            }
+            // the block holding pos: the new value at pos (prompt mode: the cached one), zeros
+            // above it (beyond this query)
 #pragma unroll
-        for (int i = 0; i < DTW; i++) {
-            const int dt = wave + 4 * i;
+            for (int i = 0; i < DTW; i++) {
+                const int dt = wave + 4 * i;
 #pragma unroll
-            for (int ts = 0; ts < 2; ts++) {
-                const int tv = t0 + 32 * ts + 8 * g;
-                if (dt < NDT && tv <= pos && pos < tv + 8) {
-                    const int e = pos - tv;
-                    const bool sub = fresh;
-                    const uint32_t vn = sub ? vnew[16 * dt + c] : 0u;
+                for (int ts = 0; ts < 2; ts++) {
+                    const int tv = t0 + 32 * ts + 8 * g;
+                    if (dt < NDT && tv <= pos && pos < tv + 8) {
+                        const int e = pos - tv;
+                        const bool sub = fresh;
+                        const uint32_t vn = sub ? vnew[16 * dt + c] : 0u;
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const uint32_t w = cur.v[i][ts][k];
-                        const uint32_t lo = 2 * k < e ? (w & 0xFFFFu)
-                                                      : (2 * k == e ? (sub ? vn : (w & 0xFFFFu)) : 0u);
-                        const uint32_t hi = 2 * k + 1 < e ? (w >> 16) : (2 * k + 1 == e ? (sub ? vn : (w >> 16)) : 0u);
-                        cur.v[i][ts][k] = lo | (hi << 16);
+                        for (int k = 0; k < 4; k++) {
+                            const uint32_t w = cur.v[i][ts][k];
+                            const uint32_t lo = 2 * k < e ? (w & 0xFFFFu)
+                                                          : (2 * k == e ? (sub ? vn : (w & 0xFFFFu)) : 0u);
+                            const uint32_t hi = 2 * k + 1 < e ? (w >> 16) : (2 * k + 1 == e ? (sub ? vn : (w >> 16)) : 0u);
+                            cur.v[i][ts][k] = lo | (hi << 16);
+                        }
                     }
                 }
             }
         }
-    }
     };
     floatx4 oacc[DTW];  // MULTI: the chunks' sums so far
 #pragma unroll
@@ -412,82 +412,84 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     lds_barrier();
     Kv nxt;
     for (int ci = 0;; ci++) {
-    if constexpr (MULTI) {  // the next chunk's rows (past the last: rows it has, unused) meanwhile
-        load_kv(t0 + kAttnChunk, nxt);
-    }
+        if constexpr (MULTI) {
+            // the next chunk's rows meanwhile (in a workgroup's last turn the next workgroup's first
+            // ones, or where there is none rows it has: not used)
+            load_kv(t0 + kAttnChunk, nxt);
+        }
 
-    // 2. Scores of positions t0 + 16 w + 4 g + r for lanes (g, col < reps).
-    floatx4 sacc = {0.f, 0.f, 0.f, 0.f};
+        // 2. Scores of positions t0 + 16 w + 4 g + r for lanes (g, col < reps).
+        floatx4 sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++)
-        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.k[ks]),
-                                                      __builtin_bit_cast(half8, qop[ks * 64 + lane]), sacc, 0, 0, 0);
-    sacc = add_lane_plus(sacc, reps);
-    if (c < reps) {
+        for (int ks = 0; ks < KS; ks++)
+            sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.k[ks]),
+                                                          __builtin_bit_cast(half8, qop[ks * 64 + lane]), sacc, 0, 0, 0);
+        sacc = add_lane_plus(sacc, reps);
+        if (c < reps) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int tl = 16 * wave + 4 * g + r, t = t0 + tl;
-            float sv = sacc[r] * a.scale;
-            if (a.softcap > 0.f) sv = tanhf(sv / a.softcap) * a.softcap;
-            p_s[c][tl] = (t >= a.t_begin && t <= pos) ? sv : -INFINITY;
+            for (int r = 0; r < 4; r++) {
+                const int tl = 16 * wave + 4 * g + r, t = t0 + tl;
+                float sv = sacc[r] * a.scale;
+                if (a.softcap > 0.f) sv = tanhf(sv / a.softcap) * a.softcap;
+                p_s[c][tl] = (t >= a.t_begin && t <= pos) ? sv : -INFINITY;
+            }
         }
-    }
-    lds_barrier();
-    // 3. Softmax partials of the chunk: one wave per head.  MULTI: relative to the largest score so
-    // far, with the factor that takes the sums so far there.
-    for (int h = wave; h < reps; h += kAttnThreads / 64) {
-        const float sc = p_s[h][lane];
-        float m = wave_max_dpp(sc), al = 0.f;
-        if constexpr (MULTI) {
-            const float m0 = ml_s[2 * h];
-            m = fmaxf(m, m0);
-            al = m0 == -INFINITY ? 0.f : expf(m0 - m);
+        lds_barrier();
+        // 3. Softmax partials of the chunk: one wave per head.  MULTI: relative to the largest score so
+        // far, with the factor that takes the sums so far there.
+        for (int h = wave; h < reps; h += kAttnThreads / 64) {
+            const float sc = p_s[h][lane];
+            float m = wave_max_dpp(sc), al = 0.f;
+            if constexpr (MULTI) {
+                const float m0 = ml_s[2 * h];
+                m = fmaxf(m, m0);
+                al = m0 == -INFINITY ? 0.f : expf(m0 - m);
+            }
+            const float p = sc == -INFINITY ? 0.f : expf(sc - m);
+            float l = wave_sum_dpp(p);
+            if constexpr (MULTI) l = fmaf(ml_s[2 * h + 1], al, l);
+            p_s[h][lane] = p;
+            if (lane == 0) {
+                ml_s[2 * h] = m;
+                ml_s[2 * h + 1] = l;
+                if constexpr (MULTI) alpha_s[h] = al;
+            }
         }
-        const float p = sc == -INFINITY ? 0.f : expf(sc - m);
-        float l = wave_sum_dpp(p);
-        if constexpr (MULTI) l = fmaf(ml_s[2 * h + 1], al, l);
-        p_s[h][lane] = p;
-        if (lane == 0) {
-            ml_s[2 * h] = m;
-            ml_s[2 * h + 1] = l;
-            if constexpr (MULTI) alpha_s[h] = al;
+        lds_barrier();
+        // P.V B operands: lane (g, col) of position step ts holds positions 32 ts + 8 g ..
+        if (tid < 2 * 64) {
+            const int ts = tid >> 6, lg = (tid >> 4) & 3, col = tid & 15;
+            v4u op = {0u, 0u, 0u, 0u};
+            if (col < 2 * reps) {
+                const int h = col < reps ? col : col - reps;
+                op = split8(&p_s[h][32 * ts + 8 * lg], col >= reps);
+            }
+            pop[tid] = op;
         }
-    }
-    lds_barrier();
-    // P.V B operands: lane (g, col) of position step ts holds positions 32 ts + 8 g ..
-    if (tid < 2 * 64) {
-        const int ts = tid >> 6, lg = (tid >> 4) & 3, col = tid & 15;
-        v4u op = {0u, 0u, 0u, 0u};
-        if (col < 2 * reps) {
-            const int h = col < reps ? col : col - reps;
-            op = split8(&p_s[h][32 * ts + 8 * lg], col >= reps);
-        }
-        pop[tid] = op;
-    }
-    lds_barrier();
-    // 4. Unnormalised P.V: dims 16 dt + 4 g + r for lanes (g, col < reps).
+        lds_barrier();
+        // 4. Unnormalised P.V: dims 16 dt + 4 g + r for lanes (g, col < reps).
 #pragma unroll
-    for (int i = 0; i < DTW; i++) {
-        const int dt = wave + 4 * i;
-        if (dt >= NDT) break;
-        floatx4 o = {0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < DTW; i++) {
+            const int dt = wave + 4 * i;
+            if (dt >= NDT) break;
+            floatx4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ts = 0; ts < 2; ts++)
-            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.v[i][ts]),
-                                                       __builtin_bit_cast(half8, pop[ts * 64 + lane]), o, 0, 0, 0);
-        o = add_lane_plus(o, reps);
-        if constexpr (MULTI) {
-            const float al = alpha_s[min(c, reps - 1)];
+            for (int ts = 0; ts < 2; ts++)
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, cur.v[i][ts]),
+                                                           __builtin_bit_cast(half8, pop[ts * 64 + lane]), o, 0, 0, 0);
+            o = add_lane_plus(o, reps);
+            if constexpr (MULTI) {
+                const float al = alpha_s[min(c, reps - 1)];
 #pragma unroll
-            for (int r = 0; r < 4; r++) o[r] = fmaf(oacc[i][r], al, o[r]);
+                for (int r = 0; r < 4; r++) o[r] = fmaf(oacc[i][r], al, o[r]);
+            }
+            oacc[i] = o;
         }
-        oacc[i] = o;
-    }
-    if (!MULTI || ci + 1 == nc || t0 + kAttnChunk > pos) break;
-    t0 += kAttnChunk;
-    owner = pos < t0 + kAttnChunk;
-    cur = nxt;
-    new_row();
+        if (!MULTI || ci + 1 == nc || t0 + kAttnChunk > pos) break;
+        t0 += kAttnChunk;
+        owner = pos < t0 + kAttnChunk;
+        cur = nxt;
+        new_row();
     }
 #pragma unroll
     for (int i = 0; i < DTW; i++) {

@@ -28,11 +28,11 @@ namespace {
 constexpr int kThreads = 256;
 
 // ── f32 scores ─────────────────────────────────────────────────────────────
-// A lane owns NF features and walks k in order, so a score is one fma chain held in one
+// A lane owns a feature and walks k in order, so a score is one fma chain held in one
 // register; a wave serves QW queries, whose values at one k come as scalar operands
 // (read through the scalar cache as they lie: one v_fmac_f32 v, s, v per term and no LDS traffic for
-// the queries).  The gate rows are staged by global_load_lds: 64 NF rows x 32 k
-// per stage, a ring of ND stages, whole 128-byte lines per row, no registers in flight.
+// the queries).  The gate rows are staged by global_load_lds: 64 rows x 32 k
+// per stage, a ring of kF32Ring stages, whole 128-byte lines per row, no registers in flight.
 // Chunk j (4 k) of row r sits in slot j ^ (r & 7) of the row's eight, so eight consecutive
 // lanes reading the same chunk of their rows touch eight different bank groups.  The NW
 // waves of a workgroup share the staged rows and serve QW queries each.
@@ -40,7 +40,7 @@ constexpr int kThreads = 256;
 // against 4.8 ms in a 64 x 256 tile that computes 256 queries whatever their number), the
 // scalar loads' latency and fp32 VALU issue for more: 608 us for 2, 700 for 8, 1.15 ms for 32,
 // 1.86 for 64, 3.46 for 128.
-constexpr int kF32Stage = 32;
+constexpr int kF32Stage = 32, kF32Ring = 4;
 
 // XT[b][k][QW] = the QW queries of block b at k: X[QW b + i][k] for existing queries and k < K, else +0 (b < Qp / QW, k < Kp).
 __global__ void queries_t_kernel(const float* __restrict__ X, float* __restrict__ XT, int Q,
@@ -76,11 +76,11 @@ __device__ __forceinline__ void ring_read4(uint32_t a, floatx4_t (&v)[4]) {
         : "memory");
 }
 
-template <int QW, int NF, int NW, int ND, bool XT>
+template <int QW, int NW, bool XT>
 __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, const float* __restrict__ X,
                                                                   float* __restrict__ S, int F, int K, int Q) {
-    constexpr int kRows = 64 * NF, kPer = 8 * NF / NW;  // rows per stage; load instructions per wave and stage
-    static_assert(kPer * NW == 8 * NF, "the waves split a stage's loads evenly");
+    constexpr int kRows = 64, kPer = 8 / NW, ND = kF32Ring;  // rows per stage; load instructions per wave and stage
+    static_assert(kPer * NW == 8, "the waves split a stage's loads evenly");
     __shared__ __align__(128) float4 ring[ND][kRows * 8];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // (waves past the last query repeat the last QW of the Q >= QW, the same scores again; XT: padding)
@@ -107,11 +107,9 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
     const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
         (__attribute__((address_space(3))) void*)&ring[0][0]));
     const uint32_t mine = ring0 + 128u * lane + 16u * (lane & 7);
-    float acc[NF][QW];
+    float acc[QW];
 #pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-        for (int q = 0; q < QW; q++) acc[f][q] = 0.f;
+    for (int q = 0; q < QW; q++) acc[q] = 0.f;
 
     const int ns = (K + kF32Stage - 1) / kF32Stage, last = ns - 1;
 #pragma unroll
@@ -122,21 +120,18 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
     // 16 k of the stage in slot `slot`
     auto half = [&](int k0, auto hc) __attribute__((always_inline)) {
         constexpr int H = decltype(hc)::value;
+        floatx4_t r[4];
+        ring_read4<H>(mine + static_cast<uint32_t>(slot) * (kRows * 128u), r);
+        float v[16];
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            floatx4_t r[4];
-            ring_read4<H>(mine + static_cast<uint32_t>(slot) * (kRows * 128u) + 8192u * f, r);
-            float v[16];
+        for (int i = 0; i < 16; i++) v[i] = r[i >> 2][i & 3];
+        if constexpr (XT) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) v[i] = r[i >> 2][i & 3];
-            if constexpr (XT) {
+            for (int i = 0; i < 16; i++)
 #pragma unroll
-                for (int i = 0; i < 16; i++)
-#pragma unroll
-                    for (int q = 0; q < QW; q++) acc[f][q] = fmaf(v[i], xq[static_cast<size_t>(k0 + 16 * H + i) * QW + q], acc[f][q]);
-            } else {
-                lane_fma16<QW>(acc[f], v, xq, K, k0 + 16 * H);
-            }
+                for (int q = 0; q < QW; q++) acc[q] = fmaf(v[i], xq[static_cast<size_t>(k0 + 16 * H + i) * QW + q], acc[q]);
+        } else {
+            lane_fma16<QW>(acc, v, xq, K, k0 + 16 * H);
         }
     };
     for (int st = 0; st < ns; st++) {
@@ -151,14 +146,10 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
     }
     wait_vmcnt<0>();  // nothing may land in LDS after the workgroup has ended
     float* Sl = S + static_cast<size_t>(l) * Q * F;
+    if (f0 + lane >= F) return;
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-        const int fo = f0 + 64 * f + lane;
-        if (fo >= F) continue;
-#pragma unroll
-        for (int q = 0; q < QW; q++)
-            if (!XT || q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + fo] = acc[f][q];
-    }
+    for (int q = 0; q < QW; q++)
+        if (!XT || q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + f0 + lane] = acc[q];
 }
 
 // More than 128 queries: the chains are bound by fp32 VALU issue and the scalar operands of the
@@ -1050,11 +1041,10 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
         launch_pad_rows_f32(X, ws, static_cast<size_t>(Q), static_cast<size_t>(K), static_cast<size_t>(Kp), 0.0f, s);
         X = ws;
     }
-    auto go = [&](auto qw, auto nf, auto nw, auto nd, auto tr) {
-        constexpr int QW = decltype(qw)::value, NF = decltype(nf)::value, NW = decltype(nw)::value,
-                      ND = decltype(nd)::value;
-        const dim3 grid((F + 64 * NF - 1) / (64 * NF), gy, n_layers);
-        gate_scores_f32_kernel<QW, NF, NW, ND, decltype(tr)::value><<<grid, dim3(64 * NW), 0, s>>>(g, X, S, F, Kp, Q);
+    auto go = [&](auto qw, auto nw, auto tr) {
+        constexpr int QW = decltype(qw)::value, NW = decltype(nw)::value;
+        gate_scores_f32_kernel<QW, NW, decltype(tr)::value>
+            <<<dim3((F + 63) / 64, gy, n_layers), dim3(64 * NW), 0, s>>>(g, X, S, F, Kp, Q);
     };
     using std::integral_constant;
     const integral_constant<int, 1> c1;
@@ -1069,18 +1059,18 @@ void launch_gate_scores_f32(const KnnLayers& g, int n_layers, const float* X, fl
         if (xt) gate_scores_f32_tile_kernel<true><<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
         else gate_scores_f32_tile_kernel<false><<<grid, dim3(kThreads), 0, s>>>(g, X, S, F, Kp, Q);
     } else if (p.nw == 1) {
-        if (p.qw == 1) go(c1, c1, c1, c4, direct);
-        else go(c2, c1, c1, c4, direct);
+        if (p.qw == 1) go(c1, c1, direct);
+        else go(c2, c1, direct);
     } else if (p.qw == 2) {
-        if (p.nw == 2) go(c2, c1, c2, c4, direct);
-        else go(c2, c1, c4, c4, direct);
+        if (p.nw == 2) go(c2, c2, direct);
+        else go(c2, c4, direct);
     } else if (p.qw == 4) {
-        if (p.nw == 4) go(c4, c1, c4, c4, direct);
-        else go(c4, c1, c8, c4, direct);
+        if (p.nw == 4) go(c4, c4, direct);
+        else go(c4, c8, direct);
     } else {
-        if (p.qw == 8 && xt) go(c8, c1, c8, c4, kmajor);
-        else if (p.qw == 8) go(c8, c1, c8, c4, direct);
-        else go(c16, c1, c8, c4, kmajor);
+        if (p.qw == 8 && xt) go(c8, c8, kmajor);
+        else if (p.qw == 8) go(c8, c8, direct);
+        else go(c16, c8, kmajor);
     }
     LARQL_HIP_CHECK(hipGetLastError());
 }
