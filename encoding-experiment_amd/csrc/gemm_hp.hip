@@ -146,8 +146,8 @@ struct PkArgs {
     int M, N, K, ntiles, mtiles, sb_per, ldy, gx, gy, gz;
 };
 
-// Measured, Q4_K [28672 x 4096] (kernel trace): 512 tokens 258 us (466
-// TFLOP/s; 311 us when each workgroup split f32 tokens into pairs itself and one wave per SIMD
+// Measured, Q4_K [28672 x 4096] (kernel trace): 512 tokens 242-250 us (481-497
+// TFLOP/s; MFMA busy 46% of the cycles, VALU 18%, 1.5 waves per SIMD; 311 us when each workgroup split f32 tokens into pairs itself and one wave per SIMD
 // waited for its own loads and LDS reads), 24 tokens 30 us (the call 83 us on the fp16 GEMM).  The
 // codes by masks take 13 VALU per eight weights; made fp16 integers by a byte permute and an fma per
 // pair, 14 (two 8B-shape layers, 512 tokens: 1137 us against 1164; bit-identical).  Left subnormal
@@ -610,9 +610,8 @@ __global__ void sum_splits_kernel(const float* __restrict__ P, float* __restrict
 // Token tiles per workgroup (the fewest workgroups of at most four, evenly filled) and K-splits
 // (1..16, whole super-blocks each): the splits with the least modelled time, rounds of workgroups
 // over the CUs x super-blocks per workgroup, ~2.2 / 3.0 / 3.6 / 4.1 us each at 1 .. 4 token tiles
-// (two workgroups on a CU take as long as one after the other: the weights' unpacking and the
-// MFMAs fill the issue slots), plus, when split, the partial sums written and summed ((splits +
-// 1) m N floats at ~5 TB/s, and a launch).
+// (workgroups past one per CU are counted as a further round), plus, when split, the partial sums
+// written and summed ((splits + 1) m N floats at ~5 TB/s, and a launch).
 struct PkPlan {
     int tt, splits, sb_per;
     double ns;  // the modelled time of the GEMM and its sums

@@ -9,8 +9,9 @@
 // workgroup is 16 TT tokens x 64 R weight rows, wave w owning R tiles; the tokens' codes (in the
 // order the weight unpack gives) and scales are staged in LDS, four blocks per stage, the next
 // stage's loads in registers meanwhile.
-// Bound: VALU issue, the reference's four operations per (row, token, block) (conversion, two
-// products, sum): Q4_0 [14336 x 4096] 29 us at 32 tokens, 65 at 128 (230 TOP/s), against 53 and
+// Bound: the reference's four operations per (row, token, block) (conversion, two products, sum) in
+// few waves (two [14336 x 4096] at 96 rows: 34,800 VALU operations per SIMD in 196,000 cycles, 1.3
+// waves per SIMD, 11% MFMA): Q4_0 [14336 x 4096] 29 us at 32 tokens, 65 at 128 (230 TOP/s), against 53 and
 // 204 us in passes of eight tokens that each stream the weights; the two matrices of a walk FFN
 // layer at 96 tokens 82 us.
 #include <type_traits>
@@ -264,7 +265,7 @@ bool int_gemm_takes(const DevWeight& w) {
 
 namespace {
 // Token tiles and weight tiles per wave: the least modelled time, rounds of workgroups over
-// the CUs times a workgroup's VALU issue per block (16 per 16 x 16 tile, ~12 to unpack a
+// the CUs times a workgroup's VALU operations per block (16 per 16 x 16 tile, ~12 to unpack a
 // weight tile, ~30 of loop, staging and waits)
 struct IgPlan {
     int TT, R;

@@ -1006,7 +1006,7 @@ __global__ __launch_bounds__(1024) void q4_0_f32_mv_kernel(const uint8_t* __rest
 // q in bit-reversed order, so that the shuffles' tree is two adds inside the four and a four-deep
 // stack of partial sums.  Weight row = operand A (output rows 4 g + r of lane (g, c)), x = operand B
 // (column c): lane (b, i) holds block b of weight row i and of x row i.
-// Bound: MFMA issue (8 passes each) and the VALU between: [4096 x 14336], 96 rows 167 us, of which the
+// Bound: MFMA issue (8 passes each) and the VALU between: [4096 x 14336], 96 rows 165 us, of which the
 // MFMAs are 78 and the VALU 62 (counters), against 306 us with a lane per block, an f32 fma per
 // weight and the shuffles, and 96 launches of the matvec for a row each; 271 us with x read as it lies
 // (16 bytes of each of 64 lines per load).
