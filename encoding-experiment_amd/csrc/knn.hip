@@ -146,10 +146,11 @@ __global__ __launch_bounds__(64 * NW) void gate_scores_f32_kernel(KnnLayers g, c
     }
     wait_vmcnt<0>();  // nothing may land in LDS after the workgroup has ended
     float* Sl = S + static_cast<size_t>(l) * Q * F;
-    if (f0 + lane >= F) return;
+    const int f = f0 + lane;
+    if (f >= F) return;
 #pragma unroll
     for (int q = 0; q < QW; q++)
-        if (!XT || q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + f0 + lane] = acc[q];
+        if (!XT || q0 + q < Q) Sl[static_cast<size_t>(q0 + q) * F + f] = acc[q];
 }
 
 // More than 128 queries: the chains are bound by fp32 VALU issue and the scalar operands of the
