@@ -207,6 +207,12 @@ def test_decode_head_geometries(hip, nq, nkv, hd, T0):
     run_sequence(hip, T0=T0, n_tokens=2, n_layers=1, nq=nq, nkv=nkv, hd=hd, hidden=512, inter=512)
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(4, 2, 64), (8, 2, 128), (4, 1, 256), (4, 1, 512)])
+def test_decode_merge_run_lengths(hip, nq, nkv, hd):
+    # 16 and 17 splits of 64 positions: the last of the short merge and the first of the long
+    run_sequence(hip, T0=1023, n_tokens=2, n_layers=1, nq=nq, nkv=nkv, hd=hd, hidden=512, inter=512)
+
+
 # per-layer head geometry: a head_dim-512 layer with one kv head between 128- and 64-wide
 # ones (Gemma-4's global layers, LC/src/pipeline.rs:100-101)
 MIXED_GEOMS = [(8, 4, 128), (4, 1, 512), (8, 2, 64)]
